@@ -58,7 +58,6 @@ def kernel_bytes(nb, n, g, V, exch_elems):
     I = n ** 3
     F = (n + 1) * n * n
     RU = I + 18 * n * n
-    recon = 8 * V * nb * (RU + 6 * (n + 2) * n * n)
     # plane kernels: part 0 reads every cell its stencils touch (interior + 3 ghost layers)
     # and writes the 3 face-flux arrays; the ghost-free part reads the interior only and writes
     # the faces between cells 3 .. n - 2 of each row; the boundary part reads the cells within
@@ -73,10 +72,7 @@ def kernel_bytes(nb, n, g, V, exch_elems):
         "recon_flux_inner": 8 * V * nb * (I + 3 * inner_faces),
         "recon_flux_outer": 8 * V * nb * (outer_cells + 3 * 6 * n * n),
         "flux_update": 8 * nb * (3 * V * F + 3 * V * I + I),
-        "recon": recon,
-        "recon_tasks": recon,
-        "fused_update": 8 * nb * (6 * V * F + 3 * V * I + I),
-        "hll_flux": 8 * V * nb * 9 * F,
+        "fluxes": 8 * V * nb * (RU + 3 * F),
         "flux_div": 8 * V * nb * (3 * F + I),
         "weighted_sum": 8 * V * nb * 3 * E,
         "derived": 8 * nb * 5 * I,

@@ -223,8 +223,8 @@ void Mesh::Adopt(Mesh &nm) {
   std::swap(channel_offset, nm.channel_offset);
   std::swap(geom, nm.geom);
   std::swap(coef, nm.coef);
-  std::swap(face, nm.face);
-  std::swap(face_V, nm.face_V);
+  std::swap(flux_scratch, nm.flux_scratch);
+  std::swap(flux_scratch_n, nm.flux_scratch_n);
   std::swap(graph, nm.graph);
   std::swap(graph_exec, nm.graph_exec);
   std::swap(scratch, nm.scratch);

@@ -1,9 +1,9 @@
 // Burgers benchmark (Parthenon-VIBE) stage kernels for gfx950, FP64.
 //
 // Task-level kernels, one launch per reference task over every block of the MeshData:
-//   ReconKernel      burgers_package::CalculateFluxes, reconstruction part
-//                    (benchmarks/burgers/burgers_package.cpp:236-303, recon.hpp:28-99)
-//   FluxKernel       the HLL part (burgers_package.cpp:307-401, burgers_package.hpp:33-43)
+//   FluxTaskKernel   burgers_package::CalculateFluxes: reconstruction
+//                    (benchmarks/burgers/burgers_package.cpp:236-303, recon.hpp:28-99) and HLL
+//                    (burgers_package.cpp:307-401, burgers_package.hpp:33-43)
 //   FluxDivKernel    Update::FluxDivergence (src/interface/update.cpp:63-84, update.hpp:43-57)
 //   WsumKernel       Update::WeightedSumData (src/interface/update.hpp:71-90)
 //   DerivedKernel    burgers_package::CalculateDerived (burgers_package.cpp:143-167)
@@ -29,106 +29,122 @@ namespace {
 
 constexpr int kWG = 256;
 
-// One thread per (block, comp, k, j, i) of the box extended by one cell around the interior.
-// face layout: [6][block][comp][k][j][i] for Ulx, Urx, Uly, Ury, Ulz, Urz.
-__global__ void __launch_bounds__(kWG)
-    ReconKernel(const double *__restrict__ U, double *__restrict__ face, Geo G, int nblocks,
-                int recon) {
-  const int dk = G.ndim > 2 ? 1 : 0, dj = G.ndim > 1 ? 1 : 0;
-  const int b0 = G.hi0 - G.lo0 + 3, b1 = G.hi1 - G.lo1 + 1 + 2 * dj,
-            b2 = G.hi2 - G.lo2 + 1 + 2 * dk;
-  const std::int64_t per = static_cast<std::int64_t>(b0) * b1 * b2;
-  const std::int64_t total = per * G.V * nblocks;
-  const std::int64_t slab = G.cells * G.V * nblocks;
-  for (std::int64_t t = static_cast<std::int64_t>(blockIdx.x) * kWG + threadIdx.x; t < total;
-       t += static_cast<std::int64_t>(gridDim.x) * kWG) {
-    std::int64_t r = t;
-    const int i = static_cast<int>(r % b0) + G.lo0 - 1;
-    r /= b0;
-    const int j = static_cast<int>(r % b1) + G.lo1 - dj;
-    r /= b1;
-    const int k = static_cast<int>(r % b2) + G.lo2 - dk;
-    r /= b2;  // r = block * V + comp
-    const double *q = U + r * G.cells;
-    const std::int64_t c = (static_cast<std::int64_t>(k) * G.e1 + j) * G.e0 + i;
-    double *f = face + r * G.cells;
-    const bool kin = k >= G.lo2 && k <= G.hi2, jin = j >= G.lo1 && j <= G.hi1,
-               iin = i >= G.lo0 && i <= G.hi0;
-    const bool xrec = kin && jin;
-    const bool yrec = kin && (G.ndim > 1) && iin;
-    const bool zrec = jin && (G.ndim > 2) && iin;
-    const std::int64_t sj = G.e0, sk = static_cast<std::int64_t>(G.e0) * G.e1;
-    double ql, qr;
-    if (xrec) {
-      if (recon == 0)
-        Weno5Z(q[c - 2], q[c - 1], q[c], q[c + 1], q[c + 2], ql, qr);
-      else
-        LinearRecon(q[c - 1], q[c], q[c + 1], ql, qr);
-      f[0 * slab + c + 1] = ql;
-      f[1 * slab + c] = qr;
-    }
-    if (yrec) {
-      if (recon == 0)
-        Weno5Z(q[c - 2 * sj], q[c - sj], q[c], q[c + sj], q[c + 2 * sj], ql, qr);
-      else
-        LinearRecon(q[c - sj], q[c], q[c + sj], ql, qr);
-      f[2 * slab + c + sj] = ql;
-      f[3 * slab + c] = qr;
-    }
-    if (zrec) {
-      if (recon == 0)
-        Weno5Z(q[c - 2 * sk], q[c - sk], q[c], q[c + sk], q[c + 2 * sk], ql, qr);
-      else
-        LinearRecon(q[c - sk], q[c], q[c + sk], ql, qr);
-      f[4 * slab + c + sk] = ql;
-      f[5 * slab + c] = qr;
-    }
+// HLL flux of component n at one face from its left and right states and those of the normal
+// velocity (burgers_package.cpp:307-401 with lr_to_flux, burgers_package.hpp:33-43).
+__device__ __forceinline__ double HllOne(int n, double upl, double upr, double l, double r) {
+  const double sl = DMin(DMin(upl, upr), 0.0);
+  const double sr = DMax(DMax(upl, upr), 0.0);
+  const double den = sr - sl + (sl * sr == 0.0);
+  if (n < 3) {
+    const double islsr = 1.0 / den;
+    return 0.5 * (sr * l * upl - sl * r * upr + sl * sr * (r - l)) * islsr;
   }
+  return (sr * upl * l - sl * upr * r + sl * sr * (r - l)) / den;
 }
 
-// One thread per (block, k, j, i) face position; HLL velocity flux then scalar fluxes that
-// reuse the face's signal speeds. flux layout: [3][block][comp][k][j][i].
+// How FluxTaskKernel splits one block: workgroups per direction and, for y and z, faces per
+// segment of a column.
+constexpr int kSegFaces = 9;
+struct FluxSplit {
+  int wgs[3], seg[3];
+};
+
+// CalculateFluxes of any block shape in one launch, from U to the fluxes [3][block][comp][k][j][i]
+// (x-face i - 1/2 at index i): the face states stay on chip. One workgroup takes a piece of one
+// block in one direction and goes through the components one after another, the normal
+// velocity first (its face states give every component's signal speeds), so any number of
+// components fits.
+//   x: a wavefront takes 64 consecutive cells of the rows extended by one cell on each side; a
+//      lane reconstructs its cell and gets the left state of its low face from the lane below
+//      (the first lane of a wavefront repeats the last one's cell of the wavefront before);
+//   y, z: a thread marches a column segment of at most kSegFaces faces with the stencil in a
+//      register window, lanes along x; the normal velocity's states wait in LDS, each thread
+//      in its own slots (no barriers).
+// A cell is reconstructed once, but for one cell per segment or wavefront. The operations are
+// those of the reference in its order, without contraction. Bound: FP64 issue (about 300
+// instructions a reconstruction with its flux, 8 IEEE divides among them). On the 960-block
+// mesh with 7 components the reconstruction and HLL as two launches, with the states in HBM
+// between them, took 1341 + 1043 us; this kernel takes
+// 1070 us.
+template <int RECON>
 __global__ void __launch_bounds__(kWG)
-    FluxKernel(const double *__restrict__ face, double *__restrict__ flux, Geo G, int nblocks) {
-  const int dk = G.ndim > 2 ? 1 : 0, dj = G.ndim > 1 ? 1 : 0;
-  const int b0 = G.hi0 - G.lo0 + 2, b1 = G.hi1 - G.lo1 + 1 + dj, b2 = G.hi2 - G.lo2 + 1 + dk;
-  const std::int64_t per = static_cast<std::int64_t>(b0) * b1 * b2;
-  const std::int64_t total = per * nblocks;
-  const std::int64_t slab = G.cells * G.V * nblocks;
-  for (std::int64_t t = static_cast<std::int64_t>(blockIdx.x) * kWG + threadIdx.x; t < total;
-       t += static_cast<std::int64_t>(gridDim.x) * kWG) {
-    std::int64_t r = t;
-    const int i = static_cast<int>(r % b0) + G.lo0;
-    r /= b0;
-    const int j = static_cast<int>(r % b1) + G.lo1;
-    r /= b1;
-    const int k = static_cast<int>(r % b2) + G.lo2;
-    r /= b2;  // block
-    const std::int64_t c = (static_cast<std::int64_t>(k) * G.e1 + j) * G.e0 + i;
-    const std::int64_t base = r * G.V * G.cells + c;
-    const bool xflux = k <= G.hi2 && j <= G.hi1;
-    const bool yflux = G.ndim > 1 && k <= G.hi2 && i <= G.hi0;
-    const bool zflux = G.ndim > 2 && j <= G.hi1 && i <= G.hi0;
-    for (int d = 0; d < 3; ++d) {
-      const bool doit = d == 0 ? xflux : (d == 1 ? yflux : zflux);
-      if (!doit) continue;
-      const double *L = face + (2 * d) * slab + base;
-      const double *R = face + (2 * d + 1) * slab + base;
-      double *F = flux + d * slab + base;
-      const double upl = L[d * G.cells], upr = R[d * G.cells];
-      const double sl = DMin(DMin(upl, upr), 0.0);
-      const double sr = DMax(DMax(upl, upr), 0.0);
-      const double islsr = 1.0 / (sr - sl + (sl * sr == 0.0));
+    FluxTaskKernel(const double *__restrict__ U, double *__restrict__ flux, Geo G, int nblocks,
+                   FluxSplit S) {
+  __shared__ double up[2][kSegFaces][kWG];
+  // one block's workgroups are adjacent and run on one XCD: the three directions read the
+  // same cells
+  const unsigned L = XcdRemap(blockIdx.x, gridDim.x);
+  const unsigned per = S.wgs[0] + S.wgs[1] + S.wgs[2];
+  const int b = static_cast<int>(L / per);
+  int r = static_cast<int>(L % per), d = 0;
+  while (r >= S.wgs[d]) r -= S.wgs[d++];
+  const int n0 = G.hi0 - G.lo0 + 1, n1 = G.hi1 - G.lo1 + 1, n2 = G.hi2 - G.lo2 + 1;
+  const double *Ub = U + static_cast<std::int64_t>(b) * G.V * G.cells;
+  double *Fb = flux + (static_cast<std::int64_t>(d) * nblocks + b) * G.V * G.cells;
+  const int tid = static_cast<int>(threadIdx.x);
+  if (d == 0) {
+    const int m = n0 + 2, cells = m * n1 * n2;
+    const int e0 = 63 * (r * (kWG / 64) + (tid >> 6)) + (tid & 63);
+    const int e = e0 < cells ? e0 : cells - 1;
+    const int a = e % m, row = e / m;
+    const unsigned c = 8u * static_cast<unsigned>(((G.lo2 + row / n1) * G.e1 + G.lo1 + row % n1) *
+                                                      G.e0 + G.lo0 - 1 + a);
+    const bool face = a > 0 && e0 < cells && (tid & 63) > 0;
+    double upl = 0.0, upr = 0.0;
+    for (int q = 0; q <= G.V; ++q) {
+      const int n = q == 0 ? 0 : q - 1;
+      if (q == 1) continue;  // the normal velocity came first
+      double ql, qr;
+      CellStates(Ub + n * G.cells, c, 8u, RECON, ql, qr);
+      const double l = __shfl_up(ql, 1, 64);
+      if (q == 0) {
+        upl = l;
+        upr = qr;
+      }
+      if (face) StoreAt(Fb + n * G.cells, c, HllOne(n, upl, upr, l, qr));
+    }
+    return;
+  }
+  const int nd = d == 1 ? n1 : n2, len = S.seg[d];
+  const int cols = n0 * (d == 1 ? n2 : n1);
+  const int t = r * kWG + tid;
+  const int f0 = t / cols * len, f1 = f0 + len < nd + 1 ? f0 + len : nd + 1;
+  if (f0 > nd) return;
+  const int o = t % cols / n0;
+  // first face's high cell: face f of the column lies below cell f
+  const unsigned st = 8u * static_cast<unsigned>(d == 1 ? G.e0 : G.e0 * G.e1);
+  const unsigned c0 =
+      8u * static_cast<unsigned>(((G.lo2 + (d == 1 ? o : f0)) * G.e1 + G.lo1 +
+                                  (d == 1 ? f0 : o)) * G.e0 + G.lo0 + t % cols % n0);
+  for (int q = 0; q <= G.V; ++q) {
+    const int n = q == 0 ? d : q - 1;
+    if (q > 0 && n == d) continue;
+    const double *u = Ub + n * G.cells;
+    // window of the cell below the first face
+    constexpr int H = RECON == 0 ? 2 : 1;
+    double w[2 * H + 1], below = 0.0;
 #pragma unroll
-      for (int n = 0; n < 3; ++n) {
-        const double ul = L[n * G.cells], ur = R[n * G.cells];
-        F[n * G.cells] = 0.5 * (sr * ul * upl - sl * ur * upr + sl * sr * (ur - ul)) * islsr;
+    for (int x = 0; x < 2 * H; ++x) w[x] = LoadAt(u, c0 + st * static_cast<unsigned>(x - 1 - H));
+    unsigned c = c0 - st;
+    double next = LoadAt(u, c + H * st);
+    for (int f = f0 - 1; f < f1; ++f, c += st) {
+      w[2 * H] = next;
+      if (f + 1 < f1) next = LoadAt(u, c + (H + 1) * st);
+      double ql, qr;
+      if constexpr (RECON == 0)
+        Weno5Z(w[0], w[1], w[2], w[3], w[4], ql, qr);
+      else
+        LinearRecon(w[0], w[1], w[2], ql, qr);
+      if (f >= f0) {
+        if (q == 0) {
+          up[0][f - f0][tid] = below;
+          up[1][f - f0][tid] = qr;
+        }
+        StoreAt(Fb + n * G.cells, c, HllOne(n, up[0][f - f0][tid], up[1][f - f0][tid], below, qr));
       }
-      for (int n = 3; n < G.V; ++n) {
-        const double ql = L[n * G.cells], qr = R[n * G.cells];
-        F[n * G.cells] =
-            (sr * upl * ql - sl * upr * qr + sl * sr * (qr - ql)) / (sr - sl + (sl * sr == 0.0));
-      }
+      below = ql;
+#pragma unroll
+      for (int x = 0; x < 2 * H; ++x) w[x] = w[x + 1];
     }
   }
 }
@@ -242,65 +258,6 @@ __global__ void __launch_bounds__(64) MinScaleKernel(const double *__restrict__ 
 }
 
 // ---- fused stage path ----------------------------------------------------------------
-//
-// ReconTaskKernel: one thread = one WENO5Z (or linear) reconstruction of one cell in one
-// direction over one brick (block, comp). Per direction the task box
-// is the interior extended by one cell along that direction only, so every lane does the same
-// amount of work. The index work around the FP64
-// reconstruction is kept small: the brick shape is a compile-time constant for the common
-// cubic blocks (N interior cells, NG ghosts; N == 0 reads the shape at run time), the direction
-// is uniform per workgroup, and loads and stores use 32-bit byte offsets from per-workgroup
-// base pointers.
-
-template <int N, int NG, int D>
-__device__ __forceinline__ void ReconTask(const double *__restrict__ q, double *__restrict__ fl,
-                                          double *__restrict__ fr, const Geo &G, int t,
-                                          int recon) {
-  const int n0 = N ? N : G.hi0 - G.lo0 + 1, n1 = N ? N : G.hi1 - G.lo1 + 1,
-            n2 = N ? N : G.hi2 - G.lo2 + 1;
-  const int lo0 = N ? NG : G.lo0, lo1 = N ? NG : G.lo1, lo2 = N ? NG : G.lo2;
-  const int e0 = N ? N + 2 * NG : G.e0, e1 = N ? N + 2 * NG : G.e1;
-  const int m0 = n0 + (D == 0 ? 2 : 0), m1 = n1 + (D == 1 ? 2 : 0), m2 = n2 + (D == 2 ? 2 : 0);
-  if (t >= m0 * m1 * m2) return;
-  const int i = t % m0 + lo0 - (D == 0 ? 1 : 0);
-  const int r = t / m0;
-  const int j = r % m1 + lo1 - (D == 1 ? 1 : 0);
-  const int k = r / m1 + lo2 - (D == 2 ? 1 : 0);
-  const unsigned c = 8u * static_cast<unsigned>((k * e1 + j) * e0 + i);
-  const unsigned st = 8u * static_cast<unsigned>(D == 0 ? 1 : D == 1 ? e0 : e0 * e1);
-  double ql, qr;
-  if (recon == 0)
-    Weno5Z(LoadAt(q, c - 2 * st), LoadAt(q, c - st), LoadAt(q, c), LoadAt(q, c + st),
-           LoadAt(q, c + 2 * st), ql, qr);
-  else
-    LinearRecon(LoadAt(q, c - st), LoadAt(q, c), LoadAt(q, c + st), ql, qr);
-  StoreAt(fl, c + st, ql);
-  StoreAt(fr, c, qr);
-}
-
-template <int N, int NG>
-__global__ void __launch_bounds__(kWG)
-    ReconTaskKernel(const double *__restrict__ U, double *__restrict__ face, Geo G, int nblocks,
-                    int recon, unsigned per_brick) {
-  // logical workgroup = (block * V + comp) * per_brick + tile * ndim + direction; consecutive
-  // logical workgroups take the directions of one tile and run on the same XCD, so the three
-  // passes over the same cells of U meet in one L2
-  const unsigned L = XcdRemap(blockIdx.x, gridDim.x);
-  const std::int64_t bc = L / per_brick;
-  const unsigned r = L % per_brick;
-  const std::int64_t slab = G.cells * G.V * nblocks;
-  const double *q = U + bc * G.cells;
-  const int d = r % G.ndim;
-  double *fl = face + 2 * d * slab + bc * G.cells;
-  double *fr = fl + slab;
-  const int t = (r / G.ndim) * kWG + threadIdx.x;
-  if (d == 0)
-    ReconTask<N, NG, 0>(q, fl, fr, G, t, recon);
-  else if (d == 1)
-    ReconTask<N, NG, 1>(q, fl, fr, G, t, recon);
-  else
-    ReconTask<N, NG, 2>(q, fl, fr, G, t, recon);
-}
 
 // HllGen over state arrays: L, R point at component 0 of the face; component stride cs.
 template <int V>
@@ -309,118 +266,15 @@ __device__ __forceinline__ void HllFace(const double *__restrict__ L, const doub
   HllGen<V>([&](int n) { return L[n * cs]; }, [&](int n) { return R[n * cs]; }, d, F);
 }
 
-constexpr int kMaxV = 16;  // components handled by the fused update kernel
-
-// FusedUpdateKernel: one thread = one interior cell. HLL fluxes on both faces of the cell in
-// every direction, flux divergence (update.hpp:43-57), the RK averaging and update in the
-// WeightedSumData form (update.hpp:71-90, 122-137), the derived field and the per-workgroup
-// CFL minimum of the updated state; optionally writes the low-face fluxes (and the last high
-// face) for flux correction. Reads face states written by ReconTaskKernel. On multilevel
-// meshes `fover` gives per block face the correction-store image whose values replace the HLL
-// fluxes of that face (SetBounds<flxcor_recv> before FluxDivergence in the reference order).
-template <int V>
-__global__ void __launch_bounds__(kWG)
-    FusedUpdateKernel(const double *__restrict__ face, const double *U0, const double *base,
-                      double *out, double *__restrict__ derived, double *__restrict__ flux,
-                      double *__restrict__ partial, const BlockCoefs *__restrict__ coef, Geo G,
-                      int nblocks, double beta, const double *__restrict__ dtvar,
-                      const int *__restrict__ fover, const double *__restrict__ fcor) {
-  __shared__ double wmin[kWG / 64];
-  const int n0 = G.hi0 - G.lo0 + 1, n1 = G.hi1 - G.lo1 + 1, n2 = G.hi2 - G.lo2 + 1;
-  const unsigned L = XcdRemap(blockIdx.x, gridDim.x);  // = block * tiles + tile
-  const int tiles = (n0 * n1 * n2 + kWG - 1) / kWG;
-  const int b = static_cast<int>(L / tiles);
-  const int t = static_cast<int>(L % tiles) * kWG + threadIdx.x;
-  double m = DBL_MAX;
-  if (t < n0 * n1 * n2) {
-    const int i = t % n0 + G.lo0;
-    const int r = t / n0;
-    const int j = r % n1 + G.lo1;
-    const int k = r / n1 + G.lo2;
-    const std::int64_t slab = G.cells * V * nblocks;
-    const std::int64_t cs = G.cells;
-    const std::int64_t c0 = static_cast<std::int64_t>(b) * V * cs + (k * G.e1 + j) * G.e0 + i;
-    const BlockCoefs &C = coef[b];
-    const std::int64_t st[3] = {1, G.e0, static_cast<std::int64_t>(G.e0) * G.e1};
-    double du[V];
-    for (int d = 0; d < G.ndim; ++d) {
-      double Flo[V], Fhi[V];
-      const double *L = face + (2 * d) * slab + c0, *R = face + (2 * d + 1) * slab + c0;
-      HllFace<V>(L, R, cs, d, Flo);
-      HllFace<V>(L + st[d], R + st[d], cs, d, Fhi);
-      if (fover) {  // flux correction: a finer neighbour's restricted fluxes replace ours
-        const int at = d == 0 ? i - G.lo0 : d == 1 ? j - G.lo1 : k - G.lo2;
-        const int top = d == 0 ? G.hi0 - i : d == 1 ? G.hi1 - j : G.hi2 - k;
-        if (at == 0 || top == 0) {
-          const int a = d == 0 ? j - G.lo1 : i - G.lo0;
-          const int q = d == 2 ? j - G.lo1 : k - G.lo2;
-          const int rows = d == 0 ? n1 : n0;
-          const int comp = rows * (d == 2 ? n1 : n2);
-          const int olo = at == 0 ? fover[6 * b + 2 * d] : -1;
-          const int ohi = top == 0 ? fover[6 * b + 2 * d + 1] : -1;
-          if (olo >= 0)
-#pragma unroll
-            for (int n = 0; n < V; ++n) Flo[n] = fcor[olo + a + q * rows + n * comp];
-          if (ohi >= 0)
-#pragma unroll
-            for (int n = 0; n < V; ++n) Fhi[n] = fcor[ohi + a + q * rows + n * comp];
-        }
-      }
-      const double A = C.area[d];
-#pragma unroll
-      for (int n = 0; n < V; ++n) {
-        const double term = (A * Fhi[n] - A * Flo[n]);
-        du[n] = d == 0 ? term : du[n] + term;
-      }
-      if (flux) {
-        double *Fo = flux + d * slab + c0;
-#pragma unroll
-        for (int n = 0; n < V; ++n) Fo[n * cs] = Flo[n];
-        const bool last = (d == 0 && i == G.hi0) || (d == 1 && j == G.hi1) || (d == 2 && k == G.hi2);
-        if (last)
-#pragma unroll
-          for (int n = 0; n < V; ++n) Fo[n * cs + st[d]] = Fhi[n];
-      }
-    }
-    const double bdt = beta * dtvar[0];
-    const double w2 = 1.0 - beta;
-    double u1[V];
-#pragma unroll
-    for (int n = 0; n < V; ++n) {
-      const double dudt = -du[n] / C.vol;
-      const double avg = beta * U0[c0 + n * cs] + w2 * base[c0 + n * cs];
-      u1[n] = 1.0 * avg + bdt * dudt;
-      out[c0 + n * cs] = u1[n];
-    }
-    if (derived)
-      derived[static_cast<std::int64_t>(b) * cs + (k * G.e1 + j) * G.e0 + i] =
-          0.5 * u1[3] * (u1[0] * u1[0] + u1[1] * u1[1] + u1[2] * u1[2]);
-    double s = fabs(u1[0]) / C.dx[0];
-    if (G.ndim > 1) s = s + fabs(u1[1]) / C.dx[1];
-    if (G.ndim > 2) s = s + fabs(u1[2]) / C.dx[2];
-    m = 1.0 / s;
-  }
-  if (!partial) return;
-  m = WaveMin(m);
-  if ((threadIdx.x & 63) == 0) wmin[threadIdx.x >> 6] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double v = wmin[0];
-#pragma unroll
-    for (int w = 1; w < kWG / 64; ++w) v = DMin(v, wmin[w]);
-    partial[L] = v;
-  }
-}
+constexpr int kMaxV = 16;  // components handled by the update kernel
 
 // ---- plane-tiled reconstruction + HLL (cubic blocks of N <= 16 cells per side) ----------
 //
 // ReconFluxKernel: one workgroup = PPW consecutive planes of one block for one direction. For
 // each plane the WENO5Z (or linear) states of the plane's cells, extended by one cell along the
 // direction, go to LDS; then the HLL flux of every face of the plane goes to the flux array
-// [3][block][comp][brick] (x-face i at index i). The operations are those of ReconTaskKernel
-// followed by HllFace, so the fluxes are the same bits, and the face states never reach HBM:
-// the flux array is half their size and the update reads it without recomputing HLL on shared
-// faces. PPW (planes per workgroup) changes only the work split and is picked by timing.
+// [3][block][comp][brick] (x-face i at index i). The operations are those of FluxTaskKernel,
+// so the fluxes are the same bits; this form also splits off the faces that read no ghost. PPW (planes per workgroup) changes only the work split and is picked by timing.
 // PART selects the cells and faces of each plane row along the direction (ext index a of the
 // N + 2 cells lo - 1 .. hi + 1; face f between ext cells f and f + 1):
 //   0: every cell and face;
@@ -536,8 +390,10 @@ __global__ void __launch_bounds__(kWG)
   }
 }
 
-// FluxUpdateKernel: FusedUpdateKernel reading stored face fluxes instead of recomputing HLL
-// (flux divergence, RK averaging and update, derived field, CFL partial); same operations.
+// FluxUpdateKernel: one thread = one interior cell. Flux divergence (update.hpp:43-57) from
+// the stored face fluxes, the RK averaging and update in the WeightedSumData form
+// (update.hpp:71-90, 122-137), the derived field and the per-workgroup CFL minimum of the
+// updated state.
 template <int V>
 __global__ void __launch_bounds__(kWG)
     FluxUpdateKernel(const double *__restrict__ flux, const double *U0, const double *base,
@@ -599,41 +455,6 @@ __global__ void __launch_bounds__(kWG)
     for (int w = 1; w < kWG / 64; ++w) v = DMin(v, wmin[w]);
     partial[L] = v;
   }
-}
-
-// flxcor_send of the fused stage: one thread per coarse face cell of a patch evaluates the HLL
-// fluxes of its 2x2 fine faces from the fine block's face states (the values CalculateFluxes
-// would store there) and writes their restriction to the correction store.
-template <int V>
-__global__ void __launch_bounds__(64)
-    FlxcorFaceKernel(const FluxPatch *__restrict__ patches, const double *__restrict__ face,
-                     double *__restrict__ store, Geo G, int nblocks) {
-  const FluxPatch &P = patches[blockIdx.x];
-  const int t = blockIdx.y * 64 + threadIdx.x;
-  if (t >= P.n[0] * P.n[1]) return;
-  const int a = t % P.n[0], c = t / P.n[0];
-  const std::int64_t cs = G.cells, slab = G.cells * V * nblocks;
-  const std::int64_t base = static_cast<std::int64_t>(P.fine) * V * cs;
-  double F[2][2][V];
-#pragma unroll
-  for (int q = 0; q < 2; ++q)
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      if (p >= P.step[0] || q >= P.step[1]) {
-#pragma unroll
-        for (int n = 0; n < V; ++n) F[q][p][n] = 0.0;
-        continue;
-      }
-      const std::int64_t o = base + PatchFineCell(P, G, a, c, p, q);
-      HllFace<V>(face + (2 * P.d) * slab + o, face + (2 * P.d + 1) * slab + o, cs, P.d,
-                 F[q][p]);
-    }
-  const std::int64_t dst = P.dst + a + static_cast<std::int64_t>(c) * P.rows;
-#pragma unroll
-  for (int n = 0; n < V; ++n)
-    store[dst + static_cast<std::int64_t>(n) * P.comp] =
-        RestrictFace(P.d, P.area, F[0][0][n], F[0][1][n], F[1][0][n], F[1][1][n], P.step[0],
-                     P.step[1]);
 }
 
 // SendBoundBufs<flxcor_send> over stored face fluxes [dir][block][comp][brick].
@@ -794,28 +615,25 @@ int Grid(std::int64_t total) {
 
 }  // namespace
 
-pth_status BurgersRecon(const Topology &t, int V, const double *U, double *face, int recon,
-                        hipStream_t s) {
-  ProfScope prof("recon", s);
+pth_status BurgersFluxes(const Topology &t, int V, const double *U, double *flux, int recon,
+                         hipStream_t s) {
+  ProfScope prof("fluxes", s);
   const Geo G = MakeGeo(t, V);
   const int nb = static_cast<int>(t.blocks.size());
-  const int dk = G.ndim > 2 ? 1 : 0, dj = G.ndim > 1 ? 1 : 0;
-  const std::int64_t total = static_cast<std::int64_t>(G.hi0 - G.lo0 + 3) *
-                             (G.hi1 - G.lo1 + 1 + 2 * dj) * (G.hi2 - G.lo2 + 1 + 2 * dk) * V * nb;
-  hipLaunchKernelGGL(ReconKernel, dim3(Grid(total)), dim3(kWG), 0, s, U, face, G, nb, recon);
-  PTH_HIP(hipGetLastError());
-  return PTH_COMPLETE;
-}
-
-pth_status BurgersFlux(const Topology &t, int V, const double *face, double *flux,
-                       hipStream_t s) {
-  ProfScope prof("hll_flux", s);
-  const Geo G = MakeGeo(t, V);
-  const int nb = static_cast<int>(t.blocks.size());
-  const int dk = G.ndim > 2 ? 1 : 0, dj = G.ndim > 1 ? 1 : 0;
-  const std::int64_t total = static_cast<std::int64_t>(G.hi0 - G.lo0 + 2) *
-                             (G.hi1 - G.lo1 + 1 + dj) * (G.hi2 - G.lo2 + 1 + dk) * nb;
-  hipLaunchKernelGGL(FluxKernel, dim3(Grid(total)), dim3(kWG), 0, s, face, flux, G, nb);
+  const int n[3] = {t.fine.n[0], t.fine.n[1], t.fine.n[2]};
+  FluxSplit S{};
+  const int waves = ((n[0] + 2) * n[1] * n[2] - 1 + 62) / 63;
+  S.wgs[0] = (waves + kWG / 64 - 1) / (kWG / 64);
+  for (int d = 1; d < G.ndim; ++d) {
+    const int segs = (n[d] + 1 + kSegFaces - 1) / kSegFaces;
+    S.seg[d] = (n[d] + 1 + segs - 1) / segs;
+    S.wgs[d] = (n[0] * n[3 - d] * segs + kWG - 1) / kWG;
+  }
+  const dim3 grid(static_cast<unsigned>(S.wgs[0] + S.wgs[1] + S.wgs[2]) * nb);
+  if (recon == 0)
+    hipLaunchKernelGGL(FluxTaskKernel<0>, grid, dim3(kWG), 0, s, U, flux, G, nb, S);
+  else
+    hipLaunchKernelGGL(FluxTaskKernel<1>, grid, dim3(kWG), 0, s, U, flux, G, nb, S);
   PTH_HIP(hipGetLastError());
   return PTH_COMPLETE;
 }
@@ -853,121 +671,9 @@ pth_status BurgersDerived(const Topology &t, int V, const double *U, double *out
   return PTH_COMPLETE;
 }
 
-pth_status BurgersReconTasks(const Topology &t, int V, const double *U, double *face, int recon,
-                             hipStream_t s) {
-  ProfScope prof("recon_tasks", s);
-  const Geo G = MakeGeo(t, V);
-  const int nb = static_cast<int>(t.blocks.size());
-  const int n0 = t.fine.n[0], n1 = t.fine.n[1], n2 = t.fine.n[2];
-  int ntask = (n0 + 2) * n1 * n2;
-  if (G.ndim > 1) ntask = std::max(ntask, n0 * (n1 + 2) * n2);
-  if (G.ndim > 2) ntask = std::max(ntask, n0 * n1 * (n2 + 2));
-  const unsigned per_brick = static_cast<unsigned>(((ntask + kWG - 1) / kWG) * G.ndim);
-  const dim3 grid(per_brick * nb * V);
-  const bool cubic = G.ndim == 3 && n0 == n1 && n1 == n2 && t.fine.g[0] == t.fine.g[1] &&
-                     t.fine.g[1] == t.fine.g[2];
-  const int g = t.fine.g[0];
-  auto run = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(kWG), 0, s, U, face, G, nb, recon, per_brick);
-  };
-  if (cubic && n0 == 16 && g == 4)
-    run(ReconTaskKernel<16, 4>);
-  else if (cubic && n0 == 16 && g == 3)
-    run(ReconTaskKernel<16, 3>);
-  else if (cubic && n0 == 32 && g == 4)
-    run(ReconTaskKernel<32, 4>);
-  else if (cubic && n0 == 8 && g == 4)
-    run(ReconTaskKernel<8, 4>);
-  else
-    run(ReconTaskKernel<0, 0>);
-  PTH_HIP(hipGetLastError());
-  return PTH_COMPLETE;
-}
-
 int FusedUpdatePartials(const Topology &t) {
   const int cells = t.fine.n[0] * t.fine.n[1] * t.fine.n[2];
   return ((cells + kWG - 1) / kWG) * static_cast<int>(t.blocks.size());
-}
-
-pth_status BurgersFusedUpdate(const Topology &t, int V, const double *face, const double *U0,
-                              const double *base, double *out, double *derived, double *flux,
-                              double *partial, const BlockCoefs *coef, double beta,
-                              const double *dtvar, const FluxCorrection *fc, hipStream_t s) {
-  if (V > kMaxV) {
-    SetError("fused Burgers update supports at most 16 components");
-    return PTH_FAIL;
-  }
-  if (V < 4) {
-    SetError("fused Burgers update needs at least 4 components");
-    return PTH_FAIL;
-  }
-  ProfScope prof("fused_update", s);
-  const Geo G = MakeGeo(t, V);
-  const int nb = static_cast<int>(t.blocks.size());
-  const int cells = t.fine.n[0] * t.fine.n[1] * t.fine.n[2];
-  const dim3 grid(((cells + kWG - 1) / kWG) * nb);
-  const bool over = fc && !fc->host.empty();
-  const int *fover = over ? fc->dev_face : nullptr;
-  const double *fcor = over ? fc->store : nullptr;
-#define PTH_FUSED_CASE(NV)                                                                     \
-  case NV:                                                                                     \
-    hipLaunchKernelGGL(FusedUpdateKernel<NV>, grid, dim3(kWG), 0, s, face, U0, base, out,      \
-                       derived, flux, partial, coef, G, nb, beta, dtvar, fover, fcor);         \
-    break;
-  switch (V) {
-    PTH_FUSED_CASE(4)
-    PTH_FUSED_CASE(5)
-    PTH_FUSED_CASE(6)
-    PTH_FUSED_CASE(7)
-    PTH_FUSED_CASE(8)
-    PTH_FUSED_CASE(9)
-    PTH_FUSED_CASE(10)
-    PTH_FUSED_CASE(11)
-    PTH_FUSED_CASE(12)
-    PTH_FUSED_CASE(13)
-    PTH_FUSED_CASE(14)
-    PTH_FUSED_CASE(15)
-    PTH_FUSED_CASE(16)
-  }
-#undef PTH_FUSED_CASE
-  PTH_HIP(hipGetLastError());
-  return PTH_COMPLETE;
-}
-
-pth_status FlxcorFromFaces(const Topology &t, int V, const FluxCorrection &fc,
-                          const double *face, hipStream_t s) {
-  if (fc.host.empty()) return PTH_COMPLETE;
-  if (V > kMaxV || V < 4 || fc.ncomp != V) {
-    SetError("flux correction from face states: component count mismatch");
-    return PTH_FAIL;
-  }
-  ProfScope prof("flxcor_faces", s);
-  const Geo G = MakeGeo(t, V);
-  const int nb = static_cast<int>(t.blocks.size());
-  const dim3 grid(static_cast<unsigned>(fc.host.size()), (fc.max_cells + 63) / 64);
-#define PTH_FLX_CASE(NV)                                                                     \
-  case NV:                                                                                   \
-    hipLaunchKernelGGL(FlxcorFaceKernel<NV>, grid, dim3(64), 0, s, fc.dev, face, fc.store, G, \
-                       nb);                                                                  \
-    break;
-  switch (V) {
-    PTH_FLX_CASE(4)
-    PTH_FLX_CASE(5)
-    PTH_FLX_CASE(6)
-    PTH_FLX_CASE(7)
-    PTH_FLX_CASE(8)
-    PTH_FLX_CASE(9)
-    PTH_FLX_CASE(10)
-    PTH_FLX_CASE(11)
-    PTH_FLX_CASE(12)
-    PTH_FLX_CASE(13)
-    PTH_FLX_CASE(14)
-    PTH_FLX_CASE(15)
-    PTH_FLX_CASE(16)
-  }
-#undef PTH_FLX_CASE
-  PTH_HIP(hipGetLastError());
-  return PTH_COMPLETE;
 }
 
 pth_status FlxcorSend(const Topology &t, const FluxCorrection &fc, const double *flux,

@@ -4,10 +4,9 @@
 
 namespace pth {
 
-pth_status BurgersRecon(const Topology &t, int V, const double *U, double *face, int recon,
-                        hipStream_t s);
-pth_status BurgersFlux(const Topology &t, int V, const double *face, double *flux,
-                       hipStream_t s);
+// CalculateFluxes: the face fluxes of every direction, any block shape and component count
+pth_status BurgersFluxes(const Topology &t, int V, const double *U, double *flux, int recon,
+                         hipStream_t s);
 pth_status FluxDivergence(const Topology &t, int V, const double *flux, double *dudt,
                           const BlockCoefs *coef, hipStream_t s);
 pth_status WeightedSum(const double *x, const double *y, double w1, double w2, double *z,
@@ -25,17 +24,9 @@ pth_status BurgersDtToDevice(const Topology &t, int V, const double *U, const Bl
                              hipStream_t s);
 
 // fused stage path
-pth_status BurgersReconTasks(const Topology &t, int V, const double *U, double *face, int recon,
-                             hipStream_t s);
 int FusedUpdatePartials(const Topology &t);
-pth_status BurgersFusedUpdate(const Topology &t, int V, const double *face, const double *U0,
-                              const double *base, double *out, double *derived, double *flux,
-                              double *partial, const BlockCoefs *coef, double beta,
-                              const double *dtvar, const FluxCorrection *fc, hipStream_t s);
-// flux correction: restricted fine fluxes into the correction store, from the face states of
-// the fused stage or from stored fluxes; and the store into the coarse blocks' stored fluxes
-pth_status FlxcorFromFaces(const Topology &t, int V, const FluxCorrection &fc,
-                           const double *face, hipStream_t s);
+// flux correction: restricted fine fluxes into the correction store, and the store into the
+// coarse blocks' stored fluxes
 pth_status FlxcorSend(const Topology &t, const FluxCorrection &fc, const double *flux,
                       hipStream_t s);
 pth_status FlxcorSet(const Topology &t, const FluxCorrection &fc, double *flux, hipStream_t s);

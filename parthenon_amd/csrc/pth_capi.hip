@@ -103,7 +103,7 @@ Mesh::~Mesh() {
   if (split_list) (void)hipFree(split_list);
   if (geom) (void)hipFree(geom);
   if (coef) (void)hipFree(coef);
-  if (face) (void)hipFree(face);
+  if (flux_scratch) (void)hipFree(flux_scratch);
   if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
   if (graph) (void)hipGraphDestroy(graph);
   if (run_stream) (void)hipStreamDestroy(run_stream);
@@ -1483,15 +1483,7 @@ pth_status pth_burgers_calculate_fluxes(pth_meshdata *mdh, int recon) {
       return PTH_FAIL;
     }
   const int V = m->fields[f].ncomp;
-  if (!m->face || m->face_V != V) {
-    if (m->face) (void)hipFree(m->face);
-    m->face = nullptr;
-    if (Alloc(&m->face, 6 * md->store[f].ndata) != PTH_COMPLETE) return PTH_FAIL;
-    m->face_V = V;
-  }
-  if (BurgersRecon(m->topo, V, md->store[f].data, m->face, recon, m->stream) != PTH_COMPLETE)
-    return PTH_FAIL;
-  return BurgersFlux(m->topo, V, m->face, md->store[f].flux, m->stream);
+  return BurgersFluxes(m->topo, V, md->store[f].data, md->store[f].flux, recon, m->stream);
 }
 
 pth_status pth_flux_divergence(pth_meshdata *inh, pth_meshdata *dudth) {

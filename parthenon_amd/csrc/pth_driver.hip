@@ -9,8 +9,8 @@
 //   clock:   time += dt; dt = min(2 dt, cfl * min)   (all on device)
 //
 // For cubic blocks of 8 or 16 cells with 4 ghosts (and 4-13 components) the reconstruction
-// and HLL run plane by plane in LDS and only the fluxes reach HBM; other shapes keep the face
-// states in HBM and evaluate HLL inside the update.
+// and HLL run plane by plane in LDS; other shapes march columns in registers. Only the fluxes
+// reach HBM.
 //
 // The simulation clock lives in device memory, so a whole cycle has no host synchronization
 // and is captured once into a hipGraph and replayed. The exchange inside a cycle uses the same
@@ -157,12 +157,13 @@ pth_status Setup(Mesh *m, Ctx &x) {
   const std::int64_t nd = x.base->store[x.fu].ndata;
   const bool planes = x.base->store[x.fu].flux && ReconFluxSupported(m->topo, x.V);
   const bool sweep = m->run_sweep && BurgersSweepSupported(m->topo, x.V);
-  if (!planes && !sweep && (!m->face || m->face_V != x.V)) {  // face states of the other path
-    if (m->face) (void)hipFree(m->face);
-    m->face = nullptr;
-    PTH_HIP(hipMalloc(&m->face, sizeof(double) * 6 * nd));
-    PTH_HIP(hipMemset(m->face, 0, sizeof(double) * 6 * nd));
-    m->face_V = x.V;
+  // the other path's fluxes: the field's own, or scratch when U was declared without them
+  if (!planes && !sweep && !x.base->store[x.fu].flux && m->flux_scratch_n != 3 * nd) {
+    if (m->flux_scratch) (void)hipFree(m->flux_scratch);
+    m->flux_scratch = nullptr;
+    m->flux_scratch_n = 0;
+    PTH_HIP(hipMalloc(&m->flux_scratch, sizeof(double) * 3 * nd));
+    m->flux_scratch_n = 3 * nd;
   }
   if (FusedUpdatePartials(m->topo) > m->scratch_n) {
     SetError("too many CFL partials for the scratch area");
@@ -194,33 +195,23 @@ pth_status Stage(Ctx &x, int stage, hipStream_t s) {
   const double beta = stage == 1 ? 1.0 : 0.5;
   double *derived = x.fd >= 0 ? x.base->store[x.fd].data : nullptr;
   double *flux = x.base->store[x.fu].flux;  // scratch of both stages
-  if (flux && ReconFluxSupported(m.topo, x.V)) {
-    // plane-tiled reconstruction + HLL into the flux array, the flux-correction tasks on the
-    // stored fluxes (LoadAndSendFluxCorrections, SetFluxCorrections), then the update
-    if (BurgersReconFlux(m.topo, x.V, mc0.store[x.fu].data, flux, m.run_recon, 0, m.rf_ppw[0], s) !=
-        PTH_COMPLETE)
-      return PTH_FAIL;
-    if (x.fc && (FlxcorSend(m.topo, *x.fc, flux, s) != PTH_COMPLETE ||
-                 FlxcorSet(m.topo, *x.fc, flux, s) != PTH_COMPLETE))
-      return PTH_FAIL;
-    if (BurgersFluxUpdate(m.topo, x.V, flux, mc0.store[x.fu].data, x.base->store[x.fu].data,
-                          mc1.store[x.fu].data, derived, stage == 2 ? m.scratch : nullptr,
-                          m.coef, beta, m.dtvar, s) != PTH_COMPLETE)
-      return PTH_FAIL;
-  } else {
-    if (BurgersReconTasks(m.topo, x.V, mc0.store[x.fu].data, m.face, m.run_recon, s) !=
-        PTH_COMPLETE)
-      return PTH_FAIL;
-    // LoadAndSendFluxCorrections / SetFluxCorrections: the restricted fine fluxes land in
-    // the correction store that the fused update reads in place of its coarse-face fluxes
-    if (x.fc && FlxcorFromFaces(m.topo, x.V, *x.fc, m.face, s) != PTH_COMPLETE)
-      return PTH_FAIL;
-    if (BurgersFusedUpdate(m.topo, x.V, m.face, mc0.store[x.fu].data,
-                           x.base->store[x.fu].data, mc1.store[x.fu].data, derived, nullptr,
-                           stage == 2 ? m.scratch : nullptr, m.coef, beta, m.dtvar, x.fc,
-                           s) != PTH_COMPLETE)
-      return PTH_FAIL;
-  }
+  const bool planes = flux && ReconFluxSupported(m.topo, x.V);
+  if (!flux) flux = m.flux_scratch;
+  // reconstruction + HLL into the flux array (plane-tiled where the block shape allows), the
+  // flux-correction tasks on the stored fluxes (LoadAndSendFluxCorrections,
+  // SetFluxCorrections), then the update
+  if ((planes ? BurgersReconFlux(m.topo, x.V, mc0.store[x.fu].data, flux, m.run_recon, 0,
+                                 m.rf_ppw[0], s)
+              : BurgersFluxes(m.topo, x.V, mc0.store[x.fu].data, flux, m.run_recon, s)) !=
+      PTH_COMPLETE)
+    return PTH_FAIL;
+  if (x.fc && (FlxcorSend(m.topo, *x.fc, flux, s) != PTH_COMPLETE ||
+               FlxcorSet(m.topo, *x.fc, flux, s) != PTH_COMPLETE))
+    return PTH_FAIL;
+  if (BurgersFluxUpdate(m.topo, x.V, flux, mc0.store[x.fu].data, x.base->store[x.fu].data,
+                        mc1.store[x.fu].data, derived, stage == 2 ? m.scratch : nullptr,
+                        m.coef, beta, m.dtvar, s) != PTH_COMPLETE)
+    return PTH_FAIL;
   if (Exchange(m, mc1, s) != PTH_COMPLETE) return PTH_FAIL;
   if (stage == 2)
     return BurgersClock(m.scratch, FusedUpdatePartials(m.topo), m.run_cfl, m.dtvar, 1, m.run_lim,

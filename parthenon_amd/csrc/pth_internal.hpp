@@ -369,8 +369,8 @@ class Mesh {
   BufState state[10] = {};
   DeviceBlockGeom *geom = nullptr;
   BlockCoefs *coef = nullptr;
-  double *face = nullptr;                       // Burgers face-state scratch
-  int face_V = 0;
+  double *flux_scratch = nullptr;               // Burgers driver: fluxes of a U without them
+  std::int64_t flux_scratch_n = 0;
   // device-resident Burgers driver state: clock (kClockSlots doubles), its limits and the
   // captured cycle
   double *dtvar = nullptr;

@@ -238,7 +238,7 @@ __global__ void __launch_bounds__(64)
 // the other forms up to FMA contraction and the folded divides, so the stage output agrees
 // with theirs to rounding, and no flux or face state reaches HBM. On
 // multilevel meshes, faces with a finer neighbour take the restricted fine fluxes from the
-// correction store (fover / fcor as in FusedUpdateKernel).
+// correction store (fover gives the face's image in fcor, or -1).
 // The grid is persistent: workgroup g takes planes [g T / G, (g + 1) T / G) of the
 // T = nblocks * N planes in block order, so every workgroup does the same number of planes
 // (a segment that starts inside a block first rebuilds the z state below its first plane).
