@@ -34,6 +34,11 @@ pth_status FlxcorSet(const Topology &t, const FluxCorrection &fc, double *flux, 
 bool ReconFluxSupported(const Topology &t, int V);
 // part 0: every face; 1: faces independent of ghost cells; 2: the remaining faces
 bool BurgersSweepSupported(const Topology &t, int V);
+// the tile form of the sweep: x and y block sizes in multiples of 16
+bool BurgersTileSweep(const Topology &t, int V);
+// whether the sweep has choices to time (register budget, spread): the tile form proper is
+// built once and runs one workgroup a CU
+bool BurgersSweepTuned(const Topology &t, int V);
 // one launch per stage: reconstruction, HLL, flux divergence, RK update, derived, CFL partial
 // per workgroup (partial[0 .. *groups), at most max_partials workgroups); faces with a finer
 // neighbour take fc's corrected fluxes; waves (3 or 4) is the register budget the kernel is
@@ -41,7 +46,7 @@ bool BurgersSweepSupported(const Topology &t, int V);
 // each workgroup takes longer plane segments (fewer z-state rebuilds on small meshes); with
 // push (27 same-level neighbours per block, or -1) the output's boundary cells are also
 // written into those neighbours' ghost cells of out; with list (nlist block ids, device
-// memory; 16^3 blocks only) the launch covers those blocks alone
+// memory; tile form only) the launch covers those blocks alone
 pth_status BurgersSweep(const Topology &t, int V, const double *U, const double *base,
                         double *out, double *derived, double *partial, int max_partials,
                         const BlockCoefs *coef, double beta, const double *dtvar, int recon,

@@ -179,8 +179,7 @@ pth_status Setup(Mesh *m, Ctx &x) {
         m->SameLevelNeighbors() != PTH_COMPLETE)
       return PTH_FAIL;
     if (ok_base && ok_one && m->pack_mode == PTH_PACK_PERSISTENT) x.push = m->same_level;
-    if (x.push && m->sweep_split && m->topo.multilevel && m->topo.fine.n[0] == 16 &&
-        m->topo.fine.g[0] == 4) {
+    if (x.push && m->sweep_split && m->topo.multilevel && BurgersTileSweep(m->topo, x.V)) {
       if (SplitLists(*m) != PTH_COMPLETE) return PTH_FAIL;
       x.split = m->split_nA > 0 && m->split_nB > 0;
     }
@@ -354,12 +353,13 @@ pth_status TuneReconFlux(Ctx &x, hipStream_t s) {
   }
   // block sweep: the register budget (built for 3 or 4 waves per SIMD); the trial writes only
   // the interior of stage "1", which the next stage overwrites
-  if (st == PTH_COMPLETE && BurgersSweepSupported(m.topo, x.V)) {
+  m.sweep_spread = 1;
+  if (st == PTH_COMPLETE && BurgersSweepSupported(m.topo, x.V) &&
+      BurgersSweepTuned(m.topo, x.V)) {
     float best = 0.0f;
-    // the register-ring kernel of 16^3 blocks is built for 3 or 2 waves per SIMD, the general
-    // one for 4 or 3
-    const bool ring = m.topo.fine.n[0] == 16 && m.topo.fine.g[0] == 4;
-    const int budgets[2] = {ring ? 3 : 4, ring ? 2 : 3};
+    // the 16^3 form is built for 3 or 2 waves per SIMD, the 8^3 one for 4 or 3
+    const bool tiled = BurgersTileSweep(m.topo, x.V);
+    const int budgets[2] = {tiled ? 3 : 4, tiled ? 2 : 3};
     for (int waves : budgets) {
       st = BurgersSweep(m.topo, x.V, U, U, x.one->store[x.fu].data, nullptr, nullptr,
                         static_cast<int>(m.scratch_n), m.coef, 1.0, m.dtvar, m.run_recon, x.fc,
@@ -384,7 +384,6 @@ pth_status TuneReconFlux(Ctx &x, hipStream_t s) {
       }
     }
     // then how many resident workgroups share the planes (longer segments on small meshes)
-    m.sweep_spread = 1;
     for (int spread : {1, 2, 3}) {
       if (st != PTH_COMPLETE) break;
       for (int r = 0; r < 4 && st == PTH_COMPLETE; ++r) {
@@ -418,7 +417,7 @@ pth_status TuneReconFlux(Ctx &x, hipStream_t s) {
 pth_status Cycle(Ctx &x, hipStream_t s);
 
 // Picks the stage form (block sweep; plane reconstruction with the exchange on a second
-// stream; plane reconstruction then update then exchange) by timing whole cycles of each on
+// stream; fluxes then update then exchange) by timing whole cycles of each on
 // the mesh's own state, which is saved first and restored afterwards (U of "base", the
 // derived field and the device clock). The two plane forms give the same bits; the sweep is
 // built with FMA contraction and agrees with them to rounding (about 1e-15 relative), so
@@ -430,14 +429,19 @@ pth_status TuneForm(Ctx &x, hipStream_t s) {
     int sweep, overlap;
   };
   std::vector<Form> forms;
-  if (BurgersSweepSupported(m.topo, x.V) &&
-      !(m.form_exact && x.base->store[x.fu].flux && ReconFluxSupported(m.topo, x.V)))
-    forms.push_back({1, 0});
-  if (x.base->store[x.fu].flux && ReconFluxSupported(m.topo, x.V)) {
-    forms.push_back({0, 1});
-    forms.push_back({0, 0});
-  }
+  const bool flux = x.base->store[x.fu].flux != nullptr;
+  const bool planes = flux && ReconFluxSupported(m.topo, x.V);
+  if (BurgersSweepSupported(m.topo, x.V) && !(m.form_exact && flux)) forms.push_back({1, 0});
+  if (planes) forms.push_back({0, 1});
+  // other block shapes: the tile sweep takes less than half the flux form's time at every size
+  // (32^3 blocks with 7 components: 135 to 332 us on 8 of them, 653 to 1538 on 64), so there
+  // is nothing to time
+  if (flux && (planes || forms.empty())) forms.push_back({0, 0});
   if (forms.size() < 2) {
+    if (!forms.empty()) {
+      m.run_sweep = forms[0].sweep;
+      m.run_overlap = forms[0].overlap;
+    }
     m.form_tuned = true;
     return PTH_COMPLETE;
   }

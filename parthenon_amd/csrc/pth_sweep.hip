@@ -46,7 +46,7 @@ __device__ __forceinline__ void SweepHll(LS l, RS r, int d, double *F) {
   }
 }
 
-// ---- helpers of the 16^3 block sweep ---------------------------------------------------
+// ---- helpers of the tile sweep ---------------------------------------------------------
 //
 // Reciprocal by v_rcp_f64 and one third-order step r <- r (1 + e + e^2), e = 1 - x r: the
 // hardware estimate is good to about 25 bits, so the step's e^3 is far below an ulp. Four
@@ -149,18 +149,28 @@ __device__ __forceinline__ double HllFluxN(int n, double a, double b, double l, 
   return fma(a, l, b * r);
 }
 
+// v, as a value the compiler knows nothing about
+__device__ __forceinline__ int Opaque(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
 __device__ __forceinline__ int DMinI(int a, int b) { return b < a ? b : a; }
 
-// value of lane - 1 / lane + 1 within each 16-lane DPP row (the row's first / last lane
-// gets 0; callers replace those)
-__device__ __forceinline__ double FromLeft16(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x111, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x111, 0xF, 0xF, false);
+// value of lane - 1 / lane + 1 within each 16-lane DPP row; the row's first / last lane gets
+// its own `edge`
+__device__ __forceinline__ double FromLeft16(double v, double edge) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(v), 0x111, 0xF,
+                                             0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(v), 0x111, 0xF,
+                                             0xF, false);
   return __hiloint2double(hi, lo);
 }
-__device__ __forceinline__ double FromRight16(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x101, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x101, 0xF, 0xF, false);
+__device__ __forceinline__ double FromRight16(double v, double edge) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(v), 0x101, 0xF,
+                                             0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(v), 0x101, 0xF,
+                                             0xF, false);
   return __hiloint2double(hi, lo);
 }
 
@@ -188,7 +198,7 @@ __global__ void __launch_bounds__(64)
     const unsigned o = 8u * static_cast<unsigned>(PatchFineCell(P, G, a, c, p, q));
     double l[V], r[V];
     if (RING) {
-      // the expressions of BlockSweep16Kernel: FastStates and the face coefficients
+      // the expressions of TileSweepKernel: FastStates and the face coefficients
 #pragma unroll
       for (int n = 0; n < V; ++n) {
         const double *q = Ub + n * cs;
@@ -456,7 +466,7 @@ __global__ void __launch_bounds__(N * N, MINW)
   }
 }
 
-// ---- block sweep for 16^3 blocks: register-ring z stencils, LDS plane, DPP neighbours ------
+// ---- block sweep for 16^3 blocks of at most 7 components ------------------------------------
 //
 // One workgroup of 256 threads marches the z planes of a block; thread (tx, ty) owns column
 // (i, j) = (tx, ty). Per plane kk:
@@ -686,7 +696,7 @@ __global__ void __launch_bounds__(256, MINW)
         const double A = C.area[0];
         double ql0, qr0;
         FastStates(RECON, own_pl[-2], own_pl[-1], own_pl[0], own_pl[1], own_pl[2], ql0, qr0);
-        double qlm = FromLeft16(ql0), qrp = FromRight16(qr0);
+        double qlm = FromLeft16(ql0, 0.0), qrp = FromRight16(qr0, 0.0);
         if (tx == 0) qlm = ext[ty * 2];
         if (tx == N - 1) qrp = ext[ty * 2 + 1];
         double alo, blo, ahi, bhi;
@@ -699,7 +709,7 @@ __global__ void __launch_bounds__(256, MINW)
             const double *cn = own_pl + n * PS;
             FastStates(RECON, cn[-2], cn[-1], cn[0], cn[1], cn[2], ql, qr);
           }
-          double lm = FromLeft16(ql), rp = FromRight16(qr);
+          double lm = FromLeft16(ql, 0.0), rp = FromRight16(qr, 0.0);
           if (tx == 0) lm = ext[(n * N + ty) * 2];
           if (tx == N - 1) rp = ext[(n * N + ty) * 2 + 1];
           double fl = HllFluxN(n, alo, blo, lm, qr);
@@ -717,7 +727,7 @@ __global__ void __launch_bounds__(256, MINW)
         double ql1, qr1;
         FastStates(RECON, c[PS - 2 * PP], c[PS - PP], c[PS], c[PS + PP], c[PS + 2 * PP], ql1,
                    qr1);
-        double qlm = FromLeft16(ql1), qrp = FromRight16(qr1);
+        double qlm = FromLeft16(ql1, 0.0), qrp = FromRight16(qr1, 0.0);
         if (tx == 0) qlm = ext[NX + (N + ty) * 2];
         if (tx == N - 1) qrp = ext[NX + (N + ty) * 2 + 1];
         double alo, blo, ahi, bhi;
@@ -730,7 +740,7 @@ __global__ void __launch_bounds__(256, MINW)
             const double *cn = c + n * PS;
             FastStates(RECON, cn[-2 * PP], cn[-PP], cn[0], cn[PP], cn[2 * PP], ql, qr);
           }
-          double lm = FromLeft16(ql), rp = FromRight16(qr);
+          double lm = FromLeft16(ql, 0.0), rp = FromRight16(qr, 0.0);
           if (tx == 0) lm = ext[NX + (n * N + ty) * 2];
           if (tx == N - 1) rp = ext[NX + (n * N + ty) * 2 + 1];
           double fl = HllFluxN(n, alo, blo, lm, qr);
@@ -811,9 +821,516 @@ __global__ void __launch_bounds__(256, MINW)
     partial[blockIdx.x] = v;
   }
 }
+// ---- tile sweep: blocks whose x and y sizes are multiples of 16 ----------------------------
+//
+// One workgroup of G groups of 256 threads (4 wavefronts each) marches the z planes of a 16 x 16
+// column tile of a block: group g owns components g, g + G, g + 2 G, ..., and thread (tx, ty) of
+// a group the tile's column (i, j) = (tx, ty). Three steps a plane, a barrier after each:
+//   1. the last plane's update: flux divergence, RK averaging and update, the output and the
+//      same-level ghost copies; then the normal velocities' states in the plane's cells (u along
+//      x, v along y, w of the cell above) and those of the cells beyond the tile's rows and
+//      columns, every component, from the plane staged in LDS;
+//   2. the face coefficients (a, b) of HllCoef of the three directions, every x and y face
+//      once; the last plane's derived field and CFL maximum;
+//   3. the fluxes, a group's components one after another. x: own cell's stencil from LDS, the
+//      neighbouring cells' states by DPP row shifts (a row of 16 cells is a 16-lane DPP row),
+//      flux = a ql + b qr; y: the same with the thread mapping transposed (thread (tx, ty)
+//      takes cell i = ty, j = tx, so a column is a row too); both differences to LDS. z: each
+//      thread keeps U of its column at planes kk - 1, kk + 1, kk + 2 and kk + 3 in registers (kk
+//      itself is in LDS), so the z stencil of the cell above needs no load; the high z
+//      face's flux becomes the next plane's low face flux. Before them the next plane is
+//      staged in the other LDS buffer (the tile's own cells from the rings, 3-cell x and y
+//      halos from HBM) and the loads that the next plane needs are issued.
+// The divergence adds x, y and z in the order of FluxDivHelper (update.hpp:43-57). A velocity's
+// flux carries a factor 1/2 against the scalars': it is applied to the face area (an exact
+// product), and corrected fluxes of velocities are doubled where they are read. Each U element
+// is read from HBM once per workgroup (plus the halos and the segment's first planes), and face
+// states and fluxes never leave the CU.
+//
+// Bound: FP64 issue, at 54% of it (2 wavefronts per SIMD from one workgroup a CU; the barriers
+// and the memory waits of the staging show). Two groups a tile, since one thread per column
+// with 8 components and more needs over 256 VGPRs: spilled registers cost most here, as each
+// reload waits for every load and store in flight. (Four groups of 128 VGPRs spill and took
+// 1105 us for the cycle below.) Measured, cycles of 128^3 cells in 32^3 blocks: 980 us with 11
+// components (fluxes, update and exchange as launches of their own: 2365), 653 us with 7
+// (1538); 16^3 blocks with 11 components: 186 us on 64 blocks, 238 by one thread per column.
+struct TileShape {
+  int n0, n1, n2;     // interior cells of a block
+  int e0;             // brick row pitch
+  int sz, cs;         // brick plane and component strides
+  int tx, tiles;      // tiles per block along x, and in all
+};
+
+template <int V, int RECON>
+__global__ void __launch_bounds__(512, 2)
+    TileSweepKernel(const double *__restrict__ U, const double *base, double *out,
+                    double *__restrict__ derived, double *__restrict__ partial,
+                    const BlockCoefs *__restrict__ coef, TileShape S, int nblocks, double beta,
+                    const double *__restrict__ dtvar, const int *__restrict__ fover,
+                    const double *__restrict__ fcor, const int *__restrict__ push,
+                    const int *__restrict__ list) {
+  constexpr int N = 16, NG = 4, G = 2, NT = 256 * G, NC = (V + G - 1) / G;
+  constexpr int H = 3;             // halo of the staged plane
+  constexpr int PW = N + 2 * H;    // staged rows / columns
+  constexpr int PP = PW + 1;       // row pitch (odd, fewer bank conflicts on column reads)
+  constexpr int PS = PW * PP;      // one component of the staged plane
+  constexpr int SP = N + 1;        // pitch of the difference tiles and of the face rows
+  constexpr int NX = V * N * 2;    // beyond-the-row states of one direction
+  constexpr int NH = V * 12 * N;   // halo cells of one staged plane (all components)
+  constexpr int QH = (NH + NT - 1) / NT;  // halo cells per thread
+  // a second staged plane and a y difference tile of its own where the LDS (160 KiB) holds
+  // them; without them a step waits for the readers of the array it reuses
+  constexpr int kFixed = V * PS + 2 * NX + V * N * SP + 6 * N * SP + 4 * V * N + 16;
+  constexpr bool DB = 8 * (kFixed + V * PS) <= 160 * 1024;
+  constexpr bool SY = DB && 8 * (kFixed + V * PS + V * N * SP) <= 160 * 1024;
+  constexpr int gW = 0, mW = 1;  // the z velocity's group and place in it
+  constexpr int gD = 1;          // the group of the derived field and CFL
+  __shared__ double pl[(DB ? 2 : 1) * V * PS];  // [plane parity][n][j + H][i + H]
+  __shared__ double ext[2 * NX];     // [dir][n][line][side]: side 0 ql of cell -1, 1 qr of cell N
+  __shared__ double sd[(SY ? 2 : 1) * V * N * SP];  // x (+ y) differences [n][j][i], then the new
+                                                    // state; the y differences
+  __shared__ double ca[3][N * SP], cb[3][N * SP];  // face coefficients [dir][line][face]
+  __shared__ double fxy[2 * V * 2 * N];  // corrected x / y face fluxes of the plane,
+                                         // [dir][n][side][line] (tiles with such faces)
+  __shared__ double wmax[NT / 64];
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int grp = wave >> 2, wrow = wave & 3;  // uniform: a wavefront takes rows 4 wrow .. + 3
+  const int tx = threadIdx.x % N, ty = (threadIdx.x / N) % N;
+  const bool last = (NC - 1) * G + grp < V;  // the group has a component at m = NC - 1
+  const int nc = last ? NC : NC - 1;
+  const double bdt = beta * dtvar[0];
+  const double w2 = 1.0 - beta;
+  const bool same_base = base == U;
+  const int n0 = S.n0, n1 = S.n1, n2 = S.n2, e0 = S.e0, tilesx = S.tx, tiles = S.tiles;
+  const std::int64_t cs = S.cs, sz = S.sz;
+  const unsigned col = 8u * static_cast<unsigned>((NG + ty) * e0 + NG + tx);  // byte offset
+  const int own = (ty + H) * PP + tx + H;  // own cell in the staged plane
+  const int osd = ty * SP + tx;            // own cell in the difference tile
+  // halo cell q of this thread (q < QH): byte offset from the tile's plane in the brick (the
+  // component's included) and place in the staged plane; cells past the last repeat it (loads
+  // are unconditional, so the compiler can count them in its memory waits)
+  unsigned hoff[QH];
+  int hloc[QH];
+#pragma unroll
+  for (int q = 0; q < QH; ++q) {
+    const int t = DMinI(static_cast<int>(threadIdx.x) + q * NT, NH - 1);
+    const int n = t / (12 * N), r = t % (12 * N);
+    int i, j;
+    if (r < 6 * N) {  // y strips: rows -3 .. -1 and N .. N + 2, all interior columns
+      const int yy = r / N;
+      i = r % N;
+      j = yy < 3 ? yy - 3 : N + yy - 3;
+    } else {          // x strips: all interior rows, columns -3 .. -1 and N .. N + 2
+      const int qq = r - 6 * N;
+      j = qq / 6;
+      const int c = qq % 6;
+      i = c < 3 ? c - 3 : N + c - 3;
+    }
+    hoff[q] = 8u * static_cast<unsigned>(n * static_cast<int>(cs) + (NG + j) * e0 + NG + i);
+    hloc[q] = n * PS + (j + H) * PP + i + H;
+  }
+  double smax = 0.0;  // largest sum of |u| / dx of the new states
+  const std::int64_t T = static_cast<std::int64_t>(nblocks) * tiles * n2;
+  std::int64_t pnext = T * blockIdx.x / gridDim.x;
+  const std::int64_t pend = T * (blockIdx.x + 1) / gridDim.x;
+  while (pnext < pend) {
+    // the planes of the launch run over its blocks' tiles in order: all blocks, or the listed
+    const int unit = static_cast<int>(pnext / n2);
+    const int k0 = static_cast<int>(pnext - static_cast<std::int64_t>(unit) * n2);
+    const int k1 = static_cast<int>(pend - pnext < n2 - k0 ? k0 + (pend - pnext) : n2);
+    pnext += k1 - k0;
+    const int bi = unit / tiles, tile = unit - bi * tiles;
+    const int b = list ? list[bi] : bi;
+    const int tj = tile / tilesx, ti = tile - tj * tilesx;
+    const bool lox = ti == 0, hix = ti == tilesx - 1, loy = tj == 0, hiy = (tj + 1) * N == n1;
+    const int toff = tj * N * e0 + ti * N;  // the tile within a plane
+    const std::int64_t at = static_cast<std::int64_t>(b) * V * cs + toff;
+    const BlockCoefs &C = coef[b];
+    const double ivol = 1.0 / C.vol;
+    const double ax = C.area[0], ay = C.area[1], az = C.area[2];
+    const double ix = 1.0 / C.dx[0], iy = 1.0 / C.dx[1], iz = 1.0 / C.dx[2];
+    // the block's same-level neighbours, one per lane, read by readlane: a load in the middle
+    // of a plane would be waited for
+    const int nbr = push ? push[27 * b + DMinI(static_cast<int>(threadIdx.x) % 64, 26)] : -1;
+    // the block's face images of corrected fluxes, where the tile touches the face
+    const int *fo = fover ? fover + 6 * b : nullptr;
+    const int ox0 = fo && lox ? fo[0] : -1, ox1 = fo && hix ? fo[1] : -1;
+    const int oy0 = fo && loy ? fo[2] : -1, oy1 = fo && hiy ? fo[3] : -1;
+    const int oz0 = fo ? fo[4] : -1, oz1 = fo ? fo[5] : -1;
+    const bool fixed = ox0 >= 0 || ox1 >= 0 || oy0 >= 0 || oy1 >= 0;
+    const int zimg = ti * N + tx + (tj * N + ty) * n0;  // this column in a z face's image
+    const int kk0 = NG + k0;
+    auto plane = [=](auto *f, int n, int kk) __attribute__((always_inline)) {
+      return Glob(f) + (at + n * cs + kk * sz);  // the tile's plane kk of component n
+    };
+    auto load = [=](const __attribute__((address_space(1))) double *p, unsigned off)
+        __attribute__((always_inline)) {
+      return *reinterpret_cast<const __attribute__((address_space(1))) double *>(
+          reinterpret_cast<const __attribute__((address_space(1))) char *>(p) + off);
+    };
+    auto store = [=](__attribute__((address_space(1))) double *p, unsigned off, double v)
+        __attribute__((always_inline)) {
+      *reinterpret_cast<__attribute__((address_space(1))) double *>(
+          reinterpret_cast<__attribute__((address_space(1))) char *>(p) + off) = v;
+    };
+    // copies of value m of v, plane k, into the same-level neighbours' ghosts: a cell within NG
+    // of a face of the block is a ghost cell of the neighbours across that face, edge or
+    // corner (push[27 b + direction]), at its index shifted by the block size along each
+    // crossed dimension. Every strip that a cell can lie in is uniform in the wavefront but for
+    // the x one, so each neighbour's copies are stores at one base address.
+    auto copies = [=](const double (&v)[NC], int k, int tx, unsigned col)
+        __attribute__((always_inline)) {
+      const int ly = loy && wrow == 0 ? -1 : hiy && wrow == 3 ? 1 : 0;
+      const int lz = k < NG ? -1 : k >= n2 - NG ? 1 : 0;
+      for (int sz_ = 0; sz_ <= (lz ? 1 : 0); ++sz_)
+        for (int sy = 0; sy <= (ly ? 1 : 0); ++sy)
+          for (int dx = lox ? -1 : 0; dx <= (hix ? 1 : 0); ++dx) {
+            const int dy = sy ? ly : 0, dz = sz_ ? lz : 0;
+            if (!(dx | dy | dz)) continue;
+            const int g = __builtin_amdgcn_readlane(nbr, (dx + 1) + 3 * (dy + 1) + 9 * (dz + 1));
+            if (g < 0) continue;
+            const std::int64_t to = static_cast<std::int64_t>(g - b) * V * cs - dz * n2 * sz -
+                                    dy * n1 * e0 - dx * n0;
+            if (dx == 0 || (dx < 0 ? tx < NG : tx >= N - NG)) {
+#pragma unroll
+              for (int m = 0; m < NC; ++m) {
+                if (m == NC - 1 && !last) break;
+                store(plane(out, G * m + grp, NG + k) + to, col, v[m]);
+              }
+            }
+          }
+    };
+    // CFL maximum and derived field of plane k from the new states in sd (group gD)
+    auto gather = [=](int k, double s, int osd, unsigned col) __attribute__((always_inline)) {
+      const double v0 = sd[osd], v1 = sd[N * SP + osd], v2 = sd[2 * N * SP + osd],
+                   v3 = sd[3 * N * SP + osd];
+      const double sp = fabs(v0) * ix + fabs(v1) * iy + fabs(v2) * iz;
+      if (derived)
+        store(Glob(derived) + (static_cast<std::int64_t>(b) * cs + toff + (NG + k) * sz), col,
+              0.5 * v3 * (v0 * v0 + v1 * v1 + v2 * v2));
+      return DMax(s, sp);
+    };
+    // corrected fluxes of plane k's x and y faces (only tiles next to finer blocks), staged in
+    // LDS so that the loops below issue no conditional load
+    auto corrected = [=](int k, int tid) __attribute__((always_inline)) {
+      for (int t = tid; t < 2 * V * 2 * N; t += NT) {
+        const int dir = t / (2 * V * N), r = t % (2 * V * N);
+        const int n = r / (2 * N), side = (r / N) & 1, line = r % N;
+        const int o = dir == 0 ? (side ? ox1 : ox0) : (side ? oy1 : oy0);
+        const int rows = dir == 0 ? n1 : n0;
+        const int a = (dir == 0 ? tj : ti) * N + line;
+        fxy[t] = o >= 0 ? (n < 3 ? 2.0 : 1.0) * fcor[o + a + (k + n * n2) * rows] : 0.0;
+      }
+    };
+    // ---- the segment's first plane kk0, staged; the rings
+    double hv[QH], r0[NC], r2[NC], r3[NC], r4[NC];
+    {
+      double *const to = pl + (DB ? (k0 & 1) * V * PS : 0);
+#pragma unroll
+      for (int q = 0; q < QH; ++q) hv[q] = load(plane(U, 0, kk0), hoff[q]);
+      double own_u[NC];
+#pragma unroll
+      for (int m = 0; m < NC; ++m) {
+        if (m == NC - 1 && !last) break;
+        const int n = G * m + grp;
+        r0[m] = load(plane(U, n, kk0 - 1), col);
+        own_u[m] = load(plane(U, n, kk0), col);
+        r2[m] = load(plane(U, n, kk0 + 1), col);
+        r3[m] = load(plane(U, n, kk0 + 2), col);
+        r4[m] = load(plane(U, n, kk0 + 3), col);
+      }
+#pragma unroll
+      for (int q = 0; q < QH; ++q) to[hloc[q]] = hv[q];
+#pragma unroll
+      for (int m = 0; m < NC; ++m) {
+        if (m == NC - 1 && !last) break;
+        to[(G * m + grp) * PS + own] = own_u[m];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < QH; ++q) hv[q] = load(plane(U, 0, kk0 + 1), hoff[q]);
+    // ---- z state at plane kk0: ql of cell kk0 (zl) and the flux of face kk0 - 1/2 (zf); the
+    // z velocity gives the face coefficients
+    double zl[NC], zf[NC];
+    {
+      auto ends = [=](int n, double &below, double &qr, double &ql)
+          __attribute__((always_inline)) {
+        double x;
+        double q[6];
+#pragma unroll
+        for (int s = 0; s < 6; ++s) q[s] = load(plane(U, n, kk0 - 3 + s), col);
+        FastStates(RECON, q[0], q[1], q[2], q[3], q[4], below, x);
+        FastStates(RECON, q[1], q[2], q[3], q[4], q[5], ql, qr);
+      };
+      double wb, wr, wl, za, zb;  // the z velocity's
+      ends(2, wb, wr, wl);
+      HllCoef(wb, wr, za, zb);
+#pragma unroll
+      for (int m = 0; m < NC; ++m) {
+        if (m == NC - 1 && !last) break;
+        const int n = G * m + grp;
+        double qb = wb, qr = wr, ql = wl;
+        if (n != 2) ends(n, qb, qr, ql);
+        double f = fma(za, qb, zb * qr);
+        if (k0 == 0 && oz0 >= 0)
+          f = (n < 3 ? 2.0 : 1.0) * fcor[oz0 + zimg + n * n0 * n1];
+        zf[m] = f;
+        zl[m] = ql;
+        // one component at a time, as in the z fluxes
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    double bv[NC], dz[NC];  // of the plane in hand: base state, z difference
+    // the update of plane k, whose differences are complete
+    auto finish = [&](int k, int tx, int osd, unsigned col) __attribute__((always_inline)) {
+      double v[NC];
+#pragma unroll
+      for (int m = 0; m < NC; ++m) {
+        if (m == NC - 1 && !last) break;
+        const int n = G * m + grp;
+        double &slot = sd[n * N * SP + osd];
+        double du = slot;
+        if (SY) du = du + sd[V * N * SP + n * N * SP + osd];
+        du = du + dz[m];
+        const double dudt = -du * ivol;
+        const double avg = beta * r0[m] + w2 * (same_base ? r0[m] : bv[m]);
+        v[m] = 1.0 * avg + bdt * dudt;
+        if (n < 4) slot = v[m];  // for the derived field and the CFL
+        store(plane(out, n, NG + k), col, v[m]);
+      }
+      if (push) copies(v, k, tx, col);
+    };
+    __syncthreads();
+    for (int k = k0; k < k1; ++k) {
+      const int kk = NG + k;
+      // the thread's place, formed anew for each plane: addresses derived from it would
+      // otherwise be hoisted out of the loop and take the registers of the stencils (a
+      // spilled register costs more than its reload: every reload waits for all the loads
+      // and stores in flight)
+      const int tid = Opaque(static_cast<int>(threadIdx.x));
+      const int tx = tid % N, ty = (tid / N) % N;
+      const int own = (ty + H) * PP + tx + H, osd = ty * SP + tx;
+      const unsigned col = 8u * static_cast<unsigned>((NG + ty) * e0 + NG + tx);
+      const double *const P = pl + (DB ? (k & 1) * V * PS : 0);
+      const double *const crow = P + own;                     // own cell
+      const double *const ccol = P + (tx + H) * PP + ty + H;  // cell i = ty, j = tx
+      // ---- 1.
+      // the next plane into the other buffer first (also past the block's last plane: ghost
+      // planes): every load in flight is waited for here, before the stores below, since a
+      // later wait would count these too
+      auto stage = [&](double *to) __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < NC; ++m) {
+          if (m == NC - 1 && !last) break;
+          to[(G * m + grp) * PS + own] = r2[m];
+        }
+#pragma unroll
+        for (int q = 0; q < QH; ++q) to[hloc[q]] = hv[q];
+      };
+      if (DB) stage(pl + ((k + 1) & 1) * V * PS);
+      if (k > k0) finish(k - 1, tx, osd, col);
+      if (fixed) corrected(k, tid);
+      double vl, vr, wl = 0.0, wr = 0.0;
+      {
+        const double *c = grp == 0 ? crow : ccol + PS;
+        const int st = grp == 0 ? 1 : PP;
+        FastStates(RECON, c[-2 * st], c[-st], c[0], c[st], c[2 * st], vl, vr);
+      }
+      if (grp == gW)
+        FastStates(RECON, r0[mW], crow[2 * PS], r2[mW], r3[mW], r4[mW], wl, wr);
+      for (int t = tid ^ (NT / 2); t < 2 * NX; t += NT) {
+        const int dir = t / NX, r = t % NX;
+        const int n = r / (2 * N), q = r % (2 * N);
+        const int line = q >> 1, side = q & 1;
+        const int cell = side ? N : -1;
+        const int st = dir ? PP : 1;
+        const double *c = P + n * PS + (dir ? (cell + H) * PP + line + H
+                                            : (line + H) * PP + cell + H);
+        double ql, qr;
+        FastStates(RECON, c[-2 * st], c[-st], c[0], c[st], c[2 * st], ql, qr);
+        ext[t] = side ? qr : ql;
+      }
+      __syncthreads();
+      // ---- 2. [line][face]: the low face of every cell and the high face of the last
+      {
+        const double *e = ext + grp * (NX + 2 * N) + ty * 2;
+        const double lm = FromLeft16(vl, e[0]);
+        double a, bb;
+        HllCoef(lm, vr, a, bb);
+        ca[grp][osd] = a;
+        cb[grp][osd] = bb;
+        if (tx == N - 1) {
+          HllCoef(vl, e[1], a, bb);
+          ca[grp][osd + 1] = a;
+          cb[grp][osd + 1] = bb;
+        }
+      }
+      if (grp == gW) {
+        double a, bb;
+        HllCoef(zl[mW], wr, a, bb);
+        ca[2][osd] = a;
+        cb[2][osd] = bb;
+      }
+      if (k > k0 && grp == gD) smax = gather(k - 1, smax, osd, col);
+      __syncthreads();
+      // ---- 3.
+      // x: own cell (tx, ty), differences to sd[n][ty][tx]
+      {
+#pragma unroll 1
+        for (int m = 0; m < nc; ++m) {
+          const int n = G * m + grp;
+          double ql = vl, qr = vr;
+          if (n != 0) {
+            const double *c = crow + n * PS;
+            FastStates(RECON, c[-2], c[-1], c[0], c[1], c[2], ql, qr);
+          }
+          const double e = ext[(n * N + ty) * 2 + (tx == N - 1)];
+          double fl = fma(ca[0][osd], FromLeft16(ql, e), cb[0][osd] * qr);
+          double fh = fma(ca[0][osd + 1], ql, cb[0][osd + 1] * FromRight16(qr, e));
+          if (fixed) {
+            if (tx == 0 && ox0 >= 0) fl = fxy[(n * 2 + 0) * N + ty];
+            if (tx == N - 1 && ox1 >= 0) fh = fxy[(n * 2 + 1) * N + ty];
+          }
+          const double A = n < 3 ? 0.5 * ax : ax;
+          sd[n * N * SP + osd] = A * fh - A * fl;
+        }
+      }
+      if (!SY) __syncthreads();  // the x differences are in the tile
+      // the loads that the next plane needs (indices in range also past the block's last
+      // plane: ghost planes); before the x fluxes they would take registers from them
+      if (DB) {
+#pragma unroll
+        for (int q = 0; q < QH; ++q) hv[q] = load(plane(U, 0, kk + 2), hoff[q]);
+      }
+      double r5[NC];
+#pragma unroll
+      for (int m = 0; m < NC; ++m) {
+        if (m == NC - 1 && !last) break;
+        r5[m] = load(plane(U, G * m + grp, kk + 4), col);
+      }
+      // y: cell i = ty, j = tx, differences to the y tile or added to sd[n][j][i]
+      {
+#pragma unroll 1
+        for (int m = 0; m < nc; ++m) {
+          const int n = G * m + grp;
+          double ql = vl, qr = vr;
+          if (n != 1) {
+            const double *c = ccol + n * PS;
+            FastStates(RECON, c[-2 * PP], c[-PP], c[0], c[PP], c[2 * PP], ql, qr);
+          }
+          const double e = ext[NX + (n * N + ty) * 2 + (tx == N - 1)];
+          double fl = fma(ca[1][osd], FromLeft16(ql, e), cb[1][osd] * qr);
+          double fh = fma(ca[1][osd + 1], ql, cb[1][osd + 1] * FromRight16(qr, e));
+          if (fixed) {
+            if (tx == 0 && oy0 >= 0) fl = fxy[((V + n) * 2 + 0) * N + ty];
+            if (tx == N - 1 && oy1 >= 0) fh = fxy[((V + n) * 2 + 1) * N + ty];
+          }
+          const double A = n < 3 ? 0.5 * ay : ay;
+          const int at_y = n * N * SP + tx * SP + ty;
+          if (SY)
+            sd[V * N * SP + at_y] = A * fh - A * fl;
+          else
+            sd[at_y] = sd[at_y] + (A * fh - A * fl);
+        }
+      }
+#pragma unroll
+      for (int m = 0; m < NC; ++m) {
+        if (m == NC - 1 && !last) break;
+        bv[m] = same_base ? 0.0 : load(plane(base, G * m + grp, kk), col);
+      }
+      // z: the cell above (kk + 1) from the ring; its low face closes this cell
+      {
+        const double za = ca[2][osd], zb = cb[2][osd];
+        const bool top = k == n2 - 1 && oz1 >= 0;
+        const int zimg = ti * N + tx + (tj * N + ty) * n0;
+#pragma unroll
+        for (int m = 0; m < NC; ++m) {
+          if (m == NC - 1 && !last) break;
+          const int n = G * m + grp;
+          const double uo = crow[n * PS];
+          double ql = wl, qr = wr;
+          if (n != 2) FastStates(RECON, r0[m], uo, r2[m], r3[m], r4[m], ql, qr);
+          double fh = fma(za, zl[m], zb * qr);
+          if (top) {  // only here a load: waited for inside the branch
+            fh = (n < 3 ? 2.0 : 1.0) * fcor[oz1 + zimg + n * n0 * n1];
+            asm volatile("" : "+v"(fh));
+          }
+          const double A = n < 3 ? 0.5 * az : az;
+          dz[m] = A * fh - A * zf[m];
+          zf[m] = fh;
+          zl[m] = ql;
+          // one component at a time: interleaving the reconstructions needs more registers
+          // than the budget holds
+          __builtin_amdgcn_sched_barrier(0);
+          if (DB || k + 1 == k1) {  // the ring moves up one plane
+            r0[m] = uo;
+            r2[m] = r3[m];
+            r3[m] = r4[m];
+            r4[m] = r5[m];
+          }
+        }
+      }
+      __syncthreads();
+      if (!DB && k + 1 < k1) {
+#pragma unroll
+        for (int m = 0; m < NC; ++m) {
+          if (m == NC - 1 && !last) break;
+          r0[m] = crow[(G * m + grp) * PS];
+        }
+        stage(pl);
+#pragma unroll
+        for (int q = 0; q < QH; ++q) hv[q] = load(plane(U, 0, kk + 2), hoff[q]);
+#pragma unroll
+        for (int m = 0; m < NC; ++m) {
+          r2[m] = r3[m];
+          r3[m] = r4[m];
+          r4[m] = r5[m];
+        }
+        __syncthreads();
+      }
+    }
+    finish(k1 - 1, tx, osd, col);
+    __syncthreads();
+    if (grp == gD) smax = gather(k1 - 1, smax, osd, col);
+    __syncthreads();  // sd and the staged planes are free for the next segment
+  }
+  if (!partial) return;
+  for (int off = 32; off > 0; off >>= 1) smax = DMax(smax, __shfl_xor(smax, off, 64));
+  if ((threadIdx.x & 63) == 0) wmax[wave] = smax;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double v = wmax[0];
+#pragma unroll
+    for (int w = 1; w < NT / 64; ++w) v = DMax(v, wmax[w]);
+    partial[blockIdx.x] = DMin(DBL_MAX, 1.0 / v);
+  }
+}
 }  // namespace
 
-bool BurgersSweepSupported(const Topology &t, int V) { return ReconFluxSupported(t, V); }
+// 16^3 blocks of at most 7 components: one thread per column, of which two workgroups fit a
+// CU's LDS and registers (960 refined blocks with 7 components: 1746 us a cycle, 1928 by the
+// tile form; from 8 on only one fits and the tile form is the faster).
+static bool RingSweep(const Topology &t, int V) {
+  const Extent &f = t.fine;
+  return f.n[0] == 16 && f.n[1] == 16 && f.n[2] == 16 && V <= 7;
+}
+
+// Blocks of the tile sweep: x and y sizes in whole 16-cell tiles, z any size whose low and
+// high ghost strips do not meet, 4 ghosts; a block's components within 32-bit byte offsets.
+bool BurgersTileSweep(const Topology &t, int V) {
+  const Extent &f = t.fine;
+  return t.ndim == 3 && f.n[0] % 16 == 0 && f.n[1] % 16 == 0 && f.n[2] >= 8 && f.g[0] == 4 &&
+         f.g[1] == 4 && f.g[2] == 4 && V >= 4 && V <= 13 &&
+         f.cells() * V < (std::int64_t(1) << 29);
+}
+
+bool BurgersSweepTuned(const Topology &t, int V) {
+  return !BurgersTileSweep(t, V) || RingSweep(t, V);
+}
+
+bool BurgersSweepSupported(const Topology &t, int V) {
+  return BurgersTileSweep(t, V) || (ReconFluxSupported(t, V) && t.fine.n[0] == 8);
+}
 
 // Workgroups of a kernel resident on the whole device at once (occupancy x compute units).
 int ResidentGroups(const void *kernel, int threads) {
@@ -839,95 +1356,109 @@ pth_status BurgersSweep(const Topology &t, int V, const double *U, const double 
     SetError("block sweep: unsupported block shape or component count");
     return PTH_FAIL;
   }
-  const int N = t.fine.n[0];
-  if (list && !(N == 16 && t.fine.g[0] == 4 && nlist > 0)) {
-    SetError("block sweep: block lists need 16^3 blocks with 4 ghosts");
+  const bool tiled = BurgersTileSweep(t, V);
+  if (list && !(tiled && nlist > 0)) {
+    SetError("block sweep: block lists need blocks of the tile sweep");
     return PTH_FAIL;
   }
   ProfScope prof("block_sweep", s);
   const int nb = list ? nlist : static_cast<int>(t.blocks.size());
-  if (N == 16 && t.fine.g[0] == 4) {
-    // register-ring kernel, compiled for 2 or 3 waves per SIMD
-    const int minw = waves >= 3 ? 3 : 2;
-    const int *fover16 = fc ? fc->dev_face : nullptr;
-    const double *fcor16 = fc ? fc->store : nullptr;
-    int grid16 = 0;
-#define PTH_S16_R(NV, W, RC)                                                                   \
-  {                                                                                            \
-    const int r =                                                                              \
-        ResidentGroups(reinterpret_cast<const void *>(&BlockSweep16Kernel<NV, W, RC>), 256);    \
-    if (r < 1) {                                                                               \
-      SetError("block sweep: occupancy query failed");                                         \
-      return PTH_FAIL;                                                                         \
-    }                                                                                          \
-    grid16 = static_cast<int>(std::min<std::int64_t>(std::min(std::max(r / spread, 1),          \
-                                                              max_partials),                   \
-                                                     static_cast<std::int64_t>(nb) * 16));     \
-    hipLaunchKernelGGL((BlockSweep16Kernel<NV, W, RC>), dim3(grid16), dim3(256), 0, s, U, base, \
-                       out, derived, partial, coef, nb, beta, dtvar, fover16, fcor16, push,   \
-                       list);                                                                  \
-  }
-#define PTH_S16_W(NV, W)                                                                       \
-  if (recon == 0)                                                                              \
-    PTH_S16_R(NV, W, 0)                                                                        \
-  else                                                                                         \
-    PTH_S16_R(NV, W, 1)
-#define PTH_S16_CASE(NV)                                                                       \
-  case NV:                                                                                     \
-    if (minw == 3)                                                                             \
-      PTH_S16_W(NV, 3)                                                                         \
-    else                                                                                       \
-      PTH_S16_W(NV, 2)                                                                         \
-    break;
-    switch (V) {
-      PTH_S16_CASE(4)
-      PTH_S16_CASE(5)
-      PTH_S16_CASE(6)
-      PTH_S16_CASE(7)
-      PTH_S16_CASE(8)
-      PTH_S16_CASE(9)
-      PTH_S16_CASE(10)
-      PTH_S16_CASE(11)
-      PTH_S16_CASE(12)
-      PTH_S16_CASE(13)
-    }
-#undef PTH_S16_CASE
-#undef PTH_S16_W
-#undef PTH_S16_R
-    PTH_HIP(hipGetLastError());
-    if (groups) *groups = grid16;
-    return PTH_COMPLETE;
-  }
-  if (waves == 2) waves = 3;
   const int *fover = fc ? fc->dev_face : nullptr;
   const double *fcor = fc ? fc->store : nullptr;
   int grid = 0;
-#define PTH_SW_LAUNCH_W(NN, NV, W)                                                            \
-  {                                                                                           \
-    const int r = ResidentGroups(reinterpret_cast<const void *>(&BlockSweepKernel<NN, 4, NV, W>), \
-                                 NN * NN);                                                    \
-    if (r < 1) {                                                                              \
-      SetError("block sweep: occupancy query failed");                                        \
-      return PTH_FAIL;                                                                        \
-    }                                                                                         \
-    grid = std::min<std::int64_t>(std::min(std::max(r / spread, 1), max_partials),             \
-                                  static_cast<std::int64_t>(nb) * NN);                        \
-    hipLaunchKernelGGL((BlockSweepKernel<NN, 4, NV, W>), dim3(grid), dim3(NN * NN), 0, s, U,  \
-                       base, out, derived, partial, coef, nb, beta, dtvar, recon, fover, fcor, \
-                       push);                                                                 \
+  // a launch takes the resident workgroups divided by spread, at most one plane each
+  auto groups_of = [&](const void *kernel, int threads, std::int64_t planes) {
+    const int r = ResidentGroups(kernel, threads);
+    if (r < 1) SetError("block sweep: occupancy query failed");
+    grid = r < 1 ? 0
+                 : static_cast<int>(std::min<std::int64_t>(
+                       std::min(std::max(r / spread, 1), max_partials), planes));
+    return grid > 0;
+  };
+  if (RingSweep(t, V)) {
+    // built for 2 or 3 waves per SIMD
+    auto run = [&](auto kernel) {
+      if (!groups_of(reinterpret_cast<const void *>(kernel), 256,
+                     static_cast<std::int64_t>(nb) * 16))
+        return PTH_FAIL;
+      hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, U, base, out, derived, partial,
+                         coef, nb, beta, dtvar, fover, fcor, push, list);
+      return PTH_COMPLETE;
+    };
+    auto pick = [&](auto v) {
+      constexpr int NV = decltype(v)::value;
+      if (waves >= 3)
+        return recon == 0 ? run(BlockSweep16Kernel<NV, 3, 0>) : run(BlockSweep16Kernel<NV, 3, 1>);
+      return recon == 0 ? run(BlockSweep16Kernel<NV, 2, 0>) : run(BlockSweep16Kernel<NV, 2, 1>);
+    };
+    const pth_status st = V == 4   ? pick(std::integral_constant<int, 4>())
+                          : V == 5 ? pick(std::integral_constant<int, 5>())
+                          : V == 6 ? pick(std::integral_constant<int, 6>())
+                                   : pick(std::integral_constant<int, 7>());
+    if (st != PTH_COMPLETE) return PTH_FAIL;
+    PTH_HIP(hipGetLastError());
+    if (groups) *groups = grid;
+    return PTH_COMPLETE;
   }
-#define PTH_SW_LAUNCH(NN, NV)                                                                 \
-  if (waves == 4)                                                                             \
-    PTH_SW_LAUNCH_W(NN, NV, (NV <= 8 ? 4 : 2))                                                \
-  else                                                                                        \
-    PTH_SW_LAUNCH_W(NN, NV, (NV <= 8 ? 3 : 2))
-#define PTH_SW_CASE(NV)                                                                       \
-  case NV:                                                                                    \
-    if (N == 16) {                                                                            \
-      PTH_SW_LAUNCH(16, NV)                                                                   \
-    } else {                                                                                  \
-      PTH_SW_LAUNCH(8, NV)                                                                    \
-    }                                                                                         \
+  if (tiled) {
+    TileShape S;
+    S.n0 = t.fine.n[0];
+    S.n1 = t.fine.n[1];
+    S.n2 = t.fine.n[2];
+    S.e0 = t.fine.ent(0);
+    S.sz = S.e0 * t.fine.ent(1);
+    S.cs = S.sz * t.fine.ent(2);
+    S.tx = S.n0 / 16;
+    S.tiles = S.tx * (S.n1 / 16);
+    const std::int64_t planes = static_cast<std::int64_t>(nb) * S.tiles * S.n2;
+    auto run = [&](auto kernel, int threads) {
+      if (!groups_of(reinterpret_cast<const void *>(kernel), threads, planes)) return PTH_FAIL;
+      hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, s, U, base, out, derived, partial,
+                         coef, S, nb, beta, dtvar, fover, fcor, push, list);
+      return PTH_COMPLETE;
+    };
+    auto pick = [&](auto v) {
+      constexpr int NV = decltype(v)::value;
+      return recon == 0 ? run(TileSweepKernel<NV, 0>, 512) : run(TileSweepKernel<NV, 1>, 512);
+    };
+    pth_status st = PTH_FAIL;
+#define PTH_TS_CASE(NV)                          \
+  case NV:                                       \
+    st = pick(std::integral_constant<int, NV>()); \
+    break;
+    switch (V) {
+      PTH_TS_CASE(4)
+      PTH_TS_CASE(5)
+      PTH_TS_CASE(6)
+      PTH_TS_CASE(7)
+      PTH_TS_CASE(8)
+      PTH_TS_CASE(9)
+      PTH_TS_CASE(10)
+      PTH_TS_CASE(11)
+      PTH_TS_CASE(12)
+      PTH_TS_CASE(13)
+    }
+#undef PTH_TS_CASE
+    if (st != PTH_COMPLETE) return PTH_FAIL;
+    PTH_HIP(hipGetLastError());
+    if (groups) *groups = grid;
+    return PTH_COMPLETE;
+  }
+  if (waves == 2) waves = 3;
+#define PTH_SW_LAUNCH_W(NV, W)                                                                \
+  {                                                                                           \
+    if (!groups_of(reinterpret_cast<const void *>(&BlockSweepKernel<8, 4, NV, W>), 64,         \
+                   static_cast<std::int64_t>(nb) * 8))                                        \
+      return PTH_FAIL;                                                                        \
+    hipLaunchKernelGGL((BlockSweepKernel<8, 4, NV, W>), dim3(grid), dim3(64), 0, s, U, base,   \
+                       out, derived, partial, coef, nb, beta, dtvar, recon, fover, fcor, push); \
+  }
+#define PTH_SW_CASE(NV)                        \
+  case NV:                                     \
+    if (waves == 4)                            \
+      PTH_SW_LAUNCH_W(NV, (NV <= 8 ? 4 : 2))   \
+    else                                       \
+      PTH_SW_LAUNCH_W(NV, (NV <= 8 ? 3 : 2))   \
     break;
   switch (V) {
     PTH_SW_CASE(4)
@@ -942,7 +1473,6 @@ pth_status BurgersSweep(const Topology &t, int V, const double *U, const double 
     PTH_SW_CASE(13)
   }
 #undef PTH_SW_CASE
-#undef PTH_SW_LAUNCH
 #undef PTH_SW_LAUNCH_W
   PTH_HIP(hipGetLastError());
   if (groups) *groups = grid;
@@ -959,7 +1489,7 @@ pth_status FlxcorDirect(const Topology &t, int V, const FluxCorrection &fc, cons
   ProfScope prof("flxcor_direct", s);
   const Geo G = MakeGeo(t, V);
   const dim3 grid(static_cast<unsigned>(fc.host.size()), (4 * fc.max_cells + 63) / 64);
-  const bool ring = t.fine.n[0] == 16 && t.fine.g[0] == 4;
+  const bool ring = BurgersTileSweep(t, V);
 #define PTH_FD_CASE(NV)                                                                       \
   case NV:                                                                                    \
     if (ring)                                                                                 \
