@@ -36,8 +36,17 @@
 // exchange x, t = w (b - (A x - diag x)) / diag + (1 - w) x with the unigrid diagonal of
 // PoissonEquation::SetDiagonal (poisson_equation.hpp:86-125), x = t.
 //
-// Transfers between levels are region tables walked by the exchange's persistent restriction,
-// prolongation and box-copy kernels. FP64 throughout.
+// Launches. The coarse levels are a few microseconds of work each, so a V-cycle costs what its
+// launches cost. A stencil reads a neighbour in another block of the same level from that
+// block's interior (a table of face neighbours) and a FixedFace ghost as -u, so a level whose
+// blocks all have one size needs no exchange: a smoothing stage is one launch from x to its
+// second array, the residual goes straight into the coarser level's b, a correction straight
+// from the coarser x. Levels with blocks of different sizes first run the part of the
+// exchange that their stencils read: the channels between levels, and the same-level ghosts of
+// blocks that restrict them for their coarse neighbours. On the mesh of 568 16^3 blocks (one
+// refined level, 8 levels) a V-cycle with its residual norm takes 468 us as a replayed graph;
+// with exchange, stage and copy back as launches of their own, 160 of them, it took 1224 us
+// and the norm 120. FP64 throughout.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -48,6 +57,7 @@
 #include <vector>
 
 #include "pth_burgers.hpp"
+#include "pth_device.hpp"
 #include "pth_internal.hpp"
 #include "pth_mgtree.hpp"
 
@@ -55,89 +65,271 @@ namespace pth {
 namespace {
 
 constexpr int kWG = 256;
-enum { kX = 0, kT = 1, kB = 2, kR = 3, kD = 4 };  // level fields: solution/correction,
-                                                  // Jacobi output, right-hand side,
-                                                  // residual, face field D (3 components)
+enum { kX = 0, kT = 1, kB = 2, kD = 3 };  // level fields: solution/correction, its second array
+                                          // (levels of one block size), right-hand side, face
+                                          // field D (3 components)
 
-struct BrickShape {
-  int e0, e1;
-  int g0, g1, g2;
-  int n0, n1, n2;
-  long long cells;
+// A level's blocks for the kernels. face[6 b + 2 d + side]: the same-level block across that
+// face, or kFixed (FixedFace-0 boundary), or kGhost (a block of another level: the ghost cell
+// holds the exchanged value).
+constexpr int kFixed = -1, kGhost = -2;
+struct LevelView {
+  int n0, n1, n2;     // interior cells of a block
+  int e0, p;          // brick row pitch, plane stride
+  int first;          // brick offset of the first interior cell
+  int per, chunks;    // interior cells of a block, and workgroups over them
+  int ndim;
+  long long cells;    // brick cells
+  const int *face;
 };
 
-BrickShape ShapeOf(const Extent &x) {
-  BrickShape s;
-  s.e0 = x.ent(0), s.e1 = x.ent(1);
-  s.g0 = x.g[0], s.g1 = x.g[1], s.g2 = x.g[2];
-  s.n0 = x.n[0], s.n1 = x.n[1], s.n2 = x.n[2];
-  s.cells = x.cells();
+// 1 / dx^2 per dimension and, for a constant D, 1 / diagonal of a block
+struct StageCoef {
+  double i2[3], rdiag;
+};
+
+struct Local {
+  int i, j, k, c;  // cell of a block and its brick offset
+};
+__device__ __forceinline__ Local At(const LevelView &V, unsigned t) {
+  Local q;
+  const unsigned r = t / static_cast<unsigned>(V.n0);
+  q.i = static_cast<int>(t - r * static_cast<unsigned>(V.n0));
+  q.k = static_cast<int>(r / static_cast<unsigned>(V.n1));
+  q.j = static_cast<int>(r - static_cast<unsigned>(q.k) * static_cast<unsigned>(V.n1));
+  q.c = V.first + q.k * V.p + q.j * V.e0 + q.i;
+  return q;
+}
+
+// A cell's value and its neighbours' along the active dimensions, [d][low, high]; every load
+// unconditional (a FixedFace neighbour reads the cell itself and becomes its negative)
+struct Near {
+  double u, v[3][2];
+};
+__device__ __forceinline__ Near LoadNear(const double *__restrict__ x, const LevelView &V, int b,
+                                         const Local &q) {
+  const double *xb = x + b * V.cells;
+  const int *f = V.face + 6 * b;
+  Near o;
+  o.u = xb[q.c];
+  auto side = [&](int at, int n, int st, int lo, int hi, double (&v)[2]) {
+    const bool in0 = at > 0, in1 = at < n - 1;
+    const long long a0 = in0 || lo == kGhost ? q.c - st
+                         : lo >= 0           ? q.c + st * (n - 1) + (lo - b) * V.cells
+                                             : q.c;
+    const long long a1 = in1 || hi == kGhost ? q.c + st
+                         : hi >= 0           ? q.c - st * (n - 1) + (hi - b) * V.cells
+                                             : q.c;
+    const double x0 = xb[a0], x1 = xb[a1];
+    v[0] = !in0 && lo == kFixed ? 0.0 - o.u : x0;
+    v[1] = !in1 && hi == kFixed ? 0.0 - o.u : x1;
+  };
+  side(q.i, V.n0, 1, f[0], f[1], o.v[0]);
+  if (V.ndim > 1) side(q.j, V.n1, V.e0, f[2], f[3], o.v[1]);
+  if (V.ndim > 2) side(q.k, V.n2, V.p, f[4], f[5], o.v[2]);
+  return o;
+}
+
+// A x at a cell, D on the cell's faces from the face field Df (the block's 3-component brick,
+// component d = D on the lower face along d) or the constant D; *diag is the operator's
+// diagonal (SetDiagonal). Inverse squares of the cell widths in place of divisions: the values
+// are the reference's to rounding.
+__device__ __forceinline__ double ApplyA(const Near &o, const LevelView &V, const StageCoef &S,
+                                         double D, const double *Df, int c, double alpha,
+                                         double *diag) {
+  double ax = -alpha * o.u, dg = -alpha;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    if (d >= V.ndim) break;
+    const int st = d == 0 ? 1 : d == 1 ? V.e0 : V.p;
+    const double Dl = Df ? Df[d * V.cells + c] : D, Dh = Df ? Df[d * V.cells + c + st] : D;
+    ax += (Dl * (o.v[d][0] - o.u) - Dh * (o.u - o.v[d][1])) * S.i2[d];
+    dg -= (Dl + Dh) * S.i2[d];
+  }
+  *diag = dg;
+  return ax;
+}
+
+// The same in the operation order of CalculateFluxes + FluxMultiplyMatrix
+// (poisson_equation.hpp:131-205), for the residual that the solve reports and stops on.
+__device__ __forceinline__ double ApplyExact(const Near &o, const LevelView &V,
+                                             const BlockCoefs &C, double D, const double *Df,
+                                             int c, double alpha) {
+  double ax = -alpha * o.u;
+  const double f1l = (Df ? Df[c] : D) / C.dx[0] * (o.v[0][0] - o.u);
+  const double f1r = (Df ? Df[c + 1] : D) / C.dx[0] * (o.u - o.v[0][1]);
+  ax += (f1l - f1r) / C.dx[0];
+  if (V.ndim > 1) {
+    const double f2l = (Df ? Df[V.cells + c] : D) * (o.v[1][0] - o.u) / C.dx[1];
+    const double f2r = (Df ? Df[V.cells + c + V.e0] : D) * (o.u - o.v[1][1]) / C.dx[1];
+    ax += (f2l - f2r) / C.dx[1];
+  }
+  if (V.ndim > 2) {
+    const double f3l = (Df ? Df[2 * V.cells + c] : D) * (o.v[2][0] - o.u) / C.dx[2];
+    const double f3r = (Df ? Df[2 * V.cells + c + V.p] : D) * (o.u - o.v[2][1]) / C.dx[2];
+    ax += (f3l - f3r) / C.dx[2];
+  }
+  return ax;
+}
+
+// One Jacobi stage out = x + w (b - A x) / diag; ZERO: from x = 0, which is not read.
+template <bool ZERO>
+__global__ void __launch_bounds__(kWG)
+    StageKernel(const double *__restrict__ x, const double *__restrict__ b,
+                double *__restrict__ out, LevelView V, const StageCoef *__restrict__ coef,
+                double D, const double *__restrict__ Df, double alpha, double w) {
+  const unsigned L = XcdRemap(blockIdx.x, gridDim.x);
+  const int blk = static_cast<int>(L / static_cast<unsigned>(V.chunks));
+  const int t = static_cast<int>(L % static_cast<unsigned>(V.chunks)) * kWG +
+                static_cast<int>(threadIdx.x);
+  if (t >= V.per) return;
+  const Local q = At(V, t);
+  const StageCoef &S = coef[blk];
+  const double *Db = Df ? Df + blk * 3 * V.cells : nullptr;
+  const long long c = blk * V.cells + q.c;
+  Near o{};
+  if (!ZERO) o = LoadNear(x, V, blk, q);
+  double diag;
+  const double r = b[c] - ApplyA(o, V, S, D, Db, q.c, alpha, &diag);
+  out[c] = o.u + w * (Df ? r / diag : r * S.rdiag);
+}
+
+// Residual of a level into the coarser level's right-hand side. The first nchild records are
+// blocks whose residual is averaged over 2^ndim cells (RestrictAverage) into octant o of block
+// cb; the others are the same block on both levels.
+struct Xfer {
+  int fb, cb;
+  int o[3];
+  int child;
+};
+__global__ void __launch_bounds__(kWG)
+    ResidualDownKernel(const double *__restrict__ x, const double *__restrict__ b, LevelView V,
+                       const StageCoef *__restrict__ coef, double D,
+                       const double *__restrict__ Df, double alpha, double *__restrict__ bc,
+                       LevelView C, const Xfer *__restrict__ recs, int nchild, int cchunks) {
+  const unsigned L = XcdRemap(blockIdx.x, gridDim.x);
+  const bool child = L < static_cast<unsigned>(nchild * cchunks);
+  const unsigned M = child ? L : L - static_cast<unsigned>(nchild * cchunks);
+  const unsigned ch = static_cast<unsigned>(child ? cchunks : V.chunks);
+  const Xfer R = recs[M / ch + (child ? 0u : static_cast<unsigned>(nchild))];
+  const int t = static_cast<int>(M % ch) * kWG + static_cast<int>(threadIdx.x);
+  const StageCoef &S = coef[R.fb];
+  const double *Db = Df ? Df + R.fb * 3 * V.cells : nullptr;
+  const double *bb = b + R.fb * V.cells;
+  double diag;
+  if (!child) {
+    if (t >= V.per) return;
+    const Local q = At(V, t);
+    bc[R.cb * C.cells + C.first + q.k * C.p + q.j * C.e0 + q.i] =
+        bb[q.c] - ApplyA(LoadNear(x, V, R.fb, q), V, S, D, Db, q.c, alpha, &diag);
+    return;
+  }
+  const int s1 = V.ndim > 1 ? 2 : 1, s2 = V.ndim > 2 ? 2 : 1;
+  const int m0 = V.n0 / 2, m1 = V.n1 / s1, m2 = V.n2 / s2;
+  if (t >= m0 * m1 * m2) return;
+  const int I = t % m0, J = t / m0 % m1, K = t / m0 / m1;
+  double sum = 0.0;
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      if (a >= s2 || e >= s1) continue;
+      double pair[2];
+#pragma unroll
+      for (int f = 0; f < 2; ++f) {
+        Local q;
+        q.i = 2 * I + f;
+        q.j = s1 * J + e;
+        q.k = s2 * K + a;
+        q.c = V.first + q.k * V.p + q.j * V.e0 + q.i;
+        pair[f] = bb[q.c] - ApplyA(LoadNear(x, V, R.fb, q), V, S, D, Db, q.c, alpha, &diag);
+      }
+      sum += pair[0] + pair[1];
+    }
+  bc[R.cb * C.cells + C.first + (R.o[2] * m2 + K) * C.p + (R.o[1] * m1 + J) * C.e0 +
+     R.o[0] * m0 + I] = sum * (V.ndim == 3 ? 0.125 : V.ndim == 2 ? 0.25 : 0.5);
+}
+
+// The coarser level's x added to a level's: prolongated (ProlongateSharedLinear: from the coarse
+// cell and its neighbour on the fine cell's side along each dimension, the terms grouped like
+// pr_ops.hpp:261-283) into child blocks, as it is into blocks that are the same on both.
+__global__ void __launch_bounds__(kWG)
+    ProlongAddKernel(double *__restrict__ x, LevelView V, const double *__restrict__ xc,
+                     LevelView C, const Xfer *__restrict__ recs) {
+  const unsigned L = XcdRemap(blockIdx.x, gridDim.x);
+  const Xfer R = recs[L / static_cast<unsigned>(V.chunks)];
+  const int t = static_cast<int>(L % static_cast<unsigned>(V.chunks)) * kWG +
+                static_cast<int>(threadIdx.x);
+  if (t >= V.per) return;
+  const Local q = At(V, t);
+  double *xf = x + R.fb * V.cells + q.c;
+  if (!R.child) {
+    *xf = *xf + xc[R.cb * C.cells + C.first + q.k * C.p + q.j * C.e0 + q.i];
+    return;
+  }
+  const int fi[3] = {q.i, q.j, q.k}, n[3] = {V.n0, V.n1, V.n2};
+  int at[3], odd[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const bool on = d < V.ndim;
+    odd[d] = on ? fi[d] & 1 : 0;
+    at[d] = on ? R.o[d] * (n[d] / 2) + (fi[d] >> 1) : fi[d];
+  }
+  Local cq;
+  cq.i = at[0];
+  cq.j = at[1];
+  cq.k = at[2];
+  cq.c = C.first + cq.k * C.p + cq.j * C.e0 + cq.i;
+  const Near o = LoadNear(xc, C, R.cb, cq);
+  double g[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+    if (d < V.ndim) g[d] = 0.25 * (odd[d] ? o.v[d][1] - o.u : o.u - o.v[d][0]);
+  const double s0 = odd[0] ? 1.0 : -1.0;
+  const double s1 = odd[0] == odd[1] ? 1.0 : -1.0, s2 = odd[0] == odd[2] ? 1.0 : -1.0;
+  *xf = *xf + (o.u + s0 * ((g[0] + s1 * g[1]) + s2 * g[2]));
+}
+
+template <int WG>
+__device__ __forceinline__ double GroupSum(double v) {
+  __shared__ double w[WG / 64];
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double s = 0.0;
+  for (int q = 0; q < WG / 64; ++q) s += w[q];
   return s;
 }
 
-unsigned Grid(long long n) { return static_cast<unsigned>((n + kWG - 1) / kWG); }
-
-// brick offset of block `blk`'s interior cell t (flattened over its [k][j][i] interior)
-__device__ __forceinline__ long long Cell(const BrickShape &s, long long t) {
-  const long long per = static_cast<long long>(s.n0) * s.n1 * s.n2;
-  const long long blk = t / per;
-  const long long r = t % per;
-  const int i = static_cast<int>(r % s.n0);
-  const long long q = r / s.n0;
-  const int j = static_cast<int>(q % s.n1);
-  const int k = static_cast<int>(q / s.n1);
-  return blk * s.cells + (static_cast<long long>(k + s.g2) * s.e1 + (j + s.g1)) * s.e0 +
-         (i + s.g0);
+// Per-workgroup sums of the squared residual of every cell (fixed order, so every call gives
+// the same bits), then their sum.
+__global__ void __launch_bounds__(kWG)
+    ResidualNormKernel(const double *__restrict__ x, const double *__restrict__ b, LevelView V,
+                       const BlockCoefs *__restrict__ coef, double D,
+                       const double *__restrict__ Df, double alpha,
+                       double *__restrict__ partial) {
+  const unsigned L = XcdRemap(blockIdx.x, gridDim.x);
+  const int blk = static_cast<int>(L / static_cast<unsigned>(V.chunks));
+  const int t = static_cast<int>(L % static_cast<unsigned>(V.chunks)) * kWG +
+                static_cast<int>(threadIdx.x);
+  double r = 0.0;
+  if (t < V.per) {
+    const Local q = At(V, t);
+    r = 1.0 * b[blk * V.cells + q.c] +
+        (-1.0) * ApplyExact(LoadNear(x, V, blk, q), V, coef[blk], D,
+                            Df ? Df + blk * 3 * V.cells : nullptr, q.c, alpha);
+  }
+  const double s = GroupSum<kWG>(r * r);
+  if (threadIdx.x == 0) partial[L] = s;
 }
 
-// MODE 0: Jacobi stage out = w (b - (A x - diag x)) / diag + (1 - w) x
-// MODE 1: residual out = 1.0 b + (-1.0) A x (AddFieldsAndStoreInteriorSelect<rhs, Ax, res>)
-// A x in the operation order of CalculateFluxes + FluxMultiplyMatrix, diag as SetDiagonal;
-// D on the cell's faces from the face field Df ([block][3] bricks, component d = D on the
-// lower face along d) or the constant D when Df is null.
-template <int MODE>
-__global__ void __launch_bounds__(kWG)
-    LevelCellKernel(const double *__restrict__ x, const double *__restrict__ b,
-                    double *__restrict__ out, BrickShape s, const BlockCoefs *__restrict__ coef,
-                    double D, const double *__restrict__ Df, double alpha, double w, int ndim,
-                    long long total) {
-  const long long t = static_cast<long long>(blockIdx.x) * kWG + threadIdx.x;
-  if (t >= total) return;
-  const long long blk = t / (static_cast<long long>(s.n0) * s.n1 * s.n2);
-  const long long c = Cell(s, t);
-  const long long p = static_cast<long long>(s.e0) * s.e1;
-  const double *d0 = Df ? Df + blk * 3 * s.cells + (c - blk * s.cells) : nullptr;  // comp 0
-  const double u = x[c];
-  const double dx1 = coef[blk].dx[0];
-  const double D1l = Df ? d0[0] : D, D1h = Df ? d0[1] : D;
-  double ax = -alpha * u;
-  const double f1l = D1l / dx1 * (x[c - 1] - u);
-  const double f1r = D1h / dx1 * (u - x[c + 1]);
-  ax += (f1l - f1r) / dx1;
-  double diag = -(D1l + D1h) / (dx1 * dx1) - alpha;
-  if (ndim > 1) {
-    const double D2l = Df ? d0[s.cells] : D, D2h = Df ? d0[s.cells + s.e0] : D;
-    const double dx2 = coef[blk].dx[1];
-    const double f2l = D2l * (x[c - s.e0] - u) / dx2;
-    const double f2r = D2h * (u - x[c + s.e0]) / dx2;
-    ax += (f2l - f2r) / dx2;
-    diag -= (D2l + D2h) / (dx2 * dx2);
-  }
-  if (ndim > 2) {
-    const double D3l = Df ? d0[2 * s.cells] : D, D3h = Df ? d0[2 * s.cells + p] : D;
-    const double dx3 = coef[blk].dx[2];
-    const double f3l = D3l * (x[c - p] - u) / dx3;
-    const double f3r = D3h * (u - x[c + p]) / dx3;
-    ax += (f3l - f3r) / dx3;
-    diag -= (D3l + D3h) / (dx3 * dx3);
-  }
-  if (MODE == 0) {
-    const double off_diag = ax - diag * u;
-    const double val = b[c] - off_diag;
-    out[c] = w * (val / diag) + (1.0 - w) * u;
-  } else {
-    out[c] = 1.0 * b[c] + (-1.0) * ax;
-  }
+constexpr int kSumWG = 1024;
+__global__ void __launch_bounds__(kSumWG)
+    SumKernel(const double *__restrict__ partial, int n, double *__restrict__ out) {
+  double v = 0.0;
+  for (int p = threadIdx.x; p < n; p += kSumWG) v += partial[p];
+  const double s = GroupSum<kSumWG>(v);
+  if (threadIdx.x == 0) *out = s;
 }
 
 // Face-field restriction (RestrictAverage on faces) from a block into its coarser-level
@@ -194,37 +386,18 @@ __global__ void __launch_bounds__(kWG)
       sum / cnt;
 }
 
-// interior cells of every block: MODE 0: a = 0; MODE 1: a += b
-template <int MODE>
-__global__ void __launch_bounds__(kWG)
-    InteriorKernel(double *__restrict__ a, const double *__restrict__ b, BrickShape s,
-                   long long total) {
-  const long long t = static_cast<long long>(blockIdx.x) * kWG + threadIdx.x;
-  if (t >= total) return;
-  const long long c = Cell(s, t);
-  if (MODE == 0)
-    a[c] = 0.0;
-  else
-    a[c] = a[c] + b[c];
+__global__ void __launch_bounds__(kWG) ZeroKernel(double *__restrict__ x, LevelView V) {
+  const int blk = static_cast<int>(blockIdx.x) / V.chunks;
+  const int t = (static_cast<int>(blockIdx.x) % V.chunks) * kWG + static_cast<int>(threadIdx.x);
+  if (t < V.per) x[blk * V.cells + At(V, t).c] = 0.0;
 }
+
+unsigned Grid(long long n) { return static_cast<unsigned>((n + kWG - 1) / kWG); }
 
 // SRJ weights of mg_solver.hpp:312-345 (Yang & Mittal 2017), by dimension and stage count
 constexpr double kSrj2[3][2] = {{0.8723, 0.5395}, {1.3895, 0.5617}, {1.7319, 0.5695}};
 constexpr double kSrj3[3][3] = {
     {0.9372, 0.6667, 0.5173}, {1.6653, 0.8000, 0.5264}, {2.2473, 0.8571, 0.5296}};
-
-std::int64_t Offset(const Extent &e, int i, int j, int k) {
-  return (static_cast<std::int64_t>(k) * e.ent(1) + j) * e.ent(0) + i;
-}
-
-Box Interior(const Extent &e) {
-  Box b;
-  for (int d = 0; d < 3; ++d) {
-    b.lo[d] = e.g[d];
-    b.hi[d] = e.g[d] + e.n[d] - 1;
-  }
-  return b;
-}
 
 Box Whole(const Extent &e) {
   Box b;
@@ -277,24 +450,40 @@ enum class Coarsen {
 
 struct TreeLevel {
   std::unique_ptr<Mesh> mesh;
-  MeshData *md = nullptr;
+  // a smoothing stage goes from x[cur] to x[1 - cur]: two containers on a level with blocks of
+  // different sizes (each with its exchange tables), fields x and t of one container elsewhere
+  MeshData *md = nullptr, *other = nullptr;
+  double *x[2] = {nullptr, nullptr};
+  int cur = 0;
+  LevelView view{};
+  StageCoef *coef = nullptr;
+  int *face = nullptr;
   Coarsen to_coarser = Coarsen::kCap;
-  // to the next coarser level: r -> r's coarse buffers (restrict), then boxes -> its b (copy);
-  // its x -> t's coarse buffers or t (copy), then t's coarse buffers -> t (prolong)
-  Table restrict_r, copy_down, copy_up, prolong_t;
+  Xfer *xfer = nullptr;  // to the next coarser level, child blocks first
+  int nxfer = 0, nchild = 0, cchunks = 1;
+  // what a stencil's exchange needs, per container: region pairs of the channels between
+  // levels and of the same-level ghosts that a block restricts for its coarse neighbours, and
+  // the coarse-buffer conditions of blocks that prolongate
+  struct Cross {
+    Table send, recv;
+    BcTable bc;
+  } cross[2];
   // the face field D to the next coarser level: same blocks copied, the others face-averaged
   Table copy_D;
   std::vector<FaceXfer> face_host;
-  FaceXfer *face = nullptr;
+  FaceXfer *face_D = nullptr;
   FaceGeom face_geom{};
   long long cells = 0;  // interior cells of all blocks
   ~TreeLevel() {
-    restrict_r.Free();
-    copy_down.Free();
-    copy_up.Free();
-    prolong_t.Free();
+    for (Cross &q : cross) {
+      q.send.Free();
+      q.recv.Free();
+      q.bc.Free();
+    }
     copy_D.Free();
-    if (face) (void)hipFree(face);
+    for (void *q : {static_cast<void *>(face_D), static_cast<void *>(coef),
+                    static_cast<void *>(face), static_cast<void *>(xfer)})
+      if (q) (void)hipFree(q);
   }
 };
 
@@ -306,10 +495,11 @@ class MgTree {
   double D = 1.0, alpha = 0.0;
   std::vector<std::unique_ptr<TreeLevel>> lv;  // finest (a copy of the user's mesh) first
   std::vector<double> w_pre, w_post;           // Jacobi weight of each smoothing stage
-  // a V-cycle is ~10 launches per level, each a few microseconds of work on the coarse
-  // levels: after one eager V-cycle (which builds every level's exchange tables) the next is
-  // captured and later V-cycles replay it
+  // a V-cycle is ~6 launches per level, each a few microseconds of work on the coarse levels:
+  // the second V-cycle, with the residual norm after it, is captured and later ones replay it
   bool use_graph = true, warmed = false;
+  double *partial = nullptr, *norm_host = nullptr;  // residual norm: partials and their sum
+  int npartial = 0;
   hipGraph_t graph = nullptr;
   hipGraphExec_t graph_exec = nullptr;
   hipStream_t capture_stream = nullptr;
@@ -318,43 +508,133 @@ class MgTree {
     if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
     if (graph) (void)hipGraphDestroy(graph);
     if (capture_stream) (void)hipStreamDestroy(capture_stream);
+    if (partial) (void)hipFree(partial);
+    if (norm_host) (void)hipHostFree(norm_host);
   }
   pth_status Build();
   pth_status Setup(MeshData &md);
   pth_status Solve(MeshData &md, int *iters, std::vector<double> *history);
 
  private:
-  pth_status VCycle();
-  pth_status NewLevel(const Topology &t, bool coarse_buffers, int x_prolong);
+  pth_status Iterate(double *rms);
+  pth_status NewLevel(const Topology &t, int x_prolong);
   pth_status BuildTransfers(int l);
-  pth_status Exchange(int l, int field);
-  pth_status Cells(int l, int mode, int in, int out, double w);
-  pth_status Smooth(int l, const std::vector<double> &w);
+  pth_status BuildCross(TreeLevel &L, MeshData &md, TreeLevel::Cross &q);
+  pth_status Exchange(int l);
+  pth_status Smooth(int l, const std::vector<double> &w, bool zero);
   pth_status Cycle(int l);
+  pth_status Norm();
   pth_status Rms(double *rms);
   double *Data(int l, int f) { return lv[l]->md->store[f].data; }
+  const double *Df(int l) { return fD >= 0 ? Data(l, kD) : nullptr; }
+  hipStream_t Stream(int l) { return lv[l]->mesh->stream; }
 };
 
-pth_status MgTree::NewLevel(const Topology &t, bool coarse_buffers, int x_prolong) {
+pth_status MgTree::NewLevel(const Topology &t, int x_prolong) {
   std::unique_ptr<TreeLevel> L(new TreeLevel());
   L->mesh.reset(new Mesh());
   Mesh &m = *L->mesh;
   m.topo = t;
-  m.force_coarse = coarse_buffers;
   m.stream = user->stream;
-  const unsigned fill = PTH_FILL_GHOST | PTH_INDEPENDENT;
-  m.fields.push_back(FieldSpec{"x", 1, fill, x_prolong});
-  m.fields.push_back(FieldSpec{"t", 1, 0u, PTH_PROLONG_LINEAR});
-  m.fields.push_back(FieldSpec{"b", 1, 0u, PTH_PROLONG_LINEAR});
-  m.fields.push_back(FieldSpec{"r", 1, 0u, PTH_PROLONG_LINEAR});
-  m.fields.push_back(FieldSpec{"D", 3, 0u, PTH_PROLONG_LINEAR});
+  m.fields.push_back(FieldSpec{"x", 1, PTH_FILL_GHOST | PTH_INDEPENDENT, x_prolong});
+  m.fields.push_back(FieldSpec{"t", 1, PTH_ONE_COPY, PTH_PROLONG_LINEAR});
+  m.fields.push_back(FieldSpec{"b", 1, PTH_ONE_COPY, PTH_PROLONG_LINEAR});
+  m.fields.push_back(FieldSpec{"D", 3, PTH_ONE_COPY, PTH_PROLONG_LINEAR});
   if (m.Finalize() != PTH_COMPLETE) return PTH_FAIL;
   L->md = m.Get("base");
   if (!L->md) return PTH_FAIL;
-  const Extent &e = m.topo.fine;
-  L->cells = static_cast<long long>(m.topo.blocks.size()) * e.n[0] * e.n[1] * e.n[2];
+  const Topology &mt = m.topo;
+  const Extent &e = mt.fine;
+  const int nb = static_cast<int>(mt.blocks.size());
+  L->cells = static_cast<long long>(nb) * e.n[0] * e.n[1] * e.n[2];
+  L->x[0] = L->md->store[kX].data;
+  L->x[1] = L->md->store[kT].data;
+  if (mt.multilevel) {
+    L->other = m.Get("other");
+    if (!L->other) return PTH_FAIL;
+    L->x[1] = L->other->store[kX].data;
+    if (BuildCross(*L, *L->md, L->cross[0]) != PTH_COMPLETE ||
+        BuildCross(*L, *L->other, L->cross[1]) != PTH_COMPLETE)
+      return PTH_FAIL;
+  }
+  LevelView &V = L->view;
+  V.n0 = e.n[0], V.n1 = e.n[1], V.n2 = e.n[2];
+  V.e0 = e.ent(0);
+  V.p = e.ent(0) * e.ent(1);
+  V.first = e.g[2] * V.p + e.g[1] * V.e0 + e.g[0];
+  V.per = e.n[0] * e.n[1] * e.n[2];
+  V.chunks = (V.per + kWG - 1) / kWG;
+  V.ndim = mt.ndim;
+  V.cells = e.cells();
+  std::vector<int> face(6 * static_cast<size_t>(nb), kGhost);
+  std::vector<StageCoef> coef(nb);
+  for (int b = 0; b < nb; ++b) {
+    const Block &B = mt.blocks[b];
+    double diag = -alpha;
+    for (int d = 0; d < 3; ++d) {
+      coef[b].i2[d] = 1.0 / (B.dx[d] * B.dx[d]);
+      if (!mt.active[d]) continue;
+      diag -= (D + D) * coef[b].i2[d];
+      const double tol = 1e-12 * (mt.xmax[d] - mt.xmin[d]);
+      if (!mt.periodic[d]) {
+        if (std::fabs(B.xmin[d] - mt.xmin[d]) <= tol) face[6 * b + 2 * d] = kFixed;
+        if (std::fabs(B.xmax[d] - mt.xmax[d]) <= tol) face[6 * b + 2 * d + 1] = kFixed;
+      }
+    }
+    coef[b].rdiag = 1.0 / diag;
+    for (const Link &l : B.links) {
+      int d = -1, faces = 0;
+      for (int q = 0; q < 3; ++q)
+        if (l.off[q]) d = q, ++faces;
+      if (faces == 1 && l.level == B.at.level) face[6 * b + 2 * d + (l.off[d] > 0)] = l.gid;
+    }
+    // on a level of one block size every face has its block or the domain's condition
+    for (int f = 0; f < 2 * mt.ndim; ++f)
+      if (!mt.multilevel && face[6 * b + f] == kGhost) {
+        SetError("MGSolver hierarchy: a block face without a neighbour");
+        return PTH_FAIL;
+      }
+  }
+  PTH_HIP(hipMalloc(&L->face, sizeof(int) * face.size()));
+  PTH_HIP(hipMemcpy(L->face, face.data(), sizeof(int) * face.size(), hipMemcpyHostToDevice));
+  PTH_HIP(hipMalloc(&L->coef, sizeof(StageCoef) * nb));
+  PTH_HIP(hipMemcpy(L->coef, coef.data(), sizeof(StageCoef) * nb, hipMemcpyHostToDevice));
+  V.face = L->face;
   lv.push_back(std::move(L));
   return PTH_COMPLETE;
+}
+
+// The exchange of x in md cut to what a stencil reads (see the head of this file).
+pth_status MgTree::BuildCross(TreeLevel &L, MeshData &md, TreeLevel::Cross &q) {
+  Mesh &m = *L.mesh;
+  if (m.BuildCache(md, PTH_BT_ANY) != PTH_COMPLETE) return PTH_FAIL;
+  BoundCache &c = md.cache[PTH_BT_ANY];
+  if (!CanExchangeDirect(c.pack, c.unpack)) {
+    SetError("MGSolver hierarchy: exchange tables do not pair up");
+    return PTH_FAIL;
+  }
+  const FieldStore &x = md.store[kX];
+  const std::int64_t cells = m.topo.fine.cells(), ccells = m.topo.coarse.cells();
+  const size_t nb = m.topo.blocks.size();
+  std::vector<char> restricts(nb, 0), prolongs(nb, 0);
+  for (const Region &r : c.restrict_set.host) restricts[(r.a - x.data) / cells] = 1;
+  for (const Table *t : {&c.prolong, &c.prolong_linear})
+    for (const Region &r : t->host) prolongs[(r.a - x.data) / cells] = 1;
+  auto fine = [&](const double *a) { return a >= x.data && a < x.data + x.ndata; };
+  for (size_t i = 0; i < c.pack.host.size(); ++i) {
+    const Region &s = c.pack.host[i], &r = c.unpack.host[i];
+    if (s.b != r.b) {
+      SetError("internal: send and receive regions do not pair up");
+      return PTH_FAIL;
+    }
+    if (fine(s.a) && fine(r.a) && !restricts[(r.a - x.data) / cells]) continue;
+    q.send.host.push_back(s);
+    q.recv.host.push_back(r);
+  }
+  for (const BcBox &b : c.bc[1].host)
+    if (prolongs[(b.slab - x.coarse) / ccells]) q.bc.host.push_back(b);
+  if (q.send.Upload() != PTH_COMPLETE || q.recv.Upload() != PTH_COMPLETE) return PTH_FAIL;
+  return q.bc.Upload();
 }
 
 pth_status MgTree::Build() {
@@ -386,7 +666,7 @@ pth_status MgTree::Build() {
     }
     t.multilevel = !t.inner.empty();
     const int xp = L == top ? user->fields[fu].prolong : PTH_PROLONG_LINEAR;
-    if (NewLevel(t, true, xp) != PTH_COMPLETE) return PTH_FAIL;
+    if (NewLevel(t, xp) != PTH_COMPLETE) return PTH_FAIL;
     lv.back()->to_coarser = Coarsen::kCap;
   }
   // below the base grid: the forest's tree levels (root_level merges of 2^d base blocks,
@@ -427,22 +707,23 @@ pth_status MgTree::Build() {
       return PTH_FAIL;
     }
     for (int f = 0; f < 6; ++f) t.bc[f] = ut.bc[f];
-    if (NewLevel(t, true, PTH_PROLONG_LINEAR) != PTH_COMPLETE) return PTH_FAIL;
+    if (NewLevel(t, PTH_PROLONG_LINEAR) != PTH_COMPLETE) return PTH_FAIL;
   }
   for (int l = 0; l + 1 < static_cast<int>(lv.size()); ++l)
     if (BuildTransfers(l) != PTH_COMPLETE) return PTH_FAIL;
+  npartial = static_cast<int>(lv[0]->mesh->topo.blocks.size()) * lv[0]->view.chunks;
+  PTH_HIP(hipMalloc(&partial, sizeof(double) * (npartial + 1)));
+  PTH_HIP(hipHostMalloc(&norm_host, sizeof(double)));
   return PTH_COMPLETE;
 }
 
 pth_status MgTree::BuildTransfers(int l) {
   TreeLevel &F = *lv[l], &C = *lv[l + 1];
   const Topology &ft = F.mesh->topo, &ct = C.mesh->topo;
-  const Extent &fe = ft.fine, &ce = ft.coarse, &Ce = ct.fine;
+  const Extent &fe = ft.fine, &Ce = ct.fine;
   int top = 0;
   for (const auto &a : ft.leaf) top = std::max(top, a.level);
-  FieldStore &r = F.md->store[kR], &t = F.md->store[kT];
-  FieldStore &cb = C.md->store[kB], &cx = C.md->store[kX];
-  for (Table *q : {&F.restrict_r, &F.prolong_t}) q->item_elems = kProResItemElems;
+  std::vector<Xfer> kids, same;
   for (int fb = 0; fb < static_cast<int>(ft.blocks.size()); ++fb) {
     const Lattice &a = ft.blocks[fb].at;
     bool child = false;
@@ -457,70 +738,48 @@ pth_status MgTree::BuildTransfers(int l) {
       for (int d = 0; d < 3; ++d) target.x[d] = ft.active[d] ? a.x[d] / 2 : a.x[d];
     }
     if (child)
-      for (int d = 0; d < 3; ++d) o[d] = ft.active[d] ? static_cast<int>(a.x[d] - 2 * target.x[d]) : 0;
+      for (int d = 0; d < 3; ++d)
+        o[d] = ft.active[d] ? static_cast<int>(a.x[d] - 2 * target.x[d]) : 0;
     auto it = ct.id.find(target);
     if (it == ct.id.end()) {
       SetError("MGSolver hierarchy: a block has no counterpart on the coarser level");
       return PTH_FAIL;
     }
     const int cbk = it->second;
-    double *r_f = r.data + fb * fe.cells(), *r_c = r.coarse + fb * ce.cells();
-    double *t_f = t.data + fb * fe.cells(), *t_c = t.coarse + fb * ce.cells();
-    double *b_C = cb.data + cbk * Ce.cells(), *x_C = cx.data + cbk * Ce.cells();
     if (F.to_coarser == Coarsen::kCap && !child) {  // the same block on both levels
       if (fe.n[0] != Ce.n[0] || fe.n[1] != Ce.n[1] || fe.n[2] != Ce.n[2]) {
         SetError("MGSolver hierarchy: block shapes differ between levels");
         return PTH_FAIL;
       }
-      F.copy_down.host.push_back(
-          Rec(r_f, b_C + Offset(Ce, Ce.g[0], Ce.g[1], Ce.g[2]), Interior(fe), fb, fe, &Ce));
-      F.copy_up.host.push_back(
-          Rec(x_C, t_f + Offset(fe, fe.g[0], fe.g[1], fe.g[2]), Interior(Ce), cbk, Ce, &fe));
+      same.push_back(Xfer{fb, cbk, {0, 0, 0}, 0});
       F.copy_D.host.push_back(Rec(F.md->store[kD].data + fb * 3 * fe.cells(),
                                   C.md->store[kD].data + cbk * 3 * Ce.cells(), Whole(fe), fb,
                                   fe, &Ce, 3));
       continue;
     }
+    for (int d = 0; d < 3; ++d)
+      if (ft.active[d] && (fe.n[d] % 2 || (o[d] + 1) * (fe.n[d] / 2) > Ce.n[d])) {
+        SetError("MGSolver hierarchy: a block does not fit its coarser block");
+        return PTH_FAIL;
+      }
     F.face_host.push_back(FaceXfer{F.md->store[kD].data + fb * 3 * fe.cells(),
                                    C.md->store[kD].data + cbk * 3 * Ce.cells(),
                                    {o[0], o[1], o[2]}, 0});
-    // restriction of the block's interior into its coarse buffer, then into the target
-    const Box ci = Interior(ce);
-    F.restrict_r.host.push_back(Rec(r_f, r_c, ci, fb, fe, &ce));
-    int dst[3], src_lo[3];
-    for (int d = 0; d < 3; ++d) {
-      dst[d] = Ce.g[d] + o[d] * ce.n[d];
-      src_lo[d] = dst[d] - ce.g[d];
-    }
-    F.copy_down.host.push_back(Rec(r_c, b_C + Offset(Ce, dst[0], dst[1], dst[2]), ci, fb, ce, &Ce));
-    // the target's cells over the block and a ghost band of m >= 1 cells (the prolongation
-    // stencil reads one) -> t's coarse buffer
-    Box sb;
-    for (int d = 0; d < 3; ++d) {
-      const int m = std::min(ce.g[d], Ce.g[d]);
-      sb.lo[d] = src_lo[d] + ce.g[d] - m;
-      sb.hi[d] = sb.lo[d] + ce.n[d] + 2 * m - 1;
-      if (sb.lo[d] < 0 || sb.hi[d] >= Ce.ent(d) || (ft.active[d] && m < 1)) {
-        SetError("MGSolver hierarchy: prolongation source outside the coarser block (level " +
-                 std::to_string(l) + ", block " + std::to_string(fb) + ", dimension " +
-                 std::to_string(d) + ": cells " + std::to_string(sb.lo[d]) + ".." +
-                 std::to_string(sb.hi[d]) + " of " + std::to_string(Ce.ent(d)) + ")");
-        return PTH_FAIL;
-      }
-    }
-    const int m0 = std::min(ce.g[0], Ce.g[0]), m1 = std::min(ce.g[1], Ce.g[1]),
-              m2 = std::min(ce.g[2], Ce.g[2]);
-    F.copy_up.host.push_back(
-        Rec(x_C, t_c + Offset(ce, ce.g[0] - m0, ce.g[1] - m1, ce.g[2] - m2), sb, cbk, Ce, &ce));
-    F.prolong_t.host.push_back(Rec(t_f, t_c, ci, fb, fe, &ce));
+    kids.push_back(Xfer{fb, cbk, {o[0], o[1], o[2]}, 1});
   }
-  for (Table *q : {&F.restrict_r, &F.copy_down, &F.copy_up, &F.prolong_t, &F.copy_D})
-    if (q->Upload() != PTH_COMPLETE) return PTH_FAIL;
+  F.nchild = static_cast<int>(kids.size());
+  kids.insert(kids.end(), same.begin(), same.end());
+  F.nxfer = static_cast<int>(kids.size());
+  F.cchunks = (F.view.per / (1 << ft.ndim) + kWG - 1) / kWG;
+  PTH_HIP(hipMalloc(&F.xfer, sizeof(Xfer) * kids.size()));
+  PTH_HIP(hipMemcpy(F.xfer, kids.data(), sizeof(Xfer) * kids.size(), hipMemcpyHostToDevice));
+  if (F.copy_D.Upload() != PTH_COMPLETE) return PTH_FAIL;
   FaceGeom &G = F.face_geom;
   G.fe0 = fe.ent(0), G.fe1 = fe.ent(1), G.ce0 = Ce.ent(0), G.ce1 = Ce.ent(1);
   G.fcells = fe.cells(), G.ccells = Ce.cells();
   for (int d = 0; d < 3; ++d) {
-    G.fg[d] = fe.g[d], G.cg[d] = Ce.g[d], G.nc[d] = ce.n[d];
+    G.fg[d] = fe.g[d], G.cg[d] = Ce.g[d];
+    G.nc[d] = ft.active[d] ? fe.n[d] / 2 : fe.n[d];
     G.act[d] = ft.active[d] ? 1 : 0;
     // the upper face of the last cell lies in the first ghost cell on both levels
     if (ft.active[d] && (fe.g[d] < 1 || Ce.g[d] < 1)) {
@@ -530,82 +789,117 @@ pth_status MgTree::BuildTransfers(int l) {
   }
   G.ndim = ft.ndim;
   if (!F.face_host.empty()) {
-    PTH_HIP(hipMalloc(&F.face, sizeof(FaceXfer) * F.face_host.size()));
-    PTH_HIP(hipMemcpy(F.face, F.face_host.data(), sizeof(FaceXfer) * F.face_host.size(),
+    PTH_HIP(hipMalloc(&F.face_D, sizeof(FaceXfer) * F.face_host.size()));
+    PTH_HIP(hipMemcpy(F.face_D, F.face_host.data(), sizeof(FaceXfer) * F.face_host.size(),
                       hipMemcpyHostToDevice));
   }
   return PTH_COMPLETE;
 }
 
-pth_status MgTree::Exchange(int l, int field) {
-  (void)field;  // x is the only FillGhost field of a level
-  return pth_exchange_fused(reinterpret_cast<pth_meshdata *>(lv[l]->md), PTH_BT_ANY);
+// x's ghost cells that the level's stencils read (none on a level of one block size)
+pth_status MgTree::Exchange(int l) {
+  TreeLevel &L = *lv[l];
+  if (!L.other) return PTH_COMPLETE;
+  Mesh &m = *L.mesh;
+  BoundCache &c = (L.cur ? L.other : L.md)->cache[PTH_BT_ANY];
+  TreeLevel::Cross &q = L.cross[L.cur];
+  if (LaunchRestrictT(c.restrict_send, m.topo, m.geom, m.stream) != PTH_COMPLETE ||
+      LaunchExchangeDirect(q.send, q.recv, m.stream) != PTH_COMPLETE ||
+      LaunchRestrictT(c.restrict_set, m.topo, m.geom, m.stream) != PTH_COMPLETE ||
+      LaunchBoundaryConditions(q.bc, m.stream) != PTH_COMPLETE ||
+      LaunchProlongT(c.prolong, m.topo, m.geom, m.stream, true) != PTH_COMPLETE)
+    return PTH_FAIL;
+  return LaunchProlongT(c.prolong_linear, m.topo, m.geom, m.stream, false);
 }
 
-pth_status MgTree::Cells(int l, int mode, int in, int out, double w) {
-  Mesh &m = *lv[l]->mesh;
-  const long long total = lv[l]->cells;
-  const BrickShape s = ShapeOf(m.topo.fine);
-  const double *Df = fD >= 0 ? Data(l, kD) : nullptr;
-  ProfScope prof(mode == 0 ? "mg_level_jacobi" : "mg_level_residual", m.stream);
-  if (mode == 0)
-    hipLaunchKernelGGL(LevelCellKernel<0>, dim3(Grid(total)), dim3(kWG), 0, m.stream,
-                       Data(l, in), Data(l, kB), Data(l, out), s, m.coef, D, Df, alpha, w,
-                       m.topo.ndim, total);
-  else
-    hipLaunchKernelGGL(LevelCellKernel<1>, dim3(Grid(total)), dim3(kWG), 0, m.stream,
-                       Data(l, in), Data(l, kB), Data(l, out), s, m.coef, D, Df, alpha, w,
-                       m.topo.ndim, total);
-  PTH_HIP(hipGetLastError());
-  return PTH_COMPLETE;
-}
-
-pth_status MgTree::Smooth(int l, const std::vector<double> &w) {
-  Mesh &m = *lv[l]->mesh;
-  for (double wk : w) {
-    if (Exchange(l, kX) != PTH_COMPLETE) return PTH_FAIL;
-    if (Cells(l, 0, kX, kT, wk) != PTH_COMPLETE) return PTH_FAIL;
-    PTH_HIP(hipMemcpyAsync(Data(l, kX), Data(l, kT), sizeof(double) * lv[l]->md->store[kX].ndata,
-                           hipMemcpyDeviceToDevice, m.stream));
+// Smoothing stages with weights w; zero: the first starts from x = 0 (which is not stored)
+pth_status MgTree::Smooth(int l, const std::vector<double> &w, bool zero) {
+  TreeLevel &L = *lv[l];
+  const dim3 grid(static_cast<unsigned>(L.mesh->topo.blocks.size()) * L.view.chunks);
+  if (zero) L.cur = 0;
+  if (zero && w.empty()) {
+    hipLaunchKernelGGL(ZeroKernel, grid, dim3(kWG), 0, Stream(l), L.x[0], L.view);
+    PTH_HIP(hipGetLastError());
+  }
+  for (size_t q = 0; q < w.size(); ++q) {
+    if (zero && q == 0) {
+      ProfScope prof("mg_level_jacobi", Stream(l));
+      hipLaunchKernelGGL(StageKernel<true>, grid, dim3(kWG), 0, Stream(l), nullptr,
+                         Data(l, kB), L.x[0], L.view, L.coef, D, Df(l), alpha, w[q]);
+    } else {
+      if (Exchange(l) != PTH_COMPLETE) return PTH_FAIL;
+      ProfScope prof("mg_level_jacobi", Stream(l));
+      hipLaunchKernelGGL(StageKernel<false>, grid, dim3(kWG), 0, Stream(l), L.x[L.cur],
+                         Data(l, kB), L.x[1 - L.cur], L.view, L.coef, D, Df(l), alpha, w[q]);
+      L.cur = 1 - L.cur;
+    }
+    PTH_HIP(hipGetLastError());
   }
   return PTH_COMPLETE;
 }
 
 pth_status MgTree::Cycle(int l) {
   const int last = static_cast<int>(lv.size()) - 1;
-  if (Smooth(l, w_pre) != PTH_COMPLETE) return PTH_FAIL;
-  if (l == last) return PTH_COMPLETE;
-  TreeLevel &F = *lv[l], &C = *lv[l + 1];
-  Mesh &fm = *F.mesh, &cm = *C.mesh;
-  // residual, restricted into the coarser level's right-hand side; zero initial correction
-  if (Exchange(l, kX) != PTH_COMPLETE) return PTH_FAIL;
-  if (Cells(l, 1, kX, kR, 0.0) != PTH_COMPLETE) return PTH_FAIL;
-  if (LaunchRestrictT(F.restrict_r, fm.topo, fm.geom, fm.stream) != PTH_COMPLETE) return PTH_FAIL;
-  if (LaunchCopy(F.copy_down, fm.stream) != PTH_COMPLETE) return PTH_FAIL;
-  const BrickShape cs = ShapeOf(cm.topo.fine);
-  hipLaunchKernelGGL(InteriorKernel<0>, dim3(Grid(C.cells)), dim3(kWG), 0, cm.stream,
-                     Data(l + 1, kX), nullptr, cs, C.cells);
-  PTH_HIP(hipGetLastError());
-  if (Cycle(l + 1) != PTH_COMPLETE) return PTH_FAIL;
-  // the coarser correction, prolongated and added
-  if (Exchange(l + 1, kX) != PTH_COMPLETE) return PTH_FAIL;
-  if (LaunchCopy(F.copy_up, fm.stream) != PTH_COMPLETE) return PTH_FAIL;
-  if (LaunchProlongT(F.prolong_t, fm.topo, fm.geom, fm.stream, false) != PTH_COMPLETE)
-    return PTH_FAIL;
-  const BrickShape fs = ShapeOf(fm.topo.fine);
-  hipLaunchKernelGGL(InteriorKernel<1>, dim3(Grid(F.cells)), dim3(kWG), 0, fm.stream,
-                     Data(l, kX), Data(l, kT), fs, F.cells);
-  PTH_HIP(hipGetLastError());
-  return Smooth(l, w_post);
+  if (Smooth(l, w_pre, l > 0) != PTH_COMPLETE) return PTH_FAIL;
+  TreeLevel &F = *lv[l];
+  if (l < last) {
+    TreeLevel &C = *lv[l + 1];
+    // residual, restricted into the coarser level's right-hand side
+    if (Exchange(l) != PTH_COMPLETE) return PTH_FAIL;
+    {
+      ProfScope prof("mg_level_residual", Stream(l));
+      const unsigned grid = static_cast<unsigned>(F.nchild * F.cchunks +
+                                                  (F.nxfer - F.nchild) * F.view.chunks);
+      hipLaunchKernelGGL(ResidualDownKernel, dim3(grid), dim3(kWG), 0, Stream(l), F.x[F.cur],
+                         Data(l, kB), F.view, F.coef, D, Df(l), alpha, Data(l + 1, kB), C.view,
+                         F.xfer, F.nchild, F.cchunks);
+      PTH_HIP(hipGetLastError());
+    }
+    if (Cycle(l + 1) != PTH_COMPLETE) return PTH_FAIL;
+    // the coarser correction, prolongated and added
+    if (Exchange(l + 1) != PTH_COMPLETE) return PTH_FAIL;
+    {
+      ProfScope prof("mg_level_prolong", Stream(l));
+      hipLaunchKernelGGL(ProlongAddKernel,
+                         dim3(static_cast<unsigned>(F.nxfer) * F.view.chunks), dim3(kWG), 0,
+                         Stream(l), F.x[F.cur], F.view, C.x[C.cur], C.view, F.xfer);
+      PTH_HIP(hipGetLastError());
+    }
+    if (Smooth(l, w_post, false) != PTH_COMPLETE) return PTH_FAIL;
+  }
+  if (l == 0 && F.cur == 1) {  // an odd number of stages: back to the first array
+    PTH_HIP(hipMemcpyAsync(F.x[0], F.x[1], sizeof(double) * F.md->store[kX].ndata,
+                           hipMemcpyDeviceToDevice, Stream(0)));
+    F.cur = 0;
+  }
+  return PTH_COMPLETE;
 }
 
-pth_status MgTree::VCycle() {
-  if (!use_graph) return Cycle(0);
-  if (!warmed) {
+// sum of squares of the leaf level's residual into partial[npartial]
+pth_status MgTree::Norm() {
+  TreeLevel &L = *lv[0];
+  if (Exchange(0) != PTH_COMPLETE) return PTH_FAIL;
+  ProfScope prof("mg_residual_norm", Stream(0));
+  hipLaunchKernelGGL(ResidualNormKernel, dim3(npartial), dim3(kWG), 0, Stream(0), L.x[0],
+                     Data(0, kB), L.view, L.mesh->coef, D, Df(0), alpha, partial);
+  hipLaunchKernelGGL(SumKernel, dim3(1), dim3(kSumWG), 0, Stream(0), partial, npartial,
+                     partial + npartial);
+  PTH_HIP(hipGetLastError());
+  return PTH_COMPLETE;
+}
+
+// one V-cycle and the RMS residual after it
+pth_status MgTree::Iterate(double *rms) {
+  auto both = [&]() -> pth_status {
+    if (Cycle(0) != PTH_COMPLETE) return PTH_FAIL;
+    return Norm();
+  };
+  if (!use_graph || !warmed) {
     warmed = true;
-    return Cycle(0);
+    if (both() != PTH_COMPLETE) return PTH_FAIL;
+    return Rms(rms);
   }
-  hipStream_t s = lv[0]->mesh->stream;
+  hipStream_t s = Stream(0);
   if (!graph_exec) {
     // the caller's stream may be the null stream, which cannot be captured: the levels launch
     // on a stream of the solver's own while the V-cycle is captured
@@ -619,7 +913,7 @@ pth_status MgTree::VCycle() {
     pth_status st = PTH_FAIL;
     hipGraph_t g = nullptr;
     if (began) {
-      st = Cycle(0);
+      st = both();
       e = hipStreamEndCapture(capture_stream, &g);
     }
     Prof().on = prof;
@@ -633,19 +927,19 @@ pth_status MgTree::VCycle() {
     graph = g;
     PTH_HIP(hipGraphInstantiate(&graph_exec, g, nullptr, nullptr, 0));
   }
-  ProfScope prof("mg_vcycle_graph", s);
-  PTH_HIP(hipGraphLaunch(graph_exec, s));
-  return PTH_COMPLETE;
+  {
+    ProfScope prof("mg_vcycle_graph", s);
+    PTH_HIP(hipGraphLaunch(graph_exec, s));
+  }
+  return Rms(rms);
 }
 
+// the RMS residual from the sum that Norm left (waits for it)
 pth_status MgTree::Rms(double *rms) {
-  if (Exchange(0, kX) != PTH_COMPLETE) return PTH_FAIL;
-  if (Cells(0, 1, kX, kR, 0.0) != PTH_COMPLETE) return PTH_FAIL;
-  double sum = 0.0;
-  if (pth_solver_dot_product(reinterpret_cast<pth_meshdata *>(lv[0]->md), "r", "r", &sum) !=
-      PTH_COMPLETE)
-    return PTH_FAIL;
-  *rms = std::sqrt(sum / static_cast<double>(lv[0]->cells));
+  PTH_HIP(hipMemcpyAsync(norm_host, partial + npartial, sizeof(double), hipMemcpyDeviceToHost,
+                         Stream(0)));
+  PTH_HIP(hipStreamSynchronize(Stream(0)));
+  *rms = std::sqrt(*norm_host / static_cast<double>(lv[0]->cells));
   return PTH_COMPLETE;
 }
 
@@ -662,6 +956,7 @@ pth_status MgTree::Setup(MeshData &md) {
       SetError("MGSolver: the mesh changed since the solver was created");
       return PTH_FAIL;
     }
+  lv[0]->cur = 0;
   const size_t n = sizeof(double) * md.store[fu].ndata;
   PTH_HIP(hipMemcpyAsync(Data(0, kX), md.store[fu].data, n, hipMemcpyDeviceToDevice, m0.stream));
   PTH_HIP(hipMemcpyAsync(Data(0, kB), md.store[frhs].data, n, hipMemcpyDeviceToDevice,
@@ -679,7 +974,7 @@ pth_status MgTree::Setup(MeshData &md) {
     for (int d = 0; d < 3; ++d) per_rec *= G.act[d] ? G.nc[d] + 1 : 1;
     const long long total = per_rec * static_cast<long long>(F.face_host.size());
     hipLaunchKernelGGL(FaceRestrictKernel, dim3(Grid(total)), dim3(kWG), 0, F.mesh->stream,
-                       F.face, G, per_rec, total);
+                       F.face_D, G, per_rec, total);
     PTH_HIP(hipGetLastError());
   }
   return PTH_COMPLETE;
@@ -688,13 +983,12 @@ pth_status MgTree::Setup(MeshData &md) {
 pth_status MgTree::Solve(MeshData &md, int *iters, std::vector<double> *history) {
   history->clear();
   double rms = 0.0;
-  if (Rms(&rms) != PTH_COMPLETE) return PTH_FAIL;
+  if (Norm() != PTH_COMPLETE || Rms(&rms) != PTH_COMPLETE) return PTH_FAIL;
   history->push_back(rms);
   int it = 0;
   do {
-    if (VCycle() != PTH_COMPLETE) return PTH_FAIL;
+    if (Iterate(&rms) != PTH_COMPLETE) return PTH_FAIL;
     ++it;
-    if (Rms(&rms) != PTH_COMPLETE) return PTH_FAIL;
     history->push_back(rms);
   } while (rms > P.residual_tolerance && it < P.max_iters);
   *iters = it;
