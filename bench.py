@@ -274,19 +274,19 @@ def gmg_bench(args, quick=False):
     kb = {"gmg_outer": 32 * c, "gmg_pre_l0": 2 * es * c, "gmg_jacobi_l0": 3 * es * c,
           "gmg_restrict_l0": 2 * es * c + es * c // 8,
           "gmg_prolong_l0": 2 * es * c + es * c // 8,
+          # one pass down (b, and x in a second inner cycle, read; x and coarse b written) and
+          # one up (x, b and coarse x read, the iterate written)
+          "gmg_pre_restrict_l0": (2 * es * c + es * c // 8 +
+                                  es * c * (args.inner_cycles - 1) // args.inner_cycles),
           "gmg_prolong_jacobi_l0": 3 * es * c + es * c // 8}
     prof = m["prof"]
     dom = max((k for k in prof if k in kb), key=lambda k: prof[k][1])
     n_l, ms = prof[dom]
     avg_s = ms / n_l * 1e-3
     achieved = kb[dom] / avg_s / 1e9
-    # per outer iteration: the finest level's traffic plus 1/7 of it for the coarser levels;
-    # a V-cycle's level traffic: pre-smoothing (b read, x written), residual-restriction (x, b
-    # read, coarse b written), prolongation inside the first post-sweep (x, b, coarse x read,
-    # t written) and the second post-sweep (x, b read, t written)
-    fused = "gmg_prolong_jacobi_l0" in prof
-    vc = (2 * es + (2 * es + es / 8) + (3 * es + es / 8) + 3 * es if fused
-          else 2 * es + 2 * 3 * es + 2 * (2 * es + es / 8))
+    # per outer iteration: the finest level's traffic plus 1/7 of it for the coarser levels; a
+    # V-cycle's level traffic is that of the two passes
+    vc = (kb["gmg_pre_restrict_l0"] + kb["gmg_prolong_jacobi_l0"]) / c
     it_bytes = int(32 * c + vc * c * 8 / 7)
     per_it = m["wall"] / m["steps"] / max(m["iters"] * args.inner_cycles, 1)
     out = {

@@ -356,8 +356,8 @@ pth_status pth_gmg_reset(pth_gmg *g);
 /* V-cycles per FP64 refinement step (default 1); cycles after the first continue from the
  * current correction on the same right-hand side. */
 pth_status pth_gmg_set_inner_cycles(pth_gmg *g, int k);
-/* Tuning (no counterpart in the reference): with on != 0 (the default) Jacobi sweeps of levels
- * whose size is a multiple of 64 run by z columns (z neighbours kept in registers); the
+/* Tuning (no counterpart in the reference): with on != 0 (the default) a level's sweeps and
+ * transfers run in one pass each way by z columns (z neighbours kept in registers); the
  * results are the same bits either way. */
 pth_status pth_gmg_set_column_sweeps(pth_gmg *h, int on);
 /* MGSolver::AddTasks iteration (mg_solver.hpp:119-161): V-cycles until the relative L2

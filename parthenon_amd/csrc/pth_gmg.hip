@@ -33,12 +33,20 @@ namespace {
 
 constexpr int kWG = 256;
 
-template <typename T>
-__device__ __forceinline__ T Ratio(T a, T b) {  // robust::ratio (utils/robust.hpp:59-62)
-  const T sgn = b >= T(0) ? T(1) : T(-1);
-  const T small = T(10) * (sizeof(T) == 8 ? T(DBL_MIN) : T(FLT_MIN));
-  return a / (b + sgn * small);
+// a / d for many a: the products with the rounded reciprocal y = 1 / d, corrected by the
+// remainder until the quotient is the correctly rounded one (Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", 1990: one step from a quotient
+// that is within one unit in the last place). The first step makes it that for any d. Infinite
+// products pass through, so an overflow gives what a division gives.
+__device__ __forceinline__ double DivBy(double a, double d, double y) {
+  double q = a * y;
+  const bool big = __builtin_isinf(q);
+  const double q0 = q;
+  q = __builtin_fma(__builtin_fma(-q, d, a), y, q);
+  q = __builtin_fma(__builtin_fma(-q, d, a), y, q);
+  return big ? q0 : q;
 }
+__device__ __forceinline__ float DivBy(float a, float d, float) { return a / d; }
 
 template <typename T>
 __device__ __forceinline__ T Diagonal(T dx) {  // SetDiagonal (poisson_equation.hpp:86-125)
@@ -49,27 +57,31 @@ __device__ __forceinline__ T Diagonal(T dx) {  // SetDiagonal (poisson_equation.
   return d;
 }
 
-// Per-level constants. Divisions by dx, by the restriction's total volume and by the coarse
-// spacing become multiplications by their inverses where that gives the same bits (n a power
-// of two: the divisors are powers of two), and always in FP32, where the inner cycle only has
-// to reduce the error; the FP64 Jacobi keeps the reference's division by the diagonal.
+// Per-level constants. With n a power of two (mul) every factor of the operator, the
+// restriction and the prolongation is a power of two, which commutes with rounding: the
+// factors are gathered into one product per cell, with the reference's bits. FP32 levels take
+// the same form for every n, since there the inner cycle only has to reduce the error.
 template <typename T>
 struct Lv {
-  T dx, idx, D, rD, tv, itv;
+  T dx, rdx, idx2, D, rD, tv;
   bool mul;
 };
 template <typename T>
 __device__ __forceinline__ Lv<T> MakeLv(int n) {
   Lv<T> o;
   o.dx = T(1) / T(n);
-  o.idx = T(n);
   o.mul = sizeof(T) == 4 || (n & (n - 1)) == 0;
-  o.D = Diagonal(o.dx);
-  const T small = T(10) * (sizeof(T) == 8 ? T(DBL_MIN) : T(FLT_MIN));
-  o.rD = T(1) / (o.D + (o.D >= T(0) ? T(1) : T(-1)) * small);
+  o.idx2 = T(n) * T(n);
+  if (o.mul) {
+    o.D = T(-6) * o.idx2;
+    o.rdx = T(n);
+  } else {
+    o.D = Diagonal(o.dx);
+    o.rdx = T(1) / o.dx;
+  }
+  o.rD = T(1) / o.D;
   const T vol = o.dx * o.dx * o.dx;
   o.tv = ((vol + vol) + (vol + vol)) + ((vol + vol) + (vol + vol));
-  o.itv = T(1) / o.tv;
   return o;
 }
 
@@ -77,30 +89,13 @@ __device__ __forceinline__ Lv<T> MakeLv(int n) {
 // across a domain face are the FixedFace-0 ghost -u.
 template <typename T>
 __device__ __forceinline__ T ApplyA(T u, T xm, T xp, T ym, T yp, T zm, T zp, const Lv<T> &o) {
-  const T D = T(1), alpha = T(0);
-  T out = -alpha * u;
-  if (o.mul) {  // D / dx == idx and x / dx == x * idx
-    const T f1l = o.idx * (xm - u);
-    const T f1r = o.idx * (u - xp);
-    out += (f1l - f1r) * o.idx;
-    const T f2l = D * (ym - u) * o.idx;
-    const T f2r = D * (u - yp) * o.idx;
-    out += (f2l - f2r) * o.idx;
-    const T f3l = D * (zm - u) * o.idx;
-    const T f3r = D * (u - zp) * o.idx;
-    out += (f3l - f3r) * o.idx;
-    return out;
-  }
+  if (o.mul)
+    return ((((xm - u) + (xp - u)) + ((ym - u) + (yp - u))) + ((zm - u) + (zp - u))) * o.idx2;
   const T dx = o.dx;
-  const T f1l = D / dx * (xm - u);
-  const T f1r = D / dx * (u - xp);
-  out += (f1l - f1r) / dx;
-  const T f2l = D * (ym - u) / dx;
-  const T f2r = D * (u - yp) / dx;
-  out += (f2l - f2r) / dx;
-  const T f3l = D * (zm - u) / dx;
-  const T f3r = D * (u - zp) / dx;
-  out += (f3l - f3r) / dx;
+  auto div = [&](T a) { return DivBy(a, dx, o.rdx); };
+  T out = div(o.rdx * (xm - u) - o.rdx * (u - xp));  // D / dx is the rounded 1 / dx
+  out += div(div(ym - u) - div(u - yp));
+  out += div(div(zm - u) - div(u - zp));
   return out;
 }
 
@@ -165,12 +160,26 @@ __device__ __forceinline__ Nbrs<T> LoadG(const T *x0, int c, const Cell &q, int 
   return v;
 }
 
+// One weighted Jacobi update: w (b - (A u - D u)) / D + (1 - w) u. In FP32 the off-diagonal part
+// is the sum of the neighbours itself (the terms in u cancel), in fused operations: 5 sums and
+// 3 products for 24 operations, with fewer roundings.
 template <typename T>
 __device__ __forceinline__ T JacobiPoint(const Nbrs<T> &v, T b, const Lv<T> &o, T w) {
-  const T off = ApplyA(v.u, v.xm, v.xp, v.ym, v.yp, v.zm, v.zp, o) - o.D * v.u;
-  const T val = b - off;
-  const T q = sizeof(T) == 4 ? val * o.rD : Ratio(val, o.D);
-  return w * q + (T(1) - w) * v.u;
+  if constexpr (sizeof(T) == 4) {
+    const T sum = ((v.xm + v.xp) + (v.ym + v.yp)) + (v.zm + v.zp);
+    return __builtin_fmaf(w * o.rD, __builtin_fmaf(-o.idx2, sum, b), (T(1) - w) * v.u);
+  } else {
+    const T off = ApplyA(v.u, v.xm, v.xp, v.ym, v.yp, v.zm, v.zp, o) - o.D * v.u;
+    return w * DivBy(b - off, o.D, o.rD) + (T(1) - w) * v.u;
+  }
+}
+
+// The first Jacobi sweep from x = 0: JacobiPoint with zero neighbours, whose operator part
+// vanishes.
+template <typename T>
+__device__ __forceinline__ T JacobiZero(T b, const Lv<T> &o, T w) {
+  if constexpr (sizeof(T) == 4) return w * o.rD * b;
+  return w * DivBy(b, o.D, o.rD);
 }
 
 // Entry q of a launch. Inline entries are selected with constant indices only, so the kernel
@@ -324,21 +333,20 @@ __global__ void __launch_bounds__(kWG)
   if (c >= n * n * n) return;
   const Cell q = Decode(c, n);
   const Lv<T> o = MakeLv<T>(n);
-  const Nbrs<T> zero = {T(0), T(0), T(0), T(0), T(0), T(0), T(0)};
   const T *b = e.b;
   if (!PRE2) {
-    Glob(e.x)[c] = JacobiPoint(zero, Glob(b)[c], o, w);
+    Glob(e.x)[c] = JacobiZero(static_cast<T>(Glob(b)[c]), o, w);
     return;
   }
   const Nbrs<T> bb = LoadG(b, c, q, n);
   Nbrs<T> x1;
-  x1.u = JacobiPoint(zero, bb.u, o, w);
-  x1.xm = q.i > 0 ? JacobiPoint(zero, bb.xm, o, w) : -x1.u;
-  x1.xp = q.i < n - 1 ? JacobiPoint(zero, bb.xp, o, w) : -x1.u;
-  x1.ym = q.j > 0 ? JacobiPoint(zero, bb.ym, o, w) : -x1.u;
-  x1.yp = q.j < n - 1 ? JacobiPoint(zero, bb.yp, o, w) : -x1.u;
-  x1.zm = q.k > 0 ? JacobiPoint(zero, bb.zm, o, w) : -x1.u;
-  x1.zp = q.k < n - 1 ? JacobiPoint(zero, bb.zp, o, w) : -x1.u;
+  x1.u = JacobiZero(bb.u, o, w);
+  x1.xm = q.i > 0 ? JacobiZero(bb.xm, o, w) : -x1.u;
+  x1.xp = q.i < n - 1 ? JacobiZero(bb.xp, o, w) : -x1.u;
+  x1.ym = q.j > 0 ? JacobiZero(bb.ym, o, w) : -x1.u;
+  x1.yp = q.j < n - 1 ? JacobiZero(bb.yp, o, w) : -x1.u;
+  x1.zm = q.k > 0 ? JacobiZero(bb.zm, o, w) : -x1.u;
+  x1.zp = q.k < n - 1 ? JacobiZero(bb.zp, o, w) : -x1.u;
   Glob(e.x)[c] = JacobiPoint(x1, bb.u, o, w);
 }
 
@@ -363,107 +371,15 @@ __global__ void __launch_bounds__(kWG)
   Glob(e.t)[c] = JacobiPoint(LoadG(static_cast<const T *>(e.x), c, q, n), Glob(e.b)[c], o, w);
 }
 
-// One Jacobi sweep x -> t by z columns: a workgroup covers 64 x 4 cells of NZ consecutive
-// planes, each thread marches its column keeping the z neighbours in registers (the x and y
-// neighbours come from the cache). Same operations as JacobiKernel; for n % 64 == 0 and
-// n % NZ == 0.
-template <typename T, int NZ>
-__global__ void __launch_bounds__(kWG) JacobiZKernel(const GmgArgs<T> A, T w) {
-  int local;
-  const GmgEntry<T> e = Find(A, local);
-  const int n = e.n, tx = n / 64, ty = n / 4;
-  const int bx = local % tx, r = local / tx, by = r % ty, bz = r / ty;
-  const int i = bx * 64 + static_cast<int>(threadIdx.x % 64);
-  const int j = by * 4 + static_cast<int>(threadIdx.x / 64);
-  const int k0 = bz * NZ;
-  const Lv<T> o = MakeLv<T>(n);
-  const int s1 = n, s2 = n * n;
-  const auto *x = Glob(static_cast<const T *>(e.x));
-  const auto *b = Glob(static_cast<const T *>(e.b));
-  auto *t = Glob(e.t);
-  int c = (k0 * n + j) * n + i;
-  // neighbours outside the array read the cell itself (unconditional loads) and are replaced
-  T cur = x[c];
-  T prev = x[k0 > 0 ? c - s2 : c];
-  T next = x[k0 + 1 < n ? c + s2 : c];
-#pragma unroll 2
-  for (int k = k0; k < k0 + NZ; ++k, c += s2) {
-    const T xm = x[i > 0 ? c - 1 : c], xp = x[i < n - 1 ? c + 1 : c];
-    const T ym = x[j > 0 ? c - s1 : c], yp = x[j < n - 1 ? c + s1 : c];
-    const T bc = b[c];
-    const T nn = x[k + 2 < n ? c + 2 * s2 : c];
-    Nbrs<T> v;
-    v.u = cur;
-    v.xm = i > 0 ? xm : -v.u;
-    v.xp = i < n - 1 ? xp : -v.u;
-    v.ym = j > 0 ? ym : -v.u;
-    v.yp = j < n - 1 ? yp : -v.u;
-    v.zm = k > 0 ? prev : -v.u;
-    v.zp = k < n - 1 ? next : -v.u;
-    t[c] = JacobiPoint(v, bc, o, w);
-    prev = cur;
-    cur = next;
-    next = nn;
-  }
-}
-
-// Column form of the fused pre-smoothing: a workgroup covers 64 x 4 cells of NZ consecutive
-// planes and each thread marches its column with the z neighbours of b in registers; the
-// operations per cell are those of PreZeroKernel<T, true>. (A column form of the FP64 outer
-// step measured slower than OuterKernel and is not used.)
-struct ZCell {
-  int i, j, k0, c;
-};
-__device__ __forceinline__ ZCell ZStart(int n, int local, int nz) {
-  const int tx = n / 64, ty = n / 4;
-  const int bx = local % tx, r = local / tx, by = r % ty, bz = r / ty;
-  ZCell z;
-  z.i = bx * 64 + static_cast<int>(threadIdx.x % 64);
-  z.j = by * 4 + static_cast<int>(threadIdx.x / 64);
-  z.k0 = bz * nz;
-  z.c = (z.k0 * n + z.j) * n + z.i;
-  return z;
-}
-
-template <typename T, int NZ>
-__global__ void __launch_bounds__(kWG) PreZero2ZKernel(const GmgArgs<T> A, T w) {
-  int local;
-  const GmgEntry<T> e = Find(A, local);
-  const int n = e.n, s1 = n, s2 = n * n;
-  const ZCell z = ZStart(n, local, NZ);
-  const int i = z.i, j = z.j;
-  int c = z.c;
-  const Lv<T> o = MakeLv<T>(n);
-  const Nbrs<T> zero = {T(0), T(0), T(0), T(0), T(0), T(0), T(0)};
-  const auto *b = Glob(static_cast<const T *>(e.b));
-  auto *x = Glob(e.x);
-  // neighbours outside the array read the cell itself (unconditional loads) and are replaced
-  T bprev = b[z.k0 > 0 ? c - s2 : c], bcur = b[c];
-  T bnext = b[z.k0 + 1 < n ? c + s2 : c];
-  for (int k = z.k0; k < z.k0 + NZ; ++k, c += s2) {
-    const T bxm = b[i > 0 ? c - 1 : c], bxp = b[i < n - 1 ? c + 1 : c];
-    const T bym = b[j > 0 ? c - s1 : c], byp = b[j < n - 1 ? c + s1 : c];
-    const T bnn = b[k + 2 < n ? c + 2 * s2 : c];
-    Nbrs<T> x1;
-    x1.u = JacobiPoint(zero, bcur, o, w);
-    x1.xm = i > 0 ? JacobiPoint(zero, bxm, o, w) : -x1.u;
-    x1.xp = i < n - 1 ? JacobiPoint(zero, bxp, o, w) : -x1.u;
-    x1.ym = j > 0 ? JacobiPoint(zero, bym, o, w) : -x1.u;
-    x1.yp = j < n - 1 ? JacobiPoint(zero, byp, o, w) : -x1.u;
-    x1.zm = k > 0 ? JacobiPoint(zero, bprev, o, w) : -x1.u;
-    x1.zp = k < n - 1 ? JacobiPoint(zero, bnext, o, w) : -x1.u;
-    x[c] = JacobiPoint(x1, bcur, o, w);
-    bprev = bcur;
-    bcur = bnext;
-    bnext = bnn;
-  }
-}
-
+// RestrictAverage of the 8 children's residuals, t[z][y][x]: the reference's sum of volume times
+// residual over the total volume.
 template <typename T>
 __device__ __forceinline__ T Restrict8(const T t[2][2][2], const Lv<T> &o) {
-  const T sum = ((t[0][0][0] + t[0][1][0]) + (t[0][0][1] + t[0][1][1])) +
-                ((t[1][0][0] + t[1][1][0]) + (t[1][0][1] + t[1][1][1]));
-  return o.mul ? sum * o.itv : sum / o.tv;
+  const T vol = o.mul ? T(1) : o.dx * o.dx * o.dx;
+  auto v = [&](int a, int b, int c) { return o.mul ? t[a][b][c] : vol * t[a][b][c]; };
+  const T sum = ((v(0, 0, 0) + v(0, 1, 0)) + (v(0, 0, 1) + v(0, 1, 1))) +
+                ((v(1, 0, 0) + v(1, 1, 0)) + (v(1, 0, 1) + v(1, 1, 1)));
+  return o.mul ? sum * T(0.125) : sum / o.tv;
 }
 
 // residual of the 8 children of one coarse cell and their average (RestrictAverage) into the
@@ -477,7 +393,6 @@ __global__ void __launch_bounds__(kWG)
   if (cc >= nc * nc * nc) return;
   const Cell p = Decode(cc, nc);
   const Lv<T> o = MakeLv<T>(n);
-  const T vol = o.dx * o.dx * o.dx;
   T t[2][2][2];
 #pragma unroll
   for (int a = 0; a < 2; ++a)
@@ -489,45 +404,46 @@ __global__ void __launch_bounds__(kWG)
         const int c = (q.k * n + q.j) * n + q.i;
         const Nbrs<T> v = LoadG(static_cast<const T *>(e.x), c, q, n);
         const T r = Glob(e.b)[c] - ApplyA(v.u, v.xm, v.xp, v.ym, v.yp, v.zm, v.zp, o);
-        t[a][bb][c2] = vol * r;
+        t[a][bb][c2] = r;
       }
   Glob(e.bc)[cc] = Restrict8(t, o);
 }
 
-// ProlongateSharedLinear of the coarse correction xc at fine cell q of an n^3 level (coarse
-// ghosts from the Dirichlet condition; pr_ops.hpp:166-289 term grouping). Every load is
-// unconditional: a coarse neighbour outside the level reads the cell itself and the ghost
-// value replaces it.
+// ProlongateSharedLinear (pr_ops.hpp:166-289) from a coarse cell fc and its neighbours f1, f2,
+// f3 (x, y, z) on the fine cell's side, the Dirichlet ghost where there is none. The reference
+// adds +/- (gradient x offset), grouped as +/- (x +/- y +/- z) with signs of the child's
+// offsets; the signs cancel against those of the one-sided gradients, and for power-of-two
+// spacings gradient x offset is a quarter of the difference.
+template <typename T>
+__device__ __forceinline__ T ProlongPoint(T fc, T f1, T f2, T f3, int oi, int oj, int ok,
+                                          const Lv<T> &oc) {
+  if (oc.mul) return fc + T(0.25) * (((f1 - fc) + (f2 - fc)) + (f3 - fc));
+  const T hc = oc.dx, df = T(0.25) * hc;
+  auto grad = [&](T diff) { return DivBy(diff, hc, oc.rdx); };
+  const T g1 = grad(oi ? f1 - fc : fc - f1);
+  const T g2 = grad(oj ? f2 - fc : fc - f2);
+  const T g3 = grad(ok ? f3 - fc : fc - f3);
+  const T so = oi ? T(1) : T(-1);
+  const T sb = oi == oj ? T(1) : T(-1);
+  const T sc = oi == ok ? T(1) : T(-1);
+  return fc + so * ((g1 * df + sb * (g2 * df)) + sc * (g3 * df));
+}
+
+// The same at fine cell q of an n^3 level. Every load is unconditional: a coarse neighbour
+// outside the level reads the cell itself and the ghost value replaces it.
 template <typename T, typename P>
-__device__ __forceinline__ T ProlongValue(const P *xc, int nc, const Cell &q) {
+__device__ __forceinline__ T ProlongValue(const P *xc, int nc, const Cell &q, const Lv<T> &oc) {
   const Cell p = {q.i >> 1, q.j >> 1, q.k >> 1};
   const int oi = q.i & 1, oj = q.j & 1, ok = q.k & 1;
   const int cc = (p.k * nc + p.j) * nc + p.i;
   const T fc = xc[cc];
-  const Lv<T> oc = MakeLv<T>(nc);
-  const T hc = oc.dx, df = T(0.25) * hc;
-  auto grad = [&](T diff) { return oc.mul ? diff * oc.idx : diff / hc; };
-  // the one-sided gradient on this child's side of the coarse cell, per dimension
   const bool in1 = oi ? p.i < nc - 1 : p.i > 0;
   const bool in2 = oj ? p.j < nc - 1 : p.j > 0;
   const bool in3 = ok ? p.k < nc - 1 : p.k > 0;
   const T l1 = xc[in1 ? cc + (oi ? 1 : -1) : cc];
   const T l2 = xc[in2 ? cc + (oj ? nc : -nc) : cc];
   const T l3 = xc[in3 ? cc + (ok ? nc * nc : -nc * nc) : cc];
-  const T f1 = in1 ? l1 : -fc;
-  const T f2 = in2 ? l2 : -fc;
-  const T f3 = in3 ? l3 : -fc;
-  const T g1 = grad(oi ? f1 - fc : fc - f1);
-  const T g2 = grad(oj ? f2 - fc : fc - f2);
-  const T g3 = grad(ok ? f3 - fc : fc - f3);
-  // fc +/- (g1 df +/- g2 df +/- g3 df) with the signs of the child's offsets, grouped like the
-  // reference's eight cases (pr_ops.hpp:261-283): the outer sign is the x offset's, the inner
-  // signs are relative to it; a product with -1 and an added negation round exactly like the
-  // subtractions they stand for
-  const T so = oi ? T(1) : T(-1);
-  const T sb = oi == oj ? T(1) : T(-1);
-  const T sc = oi == ok ? T(1) : T(-1);
-  return fc + so * ((g1 * df + sb * (g2 * df)) + sc * (g3 * df));
+  return ProlongPoint(fc, in1 ? l1 : -fc, in2 ? l2 : -fc, in3 ? l3 : -fc, oi, oj, ok, oc);
 }
 
 // x += ProlongateSharedLinear(coarse x); one thread per fine cell
@@ -538,182 +454,475 @@ __global__ void __launch_bounds__(kWG) ProlongKernel(const GmgArgs<T> A) {
   const int n = e.n, c = local * kWG + threadIdx.x;
   if (c >= n * n * n) return;
   const Cell q = Decode(c, n);
-  const T v = ProlongValue<T>(Glob(static_cast<const T *>(e.xc)), e.nc, q);
+  const T v = ProlongValue<T>(Glob(static_cast<const T *>(e.xc)), e.nc, q, MakeLv<T>(e.nc));
   Glob(e.x)[c] += v;
 }
 
-// Prolongation fused into the first post-smoothing sweep, column form: t = J(x + P xc), the
-// same values as ProlongKernel followed by JacobiZKernel. A workgroup covers 64 x 4 cells of
-// NZ consecutive planes; per plane, the corrected values x' = x + P xc of its cells and of the
-// one-cell ring around them (rows j0 - 1 and j0 + 4, columns i0 - 1 and i0 + 64) are staged
-// in LDS for the x and y neighbours, and each thread keeps x' of its column at k - 1, k, k + 1
-// in registers. The level's x is read, never written (after the launch t holds the iterate).
-template <typename T, int NZ>
-__global__ void __launch_bounds__(kWG) ProlongJacobiZKernel(const GmgArgs<T> A, T w) {
-  constexpr int TW = 66;  // tile width: 64 cells and one on each side
-  __shared__ T tile[6][TW];
+// ---- one pass over a level ------------------------------------------------------------
+// Source values, up to two Jacobi sweeps and the restriction of the residual in one kernel:
+//   kFromZero: the first sweep from x = 0, formed from b alone (writes x)
+//   kFromX:    the level's x (writes t)
+//   kFromBelow: x + P xc, the correction of the coarser level (writes t)
+// then NS sweeps, then (RES) the residual and its restriction into the coarser right-hand side.
+// A workgroup covers TX x TY cells of nz planes and marches in z. With H = NS + RES it holds
+// the tile and H cells around it: each thread owns SL columns of that area, keeps two planes of
+// every stage of them in registers for the z neighbours and leaves the newest in LDS for the x
+// and y neighbours of the next stage, which runs one plane behind; planes of LDS alternate, so
+// a plane takes one barrier. A cell's values come from the operations of the one-stage kernels
+// in the same order, so the results are the same bits.
+// Traffic per cell of a 2 + 2 cycle: 5.25 values (b; x, b and xc) against 17 (FP64) and 13
+// (FP32, prolongation inside the first sweep) with a launch per stage, and 2 launches a level
+// instead of 5 and 4; what bounds a large level now is the instructions of the overlapped area
+// (1.5 times the cells at H = 2), what bounds a small one the march. Per V-cycle, outer step and
+// bottom included (2 + 2, FP32 with 2 cycles a step, FP64 with 1): 64^3 103 -> 59 and 131 -> 81 us,
+// 128^3 156 -> 101 and 220 -> 156, 256^3 440 -> 321 and 953 -> 640.
+enum { kFromZero = 0, kFromX = 1, kFromBelow = 2 };
+
+template <int TX_, int TY_, int WG_>
+struct PassTile {
+  static constexpr int TX = TX_, TY = TY_, WG = WG_;
+};
+using PassLarge = PassTile<64, 16, 512>;
+using PassSmall = PassTile<32, 8, 512>;
+
+template <typename T, int SRC, int NS, bool RES, typename F>
+struct PassShape {
+  static constexpr int H = NS + (RES ? 1 : 0), PX = F::TX + 2 * H, PY = F::TY + 2 * H;
+  static constexpr int NC = PX * PY - 4;  // no stage reads the four corners
+  static constexpr int SL = (NC + F::WG - 1) / F::WG;
+  static constexpr int PAD = PX + 1, LP = PX * PY + 2 * PAD;  // one plane, neighbours in range
+  static constexpr int LDS = H * 2 * LP + (RES ? 2 * F::TX * F::TY : 0);
+};
+
+template <typename T, int SRC, int NS, bool RES, typename F, bool MUL>
+__device__ __forceinline__ void PassBody(const GmgEntry<T> &e, int local, int nz, T w, T *lds) {
+  using P = PassShape<T, SRC, NS, RES, F>;
+  constexpr int H = P::H, PX = P::PX, SL = P::SL, LP = P::LP;
+  const int n = e.n, nc = e.nc, s2 = n * n, c2 = nc * nc;
+  const int tx = (n + F::TX - 1) / F::TX, ty = (n + F::TY - 1) / F::TY;
+  const int x0 = local % tx * F::TX, y0 = local / tx % ty * F::TY, k0 = local / (tx * ty) * nz;
+  const int k1 = min(k0 + nz, n);
+  Lv<T> o = MakeLv<T>(n), oc = MakeLv<T>(nc);
+  o.mul = oc.mul = MUL;  // known when compiling
+  const T vol = o.dx * o.dx * o.dx;
+  const auto *gx = Glob(static_cast<const T *>(e.x));
+  const auto *gb = Glob(static_cast<const T *>(e.b));
+  const auto *gc = Glob(static_cast<const T *>(e.xc));
+  auto *go = Glob(SRC == kFromZero ? e.x : e.t);
+
+  // this thread's columns (cells past the level's edge: clamped positions whose values nobody
+  // reads; threads past the area repeat its last column)
+  unsigned col[SL], cc[SL];
+  int li[SL], ri[SL], d1[SL], d2[SL];
+  bool xl[SL], xr[SL], yl[SL], yr[SL], in[SL], in1[SL], in2[SL], oi[SL], oj[SL];
+#pragma unroll
+  for (int q = 0; q < SL; ++q) {
+    int m = min(static_cast<int>(threadIdx.x) + q * F::WG, P::NC - 1) + 1;
+    if (m >= PX - 1) ++m;
+    if (m >= (P::PY - 1) * PX) ++m;
+    const int lx = m % PX, ly = m / PX;
+    li[q] = m + P::PAD;
+    ri[q] = (ly - H) * F::TX + (lx - H);
+    const int gi = x0 + lx - H, gj = y0 + ly - H;
+    in[q] = lx >= H && lx < PX - H && ly >= H && ly < P::PY - H && gi < n && gj < n;
+    const int i = min(max(gi, 0), n - 1), j = min(max(gj, 0), n - 1);
+    xl[q] = i > 0;
+    xr[q] = i < n - 1;
+    yl[q] = j > 0;
+    yr[q] = j < n - 1;
+    col[q] = static_cast<unsigned>(j * n + i);
+    if (SRC == kFromBelow) {
+      const int pi = i >> 1, pj = j >> 1;
+      oi[q] = (i & 1) != 0;
+      oj[q] = (j & 1) != 0;
+      in1[q] = oi[q] ? pi < nc - 1 : pi > 0;
+      in2[q] = oj[q] ? pj < nc - 1 : pj > 0;
+      cc[q] = static_cast<unsigned>(pj * nc + pi);
+      d1[q] = in1[q] ? (oi[q] ? 1 : -1) : 0;
+      d2[q] = in2[q] ? (oj[q] ? nc : -nc) : 0;
+    }
+  }
+
+  T B[SL][H + 1], bn[SL];           // b of planes p, p - 1, .. and the next one
+  T X[SL], xn[SL];                  // source x of plane p and the next one
+  T a[NS + 1][SL], c[NS + 1][SL];   // stage s at planes p - s - 2 and p - s - 1
+  T lo[SL], mid[SL], hi[SL], l1[SL], l2[SL], hn[SL], l1n[SL], l2n[SL];  // coarse column
+  T half = T(0);                    // restriction: sum over the pair's lower plane
+  auto plane = [&](int k) { return min(max(k, 0), n - 1); };
+  const int p0 = k0 - H, p1 = k1 + H;
+#pragma unroll
+  for (int q = 0; q < SL; ++q) {
+    const auto *b = gb + static_cast<std::int64_t>(plane(p0)) * s2;
+    B[q][0] = b[col[q]];
+#pragma unroll
+    for (int h = 1; h <= H; ++h) B[q][h] = T(0);
+    if (SRC != kFromZero) X[q] = (gx + static_cast<std::int64_t>(plane(p0)) * s2)[col[q]];
+    if (SRC == kFromBelow) {
+      const int K = plane(p0) >> 1;
+      lo[q] = (gc + static_cast<std::int64_t>(max(K - 1, 0)) * c2)[cc[q]];
+      mid[q] = (gc + static_cast<std::int64_t>(K) * c2)[cc[q]];
+      hi[q] = (gc + static_cast<std::int64_t>(min(K + 1, nc - 1)) * c2)[cc[q]];
+      l1[q] = (gc + static_cast<std::int64_t>(K) * c2)[cc[q] + d1[q]];
+      l2[q] = (gc + static_cast<std::int64_t>(K) * c2)[cc[q] + d2[q]];
+    }
+#pragma unroll
+    for (int s = 0; s <= NS; ++s) a[s][q] = c[s][q] = T(0);
+  }
+
+  for (int p = p0; p < p1; ++p) {
+    const int pn = plane(p + 1);
+    const bool nextK = SRC == kFromBelow && (pn >> 1) != (plane(p) >> 1);
+    {  // the next plane's loads
+      const auto *b = gb + static_cast<std::int64_t>(pn) * s2;
+      const auto *x = gx + static_cast<std::int64_t>(pn) * s2;
+#pragma unroll
+      for (int q = 0; q < SL; ++q) {
+        bn[q] = b[col[q]];
+        if (SRC != kFromZero) xn[q] = x[col[q]];
+      }
+      if (nextK) {
+        const int K = pn >> 1;
+        const auto *m = gc + static_cast<std::int64_t>(K) * c2;
+        const auto *h = gc + static_cast<std::int64_t>(min(K + 1, nc - 1)) * c2;
+#pragma unroll
+        for (int q = 0; q < SL; ++q) {
+          hn[q] = h[cc[q]];
+          l1n[q] = m[cc[q] + d1[q]];
+          l2n[q] = m[cc[q] + d2[q]];
+        }
+      }
+    }
+    if (RES && p - H - 1 >= k0) {  // restriction of the plane before
+      const int r = p - H - 1;
+      if (threadIdx.x < F::TX / 2 * (F::TY / 2)) {
+        const int ci = threadIdx.x % (F::TX / 2), cj = threadIdx.x / (F::TX / 2);
+        const T *R = lds + H * 2 * LP + (r & 1) * F::TX * F::TY + 2 * cj * F::TX + 2 * ci;
+        const T sum = (R[0] + R[F::TX]) + (R[1] + R[F::TX + 1]);
+        if (r & 1) {
+          const T all = half + sum;
+          const int gi = x0 / 2 + ci, gj = y0 / 2 + cj;
+          if (gi < nc && gj < nc)
+            Glob(e.bc)[(r / 2 * nc + gj) * nc + gi] = MUL ? all * T(0.125) : all / o.tv;
+        }
+        half = sum;
+      }
+    }
+    T v[SL];  // the newest values of the stage before
+#pragma unroll
+    for (int q = 0; q < SL; ++q) {
+      if (SRC == kFromZero)
+        v[q] = JacobiZero(B[q][0], o, w);
+      else if (SRC == kFromX)
+        v[q] = X[q];
+      else {  // ProlongValue at plane p
+        const int k = plane(p), ok = k & 1, K = k >> 1;
+        const T fc = mid[q];
+        const T f3 = ok ? (K < nc - 1 ? hi[q] : -fc) : (K > 0 ? lo[q] : -fc);
+        v[q] = X[q] + ProlongPoint(fc, in1[q] ? l1[q] : -fc, in2[q] ? l2[q] : -fc, f3, oi[q],
+                                   oj[q], ok, oc);
+      }
+      if (H > 0) lds[(p & 1) * LP + li[q]] = v[q];
+    }
+    if (nextK) {
+#pragma unroll
+      for (int q = 0; q < SL; ++q) {
+        lo[q] = mid[q];
+        mid[q] = hi[q];
+        hi[q] = hn[q];
+        l1[q] = l1n[q];
+        l2[q] = l2n[q];
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < H; ++s) {  // stage s + 1 at plane k = p - s - 1
+      const int k = p - s - 1;
+      const T *L = lds + (2 * s + (k & 1)) * LP;
+      T *M = lds + (2 * (s + 1) + (k & 1)) * LP;
+#pragma unroll
+      for (int q = 0; q < SL; ++q) {
+        Nbrs<T> u;
+        u.u = c[s][q];
+        const T xm = L[li[q] - 1], xp = L[li[q] + 1], ym = L[li[q] - PX], yp = L[li[q] + PX];
+        u.xm = xl[q] ? xm : -u.u;
+        u.xp = xr[q] ? xp : -u.u;
+        u.ym = yl[q] ? ym : -u.u;
+        u.yp = yr[q] ? yp : -u.u;
+        u.zm = k > 0 ? a[s][q] : -u.u;
+        u.zp = k < n - 1 ? v[q] : -u.u;
+        a[s][q] = c[s][q];
+        c[s][q] = v[q];
+        if (s < NS) {
+          v[q] = JacobiPoint(u, B[q][s + 1], o, w);
+          if (s + 1 < H) M[li[q]] = v[q];
+        } else {
+          const T r = B[q][s + 1] - ApplyA(u.u, u.xm, u.xp, u.ym, u.yp, u.zm, u.zp, o);
+          if (in[q]) lds[H * 2 * LP + (k & 1) * F::TX * F::TY + ri[q]] = MUL ? r : vol * r;
+        }
+      }
+      if (s + 1 == NS && k >= k0 && k < k1) {
+        auto *out = go + static_cast<std::int64_t>(k) * s2;
+#pragma unroll
+        for (int q = 0; q < SL; ++q)
+          if (in[q]) out[col[q]] = v[q];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < SL; ++q) {
+#pragma unroll
+      for (int h = H; h > 0; --h) B[q][h] = B[q][h - 1];
+      B[q][0] = bn[q];
+      if (SRC != kFromZero) X[q] = xn[q];
+    }
+    __syncthreads();
+  }
+  if (RES) {  // the last plane
+    const int r = k1 - 1;
+    if (threadIdx.x < F::TX / 2 * (F::TY / 2)) {
+      const int ci = threadIdx.x % (F::TX / 2), cj = threadIdx.x / (F::TX / 2);
+      const T *R = lds + H * 2 * LP + (r & 1) * F::TX * F::TY + 2 * cj * F::TX + 2 * ci;
+      const T all = half + ((R[0] + R[F::TX]) + (R[1] + R[F::TX + 1]));
+      const int gi = x0 / 2 + ci, gj = y0 / 2 + cj;
+      if (gi < nc && gj < nc)
+        Glob(e.bc)[(r / 2 * nc + gj) * nc + gi] = MUL ? all * T(0.125) : all / o.tv;
+    }
+  }
+}
+
+template <typename T, int SRC, int NS, bool RES, typename F>
+__global__ void __launch_bounds__(F::WG) PassKernel(const GmgArgs<T> A, int nz, T w) {
+  __shared__ T lds[PassShape<T, SRC, NS, RES, F>::LDS];
   int local;
   const GmgEntry<T> e = Find(A, local);
-  const int n = e.n, nc = e.nc, s2 = n * n;
-  const ZCell z = ZStart(n, local, NZ);
-  const int i = z.i, j = z.j, lx = static_cast<int>(threadIdx.x % 64),
-            ly = static_cast<int>(threadIdx.x / 64);
-  const int i0 = i - lx, j0 = j - ly;
-  int c = z.c;
-  const Lv<T> o = MakeLv<T>(n);
-  const auto *x = Glob(static_cast<const T *>(e.x));
-  const auto *b = Glob(static_cast<const T *>(e.b));
-  const auto *xc = Glob(static_cast<const T *>(e.xc));
-  auto *t = Glob(e.t);
-  // x + P xc at a cell of the level (callers clamp positions into the level)
-  auto xp1 = [&](int ii, int jj, int kk) -> T {
-    const Cell q = {ii, jj, kk};
-    return x[(kk * n + jj) * n + ii] + ProlongValue<T>(xc, nc, q);
-  };
-  // the ring cell this thread fills: 66 + 66 cells of rows 0 and 5, then columns 0 and 65 of
-  // rows 1..4 (140 cells; threads 140..255 fill none)
-  const int h = static_cast<int>(threadIdx.x);
-  const int hr = h < TW ? 0 : h < 2 * TW ? 5 : 1 + (h - 2 * TW) / 2;
-  const int hc = h < TW ? h : h < 2 * TW ? h - TW : ((h - 2 * TW) % 2 ? TW - 1 : 0);
-  const int hi = min(max(i0 - 1 + hc, 0), n - 1), hj = min(max(j0 - 1 + hr, 0), n - 1);
-  const bool ring = h < 2 * TW + 8;
-  T prev = xp1(i, j, max(z.k0 - 1, 0));
-  T cur = xp1(i, j, z.k0);
-  T next = xp1(i, j, min(z.k0 + 1, n - 1));
-  for (int k = z.k0; k < z.k0 + NZ; ++k, c += s2) {
-    tile[ly + 1][lx + 1] = cur;
-    if (ring) tile[hr][hc] = xp1(hi, hj, k);
-    const T bc = b[c];
-    const T nn = xp1(i, j, min(k + 2, n - 1));
-    __syncthreads();
-    Nbrs<T> v;
-    v.u = cur;
-    v.xm = i > 0 ? tile[ly + 1][lx] : -v.u;
-    v.xp = i < n - 1 ? tile[ly + 1][lx + 2] : -v.u;
-    v.ym = j > 0 ? tile[ly][lx + 1] : -v.u;
-    v.yp = j < n - 1 ? tile[ly + 2][lx + 1] : -v.u;
-    v.zm = k > 0 ? prev : -v.u;
-    v.zp = k < n - 1 ? next : -v.u;
-    t[c] = JacobiPoint(v, bc, o, w);
-    __syncthreads();  // the next plane overwrites the tile
-    prev = cur;
-    cur = next;
-    next = nn;
-  }
+  if (sizeof(T) == 4 || (e.n & (e.n - 1)) == 0)
+    PassBody<T, SRC, NS, RES, F, true>(e, local, nz, w, lds);
+  else
+    PassBody<T, SRC, NS, RES, F, false>(e, local, nz, w, lds);
 }
 
 // ---- bottom of the V-cycle in one workgroup (levels of at most NB cells per side) --------
-template <typename T>
-__device__ void BSweep(T *x, T *t, const T *b, int n, T w, bool zero) {
-  const int N3 = n * n * n;
-  const Lv<T> o = MakeLv<T>(n);
-  const Nbrs<T> zn = {T(0), T(0), T(0), T(0), T(0), T(0), T(0)};
-  for (int c = threadIdx.x; c < N3; c += blockDim.x) {
-    const Cell q = Decode(c, n);
-    t[c] = JacobiPoint(zero ? zn : Load(static_cast<const T *>(x), c, q, n), b[c], o, w);
-  }
-  __syncthreads();
-  for (int c = threadIdx.x; c < N3; c += blockDim.x) x[c] = t[c];
-  __syncthreads();
-}
-
-template <typename T>
-__device__ void BRestrict(const T *x, const T *b, T *bc, T *xc, int n) {
-  const int nc = n / 2, N3 = nc * nc * nc;
-  const Lv<T> o = MakeLv<T>(n);
-  const T vol = o.dx * o.dx * o.dx;
-  for (int cc = threadIdx.x; cc < N3; cc += blockDim.x) {
-    const Cell p = Decode(cc, nc);
-    T t[2][2][2];
-    for (int a = 0; a < 2; ++a)
-      for (int bb = 0; bb < 2; ++bb)
-        for (int c2 = 0; c2 < 2; ++c2) {
-          const Cell q = {2 * p.i + c2, 2 * p.j + bb, 2 * p.k + a};
-          const int c = (q.k * n + q.j) * n + q.i;
-          const Nbrs<T> v = Load(x, c, q, n);
-          t[a][bb][c2] = vol * (b[c] - ApplyA(v.u, v.xm, v.xp, v.ym, v.yp, v.zm, v.zp, o));
-        }
-    bc[cc] = Restrict8(t, o);
-    xc[cc] = T(0);
-  }
-  __syncthreads();
-}
-
-template <typename T>
-__device__ void BProlong(T *x, const T *xc, int n) {
-  const int nc = n / 2, N3 = n * n * n;
-  const Lv<T> oc = MakeLv<T>(nc);
-  const T hc = oc.dx, df = T(0.25) * hc;
-  auto grad = [&](T diff) { return oc.mul ? diff * oc.idx : diff / hc; };
-  for (int c = threadIdx.x; c < N3; c += blockDim.x) {
-    const Cell q = Decode(c, n);
-    const Cell p = {q.i >> 1, q.j >> 1, q.k >> 1};
-    const int oi = q.i & 1, oj = q.j & 1, ok = q.k & 1;
-    const int cc = (p.k * nc + p.j) * nc + p.i;
-    const T fc = xc[cc];
-    const T g1 = oi == 0 ? grad(fc - (p.i > 0 ? xc[cc - 1] : -fc))
-                         : grad((p.i < nc - 1 ? xc[cc + 1] : -fc) - fc);
-    const T g2 = oj == 0 ? grad(fc - (p.j > 0 ? xc[cc - nc] : -fc))
-                         : grad((p.j < nc - 1 ? xc[cc + nc] : -fc) - fc);
-    const T g3 = ok == 0 ? grad(fc - (p.k > 0 ? xc[cc - nc * nc] : -fc))
-                         : grad((p.k < nc - 1 ? xc[cc + nc * nc] : -fc) - fc);
-    T v;
-    switch ((ok << 2) | (oj << 1) | oi) {
-      case 0: v = fc - (g1 * df + g2 * df + g3 * df); break;
-      case 1: v = fc + (g1 * df - g2 * df - g3 * df); break;
-      case 2: v = fc - (g1 * df - g2 * df + g3 * df); break;
-      case 3: v = fc + (g1 * df + g2 * df - g3 * df); break;
-      case 4: v = fc - (g1 * df + g2 * df - g3 * df); break;
-      case 5: v = fc + (g1 * df - g2 * df + g3 * df); break;
-      case 6: v = fc - (g1 * df - g2 * df - g3 * df); break;
-      default: v = fc + (g1 * df + g2 * df + g3 * df); break;
-    }
-    x[c] += v;
-  }
-  __syncthreads();
-}
-
 // One workgroup per entry: the V-cycle from this entry's level (rhs e.b, result in e.x) down
-// to the coarsest level, every level in LDS.
-template <typename T, int NB>
-__global__ void __launch_bounds__(1024)
-    BottomKernel(const GmgArgs<T> A, T w, int pre, int post) {
-  constexpr int kCap = NB * NB * NB + (NB / 2) * (NB / 2) * (NB / 2) * 8 / 7 + 8;
-  __shared__ T sx[kCap], st[kCap], sb[kCap];
-  const GmgEntry<T> e = At(A, blockIdx.x);
-  int nl = 0, off[8], nn[8];
-  for (int n = e.n, o = 0; nl < 8; n /= 2) {
-    off[nl] = o;
-    nn[nl] = n;
-    ++nl;
-    o += n * n * n;
-    if (n % 2 != 0 || n == 1) break;
-  }
-  const int N3 = e.n * e.n * e.n;
-  const bool warm = e.warm != 0;
-  for (int c = threadIdx.x; c < N3; c += blockDim.x) {
-    sb[c] = e.b[c];
-    if (warm) sx[c] = e.x[c];
-  }
-  __syncthreads();
-  for (int l = 0; l < nl; ++l) {
-    T *x = sx + off[l], *t = st + off[l], *b = sb + off[l];
-    const bool from_x = warm && l == 0;
-    for (int s = 0; s < pre; ++s) BSweep(x, t, b, nn[l], w, s == 0 && !from_x);
-    if (pre == 0 && !from_x) {
-      for (int c = threadIdx.x; c < nn[l] * nn[l] * nn[l]; c += blockDim.x) x[c] = T(0);
-      __syncthreads();
+// to the coarsest level. What bounds it is latency, a chain of about seven dependent steps a
+// level, so a thread keeps the x and b of its cells in registers at every level and LDS only
+// carries a level's x (or its residual) to the neighbours: 1024 threads as 256 columns by 4
+// groups of planes for levels of 5 to 16 cells per side, and one wavefront, which needs no
+// barrier, for those of at most 4. Measured 13.7 us from 16^3 in FP32 (38.7 with a launch-wide
+// loop over cells and a copy per sweep) and 19.6 from 16^3 in FP64, where 8^3 took 27.5.
+constexpr int kBottomWG = 1024;
+// cells of the levels above l (l = 31: of all)
+__host__ __device__ constexpr int BottomCells(int NB, int l) {
+  int s = 0;
+  for (int q = 0; q < l; ++q) s += (NB >> q) * (NB >> q) * (NB >> q);
+  return s;
+}
+
+template <typename T, int NB, bool MUL>
+struct Bottom {
+  T *lds;
+  T w;
+  int pre, post;
+
+  // Level l holds at most M = NB >> l cells per side, in an LDS array of M^3; a thread has SL
+  // consecutive planes of one column.
+  static constexpr int Side(int l) { return NB >> l; }
+  static constexpr int Slots(int l) { return Side(l) > 4 ? Side(l) / 4 : 1; }
+  template <int l>
+  struct Own {
+    static constexpr int M = Side(l), SL = Slots(l), S2 = M * M;
+    int n, i, j, k;  // first cell
+    int c, xm, xp, ym, yp, zm, zp;  // LDS positions: it, and its column's neighbours (clamped)
+    bool in, xl, xr, yl, yr;
+    __device__ __forceinline__ explicit Own(int n_) : n(n_) {
+      if (M <= 4) {
+        const int r = threadIdx.x / n;
+        i = threadIdx.x - r * n;
+        k = r / n;
+        j = r - k * n;
+        in = k < n && threadIdx.x < 64;
+      } else {
+        const int col = threadIdx.x % 256;
+        j = col / n;
+        i = col - j * n;
+        k = __builtin_amdgcn_readfirstlane(threadIdx.x / 256) * SL;
+        in = j < n && k < n;
+      }
+      xl = i > 0;
+      xr = i < n - 1;
+      yl = j > 0;
+      yr = j < n - 1;
+      c = (k * M + j) * M + i;
+      xm = xl ? c - 1 : c;
+      xp = xr ? c + 1 : c;
+      ym = yl ? c - M : c;
+      yp = yr ? c + M : c;
+      zm = k > 0 ? c - S2 : c;
+      zp = k + SL < n ? c + SL * S2 : c;
     }
-    if (l + 1 == nl) break;
-    BRestrict(static_cast<const T *>(x), static_cast<const T *>(b), sb + off[l + 1],
-              sx + off[l + 1], nn[l]);
+    __device__ __forceinline__ bool has(int q) const { return in && k + q < n; }
+    __device__ __forceinline__ int cell(int q) const { return ((k + q) * n + j) * n + i; }
+  };
+  // order LDS accesses: of the workgroup, or of the one wavefront that works on a small level
+  template <int l>
+  static __device__ __forceinline__ void Sync() {
+    if (Side(l) > 4) {
+      __syncthreads();
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
   }
-  for (int l = nl - 2; l >= 0; --l) {
-    T *x = sx + off[l], *t = st + off[l], *b = sb + off[l];
-    BProlong(x, static_cast<const T *>(sx + off[l + 1]), nn[l]);
-    for (int s = 0; s < post; ++s) BSweep(x, t, b, nn[l], w, false);
+
+  template <int l>
+  __device__ __forceinline__ void Put(T *X, const T (&u)[Slots(l)], const Own<l> &o) const {
+#pragma unroll
+    for (int q = 0; q < Slots(l); ++q)
+      if (o.has(q)) X[o.c + q * o.S2] = u[q];
+    Sync<l>();
   }
-  for (int c = threadIdx.x; c < N3; c += blockDim.x) e.x[c] = sx[c];
+  // fn(slot, neighbours) for this thread's cells, X holding the level's values and u this
+  // thread's. The loads are unconditional, at positions clamped into the level, so they are in
+  // flight together; a slot without a cell gets values that nobody uses.
+  template <int l, typename Fn>
+  __device__ __forceinline__ void Each(const T *X, const T (&u)[Slots(l)], const Own<l> &o,
+                                       Fn fn) const {
+    constexpr int SL = Slots(l);
+    Nbrs<T> v[SL];
+    if (o.in) {
+      const T zm = X[o.zm], zp = X[o.zp];
+#pragma unroll
+      for (int q = 0; q < SL; ++q) {
+        const T xm = X[o.xm + q * o.S2], xp = X[o.xp + q * o.S2];
+        const T ym = X[o.ym + q * o.S2], yp = X[o.yp + q * o.S2];
+        v[q] = {u[q],
+                o.xl ? xm : -u[q],
+                o.xr ? xp : -u[q],
+                o.yl ? ym : -u[q],
+                o.yr ? yp : -u[q],
+                o.k + q > 0 ? (q > 0 ? u[q > 0 ? q - 1 : 0] : zm) : -u[q],
+                o.k + q < o.n - 1 ? (q + 1 < SL ? u[q + 1 < SL ? q + 1 : 0] : zp) : -u[q]};
+      }
+    }
+    Sync<l>();  // everybody has read: X may be written again
+    if (o.in) {
+#pragma unroll
+      for (int q = 0; q < SL; ++q) fn(q, v[q]);
+    }
+  }
+
+  template <int l>
+  __device__ __forceinline__ void Sweeps(T *X, T (&u)[Slots(l)], const T (&b)[Slots(l)],
+                                         const Own<l> &o, const Lv<T> &lv, int count) const {
+    for (int s = 0; s < count; ++s) {
+      Put<l>(X, u, o);
+      Each<l>(X, u, o, [&](int q, const Nbrs<T> &v) { u[q] = JacobiPoint(v, b[q], lv, w); });
+    }
+  }
+
+  // The cycle on level l of n cells per side; b: right-hand side, u: start (from_x) and result.
+  template <int l>
+  __device__ __forceinline__ void Level(int n, T (&u)[Slots(l)], const T (&b)[Slots(l)],
+                                        bool from_x) const {
+    constexpr int M = Side(l), SL = Slots(l), S2 = M * M;
+    if (M <= 4 && threadIdx.x >= 64) return;
+    T *X = lds + BottomCells(NB, l);
+    const Own<l> o(n);
+    Lv<T> lv = MakeLv<T>(n);
+    lv.mul = MUL;  // known when compiling
+    if (!from_x) {
+#pragma unroll
+      for (int q = 0; q < SL; ++q) u[q] = pre > 0 ? JacobiZero(b[q], lv, w) : T(0);
+    }
+    Sweeps<l>(X, u, b, o, lv, pre - (from_x ? 0 : 1));
+    if constexpr (M > 1) {
+      if (n % 2 == 0) {
+        constexpr int SC = Slots(l + 1), MC = Side(l + 1);
+        const int nc = n / 2;
+        T r[SL], uc[SC], bc[SC];
+        Put<l>(X, u, o);
+        Each<l>(X, u, o, [&](int q, const Nbrs<T> &v) {
+          r[q] = b[q] - ApplyA(v.u, v.xm, v.xp, v.ym, v.yp, v.zm, v.zp, lv);
+        });
+        Put<l>(X, r, o);
+        const Own<l + 1> oc(nc);
+#pragma unroll
+        for (int q = 0; q < SC; ++q) uc[q] = bc[q] = T(0);
+        if (oc.in) {
+#pragma unroll
+          for (int q = 0; q < SC; ++q) {
+            const T *R = X + (2 * min(oc.k + q, nc - 1) * M + 2 * oc.j) * M + 2 * oc.i;
+            T t[2][2][2];
+#pragma unroll
+            for (int a = 0; a < 8; ++a)
+              t[a / 4][a / 2 % 2][a % 2] = R[a / 4 * S2 + a / 2 % 2 * M + a % 2];
+            bc[q] = Restrict8(t, lv);
+          }
+        }
+        Level<l + 1>(nc, uc, bc, false);
+        // the coarse level's x for everybody
+        T *XC = lds + BottomCells(NB, l + 1);
+#pragma unroll
+        for (int q = 0; q < SC; ++q)
+          if (oc.has(q)) XC[oc.c + q * MC * MC] = uc[q];
+        Sync<l>();
+        Lv<T> lc = MakeLv<T>(nc);
+        lc.mul = MUL;
+        if (o.in) {  // u += P xc: the coarse column's planes and its x and y neighbours
+          const int pi = o.i >> 1, pj = o.j >> 1, oi = o.i & 1, oj = o.j & 1, K = o.k >> 1;
+          const bool in1 = oi ? pi < nc - 1 : pi > 0, in2 = oj ? pj < nc - 1 : pj > 0;
+          const int c = pj * MC + pi;
+          const int c1 = in1 ? (oi ? c + 1 : c - 1) : c, c2 = in2 ? (oj ? c + MC : c - MC) : c;
+          constexpr int P = (SL + 1) / 2;
+          T f[P + 2], f1[P], f2[P];
+#pragma unroll
+          for (int p = 0; p < P + 2; ++p) f[p] = XC[min(max(K + p - 1, 0), nc - 1) * MC * MC + c];
+#pragma unroll
+          for (int p = 0; p < P; ++p) {
+            f1[p] = XC[min(K + p, nc - 1) * MC * MC + c1];
+            f2[p] = XC[min(K + p, nc - 1) * MC * MC + c2];
+          }
+#pragma unroll
+          for (int q = 0; q < SL; ++q) {
+            const int p = q / 2, ok = (o.k + q) & 1;
+            const T fc = f[p + 1];
+            const T f3 = ok ? (K + p < nc - 1 ? f[p + 2] : -fc) : (K + p > 0 ? f[p] : -fc);
+            u[q] += ProlongPoint(fc, in1 ? f1[p] : -fc, in2 ? f2[p] : -fc, f3, oi, oj, ok, lc);
+          }
+        }
+        Sweeps<l>(X, u, b, o, lv, post);
+      }
+    }
+  }
+};
+
+template <typename T, int NB, bool MUL>
+__device__ __forceinline__ void BottomBody(const GmgEntry<T> &e, T *lds, T w, int pre, int post) {
+  using B = Bottom<T, NB, MUL>;
+  constexpr int SL = B::Slots(0);
+  const bool warm = e.warm != 0;
+  const typename B::template Own<0> o(e.n);
+  T u[SL], b[SL];
+#pragma unroll
+  for (int q = 0; q < SL; ++q) {
+    u[q] = b[q] = T(0);
+    if (!o.has(q)) continue;
+    b[q] = Glob(e.b)[o.cell(q)];
+    if (warm) u[q] = Glob(e.x)[o.cell(q)];
+  }
+  const B body = {lds, w, pre, post};
+  body.template Level<0>(e.n, u, b, warm);
+#pragma unroll
+  for (int q = 0; q < SL; ++q)
+    if (o.has(q)) Glob(e.x)[o.cell(q)] = u[q];
+}
+
+template <typename T, int NB>
+__global__ void __launch_bounds__(kBottomWG)
+    BottomKernel(const GmgArgs<T> A, T w, int pre, int post) {
+  __shared__ T lds[BottomCells(NB, 31)];
+  const GmgEntry<T> e = At(A, blockIdx.x);
+  if (sizeof(T) == 4 || (e.n & (e.n - 1)) == 0)
+    BottomBody<T, NB, true>(e, lds, w, pre, post);
+  else
+    BottomBody<T, NB, false>(e, lds, w, pre, post);
 }
 
 // Right-hand side: 16 seeded Gaussian blobs at cell centres (FP64)
@@ -741,10 +950,20 @@ __global__ void __launch_bounds__(kWG) FillKernel(double *__restrict__ a, std::i
   if (c < n) a[c] = 0.0;
 }
 
+// Planes a workgroup of a pass marches through, for `planes` tile planes in the launch: as many
+// workgroups as fill the chip twice (each plane past the tile's own costs 2 H planes of
+// overlap), even, for the restriction, and from 2, where a short march beats the overlap: 32^3
+// V-cycles in FP64 take 83 / 91 / 103 / 131 us with at least 2 / 4 / 8 / 16 planes, 128^3 in FP32
+// 147 / 149 / 151 / 186, and from 256^3 up the rule gives 32.
+int PassPlanes(std::int64_t planes) {
+  const int nz = static_cast<int>(std::min<std::int64_t>((planes + 511) / 512, 32));
+  return std::max((nz + 1) / 2 * 2, 2);
+}
+
+constexpr std::int64_t kPassLarge = std::int64_t(1) << 22;
+
 int Blocks(std::int64_t cells) { return static_cast<int>((cells + kWG - 1) / kWG); }
 
-constexpr int kZCol = 8;    // planes per thread of the column Jacobi sweep
-constexpr int kPJCol = 8;   // planes per thread of the prolongation-and-sweep kernel
 
 }  // namespace
 
@@ -783,12 +1002,13 @@ std::int64_t GmgProblem<T>::Bytes(int N) {
 }
 
 template <typename T>
-pth_status GmgProblem<T>::Allocate(int N_, int bottom) {
+pth_status GmgProblem<T>::Allocate(int N_) {
+  constexpr int bottom = GmgBottom<T>::kN;
   N = N_;
   sizes = GmgLevelSizes(N);
   nbottom = 0;
   while (nbottom < static_cast<int>(sizes.size()) && sizes[nbottom] > bottom) ++nbottom;
-  if (nbottom == static_cast<int>(sizes.size())) {
+  if (sizes.back() > GmgBottom<T>::kCoarsest) {
     SetError("GMG: the coarsest level is larger than the in-LDS bottom solver");
     return PTH_FAIL;
   }
@@ -853,14 +1073,38 @@ GmgEntry<T> GmgProblem<T>::Entry(int l) const {
 
 template <typename T>
 pth_status GmgBatch<T>::Stage(const std::vector<GmgEntry<T>> &es, bool coarse_cells,
-                              GmgArgs<T> *args, int *nwg, int per_wg) {
+                              GmgArgs<T> *args, int *nwg) {
   std::vector<GmgEntry<T>> v = es;
   int wg = 0;
   for (auto &e : v) {
     e.wg_begin = wg;
     const std::int64_t n = coarse_cells ? e.nc : e.n;
-    wg += static_cast<int>((n * n * n + per_wg - 1) / per_wg);
+    wg += static_cast<int>((n * n * n + kWG - 1) / kWG);
   }
+  return Put(v, wg, args, nwg);
+}
+
+// The same for a pass: workgroups of tx x ty cells and *nz planes.
+template <typename T>
+pth_status GmgBatch<T>::StagePass(const std::vector<GmgEntry<T>> &es, int tx, int ty,
+                                  GmgArgs<T> *args, int *nwg, int *nz) {
+  std::int64_t planes = 0;
+  auto tiles = [&](int n) { return ((n + tx - 1) / tx) * ((n + ty - 1) / ty); };
+  for (const auto &e : es) planes += static_cast<std::int64_t>(tiles(e.n)) * e.n;
+  *nz = PassPlanes(planes);
+  std::vector<GmgEntry<T>> v = es;
+  int wg = 0;
+  for (auto &e : v) {
+    e.wg_begin = wg;
+    wg += tiles(e.n) * ((e.n + *nz - 1) / *nz);
+  }
+  return Put(v, wg, args, nwg);
+}
+
+// The entries of a launch into its arguments.
+template <typename T>
+pth_status GmgBatch<T>::Put(const std::vector<GmgEntry<T>> &v, int wg, GmgArgs<T> *args,
+                            int *nwg) {
   std::memset(args, 0, sizeof(*args));
   args->ne = static_cast<int>(v.size());
   *nwg = wg;
@@ -975,54 +1219,107 @@ pth_status GmgBatch<T>::Cycle(const std::vector<GmgProblem<T> *> &ps, double ome
       if (l < p->nbottom) es.push_back(p->Entry(l));
     return es;
   };
-  auto sweep = [&](int l) -> pth_status {  // x -> t, then t becomes x
-    GmgArgs<T> a;
-    int nwg;
-    const std::vector<GmgEntry<T>> es = entries(l);
-    bool zcol = jacobi_columns > 0;  // columns of kZCol planes when every size allows
-    for (const auto &e : es) zcol = zcol && e.n % 64 == 0 && e.n % kZCol == 0;
-    if (Stage(es, false, &a, &nwg, zcol ? kWG * kZCol : kWG) != PTH_COMPLETE) return PTH_FAIL;
-    ProfScope prof(l == 0 ? "gmg_jacobi_l0" : "gmg_jacobi", stream);
-    if (zcol)
-      hipLaunchKernelGGL((JacobiZKernel<T, kZCol>), dim3(nwg), dim3(kWG), 0, stream, a, w);
-    else
-      hipLaunchKernelGGL(JacobiKernel<T>, dim3(nwg), dim3(kWG), 0, stream, a, w);
-    PTH_HIP(hipGetLastError());
+  auto swap = [&](int l) {  // a sweep from x left its result in t
     for (auto *p : ps)
       if (l < p->nbottom) std::swap(p->lv[l].x, p->lv[l].t);
+  };
+  // a one-stage kernel, one thread per cell of the level (or of the next coarser one)
+  auto cells = [&](int l, bool coarse, const char *name, auto kernel, auto... arg) -> pth_status {
+    GmgArgs<T> a;
+    int nwg;
+    if (Stage(entries(l), coarse, &a, &nwg) != PTH_COMPLETE) return PTH_FAIL;
+    ProfScope prof(name, stream);
+    hipLaunchKernelGGL(kernel, dim3(nwg), dim3(kWG), 0, stream, a, arg...);
+    PTH_HIP(hipGetLastError());
+    return PTH_COMPLETE;
+  };
+  auto pass = [&](int l, const char *name, auto src, auto ns, auto res) -> pth_status {
+    const std::vector<GmgEntry<T>> es = entries(l);
+    std::int64_t total = 0;
+    for (const auto &e : es) total += static_cast<std::int64_t>(e.n) * e.n * e.n;
+    GmgArgs<T> a;
+    int nwg, nz;
+    auto run = [&](auto f) -> pth_status {
+      using F = decltype(f);
+      if (StagePass(es, F::TX, F::TY, &a, &nwg, &nz) != PTH_COMPLETE) return PTH_FAIL;
+      ProfScope prof(name, stream);
+      hipLaunchKernelGGL((PassKernel<T, decltype(src)::value, decltype(ns)::value,
+                                     decltype(res)::value, F>),
+                         dim3(nwg), dim3(F::WG), 0, stream, a, nz, w);
+      PTH_HIP(hipGetLastError());
+      return PTH_COMPLETE;
+    };
+    // below kPassLarge cells the smaller tile: more workgroups and shorter planes against less
+    // overlap (V-cycles with small / large tiles: 64^3 FP32 95 / 103 us, 128^3 FP64 196 / 208,
+    // 192^3 FP32 267 / 254, 192^3 FP64 683 / 590)
+    if ((total < kPassLarge ? run(PassSmall()) : run(PassLarge())) != PTH_COMPLETE)
+      return PTH_FAIL;
+    if (decltype(src)::value != kFromZero) swap(l);
+    return PTH_COMPLETE;
+  };
+  using std::integral_constant;
+  integral_constant<int, kFromZero> zero;
+  integral_constant<int, kFromX> from_x;
+  integral_constant<int, kFromBelow> below;
+  integral_constant<int, 1> one;
+  integral_constant<int, 2> two;
+  std::true_type res;
+  std::false_type nores;
+  const bool fused = jacobi_columns > 0;
+  auto jacobi = [&](int l) -> pth_status {
+    if (cells(l, false, l == 0 ? "gmg_jacobi_l0" : "gmg_jacobi", JacobiKernel<T>, w) !=
+        PTH_COMPLETE)
+      return PTH_FAIL;
+    swap(l);
+    return PTH_COMPLETE;
+  };
+  auto sweeps = [&](int l, int k) -> pth_status {
+    const char *name = l == 0 ? "gmg_jacobi_l0" : "gmg_jacobi";
+    while (k > 0) {
+      const int m = fused && k >= 2 ? 2 : 1;
+      if ((m == 2   ? pass(l, name, from_x, two, nores)
+           : fused  ? pass(l, name, from_x, one, nores)
+                    : jacobi(l)) != PTH_COMPLETE)
+        return PTH_FAIL;
+      k -= m;
+    }
     return PTH_COMPLETE;
   };
   for (int l = 0; l < L; ++l) {
-    GmgArgs<T> a;
-    int nwg;
-    if (warm && l == 0) {
-      for (int s = 0; s < pre; ++s)
-        if (sweep(l) != PTH_COMPLETE) return PTH_FAIL;
-    } else if (pre > 0) {
-      const std::vector<GmgEntry<T>> es = entries(l);
-      bool zcol = jacobi_columns > 0 && pre >= 2;
-      for (const auto &e : es) zcol = zcol && e.n % 64 == 0 && e.n % kZCol == 0;
-      if (Stage(es, false, &a, &nwg, zcol ? kWG * kZCol : kWG) != PTH_COMPLETE) return PTH_FAIL;
-      ProfScope prof(l == 0 ? "gmg_pre_l0" : "gmg_pre", stream);
-      if (zcol)
-        hipLaunchKernelGGL((PreZero2ZKernel<T, kZCol>), dim3(nwg), dim3(kWG), 0, stream, a, w);
-      else if (pre >= 2)
-        hipLaunchKernelGGL((PreZeroKernel<T, true>), dim3(nwg), dim3(kWG), 0, stream, a, w);
-      else
-        hipLaunchKernelGGL((PreZeroKernel<T, false>), dim3(nwg), dim3(kWG), 0, stream, a, w);
-      PTH_HIP(hipGetLastError());
-    } else {
-      if (Stage(entries(l), false, &a, &nwg) != PTH_COMPLETE) return PTH_FAIL;
-      hipLaunchKernelGGL(ZeroKernel<T>, dim3(nwg), dim3(kWG), 0, stream, a);
-      PTH_HIP(hipGetLastError());
+    const bool top = warm && l == 0;
+    const char *pname = l == 0 ? "gmg_pre_l0" : "gmg_pre";
+    const char *rname = l == 0 ? "gmg_restrict_l0" : "gmg_restrict";
+    const char *fname = l == 0 ? "gmg_pre_restrict_l0" : "gmg_pre_restrict";
+    int k = pre;  // sweeps still to do
+    if (fused && !top && pre == 2) {
+      if (pass(l, fname, zero, one, res) != PTH_COMPLETE) return PTH_FAIL;
+      continue;
     }
-    if (!(warm && l == 0))
-      for (int s = 2; s < pre; ++s)
-        if (sweep(l) != PTH_COMPLETE) return PTH_FAIL;
-    if (Stage(entries(l), true, &a, &nwg) != PTH_COMPLETE) return PTH_FAIL;
-    ProfScope prof(l == 0 ? "gmg_restrict_l0" : "gmg_restrict", stream);
-    hipLaunchKernelGGL(ResidualRestrictKernel<T>, dim3(nwg), dim3(kWG), 0, stream, a);
-    PTH_HIP(hipGetLastError());
+    if (!top) {
+      if (pre == 0) {
+        if (cells(l, false, pname, ZeroKernel<T>) != PTH_COMPLETE) return PTH_FAIL;
+      } else if (pre >= 2 && !(fused && pre == 3)) {
+        if (cells(l, false, pname, PreZeroKernel<T, true>, w) != PTH_COMPLETE) return PTH_FAIL;
+        k -= 2;
+      } else {
+        if (cells(l, false, pname, PreZeroKernel<T, false>, w) != PTH_COMPLETE) return PTH_FAIL;
+        k -= 1;
+      }
+    }
+    if (fused && k > 0) {
+      const int last = sizeof(T) == 4 && k % 2 == 0 ? 2 : 1;
+      if (sweeps(l, k - last) != PTH_COMPLETE) return PTH_FAIL;
+      if constexpr (sizeof(T) == 4) {
+        if (last == 2) {
+          if (pass(l, fname, from_x, two, res) != PTH_COMPLETE) return PTH_FAIL;
+          continue;
+        }
+      }
+      if (pass(l, fname, from_x, one, res) != PTH_COMPLETE) return PTH_FAIL;
+      continue;
+    }
+    if (sweeps(l, k) != PTH_COMPLETE) return PTH_FAIL;
+    if (cells(l, true, rname, ResidualRestrictKernel<T>) != PTH_COMPLETE) return PTH_FAIL;
   }
   {
     std::vector<GmgEntry<T>> es;
@@ -1034,36 +1331,19 @@ pth_status GmgBatch<T>::Cycle(const std::vector<GmgProblem<T> *> &ps, double ome
     int nwg;
     if (Stage(es, false, &a, &nwg) != PTH_COMPLETE) return PTH_FAIL;
     ProfScope prof("gmg_bottom", stream);
-    hipLaunchKernelGGL((BottomKernel<T, GmgBottom<T>::kN>), dim3(a.ne), dim3(1024), 0, stream,
-                       a, w, pre, post);
+    hipLaunchKernelGGL((BottomKernel<T, GmgBottom<T>::kN>), dim3(a.ne), dim3(kBottomWG), 0,
+                       stream, a, w, pre, post);
     PTH_HIP(hipGetLastError());
   }
   for (int l = L - 1; l >= 0; --l) {
-    GmgArgs<T> a;
-    int nwg;
-    const std::vector<GmgEntry<T>> es = entries(l);
-    // prolongation inside the first sweep (FP32 levels: in FP64 the recomputed neighbours'
-    // prolongation costs more than the separate pass saves, measured 208 vs 187 us at 256^3)
-    bool fuse = sizeof(T) == 4 && jacobi_columns > 0 && post >= 1;
-    for (const auto &e : es) fuse = fuse && e.n % 64 == 0 && e.n % kPJCol == 0;
-    if (fuse) {
-      if (Stage(es, false, &a, &nwg, kWG * kPJCol) != PTH_COMPLETE) return PTH_FAIL;
-      {
-        ProfScope prof(l == 0 ? "gmg_prolong_jacobi_l0" : "gmg_prolong_jacobi", stream);
-        hipLaunchKernelGGL((ProlongJacobiZKernel<T, kPJCol>), dim3(nwg), dim3(kWG), 0, stream,
-                           a, w);
-        PTH_HIP(hipGetLastError());
-      }
-      for (auto *p : ps)
-        if (l < p->nbottom) std::swap(p->lv[l].x, p->lv[l].t);
-    } else {
-      if (Stage(es, false, &a, &nwg) != PTH_COMPLETE) return PTH_FAIL;
-      ProfScope prof(l == 0 ? "gmg_prolong_l0" : "gmg_prolong", stream);
-      hipLaunchKernelGGL(ProlongKernel<T>, dim3(nwg), dim3(kWG), 0, stream, a);
-      PTH_HIP(hipGetLastError());
-    }
-    for (int s = fuse ? 1 : 0; s < post; ++s)
-      if (sweep(l) != PTH_COMPLETE) return PTH_FAIL;
+    const char *name = l == 0 ? "gmg_prolong_jacobi_l0" : "gmg_prolong_jacobi";
+    const int in = fused ? std::min(post, 2) : 0;
+    if ((in == 2   ? pass(l, name, below, two, nores)
+         : in == 1 ? pass(l, name, below, one, nores)
+                   : cells(l, false, l == 0 ? "gmg_prolong_l0" : "gmg_prolong",
+                           ProlongKernel<T>)) != PTH_COMPLETE)
+      return PTH_FAIL;
+    if (sweeps(l, post - in) != PTH_COMPLETE) return PTH_FAIL;
   }
   return PTH_COMPLETE;
 }

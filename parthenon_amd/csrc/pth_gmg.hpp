@@ -30,17 +30,11 @@ struct GmgArgs {
   int ne;
 };
 
-// largest level handled inside one workgroup in LDS (three n^3 arrays of T plus the coarser
-// levels below the 64 KiB static LDS limit)
+// kN: the largest level handled inside one workgroup; kCoarsest: the largest coarsest level
+// (cells per side, odd or 1) a problem may have
 template <typename T>
-struct GmgBottom;
-template <>
-struct GmgBottom<float> {
-  static constexpr int kN = 16;
-};
-template <>
-struct GmgBottom<double> {
-  static constexpr int kN = 8;
+struct GmgBottom {
+  static constexpr int kN = 16, kCoarsest = sizeof(T) == 4 ? 16 : 8;
 };
 
 template <typename T>
@@ -57,7 +51,7 @@ struct GmgProblem {
   double *b64 = nullptr, *partial = nullptr;
   int cur = 0;             // u[cur] is the current solution
   static std::int64_t Bytes(int N);  // device bytes one problem holds
-  pth_status Allocate(int N, int bottom);
+  pth_status Allocate(int N);
   void Free();
   GmgEntry<T> Entry(int l) const;
 };
@@ -72,10 +66,12 @@ struct GmgBatch {
   double *norms_host = nullptr, *norms_dev = nullptr;
   pth_status Init(hipStream_t s);
   void Free();
-  // per_wg: cells one workgroup of the launch covers
   pth_status Stage(const std::vector<GmgEntry<T>> &es, bool coarse_cells, GmgArgs<T> *args,
-                   int *nwg, int per_wg = 256);
-  int jacobi_columns = 1;  // Jacobi sweeps by z columns where the level size allows
+                   int *nwg);
+  pth_status StagePass(const std::vector<GmgEntry<T>> &es, int tx, int ty, GmgArgs<T> *args,
+                       int *nwg, int *nz);
+  pth_status Put(const std::vector<GmgEntry<T>> &v, int wg, GmgArgs<T> *args, int *nwg);
+  int jacobi_columns = 1;  // a level's stages in one pass each way, by z columns
   pth_status RhsNorms(const std::vector<GmgProblem<T> *> &ps, double *out);
   pth_status Residual(const std::vector<GmgProblem<T> *> &ps, const std::vector<char> &correct,
                       double *out);
@@ -92,7 +88,7 @@ struct GmgParams {
   double omega;
   int pre, post;
   int inner = 1;    // V-cycles per FP64 refinement step
-  int columns = 1;  // Jacobi sweeps by z columns where the level size allows
+  int columns = 1;  // a level's stages in one pass each way, by z columns
 };
 
 // One solve of one problem: the MGSolver::AddTasks iteration (mg_solver.hpp:119-161) as a host
@@ -112,7 +108,7 @@ struct GmgSolver1 {
   pth_status Init(int N) {
     PTH_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
     if (batch.Init(s) != PTH_COMPLETE) return PTH_FAIL;
-    return p.Allocate(N, GmgBottom<T>::kN);
+    return p.Allocate(N);
   }
   pth_status Norm() { return batch.RhsNorms({&p}, &bnorm); }
   // relative residual ||b - A u|| / ||b|| (||r|| when b = 0) below tol ends the loop once

@@ -105,7 +105,7 @@ struct Server {
       if (!Fits(need)) return nullptr;
     }
     auto *p = new GmgProblem<T>();
-    if (p->Allocate(n, GmgBottom<T>::kN) != PTH_COMPLETE) {
+    if (p->Allocate(n) != PTH_COMPLETE) {
       p->Free();
       delete p;
       return nullptr;

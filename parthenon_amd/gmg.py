@@ -25,7 +25,7 @@ class MGParams:  # src/solvers/mg_solver.hpp:37-58, with the smoother weight exp
     pre_sweeps: int = 2
     post_sweeps: int = 2
     inner_cycles: int = 1               # V-cycles per FP64 refinement step
-    column_sweeps: bool = True          # Jacobi by z columns where the level size allows
+    column_sweeps: bool = True          # a level's stages in one pass, by z columns
 
 
 class MGSolver:
