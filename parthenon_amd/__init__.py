@@ -402,6 +402,16 @@ def LoadBalancingAndAdaptiveMeshRefinement(mesh):
     return mesh.adapt()
 
 
+class _Address(int):
+    """A device address; it keeps the container whose memory it names alive, so a view made from
+    it (an array interface's data pointer) never outlives the field."""
+
+    def __new__(cls, value, owner):
+        a = super().__new__(cls, value)
+        a.owner = owner
+        return a
+
+
 class MeshData:
     def __init__(self, mesh, name, handle):
         self.mesh = mesh
@@ -446,7 +456,7 @@ class MeshData:
         d, c, f = _DP(), _DP(), _DP()
         _check(lib().pth_field_pointers(self._h, field.encode(), C.byref(d), C.byref(c),
                                         C.byref(f)), "pointers")
-        addr = lambda p: C.cast(p, C.c_void_p).value
+        addr = lambda p: _Address(C.cast(p, C.c_void_p).value, self) if p else None
         return addr(d), addr(c), addr(f)
 
 
