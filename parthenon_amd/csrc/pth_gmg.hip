@@ -224,65 +224,142 @@ __device__ __forceinline__ GmgEntry<T> Find(const GmgArgs<T> &A, int &local) {
 
 // ---- kernels --------------------------------------------------------------------------
 
-// FP64 outer step: u_new = u_old + e (e may be null), r = b - A u_new, r stored in T as the
-// inner right-hand side, per-workgroup partial sums of r^2.
-// One cell of the outer step; CORR: a correction is pending (e.x). Every load comes before
-// the first store, so a lane has its 8 (or 15) loads in flight at once.
-template <typename T, bool CORR>
-__device__ __forceinline__ double OuterCell(const GmgEntry<T> &e, int c, const Cell &q, int n) {
-  const Lv<double> o = MakeLv<double>(n);
-  const double bv = Glob(static_cast<const double *>(e.b64))[c];
-  Nbrs<double> v = LoadG(static_cast<const double *>(e.u_old), c, q, n);
-  if (CORR) {  // add the correction at the 7 points (the ghost follows the updated value)
-    const Nbrs<T> d = LoadG(static_cast<const T *>(e.x), c, q, n);
-    v.u += static_cast<double>(d.u);
-    v.xm = q.i > 0 ? v.xm + static_cast<double>(d.xm) : -v.u;
-    v.xp = q.i < n - 1 ? v.xp + static_cast<double>(d.xp) : -v.u;
-    v.ym = q.j > 0 ? v.ym + static_cast<double>(d.ym) : -v.u;
-    v.yp = q.j < n - 1 ? v.yp + static_cast<double>(d.yp) : -v.u;
-    v.zm = q.k > 0 ? v.zm + static_cast<double>(d.zm) : -v.u;
-    v.zp = q.k < n - 1 ? v.zp + static_cast<double>(d.zp) : -v.u;
-    Glob(e.u_new)[c] = v.u;
+// FP64 outer step: u = u_old + e (e may be null), r = b - A u, r stored in T as the inner
+// right-hand side, per-workgroup partial sums of r^2. A workgroup marches through nz planes of
+// 64 x 13 cells and the ring of one cell around them, 986 columns for 2 x 512 threads; u of a
+// column stays in registers for the z neighbours, the plane is left in LDS for the others, so a
+// cell's u, e and b are loaded once (1.19 times with the ring). nz depends on the entry's size
+// alone, so an entry's sum is the same alone and in a batch. What bounds it is memory: 32 bytes
+// a cell in the mixed solver, 40 in FP64. 256^3: 148 -> 129 us and 217 -> 157 against a thread
+// per cell with 15 loads, and 640 partial sums instead of 65536 (their sum 20 -> 4 us).
+constexpr int kOuterX = 64, kOuterY = 13, kOuterWG = 512;
+template <typename T, bool CORR, bool MUL>
+__device__ __forceinline__ double OuterBody(const GmgEntry<T> &e, int local, double *lds) {
+  constexpr int PX = kOuterX + 2, PY = kOuterY + 2, NC = PX * PY - 4;
+  constexpr int SL = (NC + kOuterWG - 1) / kOuterWG, PAD = PX + 1, LP = PX * PY + 2 * PAD;
+  const int n = e.n, s2 = n * n, nz = e.nz;
+  const int tx = (n + kOuterX - 1) / kOuterX, ty = (n + kOuterY - 1) / kOuterY;
+  const int x0 = local % tx * kOuterX, y0 = local / tx % ty * kOuterY;
+  const int k0 = local / (tx * ty) * nz, k1 = min(k0 + nz, n);
+  Lv<double> o = MakeLv<double>(n);
+  o.mul = MUL;  // known when compiling
+  const auto *gu = Glob(static_cast<const double *>(e.u_old));
+  const auto *gb = Glob(e.b64);
+  const auto *ge = Glob(static_cast<const T *>(e.x));
+  auto *gn = Glob(e.u_new);
+  auto *gr = Glob(e.b);
+  unsigned col[SL];
+  int li[SL];
+  bool xl[SL], xr[SL], yl[SL], yr[SL], in[SL];
+#pragma unroll
+  for (int q = 0; q < SL; ++q) {
+    const int id = threadIdx.x + q * kOuterWG;
+    int m = min(id, NC - 1) + 1;  // the four corners are not needed
+    if (m >= PX - 1) ++m;
+    if (m >= (PY - 1) * PX) ++m;
+    const int lx = m % PX, ly = m / PX, gi = x0 + lx - 1, gj = y0 + ly - 1;
+    li[q] = m + PAD;
+    in[q] = id < NC && lx >= 1 && lx < PX - 1 && ly >= 1 && ly < PY - 1 && gi < n && gj < n;
+    const int i = min(max(gi, 0), n - 1), j = min(max(gj, 0), n - 1);
+    xl[q] = i > 0;
+    xr[q] = i < n - 1;
+    yl[q] = j > 0;
+    yr[q] = j < n - 1;
+    col[q] = static_cast<unsigned>(j * n + i);
   }
-  const double r = bv - ApplyA(v.u, v.xm, v.xp, v.ym, v.yp, v.zm, v.zp, o);
-  Glob(e.b)[c] = static_cast<T>(r);
-  return r;
+  double un[SL], bn[SL], b[SL], a[SL], c[SL], rr = 0.0;
+  T en[SL];
+  auto load = [&](int p, int q) {
+    const std::int64_t at = static_cast<std::int64_t>(min(max(p, 0), n - 1)) * s2;
+    un[q] = (gu + at)[col[q]];
+    if (CORR) en[q] = (ge + at)[col[q]];
+    bn[q] = (gb + at)[col[q]];
+  };
+#pragma unroll
+  for (int q = 0; q < SL; ++q) {
+    load(k0 - 1, q);
+    a[q] = c[q] = b[q] = 0.0;
+  }
+  for (int p = k0 - 1; p <= k1; ++p) {
+    double v[SL], bp[SL];
+#pragma unroll
+    for (int q = 0; q < SL; ++q) {
+      v[q] = CORR ? un[q] + static_cast<double>(en[q]) : un[q];
+      bp[q] = bn[q];
+    }
+    if (p < k1) {
+#pragma unroll
+      for (int q = 0; q < SL; ++q) load(p + 1, q);
+    }
+#pragma unroll
+    for (int q = 0; q < SL; ++q) lds[(p & 1) * LP + li[q]] = v[q];
+    if (CORR && p >= k0 && p < k1) {
+      auto *out = gn + static_cast<std::int64_t>(p) * s2;
+#pragma unroll
+      for (int q = 0; q < SL; ++q)
+        if (in[q]) out[col[q]] = v[q];
+    }
+    const int k = p - 1;
+    if (k >= k0) {
+      const double *L = lds + (k & 1) * LP;
+      auto *out = gr + static_cast<std::int64_t>(k) * s2;
+#pragma unroll
+      for (int q = 0; q < SL; ++q) {
+        const double u = c[q];
+        const double xm = L[li[q] - 1], xp = L[li[q] + 1], ym = L[li[q] - PX], yp = L[li[q] + PX];
+        const double r = b[q] - ApplyA(u, xl[q] ? xm : -u, xr[q] ? xp : -u, yl[q] ? ym : -u,
+                                       yr[q] ? yp : -u, k > 0 ? a[q] : -u,
+                                       k < n - 1 ? v[q] : -u, o);
+        if (in[q]) {
+          out[col[q]] = static_cast<T>(r);
+          rr += r * r;
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < SL; ++q) {
+      a[q] = c[q];
+      c[q] = v[q];
+      b[q] = bp[q];
+    }
+    __syncthreads();
+  }
+  return rr;
 }
 
 template <typename T>
-__global__ void __launch_bounds__(kWG) OuterKernel(const GmgArgs<T> A) {
-  __shared__ double wsum[kWG / 64];
+__global__ void __launch_bounds__(kOuterWG) OuterKernel(const GmgArgs<T> A) {
+  constexpr int PX = kOuterX + 2, PY = kOuterY + 2;
+  __shared__ double lds[2 * (PX * PY + 2 * (PX + 1))];
+  __shared__ double wsum[kOuterWG / 64];
   int local;
   const GmgEntry<T> e = Find(A, local);
-  const int n = e.n, c = local * kWG + threadIdx.x;
-  double rr = 0.0;
-  if (c < n * n * n) {
-    const Cell q = Decode(c, n);
-    const double r = e.x ? OuterCell<T, true>(e, c, q, n) : OuterCell<T, false>(e, c, q, n);
-    rr = r * r;
-  }
+  const bool mul = (e.n & (e.n - 1)) == 0;
+  double rr = e.x ? (mul ? OuterBody<T, true, true>(e, local, lds)
+                         : OuterBody<T, true, false>(e, local, lds))
+                  : (mul ? OuterBody<T, false, true>(e, local, lds)
+                         : OuterBody<T, false, false>(e, local, lds));
   for (int off = 32; off > 0; off >>= 1) rr += __shfl_xor(rr, off, 64);
   if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = rr;
   __syncthreads();
   if (threadIdx.x == 0) {
     double s = 0.0;
-    for (int w = 0; w < kWG / 64; ++w) s += wsum[w];
+    for (int w = 0; w < kOuterWG / 64; ++w) s += wsum[w];
     e.partial[local] = s;
   }
 }
 
 // per-entry sum of the partials of OuterKernel (or of the rhs norm): one workgroup of kNormWG
 // threads per entry, each thread adding four interleaved streams of partials into separate
-// sums (independent loads in flight), then the workgroup tree; per_wg = cells per workgroup
-// of the kernel that wrote the partials. The order is fixed, so an entry's norm is the same
-// alone and in a batch.
+// sums (independent loads in flight), then the workgroup tree. The order is fixed, so an
+// entry's norm is the same alone and in a batch.
 constexpr int kNormWG = 1024;
 template <typename T>
 __global__ void __launch_bounds__(kNormWG)
-    NormKernel(const GmgArgs<T> A, double *__restrict__ out, int per_wg) {
+    NormKernel(const GmgArgs<T> A, double *__restrict__ out) {
   __shared__ double wsum[kNormWG / 64];
   const GmgEntry<T> e = At(A, blockIdx.x);
-  const int n = e.n, np = (n * n * n + per_wg - 1) / per_wg;
+  const int np = e.np;
   const double *pa = e.partial;
   double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
   for (int p = threadIdx.x; p < np; p += 4 * kNormWG) {
@@ -302,15 +379,22 @@ __global__ void __launch_bounds__(kNormWG)
   }
 }
 
-// partial sums of b^2 (the stop test's denominator)
+// partial sums of b^2 (the stop test's denominator), kRhsCells cells per workgroup
+constexpr int kRhsCells = 16 * kWG;
 template <typename T>
 __global__ void __launch_bounds__(kWG) RhsNormKernel(const GmgArgs<T> A) {
   __shared__ double wsum[kWG / 64];
   int local;
   const GmgEntry<T> e = Find(A, local);
-  const int n = e.n, c = local * kWG + threadIdx.x;
+  const int cells = e.n * e.n * e.n;
   double s = 0.0;
-  if (c < n * n * n) s = Glob(e.b64)[c] * Glob(e.b64)[c];
+#pragma unroll
+  for (int q = 0; q < kRhsCells / kWG; ++q) {
+    const std::int64_t c =
+        static_cast<std::int64_t>(local) * kRhsCells + q * kWG + threadIdx.x;
+    const double v = Glob(e.b64)[c < cells ? c : cells - 1];
+    if (c < cells) s += v * v;
+  }
   for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
   if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = s;
   __syncthreads();
@@ -474,8 +558,8 @@ __global__ void __launch_bounds__(kWG) ProlongKernel(const GmgArgs<T> A) {
 // (FP32, prolongation inside the first sweep) with a launch per stage, and 2 launches a level
 // instead of 5 and 4; what bounds a large level now is the instructions of the overlapped area
 // (1.5 times the cells at H = 2), what bounds a small one the march. Per V-cycle, outer step and
-// bottom included (2 + 2, FP32 with 2 cycles a step, FP64 with 1): 64^3 103 -> 59 and 131 -> 81 us,
-// 128^3 156 -> 101 and 220 -> 156, 256^3 440 -> 321 and 953 -> 640.
+// bottom included (2 + 2, FP32 with 2 cycles a step, FP64 with 1): 64^3 103 -> 58 and 131 -> 81 us,
+// 128^3 156 -> 98 and 220 -> 145, 256^3 440 -> 271 and 953 -> 561.
 enum { kFromZero = 0, kFromX = 1, kFromBelow = 2 };
 
 template <int TX_, int TY_, int WG_>
@@ -688,8 +772,11 @@ __device__ __forceinline__ void PassBody(const GmgEntry<T> &e, int local, int nz
   }
 }
 
+// FP32: at most 128 registers, so a CU holds two workgroups and one computes while the other
+// waits at its barrier (256^3, prolongation and two sweeps: 89 us with the compiler's 130
+// registers, 64 with 124). FP64 needs up to 210 and keeps one.
 template <typename T, int SRC, int NS, bool RES, typename F>
-__global__ void __launch_bounds__(F::WG) PassKernel(const GmgArgs<T> A, int nz, T w) {
+__global__ void __launch_bounds__(F::WG, sizeof(T) == 4 ? 4 : 1) PassKernel(const GmgArgs<T> A, int nz, T w) {
   __shared__ T lds[PassShape<T, SRC, NS, RES, F>::LDS];
   int local;
   const GmgEntry<T> e = Find(A, local);
@@ -960,6 +1047,18 @@ int PassPlanes(std::int64_t planes) {
   return std::max((nz + 1) / 2 * 2, 2);
 }
 
+// Planes a workgroup of the outer step marches through; the workgroups are never more than
+// the partial sums a problem has room for.
+int OuterTiles(int n) {
+  return ((n + kOuterX - 1) / kOuterX) * ((n + kOuterY - 1) / kOuterY);
+}
+int OuterPlanes(int n) {
+  const std::int64_t room = (static_cast<std::int64_t>(n) * n * n + kWG - 1) / kWG;
+  int nz = PassPlanes(static_cast<std::int64_t>(OuterTiles(n)) * n);
+  while (static_cast<std::int64_t>(OuterTiles(n)) * ((n + nz - 1) / nz) > room) nz += 2;
+  return nz;
+}
+
 constexpr std::int64_t kPassLarge = std::int64_t(1) << 22;
 
 int Blocks(std::int64_t cells) { return static_cast<int>((cells + kWG - 1) / kWG); }
@@ -1081,7 +1180,8 @@ pth_status GmgBatch<T>::Stage(const std::vector<GmgEntry<T>> &es, bool coarse_ce
     const std::int64_t n = coarse_cells ? e.nc : e.n;
     wg += static_cast<int>((n * n * n + kWG - 1) / kWG);
   }
-  return Put(v, wg, args, nwg);
+  *nwg = wg;
+  return Put(v, args);
 }
 
 // The same for a pass: workgroups of tx x ty cells and *nz planes.
@@ -1098,16 +1198,15 @@ pth_status GmgBatch<T>::StagePass(const std::vector<GmgEntry<T>> &es, int tx, in
     e.wg_begin = wg;
     wg += tiles(e.n) * ((e.n + *nz - 1) / *nz);
   }
-  return Put(v, wg, args, nwg);
+  *nwg = wg;
+  return Put(v, args);
 }
 
 // The entries of a launch into its arguments.
 template <typename T>
-pth_status GmgBatch<T>::Put(const std::vector<GmgEntry<T>> &v, int wg, GmgArgs<T> *args,
-                            int *nwg) {
+pth_status GmgBatch<T>::Put(const std::vector<GmgEntry<T>> &v, GmgArgs<T> *args) {
   std::memset(args, 0, sizeof(*args));
   args->ne = static_cast<int>(v.size());
-  *nwg = wg;
   if (static_cast<int>(v.size()) <= kGmgInline) {  // in the kernel arguments
     std::copy(v.begin(), v.end(), args->e);
     return PTH_COMPLETE;
@@ -1158,12 +1257,18 @@ template <typename T>
 pth_status GmgBatch<T>::RhsNorms(const std::vector<GmgProblem<T> *> &ps, double *out) {
   std::vector<GmgEntry<T>> es;
   for (auto *p : ps) es.push_back(p->Entry(0));
+  int nwg = 0;
+  for (auto &e : es) {
+    e.wg_begin = nwg;
+    e.np = static_cast<int>((static_cast<std::int64_t>(e.n) * e.n * e.n + kRhsCells - 1) /
+                            kRhsCells);
+    nwg += e.np;
+  }
   GmgArgs<T> a;
-  int nwg;
-  if (Stage(es, false, &a, &nwg) != PTH_COMPLETE) return PTH_FAIL;
+  if (Put(es, &a) != PTH_COMPLETE) return PTH_FAIL;
   const int ne = a.ne;
   hipLaunchKernelGGL(RhsNormKernel<T>, dim3(nwg), dim3(kWG), 0, stream, a);
-  hipLaunchKernelGGL(NormKernel<T>, dim3(ne), dim3(kNormWG), 0, stream, a, norms_dev, kWG);
+  hipLaunchKernelGGL(NormKernel<T>, dim3(ne), dim3(kNormWG), 0, stream, a, norms_dev);
   PTH_HIP(hipGetLastError());
   PTH_HIP(hipMemcpyAsync(norms_host, norms_dev, sizeof(double) * ne, hipMemcpyDeviceToHost,
                          stream));
@@ -1179,20 +1284,24 @@ template <typename T>
 pth_status GmgBatch<T>::Residual(const std::vector<GmgProblem<T> *> &ps,
                                  const std::vector<char> &correct, double *out) {
   std::vector<GmgEntry<T>> es;
+  int nwg = 0;
   for (size_t q = 0; q < ps.size(); ++q) {
     GmgEntry<T> e = ps[q]->Entry(0);
     if (!correct[q]) e.x = nullptr;
+    e.nz = OuterPlanes(e.n);
+    e.np = OuterTiles(e.n) * ((e.n + e.nz - 1) / e.nz);
+    e.wg_begin = nwg;
+    nwg += e.np;
     es.push_back(e);
   }
   GmgArgs<T> a;
-  int nwg;
-  if (Stage(es, false, &a, &nwg) != PTH_COMPLETE) return PTH_FAIL;
+  if (Put(es, &a) != PTH_COMPLETE) return PTH_FAIL;
   const int ne = a.ne;
   {
     ProfScope prof("gmg_outer", stream);
-    hipLaunchKernelGGL(OuterKernel<T>, dim3(nwg), dim3(kWG), 0, stream, a);
+    hipLaunchKernelGGL(OuterKernel<T>, dim3(nwg), dim3(kOuterWG), 0, stream, a);
   }
-  hipLaunchKernelGGL(NormKernel<T>, dim3(ne), dim3(kNormWG), 0, stream, a, norms_dev, kWG);
+  hipLaunchKernelGGL(NormKernel<T>, dim3(ne), dim3(kNormWG), 0, stream, a, norms_dev);
   PTH_HIP(hipGetLastError());
   PTH_HIP(hipMemcpyAsync(norms_host, norms_dev, sizeof(double) * ne, hipMemcpyDeviceToHost,
                          stream));

@@ -18,6 +18,7 @@ struct GmgEntry {
   int n, nc;              // cells per side on this and the next coarser level
   int wg_begin;           // first workgroup of this entry in the batched grid
   int warm;               // bottom solve: start from x instead of 0
+  int nz, np;             // outer step: planes per workgroup; partial sums of a norm
 };
 
 // The entries of one launch, passed as a kernel argument: inline for up to kGmgInline
@@ -70,7 +71,7 @@ struct GmgBatch {
                    int *nwg);
   pth_status StagePass(const std::vector<GmgEntry<T>> &es, int tx, int ty, GmgArgs<T> *args,
                        int *nwg, int *nz);
-  pth_status Put(const std::vector<GmgEntry<T>> &v, int wg, GmgArgs<T> *args, int *nwg);
+  pth_status Put(const std::vector<GmgEntry<T>> &v, GmgArgs<T> *args);
   int jacobi_columns = 1;  // a level's stages in one pass each way, by z columns
   pth_status RhsNorms(const std::vector<GmgProblem<T> *> &ps, double *out);
   pth_status Residual(const std::vector<GmgProblem<T> *> &ps, const std::vector<char> &correct,
