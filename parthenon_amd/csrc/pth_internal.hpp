@@ -184,7 +184,7 @@ struct Item {  // a run of consecutive elements over up to kItemRegions consecut
   int count;     // elements
 };
 constexpr int kItemRegions = 8;
-constexpr int kItemElems = 4096;
+constexpr int kItemElems = 1024;
 // restriction / prolongation items: one thread does a few coarse cells (each with 8 dependent
 // fine loads or stores), so these tables are cut finer to keep enough workgroups in flight
 constexpr int kProResItemElems = 512;
