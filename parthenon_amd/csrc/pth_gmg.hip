@@ -352,7 +352,8 @@ __global__ void __launch_bounds__(kOuterWG) OuterKernel(const GmgArgs<T> A) {
 // per-entry sum of the partials of OuterKernel (or of the rhs norm): one workgroup of kNormWG
 // threads per entry, each thread adding four interleaved streams of partials into separate
 // sums (independent loads in flight), then the workgroup tree. The order is fixed, so an
-// entry's norm is the same alone and in a batch.
+// entry's norm is the same alone and in a batch. out is pinned host memory: the value that the
+// host waits for takes no copy after the kernel (a V-cycle and step of 64^3 in FP64 81.1 -> 78.6 us).
 constexpr int kNormWG = 1024;
 template <typename T>
 __global__ void __launch_bounds__(kNormWG)
@@ -1235,8 +1236,7 @@ pth_status GmgBatch<T>::Init(hipStream_t s) {
   if (!stage_host) {
     PTH_HIP(hipHostMalloc(&stage_host, sizeof(GmgEntry<T>) * kStageCap));
     PTH_HIP(hipMalloc(&stage_dev, sizeof(GmgEntry<T>) * kStageCap));
-    PTH_HIP(hipHostMalloc(&norms_host, sizeof(double) * kMaxProblems));
-    PTH_HIP(hipMalloc(&norms_dev, sizeof(double) * kMaxProblems));
+    PTH_HIP(hipHostMalloc(&norms, sizeof(double) * kMaxProblems));
   }
   return PTH_COMPLETE;
 }
@@ -1245,12 +1245,10 @@ template <typename T>
 void GmgBatch<T>::Free() {
   if (stage_host) (void)hipHostFree(stage_host);
   if (stage_dev) (void)hipFree(stage_dev);
-  if (norms_host) (void)hipHostFree(norms_host);
-  if (norms_dev) (void)hipFree(norms_dev);
+  if (norms) (void)hipHostFree(norms);
   stage_host = nullptr;
   stage_dev = nullptr;
-  norms_host = nullptr;
-  norms_dev = nullptr;
+  norms = nullptr;
 }
 
 template <typename T>
@@ -1268,13 +1266,11 @@ pth_status GmgBatch<T>::RhsNorms(const std::vector<GmgProblem<T> *> &ps, double 
   if (Put(es, &a) != PTH_COMPLETE) return PTH_FAIL;
   const int ne = a.ne;
   hipLaunchKernelGGL(RhsNormKernel<T>, dim3(nwg), dim3(kWG), 0, stream, a);
-  hipLaunchKernelGGL(NormKernel<T>, dim3(ne), dim3(kNormWG), 0, stream, a, norms_dev);
+  hipLaunchKernelGGL(NormKernel<T>, dim3(ne), dim3(kNormWG), 0, stream, a, norms);
   PTH_HIP(hipGetLastError());
-  PTH_HIP(hipMemcpyAsync(norms_host, norms_dev, sizeof(double) * ne, hipMemcpyDeviceToHost,
-                         stream));
   PTH_HIP(hipStreamSynchronize(stream));
   stage_used = 0;  // every queued copy has run
-  for (int q = 0; q < ne; ++q) out[q] = std::sqrt(norms_host[q]);
+  for (int q = 0; q < ne; ++q) out[q] = std::sqrt(norms[q]);
   return PTH_COMPLETE;
 }
 
@@ -1301,15 +1297,13 @@ pth_status GmgBatch<T>::Residual(const std::vector<GmgProblem<T> *> &ps,
     ProfScope prof("gmg_outer", stream);
     hipLaunchKernelGGL(OuterKernel<T>, dim3(nwg), dim3(kOuterWG), 0, stream, a);
   }
-  hipLaunchKernelGGL(NormKernel<T>, dim3(ne), dim3(kNormWG), 0, stream, a, norms_dev);
+  hipLaunchKernelGGL(NormKernel<T>, dim3(ne), dim3(kNormWG), 0, stream, a, norms);
   PTH_HIP(hipGetLastError());
-  PTH_HIP(hipMemcpyAsync(norms_host, norms_dev, sizeof(double) * ne, hipMemcpyDeviceToHost,
-                         stream));
   PTH_HIP(hipStreamSynchronize(stream));
   stage_used = 0;  // every queued copy has run
   for (size_t q = 0; q < ps.size(); ++q) {
     if (correct[q]) ps[q]->cur = 1 - ps[q]->cur;
-    out[q] = std::sqrt(norms_host[q]);
+    out[q] = std::sqrt(norms[q]);
   }
   return PTH_COMPLETE;
 }

@@ -64,7 +64,7 @@ struct GmgBatch {
   hipStream_t stream = nullptr;
   GmgEntry<T> *stage_host = nullptr, *stage_dev = nullptr;
   int stage_used = 0;
-  double *norms_host = nullptr, *norms_dev = nullptr;
+  double *norms = nullptr;  // pinned host memory that the norm kernel writes
   pth_status Init(hipStream_t s);
   void Free();
   pth_status Stage(const std::vector<GmgEntry<T>> &es, bool coarse_cells, GmgArgs<T> *args,
