@@ -149,30 +149,75 @@ __global__ void __launch_bounds__(kWG)
   }
 }
 
+// FluxDivKernel's workgroups: kChunk consecutive interior cells of one brick (a block's component),
+// kCells a thread, 256 apart. The brick and the chunk's first plane are the
+// workgroup's (scalar), a thread divides 32-bit numbers below a plane's cells.
+constexpr int kCells = 4, kChunk = kCells * kWG;
+struct Chunk {
+  std::int64_t brick, t0, per;
+  int n0, plane, k0;
+  std::uint32_t x0;
+  __device__ __forceinline__ explicit Chunk(const Geo &G) {
+    n0 = G.hi0 - G.lo0 + 1;
+    plane = n0 * (G.hi1 - G.lo1 + 1);
+    per = static_cast<std::int64_t>(plane) * (G.hi2 - G.lo2 + 1);
+    const std::uint32_t chunks = static_cast<std::uint32_t>((per + kChunk - 1) / kChunk);
+    brick = blockIdx.x / chunks;
+    t0 = static_cast<std::int64_t>(blockIdx.x % chunks) * kChunk;
+    k0 = static_cast<int>(t0 / plane);
+    x0 = static_cast<std::uint32_t>(t0 % plane);
+  }
+  // slot u has a cell (the workgroup's last slots may be past the brick's end)
+  __device__ __forceinline__ bool has(int u) const { return t0 + u * kWG < per; }
+  // offset in a component of this thread's cell u; past the brick's end that of its last cell
+  __device__ __forceinline__ std::int64_t cell(const Geo &G, int u) const {
+    const int o = u * kWG + static_cast<int>(threadIdx.x);
+    const std::uint32_t x = x0 + static_cast<std::uint32_t>(t0 + o < per ? o : per - 1 - t0);
+    const int dk = static_cast<int>(x / static_cast<std::uint32_t>(plane));
+    const std::uint32_t y = x - static_cast<std::uint32_t>(dk) * plane;
+    const int j = static_cast<int>(y / static_cast<std::uint32_t>(n0));
+    const int i = static_cast<int>(y) - j * n0;
+    return (static_cast<std::int64_t>(k0 + dk + G.lo2) * G.e1 + (j + G.lo1)) * G.e0 + i + G.lo0;
+  }
+};
+unsigned ChunkGrid(const Topology &t, std::int64_t bricks) {
+  const std::int64_t per = static_cast<std::int64_t>(t.fine.n[0]) * t.fine.n[1] * t.fine.n[2];
+  return static_cast<unsigned>(bricks * ((per + kChunk - 1) / kChunk));
+}
+
+// Bound by memory: a cell takes two values of each face array, which share lines along x, and
+// writes one. 7 components in 16^3 blocks of a 64^3 mesh refined in a sphere: 402 -> 365 us
+// against four 64-bit divisions a cell and one cell at a time; 12 x 20 x 24 blocks 29 -> 22.
 __global__ void __launch_bounds__(kWG)
     FluxDivKernel(const double *__restrict__ flux, double *__restrict__ dudt,
                   const BlockCoefs *__restrict__ coef, Geo G, int nblocks) {
-  const int n0 = G.hi0 - G.lo0 + 1, n1 = G.hi1 - G.lo1 + 1, n2 = G.hi2 - G.lo2 + 1;
-  const std::int64_t total = static_cast<std::int64_t>(n0) * n1 * n2 * G.V * nblocks;
+  const Chunk K(G);
   const std::int64_t slab = G.cells * G.V * nblocks;
   const std::int64_t sj = G.e0, sk = static_cast<std::int64_t>(G.e0) * G.e1;
-  for (std::int64_t t = static_cast<std::int64_t>(blockIdx.x) * kWG + threadIdx.x; t < total;
-       t += static_cast<std::int64_t>(gridDim.x) * kWG) {
-    std::int64_t r = t;
-    const int i = static_cast<int>(r % n0) + G.lo0;
-    r /= n0;
-    const int j = static_cast<int>(r % n1) + G.lo1;
-    r /= n1;
-    const int k = static_cast<int>(r % n2) + G.lo2;
-    r /= n2;  // block * V + comp
-    const int b = static_cast<int>(r / G.V);
-    const BlockCoefs &C = coef[b];
-    const std::int64_t c = r * G.cells + (static_cast<std::int64_t>(k) * G.e1 + j) * G.e0 + i;
-    const double *fx = flux + c, *fy = flux + slab + c, *fz = flux + 2 * slab + c;
-    double du = (C.area[0] * fx[1] - C.area[0] * fx[0]);
-    if (G.ndim >= 2) du += (C.area[1] * fy[sj] - C.area[1] * fy[0]);
-    if (G.ndim == 3) du += (C.area[2] * fz[sk] - C.area[2] * fz[0]);
-    dudt[c] = -du / C.vol;
+  const BlockCoefs &C = coef[K.brick / G.V];
+  const double *f = flux + K.brick * G.cells;
+  double x0[kCells], x1[kCells], y0[kCells], y1[kCells], z0[kCells], z1[kCells];
+  std::int64_t c[kCells];
+#pragma unroll
+  for (int u = 0; u < kCells; ++u) {
+    if (!K.has(u)) break;
+    c[u] = K.cell(G, u);
+    const double *fx = f + c[u];
+    x0[u] = fx[0];
+    x1[u] = fx[1];
+    y0[u] = G.ndim >= 2 ? fx[slab] : 0.0;
+    y1[u] = G.ndim >= 2 ? fx[slab + sj] : 0.0;
+    z0[u] = G.ndim == 3 ? fx[2 * slab] : 0.0;
+    z1[u] = G.ndim == 3 ? fx[2 * slab + sk] : 0.0;
+  }
+  double *out = dudt + K.brick * G.cells;
+#pragma unroll
+  for (int u = 0; u < kCells; ++u) {
+    if (!K.has(u)) break;
+    double du = (C.area[0] * x1[u] - C.area[0] * x0[u]);
+    if (G.ndim >= 2) du += (C.area[1] * y1[u] - C.area[1] * y0[u]);
+    if (G.ndim == 3) du += (C.area[2] * z1[u] - C.area[2] * z0[u]);
+    out[c[u]] = -du / C.vol;  // past the end: the last cell's value once more
   }
 }
 
@@ -643,9 +688,9 @@ pth_status FluxDivergence(const Topology &t, int V, const double *flux, double *
   ProfScope prof("flux_div", s);
   const Geo G = MakeGeo(t, V);
   const int nb = static_cast<int>(t.blocks.size());
-  const std::int64_t total =
-      static_cast<std::int64_t>(t.fine.n[0]) * t.fine.n[1] * t.fine.n[2] * V * nb;
-  hipLaunchKernelGGL(FluxDivKernel, dim3(Grid(total)), dim3(kWG), 0, s, flux, dudt, coef, G, nb);
+  if (ChunkGrid(t, static_cast<std::int64_t>(V) * nb) == 0) return PTH_COMPLETE;
+  hipLaunchKernelGGL(FluxDivKernel, dim3(ChunkGrid(t, static_cast<std::int64_t>(V) * nb)),
+                     dim3(kWG), 0, s, flux, dudt, coef, G, nb);
   PTH_HIP(hipGetLastError());
   return PTH_COMPLETE;
 }

@@ -80,12 +80,31 @@ __global__ void __launch_bounds__(kWG)
   out[t] = b ? wa * a[t] + wb * b[t] : a[t];
 }
 
-// one thread per interior cell of every (block, component) brick
-__global__ void __launch_bounds__(kWG) ZeroKernel(double *data, Shape s, long long total) {
-  const long long t = static_cast<long long>(blockIdx.x) * kWG + threadIdx.x;
-  if (t >= total) return;
+// The interior cells of every (block, component) brick, kCells of them 256 apart a thread. A
+// workgroup stays in one brick and, but for its end, in one plane after its first, so what a
+// thread divides are 32-bit numbers: 16.8 M cells 44 -> 35 us against three 64-bit divisions.
+constexpr int kCells = 4;
+unsigned ZeroChunks(const Shape &s) {  // workgroups a brick
   const long long per = static_cast<long long>(s.n0) * s.n1 * s.n2;
-  data[(t / per) * s.cells + InteriorCell(s, t % per)] = 0.0;
+  return static_cast<unsigned>((per + kCells * kWG - 1) / (kCells * kWG));
+}
+__global__ void __launch_bounds__(kWG) ZeroKernel(double *data, Shape s, unsigned chunks) {
+  const unsigned plane = static_cast<unsigned>(s.n0 * s.n1);
+  const long long per = static_cast<long long>(plane) * s.n2;
+  const long long t0 = static_cast<long long>(blockIdx.x % chunks) * (kCells * kWG);
+  const int k0 = static_cast<int>(t0 / plane);
+  const unsigned x0 = static_cast<unsigned>(t0 % plane);
+  double *brick = data + static_cast<long long>(blockIdx.x / chunks) * s.cells;
+#pragma unroll
+  for (int u = 0; u < kCells; ++u) {
+    const int o = u * kWG + static_cast<int>(threadIdx.x);
+    if (t0 + o >= per) return;
+    const unsigned x = x0 + static_cast<unsigned>(o), dk = x / plane, y = x - dk * plane;
+    const int j = static_cast<int>(y / static_cast<unsigned>(s.n0));
+    const int i = static_cast<int>(y) - j * s.n0;
+    brick[(static_cast<long long>(k0 + static_cast<int>(dk) + s.g2) * s.e1 + (j + s.g1)) * s.e0 +
+          (i + s.g0)] = 0.0;
+  }
 }
 
 __device__ __forceinline__ double WorkgroupSum(double v, double *wsum) {
@@ -170,39 +189,53 @@ __global__ void __launch_bounds__(kWG)
   out[c] = r;
 }
 
-// level[c] = scale * brick value of global cell c = (K * N + J) * N + I; map: block id of each
-// block position (bz * nb1 + by) * nb0 + bx. Consecutive threads take consecutive I, a run
-// along x inside one brick row.
+// Brick offset of global cell c = (K * N + J) * N + I of the N^3 level (N^3 < 2^31); map: block id
+// of each block position (bz * nb1 + by) * nb0 + bx.
+__device__ __forceinline__ long long BrickCell(const int *__restrict__ map, const Shape &s,
+                                               unsigned N, unsigned c) {
+  const unsigned r = c / N, I = c - r * N, K = r / N, J = r - K * N;
+  const unsigned n0 = s.n0, n1 = s.n1, n2 = s.n2;
+  const unsigned bx = I / n0, by = J / n1, bz = K / n2;
+  const int b = map[(bz * (N / n1) + by) * (N / n0) + bx];
+  return b * s.cells +
+         (static_cast<long long>(K - bz * n2 + s.g2) * s.e1 + (J - by * n1 + s.g1)) * s.e0 +
+         (I - bx * n0 + s.g0);
+}
+
+// level[c] = scale * brick value of cell c, and back. Consecutive threads take consecutive I, a
+// run along x inside one brick row; a thread takes kCells cells, 256 apart, its loads first.
+// 256^3 in 32^3 blocks: gather 91 -> 70 us, scatter 80 -> 53 against one cell a thread and 64-bit
+// divisions.
 __global__ void __launch_bounds__(kWG)
     GatherKernel(const double *__restrict__ brick, const int *__restrict__ map, Shape s, int N,
                  double scale, double *__restrict__ level) {
-  const long long c = static_cast<long long>(blockIdx.x) * kWG + threadIdx.x;
-  if (c >= static_cast<long long>(N) * N * N) return;
-  const int I = static_cast<int>(c % N), J = static_cast<int>((c / N) % N),
-            K = static_cast<int>(c / (static_cast<long long>(N) * N));
-  const int nb0 = N / s.n0, nb1 = N / s.n1;
-  const int b = map[(K / s.n2 * nb1 + J / s.n1) * nb0 + I / s.n0];
-  const long long o = b * s.cells +
-                      (static_cast<long long>(K % s.n2 + s.g2) * s.e1 + (J % s.n1 + s.g1)) *
-                          s.e0 +
-                      (I % s.n0 + s.g0);
-  level[c] = scale * brick[o];
+  const unsigned cells = static_cast<unsigned>(N) * N * N;
+  double v[kCells];
+  unsigned c[kCells];
+#pragma unroll
+  for (int u = 0; u < kCells; ++u) {
+    c[u] = (blockIdx.x * kCells + u) * kWG + threadIdx.x;
+    v[u] = brick[BrickCell(map, s, N, c[u] < cells ? c[u] : cells - 1)];
+  }
+#pragma unroll
+  for (int u = 0; u < kCells; ++u)
+    if (c[u] < cells) level[c[u]] = scale * v[u];
 }
 
 __global__ void __launch_bounds__(kWG)
     ScatterKernel(const double *__restrict__ level, const int *__restrict__ map, Shape s, int N,
                   double *__restrict__ brick) {
-  const long long c = static_cast<long long>(blockIdx.x) * kWG + threadIdx.x;
-  if (c >= static_cast<long long>(N) * N * N) return;
-  const int I = static_cast<int>(c % N), J = static_cast<int>((c / N) % N),
-            K = static_cast<int>(c / (static_cast<long long>(N) * N));
-  const int nb0 = N / s.n0, nb1 = N / s.n1;
-  const int b = map[(K / s.n2 * nb1 + J / s.n1) * nb0 + I / s.n0];
-  const long long o = b * s.cells +
-                      (static_cast<long long>(K % s.n2 + s.g2) * s.e1 + (J % s.n1 + s.g1)) *
-                          s.e0 +
-                      (I % s.n0 + s.g0);
-  brick[o] = level[c];
+  const unsigned cells = static_cast<unsigned>(N) * N * N;
+  double v[kCells];
+  unsigned c[kCells];
+#pragma unroll
+  for (int u = 0; u < kCells; ++u) {
+    const unsigned t = (blockIdx.x * kCells + u) * kWG + threadIdx.x;
+    c[u] = t < cells ? t : cells - 1;  // past the end: the last cell once more
+    v[u] = level[c[u]];
+  }
+#pragma unroll
+  for (int u = 0; u < kCells; ++u) brick[BrickCell(map, s, N, c[u])] = v[u];
 }
 
 int SolverField(MeshData *md, const char *name, const char *what) {
@@ -337,8 +370,10 @@ pth_status pth_solver_set_to_zero(pth_meshdata *mdh, const char *var) {
   const long long total = static_cast<long long>(m->topo.blocks.size()) * m->fields[f].ncomp *
                           s.n0 * s.n1 * s.n2;
   if (total == 0) return PTH_COMPLETE;
-  hipLaunchKernelGGL(ZeroKernel, dim3(Blocks(total)), dim3(kWG), 0, m->stream,
-                     md->store[f].data, s, total);
+  const unsigned chunks = ZeroChunks(s);
+  hipLaunchKernelGGL(ZeroKernel,
+                     dim3(chunks * m->fields[f].ncomp * static_cast<unsigned>(m->topo.blocks.size())),
+                     dim3(kWG), 0, m->stream, md->store[f].data, s, chunks);
   PTH_HIP(hipGetLastError());
   return PTH_COMPLETE;
 }
@@ -537,9 +572,9 @@ pth_status pth_mg_setup(pth_mg *h, pth_meshdata *mdh) {
   const Shape s = ShapeOf(m->topo.fine);
   const long long cells = static_cast<long long>(h->N) * h->N * h->N;
   const pth_status st = h->Do([&](auto &S) -> pth_status {
-    hipLaunchKernelGGL(GatherKernel, dim3(Blocks(cells)), dim3(kWG), 0, m->stream,
+    hipLaunchKernelGGL(GatherKernel, dim3(Blocks((cells + kCells - 1) / kCells)), dim3(kWG), 0, m->stream,
                        md->store[h->frhs].data, h->map, s, h->N, h->scale, S.p.b64);
-    hipLaunchKernelGGL(GatherKernel, dim3(Blocks(cells)), dim3(kWG), 0, m->stream,
+    hipLaunchKernelGGL(GatherKernel, dim3(Blocks((cells + kCells - 1) / kCells)), dim3(kWG), 0, m->stream,
                        md->store[h->fu].data, h->map, s, h->N, 1.0, S.p.u[0]);
     PTH_HIP(hipGetLastError());
     S.p.cur = 0;
@@ -587,7 +622,7 @@ pth_status pth_mg_solve(pth_mg *h, pth_meshdata *mdh) {
     h->rms = h->history.back();
     PTH_HIP(hipEventRecord(h->ev, S.s));
     PTH_HIP(hipStreamWaitEvent(m->stream, h->ev, 0));
-    hipLaunchKernelGGL(ScatterKernel, dim3(Blocks(cells)), dim3(kWG), 0, m->stream,
+    hipLaunchKernelGGL(ScatterKernel, dim3(Blocks((cells + kCells - 1) / kCells)), dim3(kWG), 0, m->stream,
                        S.p.u[S.p.cur], h->map, s, h->N, md->store[h->fu].data);
     PTH_HIP(hipGetLastError());
     return PTH_COMPLETE;

@@ -1,0 +1,105 @@
+"""Kernels that take four cells a thread: bricks smaller than, equal to and past a workgroup's
+1024 cells, with remainders, in 1 to 3 dimensions."""
+import numpy as np
+import pytest
+
+import parthenon_amd as pa
+from parthenon_amd import gmg
+
+pytestmark = pytest.mark.gpu
+
+BLOCKS = [(4, 4, 4), (8, 8, 8), (10, 6, 8), (16, 8, 8), (12, 10, 14), (16, 16, 4), (36, 1, 1),
+          (22, 26, 1)]
+
+
+def mesh(block):
+    active = [n > 1 for n in block]
+    m = pa.Mesh(tuple(2 * n if a else 1 for n, a in zip(block, active)), block, 2)
+    m.add_field("q", 3, pa.Metadata.FillGhost | pa.Metadata.Independent | pa.Metadata.WithFluxes)
+    m.finalize()
+    n, g = m.n, m.ng
+    inner = (slice(None), slice(None)) + tuple(slice(g[2 - a], g[2 - a] + n[2 - a])
+                                               for a in range(3))
+    return m, inner
+
+
+@pytest.mark.parametrize("block", BLOCKS)
+def test_flux_divergence(block):
+    print(f"case flux divergence {block}", flush=True)
+    m, inner = mesh(block)
+    rng = np.random.default_rng(1)
+    a, b = m.mesh_data("base"), m.mesh_data("dudt")
+    shape = m.field_shape("q")
+    F = rng.standard_normal((3,) + shape)
+    a.upload("q", F, which=2)
+    b.upload("q", np.full(shape, 7.0))
+    pa.Update.FluxDivergence(a, b)
+    blk = m.block(0)
+    dx = [(blk["xmax"][d] - blk["xmin"][d]) / m.n[d] for d in range(3)]
+    area = [dx[1] * dx[2], dx[0] * dx[2], dx[0] * dx[1]]
+    du = np.zeros(shape)
+    for d in range(3):
+        if block[d] > 1:
+            du += area[d] * np.roll(F[d], -1, axis=4 - d) - area[d] * F[d]
+    exp = -du / (dx[0] * dx[1] * dx[2])
+    got = b.download("q")
+    # the widths and their products are rounded differently here: a few units in the last place
+    # of the largest term
+    tol = 64 * np.finfo(float).eps * np.abs(F).max() / min(d for d, n in zip(dx, block) if n > 1)
+    assert np.abs(got[inner] - exp[inner]).max() <= tol
+    keep = np.ones(shape, dtype=bool)
+    keep[inner] = False
+    assert (got[keep] == 7.0).all()
+
+
+@pytest.mark.parametrize("block", BLOCKS)
+def test_set_to_zero(block):
+    print(f"case zero {block}", flush=True)
+    m, inner = mesh(block)
+    md = m.mesh_data("base")
+    md.upload("q", np.full(m.field_shape("q"), 3.0))
+    gmg.set_to_zero(md, "q")
+    exp = np.full(m.field_shape("q"), 3.0)
+    exp[inner] = 0.0
+    assert np.array_equal(md.download("q"), exp)
+
+
+@pytest.mark.parametrize("n,block", [(8, (8, 8, 8)), (12, (4, 6, 12)), (20, (10, 20, 4)),
+                                     (32, (8, 16, 32))])
+def test_mesh_solve_is_the_array_solve(n, block):
+    """Gather and scatter: the FP64 solver on the blocks of a mesh gives the array solver's bits."""
+    print(f"case gather {n} {block}", flush=True)
+    m = pa.Mesh((n,) * 3, block, 2, xmin=(0.0,) * 3, xmax=(1.0,) * 3, periodic=(0, 0, 0),
+                bcs=("fixed_face",) * 6)
+    m.add_field("u", 1)
+    m.add_field("rhs", 1)
+    m.finalize()
+    md = m.mesh_data("base")
+    b = np.random.default_rng(n).standard_normal((n, n, n))
+    g, nb = m.ng, [n // block[d] for d in range(3)]
+
+    def bricks(fn):
+        for q in range(m.nblocks):
+            p = m.block(q)["l"]
+            at = tuple(slice(p[2 - a] * block[2 - a], (p[2 - a] + 1) * block[2 - a])
+                       for a in range(3))
+            fn(q, at)
+
+    rhs = np.zeros(m.field_shape("rhs"))
+    inner = tuple(slice(g[2 - a], g[2 - a] + block[2 - a]) for a in range(3))
+    bricks(lambda q, at: rhs[q, 0].__setitem__(inner, b[at]))
+    md.upload("rhs", rhs)
+    s = gmg.MeshMGSolver(m, "u", "rhs", gmg.MeshMGParams(max_iters=3, residual_tolerance=0.0,
+                                                         precision="fp64"))
+    s.setup(md)
+    s.solve(md)
+    a = gmg.MGSolver(n, "fp64", gmg.MGParams(max_iters=3, residual_tolerance=0.0))
+    a.set_rhs(b)
+    a.solve()
+    exp, u = a.solution(), md.download("u")
+    assert len(nb) == 3
+
+    def check(q, at):
+        assert np.array_equal(u[q, 0][inner], exp[at]), q
+
+    bricks(check)
