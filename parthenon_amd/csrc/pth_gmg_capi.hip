@@ -46,8 +46,15 @@ struct Request {
   double admit = -1, done = -1, rel = 0;
   int iters = 0;
   bool finished = false;
-  std::vector<double> solution;
+  // the kept solution: in pinned memory, which the device writes at full rate, while the server's
+  // share of it lasts (kPinnedMax), else in ordinary memory (a run that keeps 97 MB of solutions
+  // takes 11.5 ms for 15.6)
+  double *pinned = nullptr;
+  std::vector<double> pageable;
+  size_t kept = 0;
+  double *solution() { return pinned ? pinned : pageable.data(); }
 };
+constexpr std::int64_t kPinnedMax = std::int64_t(1) << 30;
 
 template <typename T>
 struct Server {
@@ -62,6 +69,7 @@ struct Server {
   std::vector<Request> reqs;
   std::map<int, std::vector<GmgProblem<T> *>> pool;  // free problems by grid size
   std::int64_t held = 0;                             // bytes in active + pooled problems
+  std::int64_t pinned = 0;                           // bytes of kept solutions in pinned memory
   int iterations = 0, max_batch = 0;
   double busy_s = 0.0;
   ~Server() {
@@ -70,8 +78,24 @@ struct Server {
         p->Free();
         delete p;
       }
+    for (auto &r : reqs)
+      if (r.pinned) (void)hipHostFree(r.pinned);
     batch.Free();
     if (s) (void)hipStreamDestroy(s);
+  }
+  // room for a request's solution of c cells
+  void Room(Request &r, std::int64_t c) {
+    if (r.kept) return;
+    const std::int64_t need = static_cast<std::int64_t>(sizeof(double)) * c;
+    if (pinned + need <= kPinnedMax && hipHostMalloc(&r.pinned, need) == hipSuccess)
+      pinned += need;
+    else
+      r.pinned = nullptr;
+    if (!r.pinned) {
+      (void)hipGetLastError();
+      r.pageable.resize(c);
+    }
+    r.kept = static_cast<size_t>(c);
   }
   pth_status Init() {
     PTH_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
@@ -185,8 +209,8 @@ struct Server {
         if (rel < tol || r.iters >= maxit) {
           if (keep) {
             const std::int64_t c = static_cast<std::int64_t>(r.n) * r.n * r.n;
-            r.solution.resize(c);
-            PTH_HIP(hipMemcpyAsync(r.solution.data(), a.p->u[a.p->cur], sizeof(double) * c,
+            Room(r, c);
+            PTH_HIP(hipMemcpyAsync(r.solution(), a.p->u[a.p->cur], sizeof(double) * c,
                                    hipMemcpyDeviceToHost, s));
             PTH_HIP(hipStreamSynchronize(s));
           }
@@ -212,6 +236,30 @@ struct Server {
     return PTH_COMPLETE;
   }
 };
+
+// Copies n doubles. A large copy into fresh memory waits for page after page and one thread gets
+// 10 to 17 GB/s of it, so from kCopyMin a thread it is shared by up to kCopyThreads threads, which
+// end before it returns (below, starting a thread costs what it saves: about 50 us against 1 MB
+// in 70 us). Ten solutions of the served sizes, 97 MB: 7.6 -> 2.7 ms.
+constexpr size_t kCopyMin = size_t(1) << 18;
+constexpr unsigned kCopyThreads = 8;
+void CopyOut(const double *from, double *to, size_t n) {
+  const unsigned most = std::min(kCopyThreads, std::max(1u, std::thread::hardware_concurrency()));
+  const size_t parts = std::min<size_t>(most, n / kCopyMin);
+  std::vector<std::thread> ts;
+  size_t done = 0;  // doubles given to threads so far
+  try {
+    ts.reserve(parts);
+    for (size_t q = 0; q + 1 < parts; ++q) {
+      const size_t end = n * (q + 1) / parts;
+      ts.emplace_back([from, to, done, end] { std::copy(from + done, from + end, to + done); });
+      done = end;
+    }
+  } catch (const std::exception &) {  // no more threads or memory: the rest is copied here
+  }
+  std::copy(from + done, from + n, to + done);
+  for (auto &t : ts) t.join();
+}
 
 struct ServerHandle {
   std::unique_ptr<Server<float>> f;
@@ -446,11 +494,11 @@ pth_status pth_gmg_server_result(const pth_gmg_server *h, int id, double out[5],
 pth_status pth_gmg_server_solution(const pth_gmg_server *h, int id, double *host, size_t n) {
   auto *hh = const_cast<pth_gmg_server *>(h);
   return hh->Do([&](auto &S) {
-    if (id < 0 || id >= static_cast<int>(S.reqs.size()) || S.reqs[id].solution.size() != n) {
+    if (id < 0 || id >= static_cast<int>(S.reqs.size()) || S.reqs[id].kept != n) {
       SetError("pth_gmg_server_solution: no kept solution of this size");
       return PTH_FAIL;
     }
-    std::copy(S.reqs[id].solution.begin(), S.reqs[id].solution.end(), host);
+    CopyOut(S.reqs[id].solution(), host, n);
     return PTH_COMPLETE;
   });
 }
