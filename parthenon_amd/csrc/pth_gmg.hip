@@ -230,8 +230,8 @@ __device__ __forceinline__ GmgEntry<T> Find(const GmgArgs<T> &A, int &local) {
 // column stays in registers for the z neighbours, the plane is left in LDS for the others, so a
 // cell's u, e and b are loaded once (1.19 times with the ring). nz depends on the entry's size
 // alone, so an entry's sum is the same alone and in a batch. What bounds it is memory: 32 bytes
-// a cell in the mixed solver, 40 in FP64. 256^3: 148 -> 129 us and 217 -> 157 against a thread
-// per cell with 15 loads, and 640 partial sums instead of 65536 (their sum 20 -> 4 us).
+// a cell in the mixed solver, 40 in FP64. 256^3: 148 -> 117 us and 217 -> 141 against a thread
+// per cell with 15 loads, and 1280 partial sums instead of 65536 (their sum 20 -> 4 us).
 constexpr int kOuterX = 64, kOuterY = 13, kOuterWG = 512;
 template <typename T, bool CORR, bool MUL>
 __device__ __forceinline__ double OuterBody(const GmgEntry<T> &e, int local, double *lds) {
@@ -560,7 +560,7 @@ __global__ void __launch_bounds__(kWG) ProlongKernel(const GmgArgs<T> A) {
 // instead of 5 and 4; what bounds a large level now is the instructions of the overlapped area
 // (1.5 times the cells at H = 2), what bounds a small one the march. Per V-cycle, outer step and
 // bottom included (2 + 2, FP32 with 2 cycles a step, FP64 with 1): 64^3 103 -> 58 and 131 -> 81 us,
-// 128^3 156 -> 98 and 220 -> 145, 256^3 440 -> 271 and 953 -> 561.
+// 128^3 156 -> 98 and 220 -> 145, 256^3 440 -> 262 and 953 -> 533.
 enum { kFromZero = 0, kFromX = 1, kFromBelow = 2 };
 
 template <int TX_, int TY_, int WG_>
@@ -1042,20 +1042,23 @@ __global__ void __launch_bounds__(kWG) FillKernel(double *__restrict__ a, std::i
 // workgroups as fill the chip twice (each plane past the tile's own costs 2 H planes of
 // overlap), even, for the restriction, and from 2, where a short march beats the overlap: 32^3
 // V-cycles in FP64 take 83 / 91 / 103 / 131 us with at least 2 / 4 / 8 / 16 planes, 128^3 in FP32
-// 147 / 149 / 151 / 186, and from 256^3 up the rule gives 32.
-int PassPlanes(std::int64_t planes) {
-  const int nz = static_cast<int>(std::min<std::int64_t>((planes + 511) / 512, 32));
+// 147 / 149 / 151 / 186. At most `most` planes: 32 for the passes, where 256^3 in FP32 takes
+// 270 us with 32 and 272 with 16 (192^3 158 and 180).
+int PassPlanes(std::int64_t planes, int most) {
+  const int nz = static_cast<int>(std::min<std::int64_t>((planes + 511) / 512, most));
   return std::max((nz + 1) / 2 * 2, 2);
 }
 
-// Planes a workgroup of the outer step marches through; the workgroups are never more than
-// the partial sums a problem has room for.
+// Planes a workgroup of the outer step marches through, at most 16: it is bound by memory and
+// its registers let three workgroups share a CU, which the 1280 of 256^3 fill (64 / 32 / 24 / 16 / 8
+// planes: 152 / 131 / 128 / 117 / 120 us). The workgroups are never more than the partial sums a
+// problem has room for.
 int OuterTiles(int n) {
   return ((n + kOuterX - 1) / kOuterX) * ((n + kOuterY - 1) / kOuterY);
 }
 int OuterPlanes(int n) {
   const std::int64_t room = (static_cast<std::int64_t>(n) * n * n + kWG - 1) / kWG;
-  int nz = PassPlanes(static_cast<std::int64_t>(OuterTiles(n)) * n);
+  int nz = PassPlanes(static_cast<std::int64_t>(OuterTiles(n)) * n, 16);
   while (static_cast<std::int64_t>(OuterTiles(n)) * ((n + nz - 1) / nz) > room) nz += 2;
   return nz;
 }
@@ -1192,7 +1195,7 @@ pth_status GmgBatch<T>::StagePass(const std::vector<GmgEntry<T>> &es, int tx, in
   std::int64_t planes = 0;
   auto tiles = [&](int n) { return ((n + tx - 1) / tx) * ((n + ty - 1) / ty); };
   for (const auto &e : es) planes += static_cast<std::int64_t>(tiles(e.n)) * e.n;
-  *nz = PassPlanes(planes);
+  *nz = PassPlanes(planes, 32);
   std::vector<GmgEntry<T>> v = es;
   int wg = 0;
   for (auto &e : v) {
