@@ -205,7 +205,7 @@ pth_status pth_exchange_fused(pth_meshdata *md, int bt);
 /* ---- Burgers benchmark package and Update:: tasks ---- */
 /* burgers_package::CalculateFluxes (benchmarks/burgers/burgers_package.cpp:202-404) on the
  * field "U" of md; recon 0 = WENO5Z, 1 = MC-limited linear. The reconstructed face states
- * (the reference's OneCopy Ulx..Urz) live in a library-owned scratch arena. */
+ * (the reference's OneCopy Ulx..Urz) stay on chip. */
 pth_status pth_burgers_calculate_fluxes(pth_meshdata *md, int recon);
 /* Update::FluxDivergence<MeshData> (src/interface/update.cpp:63-84). */
 pth_status pth_flux_divergence(pth_meshdata *in, pth_meshdata *dudt);

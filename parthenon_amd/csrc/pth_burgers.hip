@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <cfloat>
+#include <type_traits>
 
 #include "pth_burgers.hpp"
 #include "pth_device.hpp"
@@ -65,11 +66,13 @@ struct FluxSplit {
 // instructions a reconstruction with its flux, 8 IEEE divides among them). On the 960-block
 // mesh with 7 components the reconstruction and HLL as two launches, with the states in HBM
 // between them, took 1341 + 1043 us; this kernel takes
-// 1070 us.
-template <int RECON>
+// 1070 us. WIDE: 64-bit cell offsets, for components of 4 GB and more.
+template <int RECON, bool WIDE>
 __global__ void __launch_bounds__(kWG)
     FluxTaskKernel(const double *__restrict__ U, double *__restrict__ flux, Geo G, int nblocks,
                    FluxSplit S) {
+  using I = std::conditional_t<WIDE, std::int64_t, int>;       // cells
+  using O = std::conditional_t<WIDE, std::int64_t, unsigned>;  // byte offsets
   __shared__ double up[2][kSegFaces][kWG];
   // one block's workgroups are adjacent and run on one XCD: the three directions read the
   // same cells
@@ -83,19 +86,20 @@ __global__ void __launch_bounds__(kWG)
   double *Fb = flux + (static_cast<std::int64_t>(d) * nblocks + b) * G.V * G.cells;
   const int tid = static_cast<int>(threadIdx.x);
   if (d == 0) {
-    const int m = n0 + 2, cells = m * n1 * n2;
-    const int e0 = 63 * (r * (kWG / 64) + (tid >> 6)) + (tid & 63);
-    const int e = e0 < cells ? e0 : cells - 1;
-    const int a = e % m, row = e / m;
-    const unsigned c = 8u * static_cast<unsigned>(((G.lo2 + row / n1) * G.e1 + G.lo1 + row % n1) *
-                                                      G.e0 + G.lo0 - 1 + a);
+    const int m = n0 + 2;
+    const I cells = static_cast<I>(m) * n1 * n2;
+    const I e0 = static_cast<I>(63) * (r * (kWG / 64) + (tid >> 6)) + (tid & 63);
+    const I e = e0 < cells ? e0 : cells - 1;
+    const int a = static_cast<int>(e % m), row = static_cast<int>(e / m);
+    const O c = O(8) * static_cast<O>((static_cast<I>(G.lo2 + row / n1) * G.e1 + G.lo1 +
+                                       row % n1) * G.e0 + G.lo0 - 1 + a);
     const bool face = a > 0 && e0 < cells && (tid & 63) > 0;
     double upl = 0.0, upr = 0.0;
     for (int q = 0; q <= G.V; ++q) {
       const int n = q == 0 ? 0 : q - 1;
       if (q == 1) continue;  // the normal velocity came first
       double ql, qr;
-      CellStates(Ub + n * G.cells, c, 8u, RECON, ql, qr);
+      CellStates(Ub + n * G.cells, c, O(8), RECON, ql, qr);
       const double l = __shfl_up(ql, 1, 64);
       if (q == 0) {
         upl = l;
@@ -106,16 +110,15 @@ __global__ void __launch_bounds__(kWG)
     return;
   }
   const int nd = d == 1 ? n1 : n2, len = S.seg[d];
-  const int cols = n0 * (d == 1 ? n2 : n1);
-  const int t = r * kWG + tid;
-  const int f0 = t / cols * len, f1 = f0 + len < nd + 1 ? f0 + len : nd + 1;
+  const I cols = static_cast<I>(n0) * (d == 1 ? n2 : n1);
+  const I t = static_cast<I>(r) * kWG + tid;
+  const int f0 = static_cast<int>(t / cols) * len, f1 = f0 + len < nd + 1 ? f0 + len : nd + 1;
   if (f0 > nd) return;
-  const int o = t % cols / n0;
+  const int o = static_cast<int>(t % cols / n0);
   // first face's high cell: face f of the column lies below cell f
-  const unsigned st = 8u * static_cast<unsigned>(d == 1 ? G.e0 : G.e0 * G.e1);
-  const unsigned c0 =
-      8u * static_cast<unsigned>(((G.lo2 + (d == 1 ? o : f0)) * G.e1 + G.lo1 +
-                                  (d == 1 ? f0 : o)) * G.e0 + G.lo0 + t % cols % n0);
+  const O st = O(8) * static_cast<O>(d == 1 ? G.e0 : G.e0 * G.e1);
+  const O c0 = O(8) * static_cast<O>((static_cast<I>(G.lo2 + (d == 1 ? o : f0)) * G.e1 + G.lo1 +
+                                      (d == 1 ? f0 : o)) * G.e0 + G.lo0 + t % cols % n0);
   for (int q = 0; q <= G.V; ++q) {
     const int n = q == 0 ? d : q - 1;
     if (q > 0 && n == d) continue;
@@ -124,8 +127,8 @@ __global__ void __launch_bounds__(kWG)
     constexpr int H = RECON == 0 ? 2 : 1;
     double w[2 * H + 1], below = 0.0;
 #pragma unroll
-    for (int x = 0; x < 2 * H; ++x) w[x] = LoadAt(u, c0 + st * static_cast<unsigned>(x - 1 - H));
-    unsigned c = c0 - st;
+    for (int x = 0; x < 2 * H; ++x) w[x] = LoadAt(u, c0 + st * static_cast<O>(x - 1 - H));
+    O c = c0 - st;
     double next = LoadAt(u, c + H * st);
     for (int f = f0 - 1; f < f1; ++f, c += st) {
       w[2 * H] = next;
@@ -667,18 +670,18 @@ pth_status BurgersFluxes(const Topology &t, int V, const double *U, double *flux
   const int nb = static_cast<int>(t.blocks.size());
   const int n[3] = {t.fine.n[0], t.fine.n[1], t.fine.n[2]};
   FluxSplit S{};
-  const int waves = ((n[0] + 2) * n[1] * n[2] - 1 + 62) / 63;
-  S.wgs[0] = (waves + kWG / 64 - 1) / (kWG / 64);
+  const std::int64_t waves = (static_cast<std::int64_t>(n[0] + 2) * n[1] * n[2] - 1 + 62) / 63;
+  S.wgs[0] = static_cast<int>((waves + kWG / 64 - 1) / (kWG / 64));
   for (int d = 1; d < G.ndim; ++d) {
     const int segs = (n[d] + 1 + kSegFaces - 1) / kSegFaces;
     S.seg[d] = (n[d] + 1 + segs - 1) / segs;
-    S.wgs[d] = (n[0] * n[3 - d] * segs + kWG - 1) / kWG;
+    S.wgs[d] = static_cast<int>((static_cast<std::int64_t>(n[0]) * n[3 - d] * segs + kWG - 1) / kWG);
   }
   const dim3 grid(static_cast<unsigned>(S.wgs[0] + S.wgs[1] + S.wgs[2]) * nb);
-  if (recon == 0)
-    hipLaunchKernelGGL(FluxTaskKernel<0>, grid, dim3(kWG), 0, s, U, flux, G, nb, S);
-  else
-    hipLaunchKernelGGL(FluxTaskKernel<1>, grid, dim3(kWG), 0, s, U, flux, G, nb, S);
+  const bool wide = G.cells >= std::int64_t(1) << 29;
+  auto *kernel = recon == 0 ? (wide ? FluxTaskKernel<0, true> : FluxTaskKernel<0, false>)
+                            : (wide ? FluxTaskKernel<1, true> : FluxTaskKernel<1, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(kWG), 0, s, U, flux, G, nb, S);
   PTH_HIP(hipGetLastError());
   return PTH_COMPLETE;
 }

@@ -98,6 +98,13 @@ __device__ __forceinline__ double LoadAt(const double *base, unsigned byte_off) 
 __device__ __forceinline__ void StoreAt(double *base, unsigned byte_off, double v) {
   *reinterpret_cast<double *>(reinterpret_cast<char *>(base) + byte_off) = v;
 }
+// the same for components of 4 GB and more
+__device__ __forceinline__ double LoadAt(const double *base, std::int64_t byte_off) {
+  return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(base) + byte_off);
+}
+__device__ __forceinline__ void StoreAt(double *base, std::int64_t byte_off, double v) {
+  *reinterpret_cast<double *>(reinterpret_cast<char *>(base) + byte_off) = v;
+}
 
 // HLL flux of every component at one face from the face states (burgers_package.cpp:307-401
 // with lr_to_flux, burgers_package.hpp:33-43). l(n), r(n) give component n of the left and
@@ -182,8 +189,9 @@ __device__ __forceinline__ std::int64_t PatchCoarseCell(const FluxPatch &P, cons
 
 // Left and right states of one cell from its stencil along a direction (byte offsets c of the
 // cell and st of one step): WENO5Z or the MC-limited linear reconstruction.
-__device__ __forceinline__ void CellStates(const double *q, unsigned c, unsigned st, int recon,
-                                           double &ql, double &qr) {
+template <typename O>
+__device__ __forceinline__ void CellStates(const double *q, O c, O st, int recon, double &ql,
+                                           double &qr) {
   if (recon == 0)
     Weno5Z(LoadAt(q, c - 2 * st), LoadAt(q, c - st), LoadAt(q, c), LoadAt(q, c + st),
            LoadAt(q, c + 2 * st), ql, qr);
