@@ -13,7 +13,7 @@
 // Levels are single arrays of n^3 cells (the blocks of the reference's GMG grids are a
 // distribution artefact: on one GPU every level fits whole), so no level needs a ghost
 // exchange; the Dirichlet ghost (2 * 0 - mirror) is formed on the fly at the domain faces.
-// Levels of at most kBottom cells per side run inside one workgroup in LDS.
+// Levels of at most 16 cells per side run inside one workgroup (BottomKernel).
 //
 // Every kernel is batched: its grid covers a table of entries, one per (problem, level), so
 // the same V-cycle stage of several concurrent solves is one launch.
