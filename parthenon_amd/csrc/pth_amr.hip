@@ -156,7 +156,7 @@ pth_status Mesh::Tag(MeshData &md) {
   if (nc > 0) {
     const std::int64_t need = static_cast<std::int64_t>(nb) * nc;
     if (amr.maxd_n < need) {
-      if (amr.maxd) (void)hipFree(amr.maxd);
+      if (amr.maxd) PTH_DROP(hipFree(amr.maxd));
       amr.maxd = nullptr;
       amr.maxd_n = 0;
       PTH_HIP(hipMalloc(&amr.maxd, sizeof(double) * need));
@@ -181,9 +181,8 @@ pth_status Mesh::Tag(MeshData &md) {
       a.ndim = 1 + (a.n[1] > 1) + (a.n[2] > 1);
       a.method = c.method;
       ProfScope prof("refinement_tag", stream);
-      hipLaunchKernelGGL(DerivativeMaxKernel, dim3(nb), dim3(kTagWG), 0, stream, a, amr.maxd, nc,
-                         q);
-      PTH_HIP(hipGetLastError());
+      PTH_LAUNCH(DerivativeMaxKernel, dim3(nb), dim3(kTagWG), 0, stream, a, amr.maxd, nc,
+                 q);
     }
     PTH_HIP(hipMemcpyAsync(maxd.data(), amr.maxd, sizeof(double) * need, hipMemcpyDeviceToHost,
                            stream));
@@ -423,7 +422,7 @@ pth_status Mesh::Adapt(int *modified) {
   if (LaunchCopy(ct, stream) != PTH_COMPLETE) return fail();
   if (LaunchProlongT(pt, nt, nm->geom, stream, true) != PTH_COMPLETE) return fail();
   if (LaunchProlongT(pl, nt, nm->geom, stream, false) != PTH_COMPLETE) return fail();
-  if (hipStreamSynchronize(stream) != hipSuccess) {
+  if (Failed(hipStreamSynchronize(stream))) {
     SetError("remesh transfer failed on the device");
     return fail();
   }

@@ -681,8 +681,7 @@ pth_status BurgersFluxes(const Topology &t, int V, const double *U, double *flux
   const bool wide = G.cells >= std::int64_t(1) << 29;
   auto *kernel = recon == 0 ? (wide ? FluxTaskKernel<0, true> : FluxTaskKernel<0, false>)
                             : (wide ? FluxTaskKernel<1, true> : FluxTaskKernel<1, false>);
-  hipLaunchKernelGGL(kernel, grid, dim3(kWG), 0, s, U, flux, G, nb, S);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(kernel, grid, dim3(kWG), 0, s, U, flux, G, nb, S);
   return PTH_COMPLETE;
 }
 
@@ -692,9 +691,8 @@ pth_status FluxDivergence(const Topology &t, int V, const double *flux, double *
   const Geo G = MakeGeo(t, V);
   const int nb = static_cast<int>(t.blocks.size());
   if (ChunkGrid(t, static_cast<std::int64_t>(V) * nb) == 0) return PTH_COMPLETE;
-  hipLaunchKernelGGL(FluxDivKernel, dim3(ChunkGrid(t, static_cast<std::int64_t>(V) * nb)),
-                     dim3(kWG), 0, s, flux, dudt, coef, G, nb);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(FluxDivKernel, dim3(ChunkGrid(t, static_cast<std::int64_t>(V) * nb)),
+             dim3(kWG), 0, s, flux, dudt, coef, G, nb);
   return PTH_COMPLETE;
 }
 
@@ -702,8 +700,7 @@ pth_status WeightedSum(const double *x, const double *y, double w1, double w2, d
                        std::int64_t n, hipStream_t s) {
   if (n == 0) return PTH_COMPLETE;
   ProfScope prof("weighted_sum", s);
-  hipLaunchKernelGGL(WsumKernel, dim3(Grid(n)), dim3(kWG), 0, s, x, y, w1, w2, z, n);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(WsumKernel, dim3(Grid(n)), dim3(kWG), 0, s, x, y, w1, w2, z, n);
   return PTH_COMPLETE;
 }
 
@@ -714,8 +711,7 @@ pth_status BurgersDerived(const Topology &t, int V, const double *U, double *out
   const int nb = static_cast<int>(t.blocks.size());
   const std::int64_t total =
       static_cast<std::int64_t>(t.fine.n[0]) * t.fine.n[1] * t.fine.n[2] * nb;
-  hipLaunchKernelGGL(DerivedKernel, dim3(Grid(total)), dim3(kWG), 0, s, U, out, G, nb);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(DerivedKernel, dim3(Grid(total)), dim3(kWG), 0, s, U, out, G, nb);
   return PTH_COMPLETE;
 }
 
@@ -731,9 +727,8 @@ pth_status FlxcorSend(const Topology &t, const FluxCorrection &fc, const double 
   const Geo G = MakeGeo(t, fc.ncomp);
   const int nb = static_cast<int>(t.blocks.size());
   const dim3 grid(static_cast<unsigned>(fc.host.size()), (fc.max_cells + 63) / 64);
-  hipLaunchKernelGGL(FlxcorSendKernel, grid, dim3(64), 0, s, fc.dev, flux, fc.store, G, nb,
-                     fc.ncomp);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(FlxcorSendKernel, grid, dim3(64), 0, s, fc.dev, flux, fc.store, G, nb,
+             fc.ncomp);
   return PTH_COMPLETE;
 }
 
@@ -743,9 +738,8 @@ pth_status FlxcorSet(const Topology &t, const FluxCorrection &fc, double *flux, 
   const Geo G = MakeGeo(t, fc.ncomp);
   const int nb = static_cast<int>(t.blocks.size());
   const dim3 grid(static_cast<unsigned>(fc.host.size()), (fc.max_cells + 63) / 64);
-  hipLaunchKernelGGL(FlxcorSetKernel, grid, dim3(64), 0, s, fc.dev, fc.store, flux, G, nb,
-                     fc.ncomp);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(FlxcorSetKernel, grid, dim3(64), 0, s, fc.dev, fc.store, flux, G, nb,
+             fc.ncomp);
   return PTH_COMPLETE;
 }
 
@@ -768,8 +762,8 @@ pth_status BurgersReconFlux(const Topology &t, int V, const double *U, double *f
   const int N = t.fine.n[0];
   const dim3 grid(static_cast<unsigned>(3 * (N / ppw) * nb));
 #define PTH_RF_LAUNCH(NN, NV, PT, PW)                                                         \
-  hipLaunchKernelGGL((ReconFluxKernel<NN, 4, NV, PT, PW>), grid, dim3(kWG), 0, s, U, flux, nb, \
-                     recon)
+  PTH_LAUNCH((ReconFluxKernel<NN, 4, NV, PT, PW>), grid, dim3(kWG), 0, s, U, flux, nb, \
+             recon)
 #define PTH_RF_PPW(NN, NV, PT)                                                                \
   if (ppw == 1)                                                                               \
     PTH_RF_LAUNCH(NN, NV, PT, 1);                                                             \
@@ -809,7 +803,6 @@ pth_status BurgersReconFlux(const Topology &t, int V, const double *U, double *f
 #undef PTH_RF_PARTS
 #undef PTH_RF_PPW
 #undef PTH_RF_LAUNCH
-  PTH_HIP(hipGetLastError());
   return PTH_COMPLETE;
 }
 
@@ -828,8 +821,8 @@ pth_status BurgersFluxUpdate(const Topology &t, int V, const double *flux, const
   const dim3 grid(((cells + kWG - 1) / kWG) * nb);
 #define PTH_FU_CASE(NV)                                                                       \
   case NV:                                                                                    \
-    hipLaunchKernelGGL(FluxUpdateKernel<NV>, grid, dim3(kWG), 0, s, flux, U0, base, out,      \
-                       derived, partial, coef, G, nb, beta, dtvar);                           \
+    PTH_LAUNCH(FluxUpdateKernel<NV>, grid, dim3(kWG), 0, s, flux, U0, base, out,      \
+               derived, partial, coef, G, nb, beta, dtvar);                           \
     break;
   switch (V) {
     PTH_FU_CASE(4)
@@ -847,7 +840,6 @@ pth_status BurgersFluxUpdate(const Topology &t, int V, const double *flux, const
     PTH_FU_CASE(16)
   }
 #undef PTH_FU_CASE
-  PTH_HIP(hipGetLastError());
   return PTH_COMPLETE;
 }
 
@@ -879,19 +871,17 @@ pth_status BurgersMassHistory(const Topology &t, int V, const double *U,
       static_cast<std::int64_t>(t.fine.n[0]) * t.fine.n[1] * t.fine.n[2] * V * nb;
   int grid = Grid(total);
   if (grid > nscratch / 8) grid = nscratch / 8;
-  hipLaunchKernelGGL(MassHistoryKernel, dim3(grid), dim3(kWG), 0, s, U, geom, coef, G, nb, O,
-                     vol, scratch);
-  hipLaunchKernelGGL(SumPartials8Kernel, dim3(1), dim3(64), 0, s, scratch, grid, out);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(MassHistoryKernel, dim3(grid), dim3(kWG), 0, s, U, geom, coef, G, nb, O,
+             vol, scratch);
+  PTH_LAUNCH(SumPartials8Kernel, dim3(1), dim3(64), 0, s, scratch, grid, out);
   return PTH_COMPLETE;
 }
 
 pth_status BurgersClock(const double *partial, int n, double cfl, double *dtvar, int advance,
                         const ClockLimits &lim, hipStream_t s) {
   ProfScope prof("clock", s);
-  hipLaunchKernelGGL(ClockKernel, dim3(1), dim3(kClockWG), 0, s, partial, n, cfl, dtvar,
-                     advance, lim);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(ClockKernel, dim3(1), dim3(kClockWG), 0, s, partial, n, cfl, dtvar,
+             advance, lim);
   return PTH_COMPLETE;
 }
 
@@ -911,9 +901,8 @@ pth_status BurgersDtToDevice(const Topology &t, int V, const double *U, const Bl
     SetError("CFL reduction: more partials than the scratch holds");
     return PTH_FAIL;
   }
-  hipLaunchKernelGGL(DtKernel, dim3(grid), dim3(kWG), 0, s, U, coef, G, nb, partial);
-  hipLaunchKernelGGL(MinScaleKernel, dim3(1), dim3(64), 0, s, partial, grid, cfl, out);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(DtKernel, dim3(grid), dim3(kWG), 0, s, U, coef, G, nb, partial);
+  PTH_LAUNCH(MinScaleKernel, dim3(1), dim3(64), 0, s, partial, grid, cfl, out);
   return PTH_COMPLETE;
 }
 
@@ -926,9 +915,8 @@ pth_status BurgersDtMin(const Topology &t, int V, const double *U, const BlockCo
       static_cast<std::int64_t>(t.fine.n[0]) * t.fine.n[1] * t.fine.n[2] * nb;
   int grid = Grid(total);
   if (grid > npartial) grid = npartial;
-  hipLaunchKernelGGL(DtKernel, dim3(grid), dim3(kWG), 0, s, U, coef, G, nb, partial);
-  hipLaunchKernelGGL(MinFinalKernel, dim3(1), dim3(64), 0, s, partial, grid, out);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(DtKernel, dim3(grid), dim3(kWG), 0, s, U, coef, G, nb, partial);
+  PTH_LAUNCH(MinFinalKernel, dim3(1), dim3(64), 0, s, partial, grid, out);
   return PTH_COMPLETE;
 }
 

@@ -507,7 +507,7 @@ __global__ void __launch_bounds__(kWG) BoundaryConditionKernel(const BcBox *__re
 }  // namespace
 
 void BcTable::Free() {
-  if (dev) (void)hipFree(dev);
+  if (dev) PTH_DROP(hipFree(dev));
   dev = nullptr;
 }
 
@@ -522,9 +522,8 @@ pth_status BcTable::Upload() {
 pth_status LaunchBoundaryConditions(const BcTable &t, hipStream_t s) {
   if (t.host.empty()) return PTH_COMPLETE;
   ProfScope prof("boundary_conditions", s);
-  hipLaunchKernelGGL(BoundaryConditionKernel, dim3(static_cast<unsigned>(t.host.size())),
-                     dim3(kWG), 0, s, t.dev);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(BoundaryConditionKernel, dim3(static_cast<unsigned>(t.host.size())),
+             dim3(kWG), 0, s, t.dev);
   return PTH_COMPLETE;
 }
 
@@ -534,8 +533,8 @@ std::uint64_t Magic(int d) {
 }
 
 void Table::Free() {
-  if (dev) (void)hipFree(dev);
-  if (dev_items) (void)hipFree(dev_items);
+  if (dev) PTH_DROP(hipFree(dev));
+  if (dev_items) PTH_DROP(hipFree(dev_items));
   dev = nullptr;
   dev_items = nullptr;
 }
@@ -574,17 +573,16 @@ pth_status LaunchPack(const Table &t, double *, hipStream_t s, bool to_buffer, i
   if (mode == PTH_PACK_PER_BUFFER) {
     for (const auto &R : t.host) {
       const std::int64_t count = static_cast<std::int64_t>(R.n[0]) * R.n[1] * R.n[2] * R.nc;
-      hipLaunchKernelGGL(PackOneKernel, dim3(static_cast<unsigned>((count + kWG - 1) / kWG)),
-                         dim3(kWG), 0, s, R, to_buffer ? 1 : 0);
+      PTH_LAUNCH(PackOneKernel, dim3(static_cast<unsigned>((count + kWG - 1) / kWG)),
+                 dim3(kWG), 0, s, R, to_buffer ? 1 : 0);
     }
   } else {
     const int n = static_cast<int>(t.items.size());
     if (to_buffer)
-      hipLaunchKernelGGL(PackKernel<true>, dim3(WaveGrid(n)), dim3(kWG), 0, s, t.dev, t.dev_items, n);
+      PTH_LAUNCH(PackKernel<true>, dim3(WaveGrid(n)), dim3(kWG), 0, s, t.dev, t.dev_items, n);
     else
-      hipLaunchKernelGGL(PackKernel<false>, dim3(WaveGrid(n)), dim3(kWG), 0, s, t.dev, t.dev_items, n);
+      PTH_LAUNCH(PackKernel<false>, dim3(WaveGrid(n)), dim3(kWG), 0, s, t.dev, t.dev_items, n);
   }
-  PTH_HIP(hipGetLastError());
   return PTH_COMPLETE;
 }
 
@@ -592,8 +590,7 @@ pth_status LaunchCopy(const Table &t, hipStream_t s) {
   if (t.total == 0) return PTH_COMPLETE;
   ProfScope prof("remesh_copy", s);
   const int n = static_cast<int>(t.items.size());
-  hipLaunchKernelGGL(CopyKernel, dim3(WaveGrid(n)), dim3(kWG), 0, s, t.dev, t.dev_items, n);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(CopyKernel, dim3(WaveGrid(n)), dim3(kWG), 0, s, t.dev, t.dev_items, n);
   return PTH_COMPLETE;
 }
 
@@ -610,9 +607,8 @@ pth_status LaunchExchangeDirect(const Table &pack, const Table &unpack, hipStrea
   }
   ProfScope prof("exchange_direct", s);
   const int n = static_cast<int>(pack.items.size());
-  hipLaunchKernelGGL(ExchangeRegionKernel, dim3(WaveGrid(n)), dim3(kWG), 0, s, pack.dev,
-                     unpack.dev, pack.dev_items, n);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(ExchangeRegionKernel, dim3(WaveGrid(n)), dim3(kWG), 0, s, pack.dev,
+             unpack.dev, pack.dev_items, n);
   return PTH_COMPLETE;
 }
 
@@ -647,12 +643,11 @@ pth_status LaunchShell(const Topology &t, const std::vector<ShellBrick> &bricks,
     A.nblocks = nb;
     const dim3 grid(static_cast<unsigned>(nq) * nb);
 #define PTH_SHELL(NN, GG)                                                              \
-  if (n == NN && g == GG) hipLaunchKernelGGL((ShellKernel<NN, GG>), grid, dim3(kWG), 0, s, A);
+  if (n == NN && g == GG) PTH_LAUNCH((ShellKernel<NN, GG>), grid, dim3(kWG), 0, s, A);
     PTH_SHELL(8, 2) PTH_SHELL(8, 3) PTH_SHELL(8, 4)
     PTH_SHELL(16, 2) PTH_SHELL(16, 3) PTH_SHELL(16, 4)
     PTH_SHELL(32, 2) PTH_SHELL(32, 3) PTH_SHELL(32, 4)
 #undef PTH_SHELL
-    PTH_HIP(hipGetLastError());
   }
   return PTH_COMPLETE;
 }
@@ -668,37 +663,31 @@ static ProResParams Params(const Topology &topo) {
 }
 
 template <int OP>
-static void LaunchProRes(const Table &t, const Topology &topo, const DeviceBlockGeom *geom,
-                         hipStream_t s) {
+static pth_status LaunchProRes(const Table &t, const Topology &topo, const DeviceBlockGeom *geom,
+                               hipStream_t s) {
   const int n = static_cast<int>(t.items.size());
   const ProResParams P = Params(topo);
   if (P.act[0] && P.act[1] && P.act[2])
-    hipLaunchKernelGGL((ProResKernel<OP, true>), dim3(GridFor(n)), dim3(kWG), 0, s, t.dev,
-                       t.dev_items, n, geom, P);
+    PTH_LAUNCH((ProResKernel<OP, true>), dim3(GridFor(n)), dim3(kWG), 0, s, t.dev,
+               t.dev_items, n, geom, P);
   else
-    hipLaunchKernelGGL((ProResKernel<OP, false>), dim3(GridFor(n)), dim3(kWG), 0, s, t.dev,
-                       t.dev_items, n, geom, P);
+    PTH_LAUNCH((ProResKernel<OP, false>), dim3(GridFor(n)), dim3(kWG), 0, s, t.dev,
+               t.dev_items, n, geom, P);
+  return PTH_COMPLETE;
 }
 
 pth_status LaunchRestrictT(const Table &t, const Topology &topo, const DeviceBlockGeom *geom,
                            hipStream_t s) {
   if (t.total == 0) return PTH_COMPLETE;
   ProfScope prof("restrict", s);
-  LaunchProRes<0>(t, topo, geom, s);
-  PTH_HIP(hipGetLastError());
-  return PTH_COMPLETE;
+  return LaunchProRes<0>(t, topo, geom, s);
 }
 
 pth_status LaunchProlongT(const Table &t, const Topology &topo, const DeviceBlockGeom *geom,
                           hipStream_t s, bool minmod) {
   if (t.total == 0) return PTH_COMPLETE;
   ProfScope prof("prolong", s);
-  if (minmod)
-    LaunchProRes<1>(t, topo, geom, s);
-  else
-    LaunchProRes<2>(t, topo, geom, s);
-  PTH_HIP(hipGetLastError());
-  return PTH_COMPLETE;
+  return minmod ? LaunchProRes<1>(t, topo, geom, s) : LaunchProRes<2>(t, topo, geom, s);
 }
 
 }  // namespace pth

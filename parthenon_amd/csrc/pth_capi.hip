@@ -21,6 +21,11 @@ thread_local std::string g_error;
 void SetError(const std::string &msg) { g_error = msg; }
 const char *ErrorText() { return g_error.c_str(); }
 
+void Dropped(hipError_t e, const char *call, const char *file, int line) {
+  if (!Failed(e) || e == hipErrorDeinitialized) return;  // the process ends: nothing to free
+  std::fprintf(stderr, "parthenon_amd: %s:%d: %s: %s\n", file, line, call, hipGetErrorString(e));
+}
+
 Profiler &Prof() {
   static Profiler p;
   return p;
@@ -29,7 +34,7 @@ Profiler &Prof() {
 hipEvent_t Profiler::Take() {
   if (pool.empty()) {
     hipEvent_t e = nullptr;
-    if (hipEventCreate(&e) != hipSuccess) return nullptr;
+    if (Failed(hipEventCreate(&e))) return nullptr;
     return e;
   }
   hipEvent_t e = pool.back();
@@ -48,23 +53,23 @@ void Profiler::Clear() {
 ProfScope::ProfScope(const char *name, hipStream_t s) : name_(name), s_(s) {
   if (!Prof().on) return;
   a_ = Prof().Take();
-  if (a_) (void)hipEventRecord(a_, s_);
+  if (a_) PTH_DROP(hipEventRecord(a_, s_));
 }
 
 ProfScope::~ProfScope() {
   if (!a_) return;
   hipEvent_t b = Prof().Take();
   if (!b) return;
-  (void)hipEventRecord(b, s_);
+  PTH_DROP(hipEventRecord(b, s_));
   Prof().records.push_back(ProfRecord{name_, a_, b});
 }
 
 MeshData::~MeshData() {
   for (auto &s : store) {
     if (!s.owned) continue;
-    if (s.data) (void)hipFree(s.data);
-    if (s.coarse) (void)hipFree(s.coarse);
-    if (s.flux) (void)hipFree(s.flux);
+    if (s.data) PTH_DROP(hipFree(s.data));
+    if (s.coarse) PTH_DROP(hipFree(s.coarse));
+    if (s.flux) PTH_DROP(hipFree(s.flux));
   }
   for (auto &c : cache) {
     c.pack.Free();
@@ -79,14 +84,14 @@ MeshData::~MeshData() {
     c.unpack_rest.Free();
     c.pack_cross.Free();
     c.unpack_cross.Free();
-    if (c.shell_order) (void)hipFree(c.shell_order);
+    if (c.shell_order) PTH_DROP(hipFree(c.shell_order));
     c.shell_order = nullptr;
   }
   for (auto &kv : packs) kv.second.Free();
 }
 
 void PackEntry::Free() {
-  if (dev) (void)hipFree(dev);
+  if (dev) PTH_DROP(hipFree(dev));
   dev = nullptr;
 }
 
@@ -94,28 +99,28 @@ Mesh::~Mesh() {
   data.clear();
   for (auto &kv : flxcor) kv.second.Free();
   for (auto &s : one_copy) {
-    if (s.data) (void)hipFree(s.data);
-    if (s.coarse) (void)hipFree(s.coarse);
-    if (s.flux) (void)hipFree(s.flux);
+    if (s.data) PTH_DROP(hipFree(s.data));
+    if (s.coarse) PTH_DROP(hipFree(s.coarse));
+    if (s.flux) PTH_DROP(hipFree(s.flux));
   }
-  if (arena_base) (void)hipFree(arena_base);
-  if (same_level) (void)hipFree(same_level);
-  if (split_list) (void)hipFree(split_list);
-  if (geom) (void)hipFree(geom);
-  if (coef) (void)hipFree(coef);
-  if (flux_scratch) (void)hipFree(flux_scratch);
-  if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
-  if (graph) (void)hipGraphDestroy(graph);
-  if (run_stream) (void)hipStreamDestroy(run_stream);
+  if (arena_base) PTH_DROP(hipFree(arena_base));
+  if (same_level) PTH_DROP(hipFree(same_level));
+  if (split_list) PTH_DROP(hipFree(split_list));
+  if (geom) PTH_DROP(hipFree(geom));
+  if (coef) PTH_DROP(hipFree(coef));
+  if (flux_scratch) PTH_DROP(hipFree(flux_scratch));
+  if (graph_exec) PTH_DROP(hipGraphExecDestroy(graph_exec));
+  if (graph) PTH_DROP(hipGraphDestroy(graph));
+  if (run_stream) PTH_DROP(hipStreamDestroy(run_stream));
   for (hipEvent_t e : order_ev)
-    if (e) (void)hipEventDestroy(e);
+    if (e) PTH_DROP(hipEventDestroy(e));
   for (hipEvent_t e : fork_ev)
-    if (e) (void)hipEventDestroy(e);
-  if (side_stream) (void)hipStreamDestroy(side_stream);
-  if (dtvar) (void)hipFree(dtvar);
-  if (scratch) (void)hipFree(scratch);
-  if (pinned) (void)hipHostFree(pinned);
-  if (amr.maxd) (void)hipFree(amr.maxd);
+    if (e) PTH_DROP(hipEventDestroy(e));
+  if (side_stream) PTH_DROP(hipStreamDestroy(side_stream));
+  if (dtvar) PTH_DROP(hipFree(dtvar));
+  if (scratch) PTH_DROP(hipFree(scratch));
+  if (pinned) PTH_DROP(hipHostFree(pinned));
+  if (amr.maxd) PTH_DROP(hipFree(amr.maxd));
 }
 
 int Mesh::FieldIndex(const std::string &n) const {
@@ -578,7 +583,7 @@ pth_status Mesh::BuildCrossExchange(MeshData &md, bool *ok) {
   c.pack_cross.Free();
   c.unpack_cross.Free();
   c.shell.clear();
-  if (c.shell_order) (void)hipFree(c.shell_order);
+  if (c.shell_order) PTH_DROP(hipFree(c.shell_order));
   c.shell_order = nullptr;
   {  // blocks in Morton order of their positions on the finest level's lattice
     const int nb = static_cast<int>(topo.blocks.size());
@@ -731,9 +736,9 @@ pth_status Mesh::BuildBoundaryConditions(MeshData &md, BoundCache &c) {
 }
 
 void FluxCorrection::Free() {
-  if (dev) (void)hipFree(dev);
-  if (dev_face) (void)hipFree(dev_face);
-  if (store) (void)hipFree(store);
+  if (dev) PTH_DROP(hipFree(dev));
+  if (dev_face) PTH_DROP(hipFree(dev_face));
+  if (store) PTH_DROP(hipFree(store));
   dev = nullptr;
   dev_face = nullptr;
   store = nullptr;
@@ -832,14 +837,14 @@ FluxCorrection *Mesh::FluxPatches(int f) {
       }
   c.store_n = total;
   if (!c.host.empty()) {
-    if (hipMalloc(&c.dev, sizeof(FluxPatch) * c.host.size()) != hipSuccess ||
-        hipMalloc(&c.dev_face, sizeof(int) * c.face.size()) != hipSuccess ||
-        hipMalloc(&c.store, sizeof(double) * total) != hipSuccess ||
-        hipMemset(c.store, 0, sizeof(double) * total) != hipSuccess ||
-        hipMemcpy(c.dev, c.host.data(), sizeof(FluxPatch) * c.host.size(),
-                  hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(c.dev_face, c.face.data(), sizeof(int) * c.face.size(),
-                  hipMemcpyHostToDevice) != hipSuccess) {
+    if (Failed(hipMalloc(&c.dev, sizeof(FluxPatch) * c.host.size())) ||
+        Failed(hipMalloc(&c.dev_face, sizeof(int) * c.face.size())) ||
+        Failed(hipMalloc(&c.store, sizeof(double) * total)) ||
+        Failed(hipMemset(c.store, 0, sizeof(double) * total)) ||
+        Failed(hipMemcpy(c.dev, c.host.data(), sizeof(FluxPatch) * c.host.size(),
+                  hipMemcpyHostToDevice)) ||
+        Failed(hipMemcpy(c.dev_face, c.face.data(), sizeof(int) * c.face.size(),
+                  hipMemcpyHostToDevice))) {
       SetError("flux correction: device allocation failed");
       c.Free();
       return nullptr;
@@ -1235,10 +1240,10 @@ pth_pack *pth_pack_get(pth_meshdata *mdh, const char *const *fields, int nfields
     }
   const size_t pbytes = ptr.size() * sizeof(double *);
   const size_t bbytes = e.bounds.size() * sizeof(int);
-  if (hipMalloc(&e.dev, pbytes + bbytes) != hipSuccess ||
-      hipMemcpy(e.dev, ptr.data(), pbytes, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(static_cast<char *>(e.dev) + pbytes, e.bounds.data(), bbytes,
-                hipMemcpyHostToDevice) != hipSuccess) {
+  if (Failed(hipMalloc(&e.dev, pbytes + bbytes)) ||
+      Failed(hipMemcpy(e.dev, ptr.data(), pbytes, hipMemcpyHostToDevice)) ||
+      Failed(hipMemcpy(static_cast<char *>(e.dev) + pbytes, e.bounds.data(), bbytes,
+                hipMemcpyHostToDevice))) {
     SetError("pth_pack_get: device table upload failed");
     e.Free();
     return nullptr;
@@ -1650,9 +1655,9 @@ pth_status pth_profile_enable(int enable) {
 int pth_profile_report(char *buf, int len) {
   std::map<std::string, std::pair<int, double>> acc;
   for (auto &r : Prof().records) {
-    if (hipEventSynchronize(r.stop) != hipSuccess) continue;
+    if (Failed(hipEventSynchronize(r.stop))) continue;
     float ms = 0.f;
-    if (hipEventElapsedTime(&ms, r.start, r.stop) != hipSuccess) continue;
+    if (Failed(hipEventElapsedTime(&ms, r.start, r.stop))) continue;
     auto &a = acc[r.name];
     a.first += 1;
     a.second += ms;

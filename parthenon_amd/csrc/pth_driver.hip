@@ -111,7 +111,7 @@ pth_status SplitLists(Mesh &m) {
     }
     (inner ? a : b).push_back(q);
   }
-  if (m.split_list) (void)hipFree(m.split_list);
+  if (m.split_list) PTH_DROP(hipFree(m.split_list));
   m.split_list = nullptr;
   m.split_nA = static_cast<int>(a.size());
   m.split_nB = static_cast<int>(b.size());
@@ -159,7 +159,7 @@ pth_status Setup(Mesh *m, Ctx &x) {
   const bool sweep = m->run_sweep && BurgersSweepSupported(m->topo, x.V);
   // the other path's fluxes: the field's own, or scratch when U was declared without them
   if (!planes && !sweep && !x.base->store[x.fu].flux && m->flux_scratch_n != 3 * nd) {
-    if (m->flux_scratch) (void)hipFree(m->flux_scratch);
+    if (m->flux_scratch) PTH_DROP(hipFree(m->flux_scratch));
     m->flux_scratch = nullptr;
     m->flux_scratch_n = 0;
     PTH_HIP(hipMalloc(&m->flux_scratch, sizeof(double) * 3 * nd));
@@ -334,13 +334,13 @@ pth_status TuneReconFlux(Ctx &x, hipStream_t s) {
     for (int ppw : {1, 2, 4}) {
       st = BurgersReconFlux(m.topo, x.V, U, flux, m.run_recon, part, ppw, s);  // warm-up
       if (st != PTH_COMPLETE) break;
-      if (hipEventRecord(ev[0], s) != hipSuccess) st = PTH_FAIL;
+      if (Failed(hipEventRecord(ev[0], s))) st = PTH_FAIL;
       for (int r = 0; r < 3 && st == PTH_COMPLETE; ++r)
         st = BurgersReconFlux(m.topo, x.V, U, flux, m.run_recon, part, ppw, s);
       float ms = 0.0f;
-      if (st != PTH_COMPLETE || hipEventRecord(ev[1], s) != hipSuccess ||
-          hipEventSynchronize(ev[1]) != hipSuccess ||
-          hipEventElapsedTime(&ms, ev[0], ev[1]) != hipSuccess) {
+      if (st != PTH_COMPLETE || Failed(hipEventRecord(ev[1], s)) ||
+          Failed(hipEventSynchronize(ev[1])) ||
+          Failed(hipEventElapsedTime(&ms, ev[0], ev[1]))) {
         if (st == PTH_COMPLETE) SetError("reconstruction tuning: event timing failed");
         st = PTH_FAIL;
         break;
@@ -365,15 +365,15 @@ pth_status TuneReconFlux(Ctx &x, hipStream_t s) {
                         static_cast<int>(m.scratch_n), m.coef, 1.0, m.dtvar, m.run_recon, x.fc,
                         waves, 1, nullptr, nullptr, s);
       if (st != PTH_COMPLETE) break;
-      if (hipEventRecord(ev[0], s) != hipSuccess) st = PTH_FAIL;
+      if (Failed(hipEventRecord(ev[0], s))) st = PTH_FAIL;
       for (int r = 0; r < 3 && st == PTH_COMPLETE; ++r)
         st = BurgersSweep(m.topo, x.V, U, U, x.one->store[x.fu].data, nullptr, nullptr,
                           static_cast<int>(m.scratch_n), m.coef, 1.0, m.dtvar, m.run_recon,
                           x.fc, waves, 1, nullptr, nullptr, s);
       float ms = 0.0f;
-      if (st != PTH_COMPLETE || hipEventRecord(ev[1], s) != hipSuccess ||
-          hipEventSynchronize(ev[1]) != hipSuccess ||
-          hipEventElapsedTime(&ms, ev[0], ev[1]) != hipSuccess) {
+      if (st != PTH_COMPLETE || Failed(hipEventRecord(ev[1], s)) ||
+          Failed(hipEventSynchronize(ev[1])) ||
+          Failed(hipEventElapsedTime(&ms, ev[0], ev[1]))) {
         if (st == PTH_COMPLETE) SetError("sweep tuning: event timing failed");
         st = PTH_FAIL;
         break;
@@ -387,16 +387,16 @@ pth_status TuneReconFlux(Ctx &x, hipStream_t s) {
     for (int spread : {1, 2, 3}) {
       if (st != PTH_COMPLETE) break;
       for (int r = 0; r < 4 && st == PTH_COMPLETE; ++r) {
-        if (r == 1 && hipEventRecord(ev[0], s) != hipSuccess) st = PTH_FAIL;
+        if (r == 1 && Failed(hipEventRecord(ev[0], s))) st = PTH_FAIL;
         if (st == PTH_COMPLETE)
           st = BurgersSweep(m.topo, x.V, U, U, x.one->store[x.fu].data, nullptr, nullptr,
                             static_cast<int>(m.scratch_n), m.coef, 1.0, m.dtvar, m.run_recon,
                             x.fc, m.sweep_waves, spread, nullptr, nullptr, s);
       }
       float ms = 0.0f;
-      if (st != PTH_COMPLETE || hipEventRecord(ev[1], s) != hipSuccess ||
-          hipEventSynchronize(ev[1]) != hipSuccess ||
-          hipEventElapsedTime(&ms, ev[0], ev[1]) != hipSuccess) {
+      if (st != PTH_COMPLETE || Failed(hipEventRecord(ev[1], s)) ||
+          Failed(hipEventSynchronize(ev[1])) ||
+          Failed(hipEventElapsedTime(&ms, ev[0], ev[1]))) {
         if (st == PTH_COMPLETE) SetError("sweep tuning: event timing failed");
         st = PTH_FAIL;
         break;
@@ -408,8 +408,8 @@ pth_status TuneReconFlux(Ctx &x, hipStream_t s) {
     }
   }
   Prof().on = prof;
-  (void)hipEventDestroy(ev[0]);
-  (void)hipEventDestroy(ev[1]);
+  PTH_DROP(hipEventDestroy(ev[0]));
+  PTH_DROP(hipEventDestroy(ev[1]));
   if (st == PTH_COMPLETE) m.rf_tuned = true;
   return st;
 }
@@ -455,7 +455,7 @@ pth_status TuneForm(Ctx &x, hipStream_t s) {
   pth_status st = PTH_COMPLETE;
   auto copy = [&](double *dst, const double *src, std::int64_t n) {
     if (st == PTH_COMPLETE && n > 0 &&
-        hipMemcpyAsync(dst, src, sizeof(double) * n, hipMemcpyDeviceToDevice, s) != hipSuccess) {
+        Failed(hipMemcpyAsync(dst, src, sizeof(double) * n, hipMemcpyDeviceToDevice, s))) {
       SetError("stage-form tuning: state copy failed");
       st = PTH_FAIL;
     }
@@ -463,7 +463,7 @@ pth_status TuneForm(Ctx &x, hipStream_t s) {
   copy(save, U, nd);
   if (D) copy(save + nd, D, ndd);
   copy(save + nd + ndd, m.dtvar, kClockSlots);
-  if (hipEventCreate(&ev[0]) != hipSuccess || hipEventCreate(&ev[1]) != hipSuccess) {
+  if (Failed(hipEventCreate(&ev[0])) || Failed(hipEventCreate(&ev[1]))) {
     SetError("stage-form tuning: event creation failed");
     st = PTH_FAIL;
   }
@@ -479,12 +479,12 @@ pth_status TuneForm(Ctx &x, hipStream_t s) {
     copy(U, save, nd);
     copy(m.dtvar, save + nd + ndd, kClockSlots);
     if (st == PTH_COMPLETE) st = Cycle(x, s);  // warm-up
-    if (st == PTH_COMPLETE && hipEventRecord(ev[0], s) != hipSuccess) st = PTH_FAIL;
+    if (st == PTH_COMPLETE && Failed(hipEventRecord(ev[0], s))) st = PTH_FAIL;
     for (int c = 0; c < 2 && st == PTH_COMPLETE; ++c) st = Cycle(x, s);
     float ms = 0.0f;
-    if (st != PTH_COMPLETE || hipEventRecord(ev[1], s) != hipSuccess ||
-        hipEventSynchronize(ev[1]) != hipSuccess ||
-        hipEventElapsedTime(&ms, ev[0], ev[1]) != hipSuccess) {
+    if (st != PTH_COMPLETE || Failed(hipEventRecord(ev[1], s)) ||
+        Failed(hipEventSynchronize(ev[1])) ||
+        Failed(hipEventElapsedTime(&ms, ev[0], ev[1]))) {
       if (st == PTH_COMPLETE) SetError("stage-form tuning: event timing failed");
       st = PTH_FAIL;
       break;
@@ -498,13 +498,13 @@ pth_status TuneForm(Ctx &x, hipStream_t s) {
   copy(U, save, nd);
   if (D) copy(D, save + nd, ndd);
   copy(m.dtvar, save + nd + ndd, kClockSlots);
-  if (st == PTH_COMPLETE && hipStreamSynchronize(s) != hipSuccess) {
+  if (st == PTH_COMPLETE && Failed(hipStreamSynchronize(s))) {
     SetError("stage-form tuning: synchronize failed");
     st = PTH_FAIL;
   }
-  (void)hipFree(save);
+  PTH_DROP(hipFree(save));
   for (hipEvent_t e : ev)
-    if (e) (void)hipEventDestroy(e);
+    if (e) PTH_DROP(hipEventDestroy(e));
   if (st != PTH_COMPLETE) {
     m.run_sweep = keep_sweep;
     m.run_overlap = keep_overlap;
@@ -551,7 +551,8 @@ pth_status RunCycles(Mesh &m, Ctx &x, hipStream_t s, int ncycles, bool use_graph
     const hipError_t e = hipStreamEndCapture(s, &g);
     Prof().on = prof;
     if (st != PTH_COMPLETE) {
-      if (g) (void)hipGraphDestroy(g);
+      (void)Failed(e);  // st's text says why
+      if (g) PTH_DROP(hipGraphDestroy(g));
       return PTH_FAIL;
     }
     PTH_HIP(e);
@@ -599,8 +600,8 @@ pth_status pth_burgers_init(pth_mesh *mh, double cfl, int recon) {
     }
   m->run_cfl = cfl;
   m->run_recon = recon;
-  if (m->graph_exec) (void)hipGraphExecDestroy(m->graph_exec);
-  if (m->graph) (void)hipGraphDestroy(m->graph);
+  if (m->graph_exec) PTH_DROP(hipGraphExecDestroy(m->graph_exec));
+  if (m->graph) PTH_DROP(hipGraphDestroy(m->graph));
   m->graph_exec = nullptr;
   m->graph = nullptr;
   hipStream_t s = m->run_stream;
@@ -658,8 +659,8 @@ pth_status pth_burgers_set_tuning(pth_mesh *mh, const int planes[4]) {
   m->sweep_waves = planes[3];
   m->rf_tuned = true;  // a caller's choice is not re-tuned
   m->rf_auto = false;
-  if (m->graph_exec) (void)hipGraphExecDestroy(m->graph_exec);
-  if (m->graph) (void)hipGraphDestroy(m->graph);
+  if (m->graph_exec) PTH_DROP(hipGraphExecDestroy(m->graph_exec));
+  if (m->graph) PTH_DROP(hipGraphDestroy(m->graph));
   m->graph_exec = nullptr;
   m->graph = nullptr;
   return PTH_COMPLETE;
@@ -695,8 +696,8 @@ pth_status pth_burgers_set_sweep(pth_mesh *mh, int on) {
   Mesh *m = Impl(mh);
   m->run_sweep = on != 0;
   m->form_auto = false;
-  if (m->graph_exec) (void)hipGraphExecDestroy(m->graph_exec);
-  if (m->graph) (void)hipGraphDestroy(m->graph);
+  if (m->graph_exec) PTH_DROP(hipGraphExecDestroy(m->graph_exec));
+  if (m->graph) PTH_DROP(hipGraphDestroy(m->graph));
   m->graph_exec = nullptr;
   m->graph = nullptr;
   return PTH_COMPLETE;
@@ -705,8 +706,8 @@ pth_status pth_burgers_set_sweep(pth_mesh *mh, int on) {
 pth_status pth_burgers_set_sweep_split(pth_mesh *mh, int on) {
   Mesh *m = Impl(mh);
   m->sweep_split = on != 0;
-  if (m->graph_exec) (void)hipGraphExecDestroy(m->graph_exec);
-  if (m->graph) (void)hipGraphDestroy(m->graph);
+  if (m->graph_exec) PTH_DROP(hipGraphExecDestroy(m->graph_exec));
+  if (m->graph) PTH_DROP(hipGraphDestroy(m->graph));
   m->graph_exec = nullptr;
   m->graph = nullptr;
   return PTH_COMPLETE;
@@ -726,8 +727,8 @@ pth_status pth_burgers_set_overlap(pth_mesh *mh, int on) {
   Mesh *m = Impl(mh);
   m->run_overlap = on != 0;
   m->form_auto = false;
-  if (m->graph_exec) (void)hipGraphExecDestroy(m->graph_exec);
-  if (m->graph) (void)hipGraphDestroy(m->graph);
+  if (m->graph_exec) PTH_DROP(hipGraphExecDestroy(m->graph_exec));
+  if (m->graph) PTH_DROP(hipGraphDestroy(m->graph));
   m->graph_exec = nullptr;
   m->graph = nullptr;
   return PTH_COMPLETE;
@@ -768,8 +769,8 @@ pth_status pth_burgers_after_remesh(pth_mesh *mh) {
     if (!m->rf_tuned && TuneReconFlux(y, s) != PTH_COMPLETE) return PTH_FAIL;
     if (m->form_auto && !m->form_tuned && TuneForm(y, s) != PTH_COMPLETE) return PTH_FAIL;
     m->tuned_blocks = nb;
-    if (m->graph_exec) (void)hipGraphExecDestroy(m->graph_exec);
-    if (m->graph) (void)hipGraphDestroy(m->graph);
+    if (m->graph_exec) PTH_DROP(hipGraphExecDestroy(m->graph_exec));
+    if (m->graph) PTH_DROP(hipGraphDestroy(m->graph));
     m->graph_exec = nullptr;
     m->graph = nullptr;
   }
@@ -807,8 +808,8 @@ pth_status pth_burgers_set_time_limits(pth_mesh *mh, const double lim[6], int dt
   L.dt_init_force = dt_init_force != 0;
   m->run_lim = L;
   // the limits travel in the clock launches' arguments: a captured cycle is captured again
-  if (m->graph_exec) (void)hipGraphExecDestroy(m->graph_exec);
-  if (m->graph) (void)hipGraphDestroy(m->graph);
+  if (m->graph_exec) PTH_DROP(hipGraphExecDestroy(m->graph_exec));
+  if (m->graph) PTH_DROP(hipGraphDestroy(m->graph));
   m->graph_exec = nullptr;
   m->graph = nullptr;
   return PTH_COMPLETE;

@@ -1145,11 +1145,11 @@ pth_status GmgProblem<T>::Allocate(int N_) {
 
 template <typename T>
 void GmgProblem<T>::Free() {
-  if (levels) (void)hipFree(levels);
+  if (levels) PTH_DROP(hipFree(levels));
   for (double *&p : u)
-    if (p) (void)hipFree(p);
-  if (b64) (void)hipFree(b64);
-  if (partial) (void)hipFree(partial);
+    if (p) PTH_DROP(hipFree(p));
+  if (b64) PTH_DROP(hipFree(b64));
+  if (partial) PTH_DROP(hipFree(partial));
   levels = nullptr;
   u[0] = u[1] = b64 = partial = nullptr;
 }
@@ -1246,9 +1246,9 @@ pth_status GmgBatch<T>::Init(hipStream_t s) {
 
 template <typename T>
 void GmgBatch<T>::Free() {
-  if (stage_host) (void)hipHostFree(stage_host);
-  if (stage_dev) (void)hipFree(stage_dev);
-  if (norms) (void)hipHostFree(norms);
+  if (stage_host) PTH_DROP(hipHostFree(stage_host));
+  if (stage_dev) PTH_DROP(hipFree(stage_dev));
+  if (norms) PTH_DROP(hipHostFree(norms));
   stage_host = nullptr;
   stage_dev = nullptr;
   norms = nullptr;
@@ -1268,9 +1268,8 @@ pth_status GmgBatch<T>::RhsNorms(const std::vector<GmgProblem<T> *> &ps, double 
   GmgArgs<T> a;
   if (Put(es, &a) != PTH_COMPLETE) return PTH_FAIL;
   const int ne = a.ne;
-  hipLaunchKernelGGL(RhsNormKernel<T>, dim3(nwg), dim3(kWG), 0, stream, a);
-  hipLaunchKernelGGL(NormKernel<T>, dim3(ne), dim3(kNormWG), 0, stream, a, norms);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(RhsNormKernel<T>, dim3(nwg), dim3(kWG), 0, stream, a);
+  PTH_LAUNCH(NormKernel<T>, dim3(ne), dim3(kNormWG), 0, stream, a, norms);
   PTH_HIP(hipStreamSynchronize(stream));
   stage_used = 0;  // every queued copy has run
   for (int q = 0; q < ne; ++q) out[q] = std::sqrt(norms[q]);
@@ -1298,10 +1297,9 @@ pth_status GmgBatch<T>::Residual(const std::vector<GmgProblem<T> *> &ps,
   const int ne = a.ne;
   {
     ProfScope prof("gmg_outer", stream);
-    hipLaunchKernelGGL(OuterKernel<T>, dim3(nwg), dim3(kOuterWG), 0, stream, a);
+    PTH_LAUNCH(OuterKernel<T>, dim3(nwg), dim3(kOuterWG), 0, stream, a);
   }
-  hipLaunchKernelGGL(NormKernel<T>, dim3(ne), dim3(kNormWG), 0, stream, a, norms);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(NormKernel<T>, dim3(ne), dim3(kNormWG), 0, stream, a, norms);
   PTH_HIP(hipStreamSynchronize(stream));
   stage_used = 0;  // every queued copy has run
   for (size_t q = 0; q < ps.size(); ++q) {
@@ -1335,8 +1333,7 @@ pth_status GmgBatch<T>::Cycle(const std::vector<GmgProblem<T> *> &ps, double ome
     int nwg;
     if (Stage(entries(l), coarse, &a, &nwg) != PTH_COMPLETE) return PTH_FAIL;
     ProfScope prof(name, stream);
-    hipLaunchKernelGGL(kernel, dim3(nwg), dim3(kWG), 0, stream, a, arg...);
-    PTH_HIP(hipGetLastError());
+    PTH_LAUNCH(kernel, dim3(nwg), dim3(kWG), 0, stream, a, arg...);
     return PTH_COMPLETE;
   };
   auto pass = [&](int l, const char *name, auto src, auto ns, auto res) -> pth_status {
@@ -1349,10 +1346,9 @@ pth_status GmgBatch<T>::Cycle(const std::vector<GmgProblem<T> *> &ps, double ome
       using F = decltype(f);
       if (StagePass(es, F::TX, F::TY, &a, &nwg, &nz) != PTH_COMPLETE) return PTH_FAIL;
       ProfScope prof(name, stream);
-      hipLaunchKernelGGL((PassKernel<T, decltype(src)::value, decltype(ns)::value,
-                                     decltype(res)::value, F>),
-                         dim3(nwg), dim3(F::WG), 0, stream, a, nz, w);
-      PTH_HIP(hipGetLastError());
+      PTH_LAUNCH((PassKernel<T, decltype(src)::value, decltype(ns)::value,
+                             decltype(res)::value, F>),
+                 dim3(nwg), dim3(F::WG), 0, stream, a, nz, w);
       return PTH_COMPLETE;
     };
     // below kPassLarge cells the smaller tile: more workgroups and shorter planes against less
@@ -1437,9 +1433,8 @@ pth_status GmgBatch<T>::Cycle(const std::vector<GmgProblem<T> *> &ps, double ome
     int nwg;
     if (Stage(es, false, &a, &nwg) != PTH_COMPLETE) return PTH_FAIL;
     ProfScope prof("gmg_bottom", stream);
-    hipLaunchKernelGGL((BottomKernel<T, GmgBottom<T>::kN>), dim3(a.ne), dim3(kBottomWG), 0,
-                       stream, a, w, pre, post);
-    PTH_HIP(hipGetLastError());
+    PTH_LAUNCH((BottomKernel<T, GmgBottom<T>::kN>), dim3(a.ne), dim3(kBottomWG), 0,
+               stream, a, w, pre, post);
   }
   for (int l = L - 1; l >= 0; --l) {
     const char *name = l == 0 ? "gmg_prolong_jacobi_l0" : "gmg_prolong_jacobi";
@@ -1458,9 +1453,8 @@ template <typename T>
 pth_status GmgBatch<T>::SetBlobs(GmgProblem<T> &p, std::uint64_t seed) {
   BlobParams P;
   GmgBlobs(seed, P.v);
-  hipLaunchKernelGGL(BlobKernel, dim3(Blocks(static_cast<std::int64_t>(p.N) * p.N * p.N)),
-                     dim3(kWG), 0, stream, p.b64, p.N, P);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(BlobKernel, dim3(Blocks(static_cast<std::int64_t>(p.N) * p.N * p.N)),
+             dim3(kWG), 0, stream, p.b64, p.N, P);
   return PTH_COMPLETE;
 }
 
@@ -1468,8 +1462,7 @@ pth_status GmgBatch<T>::SetBlobs(GmgProblem<T> &p, std::uint64_t seed) {
 template <typename T>
 pth_status GmgBatch<T>::Reset(GmgProblem<T> &p) {
   const std::int64_t c = static_cast<std::int64_t>(p.N) * p.N * p.N;
-  hipLaunchKernelGGL(FillKernel, dim3(Blocks(c)), dim3(kWG), 0, stream, p.u[0], c);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(FillKernel, dim3(Blocks(c)), dim3(kWG), 0, stream, p.u[0], c);
   p.cur = 0;
   return PTH_COMPLETE;
 }

@@ -104,7 +104,7 @@ struct GmgSolver1 {
   ~GmgSolver1() {
     p.Free();
     batch.Free();
-    if (s) (void)hipStreamDestroy(s);
+    if (s) PTH_DROP(hipStreamDestroy(s));
   }
   pth_status Init(int N) {
     PTH_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));

@@ -79,20 +79,18 @@ struct Server {
         delete p;
       }
     for (auto &r : reqs)
-      if (r.pinned) (void)hipHostFree(r.pinned);
+      if (r.pinned) PTH_DROP(hipHostFree(r.pinned));
     batch.Free();
-    if (s) (void)hipStreamDestroy(s);
+    if (s) PTH_DROP(hipStreamDestroy(s));
   }
   // room for a request's solution of c cells
   void Room(Request &r, std::int64_t c) {
     if (r.kept) return;
     const std::int64_t need = static_cast<std::int64_t>(sizeof(double)) * c;
-    if (pinned + need <= kPinnedMax && hipHostMalloc(&r.pinned, need) == hipSuccess)
+    if (pinned + need <= kPinnedMax && !Failed(hipHostMalloc(&r.pinned, need))) {
       pinned += need;
-    else
+    } else {
       r.pinned = nullptr;
-    if (!r.pinned) {
-      (void)hipGetLastError();
       r.pageable.resize(c);
     }
     r.kept = static_cast<size_t>(c);
@@ -106,7 +104,7 @@ struct Server {
   bool Fits(std::int64_t need) const {
     if (budget > 0 && held + need > budget) return false;
     size_t free_b = 0, total_b = 0;
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return false;
+    if (Failed(hipMemGetInfo(&free_b, &total_b))) return false;
     return static_cast<std::int64_t>(free_b) >= need + reserve;
   }
   GmgProblem<T> *Take(int n) {

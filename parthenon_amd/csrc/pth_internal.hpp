@@ -29,14 +29,44 @@ namespace pth {
 void SetError(const std::string &msg);
 const char *ErrorText();
 
+// HIP errors. The runtime keeps a thread's last error until hipGetLastError reads it, through any
+// number of calls that succeed, and every library of the process shares it: a launch that is
+// checked by reading it fails for an error that a call long before it, or another library, left
+// behind. So a launch here is judged by what it returns itself (LaunchKernel), a failed call is
+// reported by its own status and text, and the runtime's record of it is cleared: nothing is left
+// for the next reader, and errors that others left stay theirs.
+inline bool Failed(hipError_t e) {
+  if (e == hipSuccess) return false;
+  (void)hipGetLastError();
+  return true;
+}
+
+// A call whose failure must not stop what goes on (in a destructor, or around a measurement): the
+// failure is written to stderr with its place.
+void Dropped(hipError_t e, const char *call, const char *file, int line);
+#define PTH_DROP(call) ::pth::Dropped((call), #call, __FILE__, __LINE__)
+
 #define PTH_HIP(call)                                                              \
   do {                                                                             \
     hipError_t err_ = (call);                                                      \
-    if (err_ != hipSuccess) {                                                      \
+    if (::pth::Failed(err_)) {                                                     \
       ::pth::SetError(std::string(#call) + ": " + hipGetErrorString(err_));        \
       return PTH_FAIL;                                                             \
     }                                                                              \
   } while (0)
+
+template <typename... P, typename... A>
+hipError_t LaunchKernel(void (*kernel)(P...), dim3 grid, dim3 block, unsigned lds, hipStream_t s,
+                        A &&...a) {
+  std::tuple<P...> v(std::forward<A>(a)...);
+  return std::apply(
+      [&](P &...p) {
+        void *args[] = {&p...};
+        return hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, args, lds, s);
+      },
+      v);
+}
+#define PTH_LAUNCH(kernel, ...) PTH_HIP(::pth::LaunchKernel(kernel, __VA_ARGS__))
 
 // ---------------------------------------------------------------- topology ---------------
 struct Lattice {  // a block position: level and integer coordinates on that level's lattice

@@ -483,7 +483,7 @@ struct TreeLevel {
     copy_D.Free();
     for (void *q : {static_cast<void *>(face_D), static_cast<void *>(coef),
                     static_cast<void *>(face), static_cast<void *>(xfer)})
-      if (q) (void)hipFree(q);
+      if (q) PTH_DROP(hipFree(q));
   }
 };
 
@@ -505,11 +505,11 @@ class MgTree {
   hipStream_t capture_stream = nullptr;
 
   ~MgTree() {
-    if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
-    if (graph) (void)hipGraphDestroy(graph);
-    if (capture_stream) (void)hipStreamDestroy(capture_stream);
-    if (partial) (void)hipFree(partial);
-    if (norm_host) (void)hipHostFree(norm_host);
+    if (graph_exec) PTH_DROP(hipGraphExecDestroy(graph_exec));
+    if (graph) PTH_DROP(hipGraphDestroy(graph));
+    if (capture_stream) PTH_DROP(hipStreamDestroy(capture_stream));
+    if (partial) PTH_DROP(hipFree(partial));
+    if (norm_host) PTH_DROP(hipHostFree(norm_host));
   }
   pth_status Build();
   pth_status Setup(MeshData &md);
@@ -818,22 +818,20 @@ pth_status MgTree::Smooth(int l, const std::vector<double> &w, bool zero) {
   const dim3 grid(static_cast<unsigned>(L.mesh->topo.blocks.size()) * L.view.chunks);
   if (zero) L.cur = 0;
   if (zero && w.empty()) {
-    hipLaunchKernelGGL(ZeroKernel, grid, dim3(kWG), 0, Stream(l), L.x[0], L.view);
-    PTH_HIP(hipGetLastError());
+    PTH_LAUNCH(ZeroKernel, grid, dim3(kWG), 0, Stream(l), L.x[0], L.view);
   }
   for (size_t q = 0; q < w.size(); ++q) {
     if (zero && q == 0) {
       ProfScope prof("mg_level_jacobi", Stream(l));
-      hipLaunchKernelGGL(StageKernel<true>, grid, dim3(kWG), 0, Stream(l), nullptr,
-                         Data(l, kB), L.x[0], L.view, L.coef, D, Df(l), alpha, w[q]);
+      PTH_LAUNCH(StageKernel<true>, grid, dim3(kWG), 0, Stream(l), nullptr,
+                 Data(l, kB), L.x[0], L.view, L.coef, D, Df(l), alpha, w[q]);
     } else {
       if (Exchange(l) != PTH_COMPLETE) return PTH_FAIL;
       ProfScope prof("mg_level_jacobi", Stream(l));
-      hipLaunchKernelGGL(StageKernel<false>, grid, dim3(kWG), 0, Stream(l), L.x[L.cur],
-                         Data(l, kB), L.x[1 - L.cur], L.view, L.coef, D, Df(l), alpha, w[q]);
+      PTH_LAUNCH(StageKernel<false>, grid, dim3(kWG), 0, Stream(l), L.x[L.cur],
+                 Data(l, kB), L.x[1 - L.cur], L.view, L.coef, D, Df(l), alpha, w[q]);
       L.cur = 1 - L.cur;
     }
-    PTH_HIP(hipGetLastError());
   }
   return PTH_COMPLETE;
 }
@@ -850,20 +848,18 @@ pth_status MgTree::Cycle(int l) {
       ProfScope prof("mg_level_residual", Stream(l));
       const unsigned grid = static_cast<unsigned>(F.nchild * F.cchunks +
                                                   (F.nxfer - F.nchild) * F.view.chunks);
-      hipLaunchKernelGGL(ResidualDownKernel, dim3(grid), dim3(kWG), 0, Stream(l), F.x[F.cur],
-                         Data(l, kB), F.view, F.coef, D, Df(l), alpha, Data(l + 1, kB), C.view,
-                         F.xfer, F.nchild, F.cchunks);
-      PTH_HIP(hipGetLastError());
+      PTH_LAUNCH(ResidualDownKernel, dim3(grid), dim3(kWG), 0, Stream(l), F.x[F.cur],
+                 Data(l, kB), F.view, F.coef, D, Df(l), alpha, Data(l + 1, kB), C.view,
+                 F.xfer, F.nchild, F.cchunks);
     }
     if (Cycle(l + 1) != PTH_COMPLETE) return PTH_FAIL;
     // the coarser correction, prolongated and added
     if (Exchange(l + 1) != PTH_COMPLETE) return PTH_FAIL;
     {
       ProfScope prof("mg_level_prolong", Stream(l));
-      hipLaunchKernelGGL(ProlongAddKernel,
-                         dim3(static_cast<unsigned>(F.nxfer) * F.view.chunks), dim3(kWG), 0,
-                         Stream(l), F.x[F.cur], F.view, C.x[C.cur], C.view, F.xfer);
-      PTH_HIP(hipGetLastError());
+      PTH_LAUNCH(ProlongAddKernel,
+                 dim3(static_cast<unsigned>(F.nxfer) * F.view.chunks), dim3(kWG), 0,
+                 Stream(l), F.x[F.cur], F.view, C.x[C.cur], C.view, F.xfer);
     }
     if (Smooth(l, w_post, false) != PTH_COMPLETE) return PTH_FAIL;
   }
@@ -880,11 +876,10 @@ pth_status MgTree::Norm() {
   TreeLevel &L = *lv[0];
   if (Exchange(0) != PTH_COMPLETE) return PTH_FAIL;
   ProfScope prof("mg_residual_norm", Stream(0));
-  hipLaunchKernelGGL(ResidualNormKernel, dim3(npartial), dim3(kWG), 0, Stream(0), L.x[0],
-                     Data(0, kB), L.view, L.mesh->coef, D, Df(0), alpha, partial);
-  hipLaunchKernelGGL(SumKernel, dim3(1), dim3(kSumWG), 0, Stream(0), partial, npartial,
-                     partial + npartial);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(ResidualNormKernel, dim3(npartial), dim3(kWG), 0, Stream(0), L.x[0],
+             Data(0, kB), L.view, L.mesh->coef, D, Df(0), alpha, partial);
+  PTH_LAUNCH(SumKernel, dim3(1), dim3(kSumWG), 0, Stream(0), partial, npartial,
+             partial + npartial);
   return PTH_COMPLETE;
 }
 
@@ -909,19 +904,20 @@ pth_status MgTree::Iterate(double *rms) {
     const bool prof = Prof().on;
     Prof().on = false;  // no event records inside the captured V-cycle
     hipError_t e = hipStreamBeginCapture(capture_stream, hipStreamCaptureModeThreadLocal);
-    const bool began = e == hipSuccess;
+    const bool began = !Failed(e);
     pth_status st = PTH_FAIL;
     hipGraph_t g = nullptr;
     if (began) {
       st = both();
       e = hipStreamEndCapture(capture_stream, &g);
+      (void)Failed(e);
     }
     Prof().on = prof;
     for (auto &L : lv) L->mesh->stream = s;
     if (e != hipSuccess && (!began || st == PTH_COMPLETE))
       SetError(std::string("MGSolver: V-cycle capture: ") + hipGetErrorString(e));
     if (st != PTH_COMPLETE || e != hipSuccess) {
-      if (g) (void)hipGraphDestroy(g);
+      if (g) PTH_DROP(hipGraphDestroy(g));
       return PTH_FAIL;
     }
     graph = g;
@@ -973,9 +969,8 @@ pth_status MgTree::Setup(MeshData &md) {
     long long per_rec = G.ndim;
     for (int d = 0; d < 3; ++d) per_rec *= G.act[d] ? G.nc[d] + 1 : 1;
     const long long total = per_rec * static_cast<long long>(F.face_host.size());
-    hipLaunchKernelGGL(FaceRestrictKernel, dim3(Grid(total)), dim3(kWG), 0, F.mesh->stream,
-                       F.face_D, G, per_rec, total);
-    PTH_HIP(hipGetLastError());
+    PTH_LAUNCH(FaceRestrictKernel, dim3(Grid(total)), dim3(kWG), 0, F.mesh->stream,
+               F.face_D, G, per_rec, total);
   }
   return PTH_COMPLETE;
 }

@@ -277,8 +277,8 @@ struct MgMesh {
   MgTree *tree = nullptr;       // block-mesh hierarchy (meshes other than the uniform cube)
   ~MgMesh() {
     if (tree) MgTreeDestroy(tree);
-    if (map) (void)hipFree(map);
-    if (ev) (void)hipEventDestroy(ev);
+    if (map) PTH_DROP(hipFree(map));
+    if (ev) PTH_DROP(hipEventDestroy(ev));
   }
   template <typename F>
   pth_status Do(F fn) {
@@ -308,7 +308,7 @@ struct MgMesh {
         SetError("MGSolver: the blocks do not tile the mesh");
         return PTH_FAIL;
       }
-    if (map) (void)hipFree(map);
+    if (map) PTH_DROP(hipFree(map));
     map = nullptr;
     PTH_HIP(hipMalloc(&map, sizeof(int) * h.size()));
     PTH_HIP(hipMemcpy(map, h.data(), sizeof(int) * h.size(), hipMemcpyHostToDevice));
@@ -340,10 +340,9 @@ static pth_status Linear(pth_meshdata *mdh, const char *a, const char *b, const 
     return PTH_FAIL;
   }
   const long long n = md->store[fo].ndata;
-  hipLaunchKernelGGL(LinearKernel, dim3(Blocks(n)), dim3(kWG), 0, m->stream,
-                     md->store[fa].data, b ? md->store[fb].data : nullptr, wa, wb,
-                     md->store[fo].data, n);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(LinearKernel, dim3(Blocks(n)), dim3(kWG), 0, m->stream,
+             md->store[fa].data, b ? md->store[fb].data : nullptr, wa, wb,
+             md->store[fo].data, n);
   return PTH_COMPLETE;
 }
 
@@ -371,10 +370,9 @@ pth_status pth_solver_set_to_zero(pth_meshdata *mdh, const char *var) {
                           s.n0 * s.n1 * s.n2;
   if (total == 0) return PTH_COMPLETE;
   const unsigned chunks = ZeroChunks(s);
-  hipLaunchKernelGGL(ZeroKernel,
-                     dim3(chunks * m->fields[f].ncomp * static_cast<unsigned>(m->topo.blocks.size())),
-                     dim3(kWG), 0, m->stream, md->store[f].data, s, chunks);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(ZeroKernel,
+             dim3(chunks * m->fields[f].ncomp * static_cast<unsigned>(m->topo.blocks.size())),
+             dim3(kWG), 0, m->stream, md->store[f].data, s, chunks);
   return PTH_COMPLETE;
 }
 
@@ -399,11 +397,10 @@ pth_status pth_solver_dot_product(pth_meshdata *mdh, const char *a, const char *
   const int nwg = static_cast<int>(std::max<long long>(
       1, std::min<long long>({static_cast<long long>(Blocks(total)), kDotMaxWG,
                               m->scratch_n - 8})));
-  hipLaunchKernelGGL(DotKernel, dim3(nwg), dim3(kWG), 0, m->stream, md->store[fa].data,
-                     md->store[fb].data, nc, s, total, m->scratch);
-  hipLaunchKernelGGL(SumPartialsKernel, dim3(1), dim3(kWG), 0, m->stream, m->scratch, nwg,
-                     m->scratch + m->scratch_n);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(DotKernel, dim3(nwg), dim3(kWG), 0, m->stream, md->store[fa].data,
+             md->store[fb].data, nc, s, total, m->scratch);
+  PTH_LAUNCH(SumPartialsKernel, dim3(1), dim3(kWG), 0, m->stream, m->scratch, nwg,
+             m->scratch + m->scratch_n);
   PTH_HIP(hipMemcpyAsync(m->pinned, m->scratch + m->scratch_n, sizeof(double),
                          hipMemcpyDeviceToHost, m->stream));
   PTH_HIP(hipStreamSynchronize(m->stream));
@@ -451,10 +448,9 @@ pth_status pth_poisson_ax(pth_meshdata *mdh, const pth_poisson_equation *eq, con
   const Shape s = ShapeOf(t.fine);
   const long long total = static_cast<long long>(t.blocks.size()) * s.n0 * s.n1 * s.n2;
   if (total == 0) return PTH_COMPLETE;
-  hipLaunchKernelGGL(PoissonAxKernel, dim3(Blocks(total)), dim3(kWG), 0, m->stream,
-                     md->store[fx].data, md->store[fo].data, s, m->coef, eq->D, Df,
-                     eq->diagonal_alpha, t.ndim, total);
-  PTH_HIP(hipGetLastError());
+  PTH_LAUNCH(PoissonAxKernel, dim3(Blocks(total)), dim3(kWG), 0, m->stream,
+             md->store[fx].data, md->store[fo].data, s, m->coef, eq->D, Df,
+             eq->diagonal_alpha, t.ndim, total);
   return PTH_COMPLETE;
 }
 
@@ -543,7 +539,7 @@ pth_mg *pth_mg_create(pth_mesh *mh, const char *u, const char *rhs, const pth_mg
     h->d.reset(new GmgSolver1<double>());
     st = h->d->Init(h->N);
   }
-  if (st == PTH_COMPLETE && hipEventCreateWithFlags(&h->ev, hipEventDisableTiming) != hipSuccess) {
+  if (st == PTH_COMPLETE && Failed(hipEventCreateWithFlags(&h->ev, hipEventDisableTiming))) {
     SetError("MGSolver: hipEventCreate failed");
     st = PTH_FAIL;
   }
@@ -572,11 +568,10 @@ pth_status pth_mg_setup(pth_mg *h, pth_meshdata *mdh) {
   const Shape s = ShapeOf(m->topo.fine);
   const long long cells = static_cast<long long>(h->N) * h->N * h->N;
   const pth_status st = h->Do([&](auto &S) -> pth_status {
-    hipLaunchKernelGGL(GatherKernel, dim3(Blocks((cells + kCells - 1) / kCells)), dim3(kWG), 0, m->stream,
-                       md->store[h->frhs].data, h->map, s, h->N, h->scale, S.p.b64);
-    hipLaunchKernelGGL(GatherKernel, dim3(Blocks((cells + kCells - 1) / kCells)), dim3(kWG), 0, m->stream,
-                       md->store[h->fu].data, h->map, s, h->N, 1.0, S.p.u[0]);
-    PTH_HIP(hipGetLastError());
+    PTH_LAUNCH(GatherKernel, dim3(Blocks((cells + kCells - 1) / kCells)), dim3(kWG), 0, m->stream,
+               md->store[h->frhs].data, h->map, s, h->N, h->scale, S.p.b64);
+    PTH_LAUNCH(GatherKernel, dim3(Blocks((cells + kCells - 1) / kCells)), dim3(kWG), 0, m->stream,
+               md->store[h->fu].data, h->map, s, h->N, 1.0, S.p.u[0]);
     S.p.cur = 0;
     PTH_HIP(hipEventRecord(h->ev, m->stream));
     PTH_HIP(hipStreamWaitEvent(S.s, h->ev, 0));
@@ -622,9 +617,8 @@ pth_status pth_mg_solve(pth_mg *h, pth_meshdata *mdh) {
     h->rms = h->history.back();
     PTH_HIP(hipEventRecord(h->ev, S.s));
     PTH_HIP(hipStreamWaitEvent(m->stream, h->ev, 0));
-    hipLaunchKernelGGL(ScatterKernel, dim3(Blocks((cells + kCells - 1) / kCells)), dim3(kWG), 0, m->stream,
-                       S.p.u[S.p.cur], h->map, s, h->N, md->store[h->fu].data);
-    PTH_HIP(hipGetLastError());
+    PTH_LAUNCH(ScatterKernel, dim3(Blocks((cells + kCells - 1) / kCells)), dim3(kWG), 0, m->stream,
+               S.p.u[S.p.cur], h->map, s, h->N, md->store[h->fu].data);
     return PTH_COMPLETE;
   });
   h->ready = false;

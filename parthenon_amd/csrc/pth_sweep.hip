@@ -1338,9 +1338,9 @@ int ResidentGroups(const void *kernel, int threads) {
   auto it = cache.find(kernel);
   if (it != cache.end()) return it->second;
   int dev = 0, cus = 0, per = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, 0) != hipSuccess ||
+  if (Failed(hipGetDevice(&dev)) ||
+      Failed(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) ||
+      Failed(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, 0)) ||
       per < 1 || cus < 1)
     return -1;
   cache[kernel] = per * cus;
@@ -1381,8 +1381,8 @@ pth_status BurgersSweep(const Topology &t, int V, const double *U, const double 
       if (!groups_of(reinterpret_cast<const void *>(kernel), 256,
                      static_cast<std::int64_t>(nb) * 16))
         return PTH_FAIL;
-      hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, U, base, out, derived, partial,
-                         coef, nb, beta, dtvar, fover, fcor, push, list);
+      PTH_LAUNCH(kernel, dim3(grid), dim3(256), 0, s, U, base, out, derived, partial,
+                 coef, nb, beta, dtvar, fover, fcor, push, list);
       return PTH_COMPLETE;
     };
     auto pick = [&](auto v) {
@@ -1396,7 +1396,6 @@ pth_status BurgersSweep(const Topology &t, int V, const double *U, const double 
                           : V == 6 ? pick(std::integral_constant<int, 6>())
                                    : pick(std::integral_constant<int, 7>());
     if (st != PTH_COMPLETE) return PTH_FAIL;
-    PTH_HIP(hipGetLastError());
     if (groups) *groups = grid;
     return PTH_COMPLETE;
   }
@@ -1413,8 +1412,8 @@ pth_status BurgersSweep(const Topology &t, int V, const double *U, const double 
     const std::int64_t planes = static_cast<std::int64_t>(nb) * S.tiles * S.n2;
     auto run = [&](auto kernel, int threads) {
       if (!groups_of(reinterpret_cast<const void *>(kernel), threads, planes)) return PTH_FAIL;
-      hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, s, U, base, out, derived, partial,
-                         coef, S, nb, beta, dtvar, fover, fcor, push, list);
+      PTH_LAUNCH(kernel, dim3(grid), dim3(threads), 0, s, U, base, out, derived, partial,
+                 coef, S, nb, beta, dtvar, fover, fcor, push, list);
       return PTH_COMPLETE;
     };
     auto pick = [&](auto v) {
@@ -1440,7 +1439,6 @@ pth_status BurgersSweep(const Topology &t, int V, const double *U, const double 
     }
 #undef PTH_TS_CASE
     if (st != PTH_COMPLETE) return PTH_FAIL;
-    PTH_HIP(hipGetLastError());
     if (groups) *groups = grid;
     return PTH_COMPLETE;
   }
@@ -1450,8 +1448,8 @@ pth_status BurgersSweep(const Topology &t, int V, const double *U, const double 
     if (!groups_of(reinterpret_cast<const void *>(&BlockSweepKernel<8, 4, NV, W>), 64,         \
                    static_cast<std::int64_t>(nb) * 8))                                        \
       return PTH_FAIL;                                                                        \
-    hipLaunchKernelGGL((BlockSweepKernel<8, 4, NV, W>), dim3(grid), dim3(64), 0, s, U, base,   \
-                       out, derived, partial, coef, nb, beta, dtvar, recon, fover, fcor, push); \
+    PTH_LAUNCH((BlockSweepKernel<8, 4, NV, W>), dim3(grid), dim3(64), 0, s, U, base,   \
+               out, derived, partial, coef, nb, beta, dtvar, recon, fover, fcor, push); \
   }
 #define PTH_SW_CASE(NV)                        \
   case NV:                                     \
@@ -1474,7 +1472,6 @@ pth_status BurgersSweep(const Topology &t, int V, const double *U, const double 
   }
 #undef PTH_SW_CASE
 #undef PTH_SW_LAUNCH_W
-  PTH_HIP(hipGetLastError());
   if (groups) *groups = grid;
   return PTH_COMPLETE;
 }
@@ -1493,11 +1490,11 @@ pth_status FlxcorDirect(const Topology &t, int V, const FluxCorrection &fc, cons
 #define PTH_FD_CASE(NV)                                                                       \
   case NV:                                                                                    \
     if (ring)                                                                                 \
-      hipLaunchKernelGGL((FlxcorDirectKernel<NV, true>), grid, dim3(64), 0, s, fc.dev, U,     \
-                         fc.store, G, recon);                                                 \
+      PTH_LAUNCH((FlxcorDirectKernel<NV, true>), grid, dim3(64), 0, s, fc.dev, U,     \
+                 fc.store, G, recon);                                                 \
     else                                                                                      \
-      hipLaunchKernelGGL((FlxcorDirectKernel<NV, false>), grid, dim3(64), 0, s, fc.dev, U,    \
-                         fc.store, G, recon);                                                 \
+      PTH_LAUNCH((FlxcorDirectKernel<NV, false>), grid, dim3(64), 0, s, fc.dev, U,    \
+                 fc.store, G, recon);                                                 \
     break;
   switch (V) {
     PTH_FD_CASE(4)
@@ -1515,7 +1512,6 @@ pth_status FlxcorDirect(const Topology &t, int V, const FluxCorrection &fc, cons
     PTH_FD_CASE(16)
   }
 #undef PTH_FD_CASE
-  PTH_HIP(hipGetLastError());
   return PTH_COMPLETE;
 }
 
