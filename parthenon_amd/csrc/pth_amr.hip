@@ -224,8 +224,7 @@ void Mesh::Adopt(Mesh &nm) {
   std::swap(coef, nm.coef);
   std::swap(flux_scratch, nm.flux_scratch);
   std::swap(flux_scratch_n, nm.flux_scratch_n);
-  std::swap(graph, nm.graph);
-  std::swap(graph_exec, nm.graph_exec);
+  DropGraph();  // it names the old storage
   std::swap(scratch, nm.scratch);
   std::swap(scratch_n, nm.scratch_n);
   std::swap(pinned, nm.pinned);

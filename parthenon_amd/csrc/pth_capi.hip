@@ -95,7 +95,18 @@ void PackEntry::Free() {
   dev = nullptr;
 }
 
+// The captured cycle goes once no replay of it is running or queued.
+void Mesh::DropGraph() {
+  if (!graph && !graph_exec) return;
+  if (run_stream) PTH_DROP(hipStreamSynchronize(run_stream));
+  if (graph_exec) PTH_DROP(hipGraphExecDestroy(graph_exec));
+  if (graph) PTH_DROP(hipGraphDestroy(graph));
+  graph_exec = nullptr;
+  graph = nullptr;
+}
+
 Mesh::~Mesh() {
+  DropGraph();
   data.clear();
   for (auto &kv : flxcor) kv.second.Free();
   for (auto &s : one_copy) {
@@ -109,8 +120,6 @@ Mesh::~Mesh() {
   if (geom) PTH_DROP(hipFree(geom));
   if (coef) PTH_DROP(hipFree(coef));
   if (flux_scratch) PTH_DROP(hipFree(flux_scratch));
-  if (graph_exec) PTH_DROP(hipGraphExecDestroy(graph_exec));
-  if (graph) PTH_DROP(hipGraphDestroy(graph));
   if (run_stream) PTH_DROP(hipStreamDestroy(run_stream));
   for (hipEvent_t e : order_ev)
     if (e) PTH_DROP(hipEventDestroy(e));

@@ -600,10 +600,7 @@ pth_status pth_burgers_init(pth_mesh *mh, double cfl, int recon) {
     }
   m->run_cfl = cfl;
   m->run_recon = recon;
-  if (m->graph_exec) PTH_DROP(hipGraphExecDestroy(m->graph_exec));
-  if (m->graph) PTH_DROP(hipGraphDestroy(m->graph));
-  m->graph_exec = nullptr;
-  m->graph = nullptr;
+  m->DropGraph();
   hipStream_t s = m->run_stream;
   // order after any work the caller queued on the mesh stream
   PTH_HIP(hipStreamSynchronize(m->stream));
@@ -659,10 +656,7 @@ pth_status pth_burgers_set_tuning(pth_mesh *mh, const int planes[4]) {
   m->sweep_waves = planes[3];
   m->rf_tuned = true;  // a caller's choice is not re-tuned
   m->rf_auto = false;
-  if (m->graph_exec) PTH_DROP(hipGraphExecDestroy(m->graph_exec));
-  if (m->graph) PTH_DROP(hipGraphDestroy(m->graph));
-  m->graph_exec = nullptr;
-  m->graph = nullptr;
+  m->DropGraph();
   return PTH_COMPLETE;
 }
 
@@ -696,20 +690,14 @@ pth_status pth_burgers_set_sweep(pth_mesh *mh, int on) {
   Mesh *m = Impl(mh);
   m->run_sweep = on != 0;
   m->form_auto = false;
-  if (m->graph_exec) PTH_DROP(hipGraphExecDestroy(m->graph_exec));
-  if (m->graph) PTH_DROP(hipGraphDestroy(m->graph));
-  m->graph_exec = nullptr;
-  m->graph = nullptr;
+  m->DropGraph();
   return PTH_COMPLETE;
 }
 
 pth_status pth_burgers_set_sweep_split(pth_mesh *mh, int on) {
   Mesh *m = Impl(mh);
   m->sweep_split = on != 0;
-  if (m->graph_exec) PTH_DROP(hipGraphExecDestroy(m->graph_exec));
-  if (m->graph) PTH_DROP(hipGraphDestroy(m->graph));
-  m->graph_exec = nullptr;
-  m->graph = nullptr;
+  m->DropGraph();
   return PTH_COMPLETE;
 }
 
@@ -727,10 +715,7 @@ pth_status pth_burgers_set_overlap(pth_mesh *mh, int on) {
   Mesh *m = Impl(mh);
   m->run_overlap = on != 0;
   m->form_auto = false;
-  if (m->graph_exec) PTH_DROP(hipGraphExecDestroy(m->graph_exec));
-  if (m->graph) PTH_DROP(hipGraphDestroy(m->graph));
-  m->graph_exec = nullptr;
-  m->graph = nullptr;
+  m->DropGraph();
   return PTH_COMPLETE;
 }
 
@@ -769,10 +754,7 @@ pth_status pth_burgers_after_remesh(pth_mesh *mh) {
     if (!m->rf_tuned && TuneReconFlux(y, s) != PTH_COMPLETE) return PTH_FAIL;
     if (m->form_auto && !m->form_tuned && TuneForm(y, s) != PTH_COMPLETE) return PTH_FAIL;
     m->tuned_blocks = nb;
-    if (m->graph_exec) PTH_DROP(hipGraphExecDestroy(m->graph_exec));
-    if (m->graph) PTH_DROP(hipGraphDestroy(m->graph));
-    m->graph_exec = nullptr;
-    m->graph = nullptr;
+    m->DropGraph();
   }
   PTH_HIP(hipStreamSynchronize(s));
   return PTH_COMPLETE;
@@ -808,10 +790,7 @@ pth_status pth_burgers_set_time_limits(pth_mesh *mh, const double lim[6], int dt
   L.dt_init_force = dt_init_force != 0;
   m->run_lim = L;
   // the limits travel in the clock launches' arguments: a captured cycle is captured again
-  if (m->graph_exec) PTH_DROP(hipGraphExecDestroy(m->graph_exec));
-  if (m->graph) PTH_DROP(hipGraphDestroy(m->graph));
-  m->graph_exec = nullptr;
-  m->graph = nullptr;
+  m->DropGraph();
   return PTH_COMPLETE;
 }
 

@@ -73,6 +73,7 @@ struct Server {
   int iterations = 0, max_batch = 0;
   double busy_s = 0.0;
   ~Server() {
+    if (s) PTH_DROP(hipStreamSynchronize(s));  // a run that failed may have left work behind
     for (auto &kv : pool)
       for (auto *p : kv.second) {
         p->Free();

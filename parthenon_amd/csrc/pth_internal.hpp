@@ -443,6 +443,7 @@ class Mesh {
   BufState flxcor_state = BufState::kStale;
 
   ~Mesh();
+  void DropGraph();
   int FieldIndex(const std::string &n) const;
   pth_status Plan();
   pth_status Finalize();

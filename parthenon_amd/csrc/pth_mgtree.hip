@@ -505,10 +505,10 @@ class MgTree {
   hipStream_t capture_stream = nullptr;
 
   ~MgTree() {
+    if (partial) PTH_DROP(hipFree(partial));  // waits for the device: nothing runs past here
     if (graph_exec) PTH_DROP(hipGraphExecDestroy(graph_exec));
     if (graph) PTH_DROP(hipGraphDestroy(graph));
     if (capture_stream) PTH_DROP(hipStreamDestroy(capture_stream));
-    if (partial) PTH_DROP(hipFree(partial));
     if (norm_host) PTH_DROP(hipHostFree(norm_host));
   }
   pth_status Build();
