@@ -251,9 +251,11 @@ pth_status pth_burgers_run_cycles(pth_mesh *m, int ncycles, int use_graph);
 pth_status pth_burgers_set_overlap(pth_mesh *m, int on);
 pth_status pth_burgers_set_sweep(pth_mesh *m, int on);
 pth_status pth_burgers_form(pth_mesh *m, int *sweep, int *overlap);
-/* With on != 0 the automatic choice of pth_burgers_init considers only the bit-exact plane
- * forms (when the mesh supports them), so a run's bits cannot depend on timing noise; must
- * precede pth_burgers_init. No counterpart in the reference. */
+/* With on != 0 the automatic choice of pth_burgers_init considers only the bit-exact forms (the
+ * plane forms where the mesh supports them, else fluxes, update and exchange one after another;
+ * a U declared without fluxes takes the latter with an array of the driver's own), so a run's
+ * bits cannot depend on timing noise; must precede pth_burgers_init. No counterpart in the
+ * reference. */
 pth_status pth_burgers_set_bit_exact(pth_mesh *m, int on);
 /* Sweep form on statically refined meshes of 16^3 blocks with 4 ghosts (on by default; no
  * counterpart in the reference): each stage sweeps the blocks without a neighbour at another

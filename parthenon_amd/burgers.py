@@ -100,7 +100,7 @@ class DeviceBurgersDriver:
         # others to rounding); otherwise the plane reconstruction (bit-exact), with overlap =
         # the stage input's exchange beside the ghost-free reconstruction on a second stream.
         # Left as None, initialize() times the forms and keeps the fastest; bit_exact limits
-        # that choice to the bit-exact plane forms.
+        # that choice to the bit-exact forms.
         if bit_exact:
             _check(lib().pth_burgers_set_bit_exact(mesh._h, 1), "set_bit_exact")
         if overlap is not None:

@@ -157,8 +157,10 @@ pth_status Setup(Mesh *m, Ctx &x) {
   const std::int64_t nd = x.base->store[x.fu].ndata;
   const bool planes = x.base->store[x.fu].flux && ReconFluxSupported(m->topo, x.V);
   const bool sweep = m->run_sweep && BurgersSweepSupported(m->topo, x.V);
-  // the other path's fluxes: the field's own, or scratch when U was declared without them
-  if (!planes && !sweep && !x.base->store[x.fu].flux && m->flux_scratch_n != 3 * nd) {
+  // the other path's fluxes: the field's own, or scratch when U was declared without them (also
+  // for a choice of form that leaves the sweep out)
+  const bool may_flux = !sweep || (m->form_auto && m->form_exact);
+  if (!planes && may_flux && !x.base->store[x.fu].flux && m->flux_scratch_n != 3 * nd) {
     if (m->flux_scratch) PTH_DROP(hipFree(m->flux_scratch));
     m->flux_scratch = nullptr;
     m->flux_scratch_n = 0;
@@ -421,8 +423,8 @@ pth_status Cycle(Ctx &x, hipStream_t s);
 // the mesh's own state, which is saved first and restored afterwards (U of "base", the
 // derived field and the device clock). The two plane forms give the same bits; the sweep is
 // built with FMA contraction and agrees with them to rounding (about 1e-15 relative), so
-// with form_exact set only the plane forms are candidates and the result cannot depend on
-// which form the timing picked.
+// with form_exact set the sweep is no candidate and the result cannot depend on which form the
+// timing picked; a U without fluxes then takes the flux form over the driver's own flux array.
 pth_status TuneForm(Ctx &x, hipStream_t s) {
   Mesh &m = *x.m;
   struct Form {
@@ -431,12 +433,12 @@ pth_status TuneForm(Ctx &x, hipStream_t s) {
   std::vector<Form> forms;
   const bool flux = x.base->store[x.fu].flux != nullptr;
   const bool planes = flux && ReconFluxSupported(m.topo, x.V);
-  if (BurgersSweepSupported(m.topo, x.V) && !(m.form_exact && flux)) forms.push_back({1, 0});
+  if (BurgersSweepSupported(m.topo, x.V) && !m.form_exact) forms.push_back({1, 0});
   if (planes) forms.push_back({0, 1});
   // other block shapes: the tile sweep takes less than half the flux form's time at every size
   // (32^3 blocks with 7 components: 135 to 332 us on 8 of them, 653 to 1538 on 64), so there
   // is nothing to time
-  if (flux && (planes || forms.empty())) forms.push_back({0, 0});
+  if ((flux || m.form_exact) && (planes || forms.empty())) forms.push_back({0, 0});
   if (forms.size() < 2) {
     if (!forms.empty()) {
       m.run_sweep = forms[0].sweep;
