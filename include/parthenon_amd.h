@@ -131,9 +131,16 @@ pth_status pth_mesh_exchange_counts(const pth_mesh *m, int bt, int64_t *nbuffers
 pth_meshdata *pth_meshdata_get(pth_mesh *m, const char *name);
 
 /* Device pointers of a field: data [nblocks][ncomp][Ek][Ej][Ei]; coarse (multilevel) in the
- * c_cellbounds shape; flux [3][nblocks][ncomp][Ek][Ej][Ei] (x-face i at index i). */
+ * c_cellbounds shape; flux [3][nblocks][ncomp][Ek][Ej][Ei] (x-face i at index i). They name the
+ * field's present memory, which lasts until the mesh changes (pth_mesh_adapt) or is destroyed. */
 pth_status pth_field_pointers(pth_meshdata *md, const char *field, double **data,
                               double **coarse, double **flux);
+/* Keeps the memory that pth_field_pointers names now until pth_field_release, also past a remesh
+ * (which moves the field to new memory: the held one stays as it was) and past the mesh. No
+ * counterpart in the reference. */
+typedef struct pth_hold pth_hold;
+pth_hold *pth_field_hold(pth_meshdata *md, const char *field);
+void pth_field_release(pth_hold *h);
 /* Synchronous host<->device copies of a whole field (n = number of doubles). which: 0 data,
  * 1 coarse, 2 flux. */
 pth_status pth_field_upload(pth_meshdata *md, const char *field, int which, const double *host,

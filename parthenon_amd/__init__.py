@@ -17,6 +17,7 @@ the compute API fails loudly.
 import ctypes as C
 import enum
 import os
+import weakref
 
 import numpy as np
 
@@ -117,6 +118,8 @@ _SIGNATURES = {
     "pth_mesh_exchange_counts": (_I, [_P, _I, C.POINTER(_I64), C.POINTER(_I64)]),
     "pth_meshdata_get": (_P, [_P, C.c_char_p]),
     "pth_field_pointers": (_I, [_P, C.c_char_p, C.POINTER(_DP), C.POINTER(_DP), C.POINTER(_DP)]),
+    "pth_field_hold": (_P, [_P, C.c_char_p]),
+    "pth_field_release": (None, [_P]),
     "pth_pack_get": (_P, [_P, C.POINTER(C.c_char_p), _I, C.c_uint]),
     "pth_pack_view_get": (_I, [_P, C.POINTER(PackView)]),
     "pth_pack_bounds": (_I, [_P, _I, C.POINTER(_I), C.POINTER(_I)]),
@@ -379,7 +382,11 @@ class Mesh:
 
     def adapt(self):
         """Mesh::LoadBalancingAndAdaptiveMeshRefinement: True when the mesh changed. Block
-        ids and counts change; MeshData objects stay valid."""
+        ids and counts change; MeshData objects stay valid. Addresses taken before keep naming
+        the memory as it was; MeshData.pointers gives the new ones."""
+        for md in self._data.values():
+            for held in md._held:
+                held.keep()
         mod = _I()
         _check(lib().pth_mesh_adapt(self._h, C.byref(mod)), "adapt")
         if mod.value:
@@ -402,9 +409,29 @@ def LoadBalancingAndAdaptiveMeshRefinement(mesh):
     return mesh.adapt()
 
 
+class _Held:
+    """What the addresses of one pointers() call refer to: the container, and, once a remesh is
+    about to move the field to new memory, the memory that they name."""
+
+    def __init__(self, md, field):
+        self.md, self.field, self.hold = md, field, None
+
+    def keep(self):
+        if self.hold is None:
+            self.hold = lib().pth_field_hold(self.md._h, self.field.encode())
+            if not self.hold:
+                raise RuntimeError("pth_field_hold failed: " + lib().pth_last_error().decode())
+
+    def __del__(self):
+        if self.hold and _LIB is not None:
+            _LIB.pth_field_release(self.hold)
+
+
 class _Address(int):
-    """A device address; it keeps the container whose memory it names alive, so a view made from
-    it (an array interface's data pointer) never outlives the field."""
+    """A device address. It keeps the memory that it names: the container and its mesh are not
+    collected before it, and a remesh, which moves the field to new memory, leaves it the old one
+    as it was. A view made from it (an array interface's data pointer) may hold it; a number
+    computed from it is a bare one, which keeps nothing."""
 
     def __new__(cls, value, owner):
         a = super().__new__(cls, value)
@@ -417,6 +444,7 @@ class MeshData:
         self.mesh = mesh
         self.name = name
         self._h = handle
+        self._held = weakref.WeakSet()  # of addresses that somebody has
 
     def _shape(self, field, which):
         if which == 1:
@@ -456,7 +484,9 @@ class MeshData:
         d, c, f = _DP(), _DP(), _DP()
         _check(lib().pth_field_pointers(self._h, field.encode(), C.byref(d), C.byref(c),
                                         C.byref(f)), "pointers")
-        addr = lambda p: _Address(C.cast(p, C.c_void_p).value, self) if p else None
+        held = _Held(self, field)
+        self._held.add(held)
+        addr = lambda p: _Address(C.cast(p, C.c_void_p).value, held) if p else None
         return addr(d), addr(c), addr(f)
 
 

@@ -64,13 +64,12 @@ ProfScope::~ProfScope() {
   Prof().records.push_back(ProfRecord{name_, a_, b});
 }
 
+FieldMemory::~FieldMemory() {
+  for (double *p : {data, coarse, flux})
+    if (p) PTH_DROP(hipFree(p));
+}
+
 MeshData::~MeshData() {
-  for (auto &s : store) {
-    if (!s.owned) continue;
-    if (s.data) PTH_DROP(hipFree(s.data));
-    if (s.coarse) PTH_DROP(hipFree(s.coarse));
-    if (s.flux) PTH_DROP(hipFree(s.flux));
-  }
   for (auto &c : cache) {
     c.pack.Free();
     c.unpack.Free();
@@ -109,11 +108,6 @@ Mesh::~Mesh() {
   DropGraph();
   data.clear();
   for (auto &kv : flxcor) kv.second.Free();
-  for (auto &s : one_copy) {
-    if (s.data) PTH_DROP(hipFree(s.data));
-    if (s.coarse) PTH_DROP(hipFree(s.coarse));
-    if (s.flux) PTH_DROP(hipFree(s.flux));
-  }
   if (arena_base) PTH_DROP(hipFree(arena_base));
   if (same_level) PTH_DROP(hipFree(same_level));
   if (split_list) PTH_DROP(hipFree(split_list));
@@ -157,9 +151,14 @@ pth_status AllocStore(const Mesh &m, const FieldSpec &f, FieldStore &s) {
   s.ndata = nb * f.ncomp * m.topo.fine.cells();
   s.ncoarse = m.topo.multilevel ? nb * f.ncomp * m.topo.coarse.cells() : 0;
   s.nflux = (f.flags & PTH_WITH_FLUXES) ? 3 * s.ndata : 0;
-  if (Alloc(&s.data, s.ndata) != PTH_COMPLETE) return PTH_FAIL;
-  if (Alloc(&s.coarse, s.ncoarse) != PTH_COMPLETE) return PTH_FAIL;
-  if (Alloc(&s.flux, s.nflux) != PTH_COMPLETE) return PTH_FAIL;
+  s.memory = std::make_shared<FieldMemory>();
+  FieldMemory &mem = *s.memory;
+  if (Alloc(&mem.data, s.ndata) != PTH_COMPLETE ||
+      Alloc(&mem.coarse, s.ncoarse) != PTH_COMPLETE || Alloc(&mem.flux, s.nflux) != PTH_COMPLETE)
+    return PTH_FAIL;
+  s.data = mem.data;
+  s.coarse = mem.coarse;
+  s.flux = mem.flux;
   return PTH_COMPLETE;
 }
 
@@ -305,7 +304,6 @@ MeshData *Mesh::Get(const std::string &name) {
   for (size_t f = 0; f < fields.size(); ++f) {
     if (fields[f].flags & PTH_ONE_COPY) {
       md->store[f] = one_copy[f];
-      md->store[f].owned = false;
     } else if (AllocStore(*this, fields[f], md->store[f]) != PTH_COMPLETE) {
       return nullptr;
     }
@@ -1181,6 +1179,18 @@ pth_status pth_field_pointers(pth_meshdata *mdh, const char *field, double **dat
   if (flux) *flux = md->store[f].flux;
   return PTH_COMPLETE;
 }
+
+pth_hold *pth_field_hold(pth_meshdata *mdh, const char *field) {
+  MeshData *md = Impl(mdh);
+  const int f = md->mesh->FieldIndex(field ? field : "");
+  if (f < 0) {
+    SetError(std::string("no field ") + (field ? field : "(null)"));
+    return nullptr;
+  }
+  return reinterpret_cast<pth_hold *>(new std::shared_ptr<FieldMemory>(md->store[f].memory));
+}
+
+void pth_field_release(pth_hold *h) { delete reinterpret_cast<std::shared_ptr<FieldMemory> *>(h); }
 
 // ---- packs ------------------------------------------------------------------------------
 pth_pack *pth_pack_get(pth_meshdata *mdh, const char *const *fields, int nfields,

@@ -274,10 +274,17 @@ struct FieldSpec {
   int prolong = PTH_PROLONG_MINMOD;  // registered shared-prolongation operator
 };
 
+// The device memory of a field in a container: freed with its last owner, which are the containers
+// (a OneCopy field's share one) and the holds of pth_field_hold.
+struct FieldMemory {
+  double *data = nullptr, *coarse = nullptr, *flux = nullptr;
+  ~FieldMemory();
+};
+
 struct FieldStore {
+  std::shared_ptr<FieldMemory> memory;
   double *data = nullptr, *coarse = nullptr, *flux = nullptr;
   std::int64_t ndata = 0, ncoarse = 0, nflux = 0;
-  bool owned = true;
 };
 
 class Mesh;
