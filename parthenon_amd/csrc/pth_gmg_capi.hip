@@ -166,6 +166,10 @@ struct Server {
         waiting.erase(waiting.begin());
         if (batch.SetBlobs(*p, r.seed) != PTH_COMPLETE) return PTH_FAIL;
         if (batch.Reset(*p) != PTH_COMPLETE) return PTH_FAIL;
+        // a request of an earlier run is solved again, with a count of its own
+        r.iters = 0;
+        r.rel = 0.0;
+        r.finished = false;
         r.admit = now();
         fresh.push_back({r.id, p, 0.0, false});
       }
