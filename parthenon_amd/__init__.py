@@ -14,10 +14,10 @@ Every task returns a TaskStatus like the reference; a failure raises RuntimeErro
 the library's message. There is no CPU fallback: if the HIP library is missing, importing
 the compute API fails loudly.
 """
+import collections
 import ctypes as C
 import enum
 import os
-import weakref
 
 import numpy as np
 
@@ -237,6 +237,50 @@ def _dptr(a):
     return a.ctypes.data_as(_DP)
 
 
+class _Kept:
+    """Field memory that outlives its mesh for a while. A mesh and its containers refer to each
+    other, so the collector destroys them at a time of its own, which may fall between the moment
+    a program drops them and its last look at a view of a field (a tensor over MeshData.pointers).
+    The memory of fields whose addresses were given out is therefore held when a mesh is destroyed
+    or changes, and released when the next mesh is finalized or changes: a view of a mesh that is
+    gone may be read until then. Past LIMIT bytes the oldest goes first. An address cannot keep the
+    mesh itself: torch.as_tensor never drops the tuple of the array interface that it read the
+    address from, so no mesh with such a view would ever be freed."""
+
+    LIMIT = 8 << 30
+    holds = collections.deque()
+
+    def __init__(self, md, field):
+        self.hold = None
+        ncomp, flags = md.mesh.fields[field]
+        cells = md.mesh.ent[0] * md.mesh.ent[1] * md.mesh.ent[2]
+        copies = 1 + md.mesh.multilevel + 3 * bool(flags & Metadata.WithFluxes)
+        self.bytes = 8 * md.mesh.nblocks * ncomp * cells * copies
+        self.hold = _LIB.pth_field_hold(md._h, field.encode())
+
+    def __del__(self):
+        if self.hold and _LIB is not None:
+            _LIB.pth_field_release(self.hold)
+
+    @classmethod
+    def of(cls, mesh):
+        return [cls(md, f) for md in mesh._data.values() for f in md._given]
+
+    @classmethod
+    def add(cls, kept):
+        cls.holds.extend(kept)
+        while sum(k.bytes for k in list(cls.holds)) > cls.LIMIT:
+            try:
+                cls.holds.popleft()
+            except IndexError:  # another thread was faster
+                break
+
+    @classmethod
+    def replace(cls, kept):
+        cls.holds.clear()
+        cls.add(kept)
+
+
 class Mesh:
     """A uniform or statically refined Cartesian mesh of equal-size meshblocks."""
 
@@ -246,6 +290,9 @@ class Mesh:
         a BoundaryCondition or its name; faces of non-periodic dimensions default to
         outflow, faces of periodic dimensions must stay periodic."""
         L = lib()
+        self.fields = {}
+        self._data = {}
+        self.finalized = False
         arr3 = lambda v, t: (t * 3)(*v)
         self._h = L.pth_mesh_create(arr3(nx, _I), arr3(block, _I), nghost, arr3(xmin, _D),
                                     arr3(xmax, _D), arr3([int(bool(p)) for p in periodic], _I))
@@ -260,12 +307,10 @@ class Mesh:
         for center, radius, level in refine_spheres:
             _check(L.pth_mesh_refine_sphere(self._h, arr3(center, _D), radius, level),
                    "refine_sphere")
-        self.fields = {}
-        self._data = {}
-        self.finalized = False
 
     def __del__(self):
         if getattr(self, "_h", None) and _LIB is not None:
+            _Kept.add(_Kept.of(self))
             self._data.clear()
             _LIB.pth_mesh_destroy(self._h)
             self._h = None
@@ -288,6 +333,7 @@ class Mesh:
         self._shapes()
 
     def finalize(self):
+        _Kept.replace(())
         _check(lib().pth_mesh_finalize(self._h), "finalize")
         self._shapes()
         self.finalized = True
@@ -382,14 +428,13 @@ class Mesh:
 
     def adapt(self):
         """Mesh::LoadBalancingAndAdaptiveMeshRefinement: True when the mesh changed. Block
-        ids and counts change; MeshData objects stay valid. Addresses taken before keep naming
-        the memory as it was; MeshData.pointers gives the new ones."""
-        for md in self._data.values():
-            for held in md._held:
-                held.keep()
+        ids and counts change; MeshData objects stay valid. Addresses taken before name the old
+        memory, which the next change or mesh ends; MeshData.pointers gives the new ones."""
         mod = _I()
+        kept = _Kept.of(self)
         _check(lib().pth_mesh_adapt(self._h, C.byref(mod)), "adapt")
         if mod.value:
+            _Kept.replace(kept)
             self._shapes()
         return bool(mod.value)
 
@@ -409,42 +454,12 @@ def LoadBalancingAndAdaptiveMeshRefinement(mesh):
     return mesh.adapt()
 
 
-class _Held:
-    """What the addresses of one pointers() call refer to: the container, and, once a remesh is
-    about to move the field to new memory, the memory that they name."""
-
-    def __init__(self, md, field):
-        self.md, self.field, self.hold = md, field, None
-
-    def keep(self):
-        if self.hold is None:
-            self.hold = lib().pth_field_hold(self.md._h, self.field.encode())
-            if not self.hold:
-                raise RuntimeError("pth_field_hold failed: " + lib().pth_last_error().decode())
-
-    def __del__(self):
-        if self.hold and _LIB is not None:
-            _LIB.pth_field_release(self.hold)
-
-
-class _Address(int):
-    """A device address. It keeps the memory that it names: the container and its mesh are not
-    collected before it, and a remesh, which moves the field to new memory, leaves it the old one
-    as it was. A view made from it (an array interface's data pointer) may hold it; a number
-    computed from it is a bare one, which keeps nothing."""
-
-    def __new__(cls, value, owner):
-        a = super().__new__(cls, value)
-        a.owner = owner
-        return a
-
-
 class MeshData:
     def __init__(self, mesh, name, handle):
         self.mesh = mesh
         self.name = name
         self._h = handle
-        self._held = weakref.WeakSet()  # of addresses that somebody has
+        self._given = set()  # fields whose addresses were given out
 
     def _shape(self, field, which):
         if which == 1:
@@ -481,12 +496,14 @@ class MeshData:
         return lo.value, hi.value
 
     def pointers(self, field):
+        """Device addresses of the field's data, coarse buffer and fluxes (None where there is
+        none). They are bare numbers, valid as long as the mesh exists and does not change; see
+        _Kept for what a view made from them may still read afterwards."""
         d, c, f = _DP(), _DP(), _DP()
         _check(lib().pth_field_pointers(self._h, field.encode(), C.byref(d), C.byref(c),
                                         C.byref(f)), "pointers")
-        held = _Held(self, field)
-        self._held.add(held)
-        addr = lambda p: _Address(C.cast(p, C.c_void_p).value, held) if p else None
+        self._given.add(field)
+        addr = lambda p: C.cast(p, C.c_void_p).value
         return addr(d), addr(c), addr(f)
 
 
