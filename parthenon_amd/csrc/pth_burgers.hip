@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <cfloat>
+#include <cmath>
 #include <type_traits>
 
 #include "pth_burgers.hpp"
@@ -43,85 +44,128 @@ __device__ __forceinline__ double HllOne(int n, double upl, double upr, double l
   return (sr * upl * l - sl * upr * r + sl * sr * (r - l)) / den;
 }
 
-// How FluxTaskKernel splits one block: workgroups per direction and, for y and z, faces per
-// segment of a column.
+// How FluxTaskKernel splits the work: units of `pack` consecutive blocks, `chunks` groups of
+// `comps` components (one of all, by segments); per unit and group workgroups of each direction, in `stripes`; y and z by rows
+// or by segments of `seg` faces.
 constexpr int kSegFaces = 9;
 struct FluxSplit {
   int wgs[3], seg[3];
+  int pack, chunks, comps, stripes, rows;
 };
 
 // CalculateFluxes of any block shape in one launch, from U to the fluxes [3][block][comp][k][j][i]
 // (x-face i - 1/2 at index i): the face states stay on chip. One workgroup takes a piece of one
-// block in one direction and goes through the components one after another, the normal
-// velocity first (its face states give every component's signal speeds), so any number of
-// components fits.
-//   x: a wavefront takes 64 consecutive cells of the rows extended by one cell on each side; a
-//      lane reconstructs its cell and gets the left state of its low face from the lane below
-//      (the first lane of a wavefront repeats the last one's cell of the wavefront before);
-//   y, z: a thread marches a column segment of at most kSegFaces faces with the stencil in a
-//      register window, lanes along x; the normal velocity's states wait in LDS, each thread
+// block (of several, where one would leave most of its lanes idle) in one direction and goes
+// through its components one after another, the normal velocity first (its face states give every
+// component's signal speeds), so any number of components fits.
+//   rows (x; y and z where the mesh is small): a wavefront takes 64 consecutive cells of the rows
+//      along the direction, extended by one cell on each side; a lane reconstructs its cell and
+//      gets the left state of its low face from the lane below (the first lane of a wavefront
+//      repeats the last one's cell of the wavefront before; the first cell of a row, and so of a
+//      block, has no low face);
+//   segments (y, z): a thread marches a column segment of at most kSegFaces faces with the stencil
+//      in a register window, lanes along x; the normal velocity's states wait in LDS, each thread
 //      in its own slots (no barriers).
-// A cell is reconstructed once, but for one cell per segment or wavefront. The operations are
+// A cell is reconstructed once, but for two cells a row or one a segment or wavefront. The
+// operations are
 // those of the reference in its order, without contraction. Bound: FP64 issue (about 300
 // instructions a reconstruction with its flux, 8 IEEE divides among them). On the 960-block
 // mesh with 7 components the reconstruction and HLL as two launches, with the states in HBM
 // between them, took 1341 + 1043 us; this kernel takes
-// 1070 us. WIDE: 64-bit cell offsets, for components of 4 GB and more.
-template <int RECON, bool WIDE>
+// 1070 us. One block of 128^3: 1417 us with the directions one after another, which leaves XCDs
+// with long workgroups alone, 509 in stripes. WIDE: 64-bit cell offsets, for components of 4 GB and more.
+// ROWS: y and z by rows too.
+template <int RECON, bool WIDE, bool ROWS>
 __global__ void __launch_bounds__(kWG)
     FluxTaskKernel(const double *__restrict__ U, double *__restrict__ flux, Geo G, int nblocks,
                    FluxSplit S) {
   using I = std::conditional_t<WIDE, std::int64_t, int>;       // cells
   using O = std::conditional_t<WIDE, std::int64_t, unsigned>;  // byte offsets
-  __shared__ double up[2][kSegFaces][kWG];
-  // one block's workgroups are adjacent and run on one XCD: the three directions read the
+  // one unit's workgroups are adjacent and run on one XCD: the three directions read the
   // same cells
   const unsigned L = XcdRemap(blockIdx.x, gridDim.x);
   const unsigned per = S.wgs[0] + S.wgs[1] + S.wgs[2];
-  const int b = static_cast<int>(L / per);
+  const int chunk = ROWS ? static_cast<int>(L / per) % S.chunks : 0;
+  const int b0 = static_cast<int>(L / per) / (ROWS ? S.chunks : 1) * S.pack;
+  const int nb = nblocks - b0 < S.pack ? nblocks - b0 : S.pack;  // blocks of this unit
+  const int na = ROWS ? chunk * S.comps : 0;
+  const int nz = ROWS && na + S.comps < G.V ? na + S.comps : G.V;
+  // the unit's stripes, each with its share of the x, the y and the z workgroups
+  auto from = [&](int d, std::uint64_t s) { return static_cast<int>(s * S.wgs[d] / S.stripes); };
+  auto start = [&](std::uint64_t s) { return from(0, s) + from(1, s) + from(2, s); };
   int r = static_cast<int>(L % per), d = 0;
-  while (r >= S.wgs[d]) r -= S.wgs[d++];
+  std::uint64_t s = static_cast<std::uint64_t>(r) * S.stripes / per;
+  while (start(s) > r) --s;
+  while (start(s + 1) <= r) ++s;
+  r -= start(s);
+  while (r >= from(d, s + 1) - from(d, s)) r -= from(d, s + 1) - from(d, s), ++d;
+  r += from(d, s);
+  // the normal velocity is one of this chunk's components
+  const bool own = !ROWS || (d >= na && d < nz);
   const int n0 = G.hi0 - G.lo0 + 1, n1 = G.hi1 - G.lo1 + 1, n2 = G.hi2 - G.lo2 + 1;
-  const double *Ub = U + static_cast<std::int64_t>(b) * G.V * G.cells;
-  double *Fb = flux + (static_cast<std::int64_t>(d) * nblocks + b) * G.V * G.cells;
+  const double *Ub = U + static_cast<std::int64_t>(b0) * G.V * G.cells;
+  double *Fb = flux + (static_cast<std::int64_t>(d) * nblocks + b0) * G.V * G.cells;
   const int tid = static_cast<int>(threadIdx.x);
-  if (d == 0) {
-    const int m = n0 + 2;
-    const I cells = static_cast<I>(m) * n1 * n2;
+  const int nd = d == 0 ? n0 : d == 1 ? n1 : n2;
+  const O st = O(8) * static_cast<O>(d == 0 ? 1 : d == 1 ? G.e0 : G.e0 * G.e1);
+  if (ROWS || d == 0) {
+    const int m = nd + 2, across = d == 0 ? n1 : n0;
+    const I cells = static_cast<I>(m) * across * (d == 2 ? n1 : n2), all = cells * nb;
     const I e0 = static_cast<I>(63) * (r * (kWG / 64) + (tid >> 6)) + (tid & 63);
-    const I e = e0 < cells ? e0 : cells - 1;
-    const int a = static_cast<int>(e % m), row = static_cast<int>(e / m);
-    const O c = O(8) * static_cast<O>((static_cast<I>(G.lo2 + row / n1) * G.e1 + G.lo1 +
-                                       row % n1) * G.e0 + G.lo0 - 1 + a);
-    const bool face = a > 0 && e0 < cells && (tid & 63) > 0;
-    double upl = 0.0, upr = 0.0;
-    for (int q = 0; q <= G.V; ++q) {
-      const int n = q == 0 ? 0 : q - 1;
-      if (q == 1) continue;  // the normal velocity came first
-      double ql, qr;
-      CellStates(Ub + n * G.cells, c, O(8), RECON, ql, qr);
-      const double l = __shfl_up(ql, 1, 64);
-      if (q == 0) {
-        upl = l;
-        upr = qr;
-      }
-      if (face) StoreAt(Fb + n * G.cells, c, HllOne(n, upl, upr, l, qr));
+    I e = e0 < all ? e0 : all - 1, at = 0;
+    if (S.pack > 1) {
+      const I lb = e / cells;
+      e -= lb * cells;
+      at = lb * static_cast<I>(G.V) * static_cast<I>(G.cells);
     }
+    const int a = static_cast<int>(e % m), row = static_cast<int>(e / m);
+    const int p = row % across, o = row / across;  // the other two directions, in order
+    const int i = d == 0 ? a - 1 : p, j = d == 0 ? p : d == 1 ? a - 1 : o, k = d == 2 ? a - 1 : o;
+    const O c = O(8) * static_cast<O>(at + (static_cast<I>(G.lo2 + k) * G.e1 + G.lo1 + j) * G.e0 +
+                                      G.lo0 + i);
+    const bool face = a > 0 && e0 < all && (tid & 63) > 0;
+    auto fluxes = [&](auto step) {  // x's step as a constant: it goes into the loads' offsets
+      double upl = 0.0, upr = 0.0;
+      for (int q = na - 1; q < nz; ++q) {
+        const int n = q < na ? d : q;
+        if (q >= na && n == d) continue;  // the normal velocity came first
+        double ql, qr;
+        CellStates(Ub + n * G.cells, c, static_cast<O>(step), RECON, ql, qr);
+        const double l = __shfl_up(ql, 1, 64);
+        if (q < na) {
+          upl = l;
+          upr = qr;
+          if (!own) continue;
+        }
+        if (face) StoreAt(Fb + n * G.cells, c, HllOne(n, upl, upr, l, qr));
+      }
+    };
+    if (d == 0)
+      fluxes(std::integral_constant<O, 8>());
+    else
+      fluxes(st);
     return;
   }
-  const int nd = d == 1 ? n1 : n2, len = S.seg[d];
-  const I cols = static_cast<I>(n0) * (d == 1 ? n2 : n1);
-  const I t = static_cast<I>(r) * kWG + tid;
-  const int f0 = static_cast<int>(t / cols) * len, f1 = f0 + len < nd + 1 ? f0 + len : nd + 1;
+  __shared__ double up[2][kSegFaces][kWG];
+  const int len = S.seg[d];
+  const I cols = static_cast<I>(n0) * (d == 1 ? n2 : n1), all = cols * S.pack;
+  I t = static_cast<I>(r) * kWG + tid, at = 0;
+  const int f0 = static_cast<int>(t / all) * len, f1 = f0 + len < nd + 1 ? f0 + len : nd + 1;
   if (f0 > nd) return;
-  const int o = static_cast<int>(t % cols / n0);
+  t %= all;
+  if (S.pack > 1) {
+    const I lb = t / cols;
+    if (lb >= nb) return;
+    t -= lb * cols;
+    at = lb * static_cast<I>(G.V) * static_cast<I>(G.cells);
+  }
+  const int o = static_cast<int>(t / n0);
   // first face's high cell: face f of the column lies below cell f
-  const O st = O(8) * static_cast<O>(d == 1 ? G.e0 : G.e0 * G.e1);
-  const O c0 = O(8) * static_cast<O>((static_cast<I>(G.lo2 + (d == 1 ? o : f0)) * G.e1 + G.lo1 +
-                                      (d == 1 ? f0 : o)) * G.e0 + G.lo0 + t % cols % n0);
-  for (int q = 0; q <= G.V; ++q) {
-    const int n = q == 0 ? d : q - 1;
-    if (q > 0 && n == d) continue;
+  const O c0 = O(8) * static_cast<O>(at + (static_cast<I>(G.lo2 + (d == 1 ? o : f0)) * G.e1 +
+                                           G.lo1 + (d == 1 ? f0 : o)) * G.e0 + G.lo0 + t % n0);
+  for (int q = na - 1; q < nz; ++q) {
+    const int n = q < na ? d : q;
+    if (q >= na && n == d) continue;
     const double *u = Ub + n * G.cells;
     // window of the cell below the first face
     constexpr int H = RECON == 0 ? 2 : 1;
@@ -139,7 +183,7 @@ __global__ void __launch_bounds__(kWG)
       else
         LinearRecon(w[0], w[1], w[2], ql, qr);
       if (f >= f0) {
-        if (q == 0) {
+        if (q < na) {
           up[0][f - f0][tid] = below;
           up[1][f - f0][tid] = qr;
         }
@@ -663,26 +707,89 @@ int Grid(std::int64_t total) {
 
 }  // namespace
 
+// The split for nb blocks, by rows or by column segments: the one for which these two, squared and
+// added, are least:
+//   * the reconstructions of all wavefronts over the chip's SIMDs, those of y and z rows counted 1.1
+//     times, more on long rows (their loads are strided, and fewer rows meet in a CU's cache);
+//     segments share evenly among the XCDs, which take equal numbers of workgroups in their
+//     order, only if the stripes divide by them or are many;
+//   * 2.2 times the longest chain of a thread, which small meshes end with.
+// Rows win until a mesh fills the chip many times over, and on blocks of up to 32. Measured, segments /
+// rows: 8 blocks of 24^3 with 4 components 44.5 / 26.5 us, 64 blocks of 16^3 with 7 149 / 72, 960
+// 1012 / 1065, 512 of 12^3 392 / 231, one of 128^3 526 / 743. Small meshes take their components in
+// groups (the normal velocity repeated: 8 blocks of 8^3, 7 components 12.7 us in one, 9.8 in four), small
+// blocks share workgroups (1024 blocks of 8^2: 43 us alone, 24 in units of 8).
+static FluxSplit SplitFluxes(const Geo &G, const int n[3], int nb) {
+  constexpr double kSimds = 1024.0, kWaves = kWG / 64, kStripe = 192.0;
+  auto up = [](double a, double b) { return std::ceil(a / b); };
+  FluxSplit best{};
+  double least = 0.0;
+  for (int pack = 1; pack <= 32 && pack <= std::max(nb, 1); pack *= 2) {
+    // a packed unit's offsets are 32-bit
+    if (pack > 1 && pack * G.V * G.cells >= std::int64_t(1) << 29) break;
+    for (bool rows : {false, true}) {
+      FluxSplit S{};
+      S.pack = pack;
+      S.rows = rows;
+      double steps = 0.0, longest = 1.0, wgs = 0.0;
+      for (int d = 0; d < G.ndim; ++d) {
+        const double cols = static_cast<double>(n[d == 0 ? 1 : 0]) * n[d == 2 ? 1 : 2];
+        double w;
+        if (rows || d == 0) {
+          w = up(up((n[d] + 2.0) * cols * pack - 1.0, 63.0), kWaves);
+          steps += w * (d == 0 ? 1.0 : 1.1 + 0.006 * std::max(n[d] - 16, 0));
+        } else {
+          const double segs = up(n[d] + 1.0, kSegFaces);
+          S.seg[d] = static_cast<int>(up(n[d] + 1.0, segs));
+          w = up(cols * segs * pack, kWG);
+          steps += w * (S.seg[d] + 1.0);
+          longest = std::max(longest, S.seg[d] + 1.0);
+        }
+        S.wgs[d] = static_cast<int>(w);
+        wgs += w;
+      }
+      S.stripes = rows ? 1 : std::max(1, static_cast<int>(wgs / kStripe));
+      for (int groups : {1, 2, 4}) {
+        if (groups > G.V || (groups > 1 && !rows)) continue;
+        S.comps = (G.V + groups - 1) / groups;
+        S.chunks = (G.V + S.comps - 1) / S.comps;
+        const double comps = S.comps + (S.chunks > 1), units = up(nb, pack) * S.chunks;
+        const double parts = units * S.stripes;
+        const double uneven = rows ? 1.0 : up(parts, kXcds) * kXcds / parts;
+        const double cost =
+            comps * std::hypot(steps * kWaves * units / kSimds * uneven, 2.2 * longest);
+        // by rows, blocks share workgroups only for a gain: the order suits the caches less (27
+        // blocks of 32^3 228 us alone, 265 in units of 8)
+        if (least > 0.0 && cost >= least * (rows && pack > best.pack ? 0.97 : 1.0)) continue;
+        least = cost;
+        best = S;
+      }
+    }
+  }
+  return best;
+}
+
 pth_status BurgersFluxes(const Topology &t, int V, const double *U, double *flux, int recon,
                          hipStream_t s) {
   ProfScope prof("fluxes", s);
   const Geo G = MakeGeo(t, V);
   const int nb = static_cast<int>(t.blocks.size());
   const int n[3] = {t.fine.n[0], t.fine.n[1], t.fine.n[2]};
-  FluxSplit S{};
-  const std::int64_t waves = (static_cast<std::int64_t>(n[0] + 2) * n[1] * n[2] - 1 + 62) / 63;
-  S.wgs[0] = static_cast<int>((waves + kWG / 64 - 1) / (kWG / 64));
-  for (int d = 1; d < G.ndim; ++d) {
-    const int segs = (n[d] + 1 + kSegFaces - 1) / kSegFaces;
-    S.seg[d] = (n[d] + 1 + segs - 1) / segs;
-    S.wgs[d] = static_cast<int>((static_cast<std::int64_t>(n[0]) * n[3 - d] * segs + kWG - 1) / kWG);
-  }
-  const dim3 grid(static_cast<unsigned>(S.wgs[0] + S.wgs[1] + S.wgs[2]) * nb);
+  const FluxSplit S = SplitFluxes(G, n, nb);
+  const dim3 grid(static_cast<unsigned>(S.wgs[0] + S.wgs[1] + S.wgs[2]) *
+                  static_cast<unsigned>(S.chunks * ((nb + S.pack - 1) / S.pack)));
   const bool wide = G.cells >= std::int64_t(1) << 29;
-  auto *kernel = recon == 0 ? (wide ? FluxTaskKernel<0, true> : FluxTaskKernel<0, false>)
-                            : (wide ? FluxTaskKernel<1, true> : FluxTaskKernel<1, false>);
-  PTH_LAUNCH(kernel, grid, dim3(kWG), 0, s, U, flux, G, nb, S);
-  return PTH_COMPLETE;
+  auto run = [&](auto kernel) -> pth_status {
+    PTH_LAUNCH(kernel, grid, dim3(kWG), 0, s, U, flux, G, nb, S);
+    return PTH_COMPLETE;
+  };
+  auto form = [&](auto rows) -> pth_status {
+    constexpr bool ROWS = decltype(rows)::value;
+    if (recon == 0)
+      return wide ? run(FluxTaskKernel<0, true, ROWS>) : run(FluxTaskKernel<0, false, ROWS>);
+    return wide ? run(FluxTaskKernel<1, true, ROWS>) : run(FluxTaskKernel<1, false, ROWS>);
+  };
+  return S.rows ? form(std::true_type()) : form(std::false_type());
 }
 
 pth_status FluxDivergence(const Topology &t, int V, const double *flux, double *dudt,

@@ -59,3 +59,23 @@ def test_driver_other_blocks_matches_oracle(nx, block, boxes):
         ob.cycles(2)
         assert np.array_equal(d.base.download("U").ravel(), ob.get(0))
     assert d.clock()[0] == ob.dt
+
+
+# the flux kernel's splits: small blocks that share workgroups (the last unit not full), components
+# in groups, 2-D and 1-D; and meshes that it takes by column segments: 2304 blocks of one segment of
+# 9 faces in units of several blocks, large blocks whose last segments are short, in stripes, 2-D
+SPLITS = [
+    ((88, 8, 8), (8, 8, 8), 6, 0),
+    ((40, 40, 40), (10, 10, 10), 1, 1),
+    ((72, 40, 1), (8, 8, 1), 5, 0),
+    ((96, 1, 1), (8, 1, 1), 2, 0),
+    ((128, 96, 96), (8, 8, 8), 1, 0),
+    ((192, 100, 76), (96, 100, 76), 1, 1),
+    ((1024, 1024, 1), (128, 128, 1), 1, 0),
+]
+
+
+@pytest.mark.parametrize("nx,block,ns,recon", SPLITS)
+def test_flux_splits_match_oracle_bit_for_bit(nx, block, ns, recon):
+    print(f"case flux split {nx} {block} scalars {ns} recon {recon}", flush=True)
+    test_fluxes_match_oracle_bit_for_bit(nx, block, ns, recon)
