@@ -9,7 +9,7 @@ from parthenon_amd import gmg
 pytestmark = pytest.mark.gpu
 
 BLOCKS = [(4, 4, 4), (8, 8, 8), (10, 6, 8), (16, 8, 8), (12, 10, 14), (16, 16, 4), (36, 1, 1),
-          (22, 26, 1)]
+          (22, 26, 1), (14, 18, 1), (6, 1, 1)]
 
 
 def mesh(block):
