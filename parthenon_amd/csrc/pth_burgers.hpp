@@ -36,6 +36,8 @@ bool ReconFluxSupported(const Topology &t, int V);
 bool BurgersSweepSupported(const Topology &t, int V);
 // the tile form of the sweep: x and y block sizes in multiples of 16
 bool BurgersTileSweep(const Topology &t, int V);
+// planes of 16 x 16 cells that it has to share out
+std::int64_t BurgersTilePlanes(const Topology &t);
 // whether the sweep has choices to time (register budget, spread): the tile form proper is
 // built once and runs one workgroup a CU
 bool BurgersSweepTuned(const Topology &t, int V);

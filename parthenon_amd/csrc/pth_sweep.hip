@@ -1308,8 +1308,10 @@ __global__ void __launch_bounds__(512, 2)
 }  // namespace
 
 // 16^3 blocks of at most 7 components: one thread per column, of which two workgroups fit a
-// CU's LDS and registers (960 refined blocks with 7 components: 1746 us a cycle, 1928 by the
-// tile form; from 8 on only one fits and the tile form is the faster).
+// CU's LDS and registers; from 8 on only one fits and the tile form is the faster. Cycles by this form
+// and by the tile form, WENO5: 7 components 61 / 69 us on 8 blocks, 86 / 117 on 27, 135 / 144 on 64, 396 /
+// 363 on 216, 729 / 982 on 512, 1723 / 1916 on 960 refined ones; 4 components 46 / 47, 60 / 76, 86 / 95, 215 /
+// 234, 446 / 534, 1013 / 1121. The linear reconstruction gains more (7 components, 64 blocks 83 / 106).
 static bool RingSweep(const Topology &t, int V) {
   const Extent &f = t.fine;
   return f.n[0] == 16 && f.n[1] == 16 && f.n[2] == 16 && V <= 7;
@@ -1322,6 +1324,11 @@ bool BurgersTileSweep(const Topology &t, int V) {
   return t.ndim == 3 && f.n[0] % 16 == 0 && f.n[1] % 16 == 0 && f.n[2] >= 8 && f.g[0] == 4 &&
          f.g[1] == 4 && f.g[2] == 4 && V >= 4 && V <= 13 &&
          f.cells() * V < (std::int64_t(1) << 29);
+}
+
+std::int64_t BurgersTilePlanes(const Topology &t) {
+  const Extent &f = t.fine;
+  return static_cast<std::int64_t>(t.blocks.size()) * (f.n[0] / 16) * (f.n[1] / 16) * f.n[2];
 }
 
 bool BurgersSweepTuned(const Topology &t, int V) {

@@ -71,3 +71,23 @@ def test_bit_exact_choice_excludes_the_tile_sweep():
     d.cycles(2)
     ob.cycles(2)
     assert np.array_equal(d.base.download("U").ravel(), ob.get(0))
+
+
+@pytest.mark.parametrize("nx,block,ns,recon,form", [
+    ((16, 16, 8), (16, 16, 8), 1, 0, "serial"), ((16, 32, 16), (16, 32, 16), 1, 0, "sweep"),
+    ((32, 32, 24), (16, 16, 24), 3, 0, "serial"), ((32, 32, 25), (16, 16, 25), 3, 0, "sweep"),
+    ((16, 16, 8), (16, 16, 8), 10, 1, "sweep")])
+def test_few_planes_take_the_flux_form(nx, block, ns, recon, form):
+    # below 100 planes of 16 x 16 cells (32 with up to 5 components), WENO5
+    print(f"case few planes {nx} {block}", flush=True)
+    ob = OracleBurgers(OracleMesh(nx, block, 4), ns, 0.4, recon)
+    lib().orc_burgers_pgen_sinusoid(ob.h, 6)
+    lib().orc_burgers_initialize(ob.h)
+    d = DeviceBurgersDriver(make_burgers_mesh(nx, block, 4, ns), cfl=0.4, recon=recon)
+    d.initialize("sinusoid", seed=6)
+    assert d.form() == form
+    d.cycles(4)
+    ob.cycles(4)
+    exp = ob.get(0)
+    assert np.max(np.abs(d.base.download("U").ravel() - exp)) <= 1e-13 * np.max(np.abs(exp))
+    assert abs(d.clock()[0] - ob.dt) <= 1e-13 * ob.dt
