@@ -423,9 +423,11 @@ pth_status pth_poisson_ax(pth_meshdata *md, const pth_poisson_equation *eq, cons
  * - every other mesh or equation (static refinement, 1-D / 2-D, periodic faces, a face field
  *   D, diagonal_alpha != 0, or smoother 1-3): a hierarchy of block meshes (the leaf mesh, the
  *   mesh capped at each coarser refinement level, then the forest's merged and cell-halved
- *   levels below the base grid) in FP64 (precision 1 only); each level's ghosts come from
- *   its own boundary exchange with the faces' conditions, restriction is RestrictAverage and
- *   prolongation of the correction ProlongateSharedLinear; a face field D is read at pth_mg_setup and restricted down the
+ *   levels below the base grid) in FP64 (precision 1 only); a stencil reads
+ *   its neighbours in other blocks of the same size in place and a fixed_face ghost as the
+ *   negated cell; only blocks beside coarser or finer ones get ghosts from their level's boundary
+ *   exchange. Restriction is RestrictAverage and prolongation of the correction
+ *   ProlongateSharedLinear; a face field D is read at pth_mg_setup and restricted down the
  *   levels by face averages (D is GMGRestrict in the reference, AddSetupTasks restricts it,
  *   mg_solver.hpp:188-203). u's registered prolongation operator defines the leaf problem's
  *   fine-coarse ghosts (the poisson_gmg package registers ProlongateSharedLinear). */

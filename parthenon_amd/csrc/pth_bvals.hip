@@ -555,7 +555,7 @@ pth_status Table::Upload() {
     }
     const int step = std::min(std::max(item_elems, 1), kItemElems);
     for (std::int64_t b = 0; b < count; b += step)
-      items.push_back(Item{static_cast<int>(q), 1, static_cast<int>(b),
+      items.push_back(Item{static_cast<int>(q), 0, static_cast<int>(b),
                            static_cast<int>(std::min<std::int64_t>(count - b, step))});
     total += count;
   }

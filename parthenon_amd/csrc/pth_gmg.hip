@@ -123,21 +123,7 @@ template <typename T>
 struct Nbrs {
   T u, xm, xp, ym, yp, zm, zp;
 };
-template <typename T>
-__device__ __forceinline__ Nbrs<T> Load(const T *__restrict__ x, int c, const Cell &q, int n) {
-  Nbrs<T> v;
-  const int s1 = n, s2 = n * n;
-  v.u = x[c];
-  v.xm = q.i > 0 ? x[c - 1] : -v.u;
-  v.xp = q.i < n - 1 ? x[c + 1] : -v.u;
-  v.ym = q.j > 0 ? x[c - s1] : -v.u;
-  v.yp = q.j < n - 1 ? x[c + s1] : -v.u;
-  v.zm = q.k > 0 ? x[c - s2] : -v.u;
-  v.zp = q.k < n - 1 ? x[c + s2] : -v.u;
-  return v;
-}
-
-// The same from an array in global memory, every load unconditional: a neighbour outside the
+// Those of an array in global memory, every load unconditional: a neighbour outside the
 // array reads the cell itself and the ghost value -u replaces it afterwards. (gfx9 counts
 // loads and stores on one in-order counter; loads under a per-lane branch make the compiler
 // wait for each before the next.)

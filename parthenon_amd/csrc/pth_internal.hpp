@@ -207,13 +207,12 @@ struct ShellArgs {
   int nblocks;
 };
 
-struct Item {  // a run of consecutive elements over up to kItemRegions consecutive regions
-  int region;    // first region
-  int nreg;      // regions touched
-  int begin;     // element offset within the first region
+struct Item {  // a run of consecutive elements of a region; 16 bytes, one scalar load
+  int region;
+  int pad;
+  int begin;     // element offset within the region
   int count;     // elements
 };
-constexpr int kItemRegions = 8;
 constexpr int kItemElems = 1024;
 // restriction / prolongation items: one thread does a few coarse cells (each with 8 dependent
 // fine loads or stores), so these tables are cut finer to keep enough workgroups in flight

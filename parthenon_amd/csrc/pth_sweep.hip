@@ -878,14 +878,14 @@ __global__ void __launch_bounds__(512, 2)
   constexpr int NX = V * N * 2;    // beyond-the-row states of one direction
   constexpr int NH = V * 12 * N;   // halo cells of one staged plane (all components)
   constexpr int QH = (NH + NT - 1) / NT;  // halo cells per thread
-  // a second staged plane and a y difference tile of its own where the LDS (160 KiB) holds
-  // them; without them a step waits for the readers of the array it reuses
-  constexpr int kFixed = V * PS + 2 * NX + V * N * SP + 6 * N * SP + 4 * V * N + 16;
-  constexpr bool DB = 8 * (kFixed + V * PS) <= 160 * 1024;
-  constexpr bool SY = DB && 8 * (kFixed + V * PS + V * N * SP) <= 160 * 1024;
+  // a y difference tile of its own where the LDS (160 KiB) holds it beside the two staged
+  // planes, up to 11 components; without it the y pass waits for the x differences and adds
+  constexpr int kLds = 2 * V * PS + 2 * NX + V * N * SP + 6 * N * SP + 4 * V * N + 16;
+  static_assert(8 * kLds <= 160 * 1024);
+  constexpr bool SY = 8 * (kLds + V * N * SP) <= 160 * 1024;
   constexpr int gW = 0, mW = 1;  // the z velocity's group and place in it
   constexpr int gD = 1;          // the group of the derived field and CFL
-  __shared__ double pl[(DB ? 2 : 1) * V * PS];  // [plane parity][n][j + H][i + H]
+  __shared__ double pl[2 * V * PS];  // [plane parity][n][j + H][i + H]
   __shared__ double ext[2 * NX];     // [dir][n][line][side]: side 0 ql of cell -1, 1 qr of cell N
   __shared__ double sd[(SY ? 2 : 1) * V * N * SP];  // x (+ y) differences [n][j][i], then the new
                                                     // state; the y differences
@@ -1025,7 +1025,7 @@ __global__ void __launch_bounds__(512, 2)
     // ---- the segment's first plane kk0, staged; the rings
     double hv[QH], r0[NC], r2[NC], r3[NC], r4[NC];
     {
-      double *const to = pl + (DB ? (k0 & 1) * V * PS : 0);
+      double *const to = pl + (k0 & 1) * V * PS;
 #pragma unroll
       for (int q = 0; q < QH; ++q) hv[q] = load(plane(U, 0, kk0), hoff[q]);
       double own_u[NC];
@@ -1111,14 +1111,15 @@ __global__ void __launch_bounds__(512, 2)
       const int tx = tid % N, ty = (tid / N) % N;
       const int own = (ty + H) * PP + tx + H, osd = ty * SP + tx;
       const unsigned col = 8u * static_cast<unsigned>((NG + ty) * e0 + NG + tx);
-      const double *const P = pl + (DB ? (k & 1) * V * PS : 0);
+      const double *const P = pl + (k & 1) * V * PS;
       const double *const crow = P + own;                     // own cell
       const double *const ccol = P + (tx + H) * PP + ty + H;  // cell i = ty, j = tx
       // ---- 1.
       // the next plane into the other buffer first (also past the block's last plane: ghost
       // planes): every load in flight is waited for here, before the stores below, since a
       // later wait would count these too
-      auto stage = [&](double *to) __attribute__((always_inline)) {
+      {
+        double *const to = pl + ((k + 1) & 1) * V * PS;
 #pragma unroll
         for (int m = 0; m < NC; ++m) {
           if (m == NC - 1 && !last) break;
@@ -1126,8 +1127,7 @@ __global__ void __launch_bounds__(512, 2)
         }
 #pragma unroll
         for (int q = 0; q < QH; ++q) to[hloc[q]] = hv[q];
-      };
-      if (DB) stage(pl + ((k + 1) & 1) * V * PS);
+      }
       if (k > k0) finish(k - 1, tx, osd, col);
       if (fixed) corrected(k, tid);
       double vl, vr, wl = 0.0, wr = 0.0;
@@ -1198,10 +1198,8 @@ __global__ void __launch_bounds__(512, 2)
       if (!SY) __syncthreads();  // the x differences are in the tile
       // the loads that the next plane needs (indices in range also past the block's last
       // plane: ghost planes); before the x fluxes they would take registers from them
-      if (DB) {
 #pragma unroll
-        for (int q = 0; q < QH; ++q) hv[q] = load(plane(U, 0, kk + 2), hoff[q]);
-      }
+      for (int q = 0; q < QH; ++q) hv[q] = load(plane(U, 0, kk + 2), hoff[q]);
       double r5[NC];
 #pragma unroll
       for (int m = 0; m < NC; ++m) {
@@ -1262,32 +1260,13 @@ __global__ void __launch_bounds__(512, 2)
           // one component at a time: interleaving the reconstructions needs more registers
           // than the budget holds
           __builtin_amdgcn_sched_barrier(0);
-          if (DB || k + 1 == k1) {  // the ring moves up one plane
-            r0[m] = uo;
-            r2[m] = r3[m];
-            r3[m] = r4[m];
-            r4[m] = r5[m];
-          }
-        }
-      }
-      __syncthreads();
-      if (!DB && k + 1 < k1) {
-#pragma unroll
-        for (int m = 0; m < NC; ++m) {
-          if (m == NC - 1 && !last) break;
-          r0[m] = crow[(G * m + grp) * PS];
-        }
-        stage(pl);
-#pragma unroll
-        for (int q = 0; q < QH; ++q) hv[q] = load(plane(U, 0, kk + 2), hoff[q]);
-#pragma unroll
-        for (int m = 0; m < NC; ++m) {
+          r0[m] = uo;  // the ring moves up one plane
           r2[m] = r3[m];
           r3[m] = r4[m];
           r4[m] = r5[m];
         }
-        __syncthreads();
       }
+      __syncthreads();
     }
     finish(k1 - 1, tx, osd, col);
     __syncthreads();

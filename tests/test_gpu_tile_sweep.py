@@ -1,7 +1,7 @@
 """The tile sweep (x and y block sizes in multiples of 16, any component count that the sweep
 takes) against the oracle: several tiles a block, non-cubic blocks, the smallest z size, every
-LDS layout (two staged planes and a y tile up to 10 components, without the y tile at 11 and 12,
-one plane at 13), same-level copies to other blocks and to the block itself, corrected fluxes
+LDS layout (a y difference tile beside the two staged planes up to 11 components, none at 12 and
+13), same-level copies to other blocks and to the block itself, corrected fluxes
 on refined meshes and physical faces. Bound 1e-13 relative, as for every sweep test."""
 import numpy as np
 import pytest
