@@ -779,8 +779,9 @@ __global__ void __launch_bounds__(F::WG, sizeof(T) == 4 ? 4 : 1) PassKernel(cons
 // level, so a thread keeps the x and b of its cells in registers at every level and LDS only
 // carries a level's x (or its residual) to the neighbours: 1024 threads as 256 columns by 4
 // groups of planes for levels of 5 to 16 cells per side, and one wavefront, which needs no
-// barrier, for those of at most 4. Measured 13.7 us from 16^3 in FP32 (38.7 with a launch-wide
-// loop over cells and a copy per sweep) and 19.6 from 16^3 in FP64, where 8^3 took 27.5.
+// barrier, for those of at most 4. Measured between events 13.7 us from 16^3 in FP32 (38.7 with a
+// launch-wide loop over cells and a copy per sweep) and 19.6 from 16^3 in FP64, where 8^3 took
+// 27.5; the kernels alone, from a trace, 12.1 and 17.6.
 constexpr int kBottomWG = 1024;
 // cells of the levels above l (l = 31: of all)
 __host__ __device__ constexpr int BottomCells(int NB, int l) {

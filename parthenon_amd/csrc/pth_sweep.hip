@@ -847,10 +847,11 @@ __global__ void __launch_bounds__(256, MINW)
 // is read from HBM once per workgroup (plus the halos and the segment's first planes), and face
 // states and fluxes never leave the CU.
 //
-// Bound: FP64 issue, at 54% of it (2 wavefronts per SIMD from one workgroup a CU; the barriers
-// and the memory waits of the staging show). Two groups a tile, since one thread per column
-// with 8 components and more needs over 256 VGPRs: spilled registers cost most here, as each
-// reload waits for every load and store in flight. (Four groups of 128 VGPRs spill and took
+// Bound: FP64 issue, at 59% of it (180 M wave64 instructions in a launch of 495 us, 11
+// components, at 4 cycles each and 2.4 GHz; 2 wavefronts per SIMD from one workgroup a CU; the
+// barriers and the memory waits of the staging show). Two groups a tile, since one thread per
+// column with 8 components and more needs over 256 VGPRs: spilled registers cost most here, as
+// each reload waits for every load and store in flight. (Four groups of 128 VGPRs spill and took
 // 1105 us for the cycle below.) Measured, cycles of 128^3 cells in 32^3 blocks: 980 us with 11
 // components (fluxes, update and exchange as launches of their own: 2365), 653 us with 7
 // (1538); 16^3 blocks with 11 components: 186 us on 64 blocks, 238 by one thread per column.
@@ -1118,8 +1119,9 @@ __global__ void __launch_bounds__(512, 2)
       // the next plane into the other buffer first (also past the block's last plane: ghost
       // planes): every load in flight is waited for here, before the stores below, since a
       // later wait would count these too
-      {
-        double *const to = pl + ((k + 1) & 1) * V * PS;
+      // (as a lambda, which the compiler schedules better: the same lines in place cost 0.7% of
+      // the cycle below)
+      auto stage = [&](double *to) __attribute__((always_inline)) {
 #pragma unroll
         for (int m = 0; m < NC; ++m) {
           if (m == NC - 1 && !last) break;
@@ -1127,7 +1129,8 @@ __global__ void __launch_bounds__(512, 2)
         }
 #pragma unroll
         for (int q = 0; q < QH; ++q) to[hloc[q]] = hv[q];
-      }
+      };
+      stage(pl + ((k + 1) & 1) * V * PS);
       if (k > k0) finish(k - 1, tx, osd, col);
       if (fixed) corrected(k, tid);
       double vl, vr, wl = 0.0, wr = 0.0;
