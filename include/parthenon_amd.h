@@ -474,7 +474,12 @@ pth_status pth_mg_set_graph(pth_mg *mg, int on);
  * HBM (hipMemGetInfo) holds the request's hierarchy plus a reserve (default 1 GiB); a
  * budget_bytes > 0 also caps the bytes the server holds (<= 0: no cap). Pooled hierarchies of
  * other sizes are freed first when memory is short. Every outer iteration runs the same
- * V-cycle stage of all active solves as one launch. */
+ * V-cycle stage of all active solves as one launch.
+ *
+ * keep_solutions: each request's solution is copied to host memory that the server holds until
+ * it is destroyed, in page-locked memory up to 1 GiB of them and in ordinary memory past that
+ * or where page-locked memory is refused. pth_gmg_server_solution shares a copy of 4 MiB and
+ * more among up to eight threads, which end before it returns. */
 typedef struct pth_gmg_server pth_gmg_server;
 pth_gmg_server *pth_gmg_server_create(int precision, double omega, int pre, int post, double tol,
                                       int max_iters, int64_t budget_bytes, int max_active,

@@ -847,7 +847,7 @@ __global__ void __launch_bounds__(256, MINW)
 // is read from HBM once per workgroup (plus the halos and the segment's first planes), and face
 // states and fluxes never leave the CU.
 //
-// Bound: FP64 issue, at 59% of it (180 M wave64 instructions in a launch of 495 us, 11
+// Bound: FP64 issue, at 59% of it (176 M wave64 instructions in a launch of 488 us, 11
 // components, at 4 cycles each and 2.4 GHz; 2 wavefronts per SIMD from one workgroup a CU; the
 // barriers and the memory waits of the staging show). Two groups a tile, since one thread per
 // column with 8 components and more needs over 256 VGPRs: spilled registers cost most here, as
