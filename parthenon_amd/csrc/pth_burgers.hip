@@ -67,14 +67,12 @@ struct FluxSplit {
 //      in a register window, lanes along x; the normal velocity's states wait in LDS, each thread
 //      in its own slots (no barriers).
 // A cell is reconstructed once, but for two cells a row or one a segment or wavefront. The
-// operations are
-// those of the reference in its order, without contraction. Bound: FP64 issue (about 300
-// instructions a reconstruction with its flux, 8 IEEE divides among them). On the 960-block
-// mesh with 7 components the reconstruction and HLL as two launches, with the states in HBM
-// between them, took 1341 + 1043 us; this kernel takes
-// 1070 us. One block of 128^3: 1417 us with the directions one after another, which leaves XCDs
-// with long workgroups alone, 509 in stripes. WIDE: 64-bit cell offsets, for components of 4 GB and more.
-// ROWS: y and z by rows too.
+// operations are those of the reference in its order, without contraction. Bound: FP64 issue
+// (about 300 instructions a reconstruction with its flux, 8 IEEE divides among them). On the
+// 960-block mesh with 7 components the reconstruction and HLL as two launches, with the states in
+// HBM between them, took 1341 + 1043 us; this kernel takes 1070. One block of 128^3: 1417 us with
+// the directions one after another, which leaves XCDs with long workgroups alone, 509 in stripes.
+// WIDE: 64-bit cell offsets, for components of 4 GB and more. ROWS: y and z by rows too.
 template <int RECON, bool WIDE, bool ROWS>
 __global__ void __launch_bounds__(kWG)
     FluxTaskKernel(const double *__restrict__ U, double *__restrict__ flux, Geo G, int nblocks,
@@ -197,8 +195,8 @@ __global__ void __launch_bounds__(kWG)
 }
 
 // FluxDivKernel's workgroups: kChunk consecutive interior cells of one brick (a block's component),
-// kCells a thread, 256 apart. The brick and the chunk's first plane are the
-// workgroup's (scalar), a thread divides 32-bit numbers below a plane's cells. SMALL: bricks of
+// kCells a thread, 256 apart. The brick and the chunk's first plane are the workgroup's (scalar),
+// a thread divides 32-bit numbers below a plane's cells. SMALL: bricks of
 // fewer than kChunk / 4 cells, of which a workgroup takes several, one after another (1024 blocks of
 // 8^2, 7 components: 9.9 us alone, 5.7; 512 of 8^3 20.0 alone, 20.8).
 constexpr int kCells = 4, kChunk = kCells * kWG;
@@ -392,7 +390,8 @@ constexpr int kMaxV = 16;  // components handled by the update kernel
 // each plane the WENO5Z (or linear) states of the plane's cells, extended by one cell along the
 // direction, go to LDS; then the HLL flux of every face of the plane goes to the flux array
 // [3][block][comp][brick] (x-face i at index i). The operations are those of FluxTaskKernel,
-// so the fluxes are the same bits; this form also splits off the faces that read no ghost. PPW (planes per workgroup) changes only the work split and is picked by timing.
+// so the fluxes are the same bits; this form also splits off the faces that read no ghost. PPW
+// (planes per workgroup) changes only the work split and is picked by timing.
 // PART selects the cells and faces of each plane row along the direction (ext index a of the
 // N + 2 cells lo - 1 .. hi + 1; face f between ext cells f and f + 1):
 //   0: every cell and face;

@@ -434,11 +434,11 @@ pth_status TuneForm(Ctx &x, hipStream_t s) {
   const bool flux = x.base->store[x.fu].flux != nullptr;
   const bool planes = flux && ReconFluxSupported(m.topo, x.V);
   // block shapes without plane forms are not timed. The tile sweep takes 0.4 to 1 of the flux
-  // form's time from 100 planes on (32^3 blocks with 7 components: 67 us for 123 on one, 134 for 257 on 8,
-  // 648 for 1612 on 64; 48 x 16 x 12 with 13 on 32 362 for 407; 16 x 32 x 8 with 7 on 8 69 for 69) and with the
-  // linear reconstruction (0.4 to 1.1); on fewer planes, which leave most CUs idle, 1 to 1.6 (one
-  // block of 16 x 16 x 8 with 13 89 for 57, one of 48 x 16 x 12 with 7 57 for 48), with up to 5 components
-  // from 32 planes on 0.9 to 1
+  // form's time from 100 planes on (32^3 blocks with 7 components: 67 us for 123 on one, 134 for
+  // 257 on 8, 648 for 1612 on 64; 48 x 16 x 12 with 13 on 32 362 for 407; 16 x 32 x 8 with 7 on 8
+  // 69 for 69) and with the linear reconstruction (0.4 to 1.1); on fewer planes, which leave most
+  // CUs idle, 1 to 1.6 (one block of 16 x 16 x 8 with 13 89 for 57, one of 48 x 16 x 12 with 7 57
+  // for 48), with up to 5 components from 32 planes on 0.9 to 1
   const bool small = flux && !planes && m.run_recon == 0 && BurgersTileSweep(m.topo, x.V) &&
                      BurgersTilePlanes(m.topo) < (x.V < 6 ? 32 : 100);
   if (BurgersSweepSupported(m.topo, x.V) && !m.form_exact && !small) forms.push_back({1, 0});
